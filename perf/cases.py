@@ -1,0 +1,706 @@
+"""Performance cases: the calls a program built on this package makes, with
+inputs, sizes, work and accuracy of each.
+
+``listed()`` names the cases, ``draw(rng)`` gives more of the same ranges,
+``prepare`` / ``run`` execute one, ``work`` counts what a pass cannot do
+without, ``tolerance`` states how far two correct implementations of the same
+precision are apart and ``exact`` evaluates a case in 64 bits with plain torch.
+
+The model, codec and style-model handles hold seeded random weights of the
+reference architecture (there are no checkpoints here); a process builds each
+once, as a server does, and every state, token and activation comes from the
+case's seed.
+"""
+
+import math
+import pathlib
+import sys
+import zlib
+
+import numpy as np
+import torch
+
+PKG = str(pathlib.Path(__file__).resolve().parents[1] / "magenta-realtime-mlx-cpp_amd")
+if PKG not in sys.path:
+    sys.path.insert(0, PKG)
+
+import mrt_df  # noqa: E402
+
+DEV = "cuda:0"
+LEVELS, CODES, OFFSET = 16, 1024, 2     # RVQ levels per frame, codes per level, first codec id
+CHUNK, CONTEXT = 50, 1006               # frames of a 2 s chunk, encoder ids of the 10 s context + style
+STYLE = 17410                           # first style id
+TOP_K, TEMPERATURE, GUIDANCE = 40, 1.1, 5.0
+TORCH = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}
+BYTES = {"bf16": 2, "fp16": 2, "fp32": 4}
+
+
+# ---------------------------------------------------------------------------
+# The cases
+
+
+def listed():
+    return [
+        # One RVQ level of a host-driven decode loop: the smallest call, all launch and latency.
+        dict(name="depth_step", path="depth_step", model="bench", dtype="bf16", pos=7, level=7),
+        # One frame step of a host-driven loop, mid chunk, on the smaller published configuration in fp16.
+        dict(name="temporal_step", path="temporal_step", model="base", dtype="fp16", pos=24, enc_len=CONTEXT),
+        # A frame's depth pass in one call (scoring, draft verification), full vocabulary.
+        dict(name="depth_full", path="depth_full", model="bench", dtype="bf16", k=LEVELS),
+        # The once-per-chunk prefill of a live stream.
+        dict(name="encode", path="encode", model="bench", dtype="bf16", enc_len=CONTEXT),
+        # The same in fp32, the bundles' own type (--dtype fp32: offline rendering, parity checks).
+        dict(name="encode_fp32", path="encode", model="bench", dtype="fp32", enc_len=CONTEXT),
+        # The headline: prefill and 50 frames x 16 levels of one live stream.
+        dict(name="chunk", path="chunk", model="bench", dtype="bf16", frames=CHUNK, enc_len=CONTEXT),
+        # A server's prefill of 32 streams.
+        dict(name="batch_encode_32", path="batch_encode", model="bench", dtype="bf16", streams=32, enc_len=CONTEXT),
+        # A server's chunk decode of 32 streams.
+        dict(name="batch_decode_32", path="batch_decode", model="bench", dtype="bf16", streams=32, frames=CHUNK,
+             enc_len=CONTEXT),
+        # A few streams with a short context that fills no tile, half a chunk.
+        dict(name="batch_decode_5", path="batch_decode", model="bench", dtype="bf16", streams=5, frames=25,
+             enc_len=517),
+        # Audio of one chunk with its crossfade frame.
+        dict(name="codec_chunk", path="codec", frames=51),
+        # Audio of a fifth of a second (previews, low-latency playback).
+        dict(name="codec_short", path="codec", frames=5),
+        # A text prompt to style ids.
+        dict(name="style", path="style", ids=12),
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return min(hi, max(lo, int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))))
+
+
+def draw(rng):
+    path = rng.choice(["depth_step", "temporal_step", "depth_full", "encode", "encode", "chunk", "batch_encode",
+                       "batch_decode", "batch_decode", "codec", "codec", "style"])
+    if path == "codec":
+        return dict(path=path, frames=_log_int(rng, 1, 51))
+    if path == "style":
+        return dict(path=path, ids=_log_int(rng, 1, 127))
+    model, dtype = rng.choice([("bench", "bf16"), ("bench", "bf16"), ("base", "fp16"), ("bench", "fp32")])
+    enc_len = _log_int(rng, 64, CONTEXT)
+    if path == "depth_step":
+        return dict(path=path, model=model, dtype=dtype, pos=rng.randrange(LEVELS),
+                    level=rng.choice([-1, rng.randrange(LEVELS)]))
+    if path == "temporal_step":
+        return dict(path=path, model=model, dtype=dtype, pos=rng.randrange(CHUNK), enc_len=enc_len)
+    if path == "depth_full":
+        return dict(path=path, model=model, dtype=dtype, k=rng.randrange(1, LEVELS + 1))
+    if path == "encode":
+        return dict(path=path, model=model, dtype=dtype, enc_len=enc_len)
+    if path == "chunk":
+        return dict(path=path, model=model, dtype=dtype, frames=_log_int(rng, 1, CHUNK), enc_len=enc_len)
+    streams = _log_int(rng, 1, 32)  # batched streams are bf16 only
+    if path == "batch_encode":
+        return dict(path=path, model="bench", dtype="bf16", streams=streams, enc_len=enc_len)
+    return dict(path=path, model="bench", dtype="bf16", streams=streams, frames=_log_int(rng, 1, CHUNK),
+                enc_len=enc_len)
+
+
+# ---------------------------------------------------------------------------
+# Weights: seeded, made on the device, in the bundles' layouts
+
+
+def _config(model):
+    return getattr(mrt_df.Config, model)()
+
+
+def _normal(name, shape):
+    g = torch.Generator(device=DEV)
+    g.manual_seed(zlib.crc32(name.encode()))
+    return torch.randn(tuple(shape), generator=g, device=DEV)
+
+
+def _depthformer_shapes(c):
+    D, HD, F = c.d_model, c.num_heads * c.d_kv, c.d_ff
+    out = {"token_embedding.weight": (c.vocab_size, D), "lm_head.weight": (c.vocab_size, D),
+           "encoder_norm.weight": (D,), "decoder_norm.weight": (D,),
+           "temporal_rel_pos.relative_attention_bias.weight": (c.temporal_num_buckets, c.num_heads),
+           "depth_rel_pos.relative_attention_bias.weight": (c.depth_num_buckets, c.num_heads)}
+    stacks = (("encoder", c.num_encoder_layers, [("self_attn", "pre_attn_norm")]),
+              ("temporal", c.num_temporal_layers, [("self_attn", "pre_self_attn_norm"),
+                                                   ("cross_attn", "pre_cross_attn_norm")]),
+              ("depth", c.num_depth_layers, [("self_attn", "pre_self_attn_norm")]))
+    for stack, n, attns in stacks:
+        for i in range(n):
+            p = f"{stack}_layers.{i}."
+            for a, norm in attns:
+                out[p + norm + ".weight"] = (D,)
+                for x in "qkv":
+                    out[f"{p}{a}.{x}_proj.weight"] = (HD, D)
+                out[f"{p}{a}.o_proj.weight"] = (D, HD)
+            out[p + "pre_ffn_norm.weight"] = (D,)
+            out[p + "ffn.wi_0.weight"] = out[p + "ffn.wi_1.weight"] = (F, D)
+            out[p + "ffn.wo.weight"] = (D, F)
+    return out
+
+
+def _depthformer_weight(c, name, shape):
+    w = _normal(name, shape)
+    if name.endswith("norm.weight"):
+        return 1.0 + 0.1 * w
+    if name == "token_embedding.weight":
+        return w
+    if "relative_attention_bias" in name:
+        return 0.2 * w
+    w = w.clamp_(-2.0, 2.0) / math.sqrt(shape[1])
+    return w / math.sqrt(c.d_kv) if name.endswith("q_proj.weight") else w  # the attention scale is in q
+
+
+# (in, out, stride, transposed kernel, kernel) of the codec decoder's blocks
+CODEC_BLOCKS = [(512, 1024, (2, 1), (4, 3)), (512, 256, (2, 2), (4, 4)), (256, 256, (1, 2), (3, 4)),
+                (256, 256, (1, 2), (3, 4)), (256, 128, (1, 3), (3, 6)), (128, 128, (1, 2), (3, 4)),
+                (128, 64, (1, 2), (3, 4))]
+EMB, PROJ, UNFOLD, NFFT, HOP = 256, 2560, 5, 960, 480
+
+
+def _codec_shapes():
+    out = {}
+
+    def conv(n, o, i, kh, kw):
+        out[n + ".weight"], out[n + ".bias"] = (o, i, kh, kw), (o,)
+
+    conv("input_proj.conv1", PROJ, EMB, 1, 1)
+    conv("input_proj.conv2", PROJ, PROJ, 1, 1)
+    conv("input_proj.shortcut", PROJ, EMB, 1, 1)
+    conv("input_conv.conv1", PROJ // UNFOLD, PROJ // UNFOLD, 3, 3)
+    conv("input_conv.conv2", PROJ // UNFOLD, PROJ // UNFOLD, 3, 3)
+    for i, (ci, co, _, kt) in enumerate(CODEC_BLOCKS):
+        p = f"decoder_blocks.{i}"
+        out[p + ".conv_transpose.weight"], out[p + ".conv_transpose.bias"] = (ci, co) + kt, (co,)
+        conv(p + ".conv", co, co, 3, 3)
+        if ci != co:
+            conv(p + ".shortcut", co, ci, 1, 1)
+    conv("output_conv", 2, CODEC_BLOCKS[-1][1], 7, 7)
+    out["codebooks"] = (LEVELS, CODES, EMB)
+    return out
+
+
+def _codec_weight(name, shape):
+    w = _normal("codec." + name, shape)
+    if name == "codebooks":
+        return 0.25 * w
+    if name.endswith(".bias"):
+        return 0.02 * w
+    return w / math.sqrt((shape[0] if ".conv_transpose." in name else shape[1]) * shape[2] * shape[3])
+
+
+def _style_shapes():
+    c = mrt_df.CocaConfig()
+    D, F, HD, PD = c.d_model, c.d_ff, c.num_heads * c.d_head, c.num_heads * c.pooler_d_head
+    out = {"token_embedding.weight": (c.vocab_size, D)}
+
+    def lin(n, o, i):
+        out[n + ".weight"], out[n + ".bias"] = (o, i), (o,)
+
+    def attn(n, width):
+        for x in "qkv":
+            lin(f"{n}.{x}_proj", width, D)
+        lin(n + ".o_proj", D, width)
+
+    def ln(n):
+        out[n + ".weight"], out[n + ".bias"] = (D,), (D,)
+
+    for i in range(c.num_layers):
+        p = f"text_layers.{i}"
+        ln(p + ".attn_ln")
+        attn(p + ".attn", HD)
+        ln(p + ".ffn_ln")
+        lin(p + ".ffn_w1", F, D)
+        lin(p + ".ffn_w2", D, F)
+    ln("text_exit_ln")
+    ln("text_pooler.ln")
+    attn("text_pooler.attn", PD)
+    out["text_pooler.query"] = (1, 1, D)
+    out["text_pooler.attn._per_dim_scale"] = (c.pooler_d_head,)
+    out["codebooks"] = (c.rvq_depth, c.codebook_size, D)
+    return out
+
+
+def _style_weight(name, shape):
+    w = _normal("style." + name, shape)
+    if name == "token_embedding.weight":
+        return w / math.sqrt(shape[1])
+    if name.endswith("ln.weight"):
+        return 1.0 + 0.1 * w
+    if name.endswith(".bias"):
+        return 0.02 * w
+    if name == "codebooks":
+        return 0.05 * w
+    if name.endswith("_per_dim_scale"):
+        return 0.1 * w
+    return w / math.sqrt(shape[1]) if len(shape) == 2 else w
+
+
+_handles = {}
+
+
+def _handle(kind, model=None, dtype=None):
+    """The process's model, codec or style model (built once)."""
+    key = (kind, model, dtype)
+    if key not in _handles:
+        if kind == "depthformer":
+            c = _config(model)
+            w = {n: _depthformer_weight(c, n, s).cpu().numpy() for n, s in _depthformer_shapes(c).items()}
+            _handles[key] = mrt_df.Depthformer(w, c, dtype=dtype)
+        elif kind == "codec":
+            w = {n: _codec_weight(n, s).cpu().numpy() for n, s in _codec_shapes().items()}
+            _handles[key] = mrt_df.Codec(w, max_frames=51)
+        else:
+            w = {n: _style_weight(n, s).cpu().numpy() for n, s in _style_shapes().items()}
+            _handles[key] = mrt_df.StyleModel(w)
+    return _handles[key]
+
+
+# ---------------------------------------------------------------------------
+# Inputs
+
+
+def _context(rng, streams, enc_len):
+    """Encoder ids of CFG pairs: context codes of the first 4 levels, then 6
+    style ids (masked in the unconditional row), as the streaming session
+    builds them; short contexts keep the tail."""
+    n = CONTEXT - 6
+    codes = OFFSET + CODES * (np.arange(n) % 4) + rng.integers(0, CODES, (streams, n))
+    style = STYLE + CODES * np.arange(6) + rng.integers(0, CODES, (streams, 6))
+    ids = np.ones((streams, 2, CONTEXT), np.int32)
+    ids[:, :, :n] = codes[:, None]
+    ids[:, 0, n:] = style
+    return np.ascontiguousarray(ids.reshape(2 * streams, CONTEXT)[:, CONTEXT - enc_len:])
+
+
+def _inputs(case, seed):
+    """Every input array of a case, from the seed alone (host)."""
+    rng = np.random.default_rng([seed, zlib.crc32(case["path"].encode())])
+    path = case["path"]
+    if path == "codec":
+        return {"codes": rng.integers(0, CODES, (case["frames"], LEVELS)).astype(np.int32)}
+    if path == "style":
+        c = mrt_df.CocaConfig()
+        ids, pad = np.zeros(c.max_text_len, np.int32), np.ones(c.max_text_len, np.float32)
+        ids[0] = 1
+        ids[1:case["ids"] + 1] = rng.integers(3, c.vocab_size, case["ids"])
+        pad[:case["ids"] + 1] = 0
+        return {"ids": ids, "padding": pad}
+    D = _config(case["model"]).d_model
+    if path == "depth_step":  # a temporal output, then the embeddings of fed tokens on both rows
+        first = rng.standard_normal((1, 2, D), dtype=np.float32)
+        fed = rng.standard_normal((case["pos"], 1, D), dtype=np.float32).repeat(2, 1)
+        return {"embs": np.concatenate([first, fed])}
+    if path == "depth_full":
+        first = rng.standard_normal((2, 1, D), dtype=np.float32)
+        fed = rng.standard_normal((1, case["k"] - 1, D), dtype=np.float32).repeat(2, 0)
+        return {"embs": np.concatenate([first, fed], 1)}
+    streams = case.get("streams", 1)
+    out = {"context": _context(rng, streams, case["enc_len"])}
+    if path == "temporal_step":  # means of 16 token embeddings
+        out["embs"] = (0.25 * rng.standard_normal((case["pos"] + 1, 1, D), dtype=np.float32)).repeat(2, 1)
+    if path in ("chunk", "batch_decode"):
+        out["teacher"] = (OFFSET + CODES * np.arange(LEVELS) +
+                          rng.integers(0, CODES, (streams, case["frames"], LEVELS))).astype(np.int32)
+    return out
+
+
+def _options(frames, seed):
+    return mrt_df.GenOptions(num_frames=frames, rvq_depth=LEVELS, temperature=TEMPERATURE, top_k=TOP_K,
+                             guidance_weight=GUIDANCE, seed=seed, codebook_size=CODES, codec_offset=OFFSET)
+
+
+def prepare(case, seed):
+    path = case["path"]
+    s = {"case": case, **_inputs(case, seed)}
+    if path == "codec":
+        s["codec"] = _handle("codec")
+        return s
+    if path == "style":
+        s["model"] = _handle("style")
+        return s
+    dtype = case["dtype"]
+    m = s["model"] = _handle("depthformer", case["model"], dtype)
+    D = m.config.d_model
+    if "embs" in s:
+        s["embs"] = torch.from_numpy(s["embs"]).to(DEV).to(TORCH[dtype])
+    if path == "depth_step":
+        st = s["state"] = m.new_state()
+        s["level"] = None if case["level"] < 0 else case["level"]
+        s["out"] = torch.empty((2, CODES if case["level"] >= 0 else m.config.vocab_size), device=DEV)
+        for i in range(case["pos"]):
+            st.depth_step(s["embs"][i], i, level=0)
+    elif path == "depth_full":
+        s["state"] = m.new_state()
+    elif path == "temporal_step":
+        st = s["state"] = m.new_state(max_frames=CHUNK, enc_len=case["enc_len"])
+        s["out"] = torch.empty((2, D), dtype=TORCH[dtype], device=DEV)
+        st.encode(s["context"])
+        for i in range(case["pos"]):
+            st.temporal_step(s["embs"][i], i)
+    elif path == "encode":
+        s["state"] = m.new_state(enc_len=case["enc_len"])
+    elif path == "chunk":
+        s["state"] = m.new_state(max_frames=case["frames"], enc_len=case["enc_len"])
+        s["opts"] = _options(case["frames"], seed)
+        s["record"] = {"slices": torch.empty((case["frames"], LEVELS, 2, CODES), device=DEV),
+                       "temporal": torch.empty((case["frames"], 2, D), dtype=TORCH[dtype], device=DEV),
+                       "drawn": torch.empty((case["frames"], LEVELS), dtype=torch.int32, device=DEV)}
+    else:
+        B = case["streams"]
+        b = s["batch"] = mrt_df.Batch(m, B, max_frames=case.get("frames", 1), enc_len=case["enc_len"])
+        if path == "batch_decode":
+            b.encode(s["context"])
+            s["opts"] = _options(case["frames"], seed)
+            s["seeds"] = [seed + i for i in range(B)]
+            s["record"] = {"slices": torch.empty((case["frames"], LEVELS, 2 * B, CODES), device=DEV),
+                           "temporal": torch.empty((case["frames"], 2 * B, D), dtype=TORCH[dtype], device=DEV)}
+    return s
+
+
+def run(s):
+    case = s["case"]
+    path = case["path"]
+    if path == "codec":
+        return s["codec"].decode(s["codes"])
+    if path == "style":
+        emb = s["model"].embed_text(s["ids"], s["padding"])
+        return {"embedding": emb, "tokens": s["model"].tokenize()}
+    if path == "depth_step":
+        s["state"].set_cache_length(1, case["pos"])  # the step before this one, again
+        return s["state"].depth_step(s["embs"][-1], case["pos"], level=s["level"], out=s["out"], sync=False)
+    if path == "temporal_step":
+        s["state"].set_cache_length(0, case["pos"])
+        return s["state"].temporal_step(s["embs"][-1], case["pos"], out=s["out"], sync=False)
+    if path == "depth_full":
+        return s["state"].depth_forward_full(s["embs"])
+    if path == "encode":
+        st, last = s["state"], s["model"].config.num_temporal_layers - 1
+        st.encode(s["context"])
+        return {"out": st.read(mrt_df.BUF_ENC_OUT), "k": st.read(mrt_df.BUF_CROSS_K, last),
+                "v": st.read(mrt_df.BUF_CROSS_V, last)}
+    if path == "chunk":
+        tokens = s["state"].generate_tokens(s["context"], s["opts"], teacher=s["teacher"][0], record=s["record"])
+        return {"tokens": tokens, **s["record"]}
+    if path == "batch_encode":
+        s["batch"].encode(s["context"])
+        return s["batch"].read_enc_out()
+    tokens = s["batch"].generate_tokens(None, s["opts"], s["seeds"], teacher=s["teacher"], record=s["record"])
+    return {"tokens": tokens, **s["record"]}
+
+
+# ---------------------------------------------------------------------------
+# Work and accuracy
+
+
+def _encoder_work(c, e, rows, S):
+    D, HD, F, M = c.d_model, c.num_heads * c.d_kv, c.d_ff, rows * S
+    layer, cross = 4 * D * HD + 3 * D * F, 2 * D * HD * c.num_temporal_layers
+    flops = 2.0 * M * (c.num_encoder_layers * layer + cross) + c.num_encoder_layers * 4.0 * rows * S * S * HD
+    return {"bytes": e * (c.num_encoder_layers * layer + cross + M * (D + 2 * HD * c.num_temporal_layers)),
+            "flops": flops}
+
+
+def _temporal_work(c, e, rows, S, pos):
+    """One temporal step: every weight, the rows' cross K/V and their history."""
+    D, HD, n = c.d_model, c.num_heads * c.d_kv, c.num_temporal_layers
+    w = n * (6 * D * HD + 3 * D * c.d_ff)
+    kv = n * rows * 2 * HD * (S + pos + 1)
+    return {"bytes": e * (w + kv + 2 * rows * D), "flops": 2.0 * rows * w + 2.0 * kv}
+
+
+def _depth_work(c, e, rows, pos, head):
+    D, HD, n = c.d_model, c.num_heads * c.d_kv, c.num_depth_layers
+    w = n * (4 * D * HD + 3 * D * c.d_ff) + head * D
+    kv = n * rows * 2 * HD * (pos + 1)
+    return {"bytes": e * (w + kv + rows * D) + 4 * rows * head, "flops": 2.0 * rows * w + 2.0 * kv}
+
+
+def _sum(works):
+    works = list(works)
+    return {k: sum(w[k] for w in works) for k in ("bytes", "flops")}
+
+
+def _codec_flops(frames):
+    H, W, C = frames + 1, UNFOLD, PROJ // UNFOLD
+    fl = 2.0 * H * (2 * EMB * PROJ + PROJ * PROJ) + 2.0 * 2 * H * W * 9 * C * C
+    n = 1
+    for i, (ci, co, (sh, sw), (kh, kw)) in enumerate(CODEC_BLOCKS):
+        n = 1 if i == 0 else 2
+        fl += 2.0 * n * H * W * ci * co * (kh * kw + (ci != co))  # the 1 x 1 shortcut on the input grid
+        H, W = H * sh, W * sw
+        fl += 2.0 * n * H * W * 9 * co * co
+    H -= 4
+    return fl + 2.0 * n * H * W * 49 * CODEC_BLOCKS[-1][1] * 2 + 2.0 * 2 * H * NFFT * NFFT
+
+
+def work(case):
+    path = case["path"]
+    if path == "codec":
+        shapes = _codec_shapes()
+        n = sum(math.prod(s) for k, s in shapes.items() if k != "codebooks")
+        f = case["frames"]
+        return {"bytes": 4.0 * (n + f * LEVELS * (EMB + 1) + f * 1920 * 2), "flops": _codec_flops(f)}
+    if path == "style":
+        c = mrt_df.CocaConfig()
+        n = sum(math.prod(s) for k, s in _style_shapes().items() if k != "token_embedding.weight")
+        L, D, HD, PD = c.max_text_len, c.d_model, c.num_heads * c.d_head, c.num_heads * c.pooler_d_head
+        fl = c.num_layers * (2.0 * L * (4 * D * HD + 2 * D * c.d_ff) + 4.0 * L * L * HD)
+        fl += 2.0 * (2 * D * PD + 2 * L * D * PD) + 4.0 * L * PD + 2.0 * c.rvq_depth * c.codebook_size * D
+        return {"bytes": 4.0 * (n + L * D), "flops": fl}
+    c, e = _config(case["model"]), BYTES[case["dtype"]]
+    if path == "depth_step":
+        return _depth_work(c, e, 2, case["pos"], CODES if case["level"] >= 0 else c.vocab_size)
+    if path == "temporal_step":
+        return _temporal_work(c, e, 2, case["enc_len"], case["pos"])
+    if path == "depth_full":
+        k, HD = case["k"], c.num_heads * c.d_kv
+        w = _depth_work(c, e, 2, k - 1, c.vocab_size)
+        return {"bytes": w["bytes"] + (k - 1) * 2 * (e * c.d_model + 4 * c.vocab_size),
+                "flops": k * w["flops"] - c.num_depth_layers * 4.0 * 2 * HD * k * (k - 1) / 2}
+    rows = 2 * case.get("streams", 1)
+    if path in ("encode", "batch_encode"):
+        return _encoder_work(c, e, rows, case["enc_len"])
+    frame = [_depth_work(c, e, rows, l, CODES) for l in range(LEVELS)]
+    total = _sum([_temporal_work(c, e, rows, case["enc_len"], f) for f in range(case["frames"])] +
+                 frame * case["frames"])
+    return _sum([total, _encoder_work(c, e, rows, case["enc_len"])]) if path == "chunk" else total
+
+
+def tolerance(case):
+    """Four times the distance from 64 bits that the paths show (16-bit types
+    round every layer's outputs; fp32 paths differ by the order of sums).  A
+    drawn token follows its logits' rounding: 16-bit evaluations of a chunk
+    pick another of the 40 candidates in about a tenth of the draws."""
+    path = case["path"]
+    if path in ("codec", "style"):
+        return {"rel": 1e-5, "differ": 0.1}
+    rel = {"bf16": 6e-2, "fp16": 8e-3, "fp32": 2e-5}[case["dtype"]]
+    if path == "chunk":
+        return {"rel": rel, "differ": 0.25 if case["dtype"] != "fp32" else 0.02}
+    return {"rel": rel}
+
+
+# ---------------------------------------------------------------------------
+# The same in 64 bits
+
+_exact_weights = {}
+
+
+def _depthformer64(case):
+    """Weights rounded to the model's type, as float64 on demand."""
+    key = (case["model"], case["dtype"])
+    c, t = _config(case["model"]), TORCH[case["dtype"]]
+    if key not in _exact_weights:
+        _exact_weights.clear()
+        _exact_weights[key] = {n: _depthformer_weight(c, n, s).to(t) for n, s in _depthformer_shapes(c).items()}
+    w = _exact_weights[key]
+    return c, lambda name: w[name + ".weight"].double()
+
+
+def _rms(x, g):
+    return x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6) * g
+
+
+def _ffn(w, p, x):
+    a, b = x @ w(p + "wi_0").T, x @ w(p + "wi_1").T
+    gelu = 0.5 * a * (1.0 + torch.tanh(0.7978845608028654 * (a + 0.044715 * a ** 3)))
+    return (gelu * b) @ w(p + "wo").T
+
+
+def _heads(x, H):
+    return x.unflatten(-1, (H, -1)).transpose(-2, -3).contiguous()
+
+
+def _attend(q, k, v, bias=None):
+    """q (..., H, T, d), k / v (..., H, S, d), no scale; one leading row at a time to bound the memory."""
+    out = torch.empty_like(q)
+    for i in range(q.shape[0]):
+        s = q[i] @ k[i].transpose(-1, -2).contiguous()
+        out[i] = torch.softmax(s if bias is None else s + bias, -1) @ v[i]
+    return out.transpose(-2, -3).flatten(-2)
+
+
+def _sinusoid(n, D, dtype):
+    half = D // 2
+    f = torch.exp(torch.arange(half, dtype=torch.float64, device=DEV) * (-math.log(10000.0) / (half - 1)))
+    a = torch.arange(n, dtype=torch.float64, device=DEV)[:, None] * f
+    return torch.cat([a.sin(), a.cos()], -1).to(dtype).double()
+
+
+def _bias(w, c, stack, n):
+    """(H, n, n) causal relative-position bias of a decoder stack."""
+    nb, md = (c.temporal_num_buckets, c.temporal_max_distance) if stack == "temporal" else \
+        (c.depth_num_buckets, c.depth_max_distance)
+    dist = torch.arange(n, device=DEV)[:, None] - torch.arange(n, device=DEV)[None, :]
+    d = dist.clamp(min=0)
+    exact = nb // 2
+    far = exact + (torch.log(d.clamp(min=1).float() / exact) / math.log(md / exact) * (nb - exact))
+    bucket = torch.where(d < exact, d, far.int().clamp(max=nb - 1).long())
+    bias = w(stack + "_rel_pos.relative_attention_bias")[bucket].permute(2, 0, 1)
+    return bias.masked_fill(dist[None] < 0, -math.inf)
+
+
+def _encoder64(c, w, ids, dtype):
+    ids = torch.from_numpy(ids).to(DEV).long()
+    H = c.num_heads
+    x = w("token_embedding")[ids] + _sinusoid(ids.shape[1], c.d_model, TORCH[dtype])
+    for i in range(c.num_encoder_layers):
+        p = f"encoder_layers.{i}."
+        h = _rms(x, w(p + "pre_attn_norm"))
+        q, k, v = (_heads(h @ w(f"{p}self_attn.{n}_proj").T, H) for n in "qkv")
+        x = x + _attend(q, k, v) @ w(p + "self_attn.o_proj").T
+        x = x + _ffn(w, p + "ffn.", _rms(x, w(p + "pre_ffn_norm")))
+    return _rms(x, w("encoder_norm"))
+
+
+def _decoder64(c, w, stack, x, enc=None):
+    """Causal pass over x (rows, T, D); enc (rows, S, D) for the temporal stack."""
+    H, bias = c.num_heads, _bias(w, c, stack, x.shape[1])
+    for i in range(c.num_temporal_layers if stack == "temporal" else c.num_depth_layers):
+        p = f"{stack}_layers.{i}."
+        h = _rms(x, w(p + "pre_self_attn_norm"))
+        q, k, v = (_heads(h @ w(f"{p}self_attn.{n}_proj").T, H) for n in "qkv")
+        if x.shape[0] > 64:  # many short frames: all at once
+            a = (torch.softmax(q @ k.transpose(-1, -2).contiguous() + bias, -1) @ v).transpose(-2, -3).flatten(-2)
+        else:
+            a = _attend(q, k, v, bias)
+        x = x + a @ w(p + "self_attn.o_proj").T
+        if enc is not None:
+            q = _heads(_rms(x, w(p + "pre_cross_attn_norm")) @ w(p + "cross_attn.q_proj").T, H)
+            k, v = (_heads(enc @ w(f"{p}cross_attn.{n}_proj").T, H) for n in "kv")
+            x = x + _attend(q, k, v) @ w(p + "cross_attn.o_proj").T
+        x = x + _ffn(w, p + "ffn.", _rms(x, w(p + "pre_ffn_norm")))
+    return x
+
+
+def _chunk64(c, w, enc, teacher):
+    """Teacher-forced temporal outputs and level slices: (F, rows, D), (F, L, rows, codes)."""
+    B, F, L = teacher.shape
+    ids = torch.from_numpy(teacher).to(DEV).long()
+    emb = w("token_embedding")
+    fed = emb[ids]                                                     # (B, F, L, D)
+    x = torch.cat([emb[0].expand(B, 1, -1), fed.mean(2)[:, :-1]], 1)   # frame 0: PAD, then the frame means
+    t = _decoder64(c, w, "temporal", x.repeat_interleave(2, 0), enc)   # (2B, F, D)
+    head, slices = w("lm_head"), torch.empty((F, L, 2 * B, CODES), dtype=torch.float64, device=DEV)
+    for b in range(B):
+        rows = torch.stack([t[2 * b], t[2 * b + 1]], 1)                # (F, 2, D)
+        d = torch.cat([rows[:, :, None], fed[b, :, None, :-1].expand(F, 2, L - 1, -1)], 2).flatten(0, 1)
+        d = _rms(_decoder64(c, w, "depth", d), w("decoder_norm")).unflatten(0, (F, 2))
+        for l in range(L):
+            lo = OFFSET + CODES * l
+            slices[:, l, 2 * b:2 * b + 2] = d[:, :, l] @ head[lo:lo + CODES].T
+    return t.transpose(0, 1).contiguous(), slices
+
+
+def _conv64(x, wt, b, top, left, right):
+    """Stride-1 cross-correlation, x (n, H, W, C), zero padding at the top and sides."""
+    x = torch.nn.functional.pad(x, (0, 0, left, right, top, 0))
+    O, _, kh, kw = wt.shape
+    H, W = x.shape[1] - kh + 1, x.shape[2] - kw + 1
+    y = b.expand(x.shape[0], H, W, O).clone()
+    for i in range(kh):
+        for j in range(kw):
+            y += x[:, i:i + H, j:j + W].reshape(-1, x.shape[3]).mm(wt[:, :, i, j].T).view(y.shape)
+    return y
+
+
+def _codec64(codes):
+    if "codec" not in _exact_weights:
+        _exact_weights.clear()
+        _exact_weights["codec"] = {n: _codec_weight(n, s).double() for n, s in _codec_shapes().items()}
+    w = _exact_weights["codec"]
+    elu = torch.nn.functional.elu
+
+    def conv(n, x, top=0, left=0, right=0):
+        return _conv64(x, w[n + ".weight"], w[n + ".bias"], top, left, right)
+
+    ids = torch.from_numpy(codes).to(DEV).long()
+    x = sum(w["codebooks"][l][ids[:, l]] for l in range(LEVELS))
+    x = torch.cat([x, x.new_zeros(1, EMB)])[None, :, None]
+    x = conv("input_proj.conv2", elu(conv("input_proj.conv1", x))) + conv("input_proj.shortcut", x)
+    x = x.reshape(1, x.shape[1], UNFOLD, PROJ // UNFOLD)
+    x = x + conv("input_conv.conv2", elu(conv("input_conv.conv1", elu(x), 2, 1, 1)), 2, 1, 1)
+    for i, (ci, co, (sh, sw), (kh, kw)) in enumerate(CODEC_BLOCKS):
+        p = f"decoder_blocks.{i}"
+        n, H, W, _ = x.shape
+        wt = w[p + ".conv_transpose.weight"]
+        y = x.new_zeros(n, (H - 1) * sh + kh, (W - 1) * sw + kw, co)
+        for a in range(kh):
+            for b in range(kw):
+                y[:, a:a + sh * (H - 1) + 1:sh, b:b + sw * (W - 1) + 1:sw] += \
+                    elu(x).reshape(-1, ci).mm(wt[:, :, a, b]).view(n, H, W, co)
+        cut = (kw - sw) // 2
+        y = elu((y + w[p + ".conv_transpose.bias"])[:, :H * sh, cut:cut + W * sw])
+        r = conv(p + ".shortcut", x) if ci != co else x
+        x = conv(p + ".conv", y, 2, 1, 1) + r.repeat_interleave(sh, 1).repeat_interleave(sw, 2)
+        if i == 0:
+            x = torch.cat(x.split(co // 2, -1))  # stereo halves
+    x = conv("output_conv", elu(x), 6, 3, 3)[:, 4:]
+    win = torch.hann_window(NFFT, periodic=True, dtype=torch.float64, device=DEV)
+    syn = win / (win.square().view(2, HOP).sum(0).repeat(2))
+    f = torch.fft.irfft(torch.nn.functional.pad(torch.complex(x[..., 0], x[..., 1]), (0, 1)), n=NFFT) * syn
+    audio = f[:, :, :HOP].clone()
+    audio[:, 1:] += f[:, :-1, HOP:]
+    audio = torch.cat([audio.flatten(1), f[:, -1, HOP:]], -1)
+    return audio[:, :codes.shape[0] * 1920].T
+
+
+def _style64(ids, padding):
+    if "style" not in _exact_weights:
+        _exact_weights.clear()
+        _exact_weights["style"] = {n: _style_weight(n, s) for n, s in _style_shapes().items()}
+    ws, c = _exact_weights["style"], mrt_df.CocaConfig()
+
+    def lin(n, x):
+        return x @ ws[n + ".weight"].double().T + ws[n + ".bias"].double()
+
+    def ln(n, x):
+        return torch.nn.functional.layer_norm(x, (c.d_model,), ws[n + ".weight"].double(), ws[n + ".bias"].double())
+
+    def attn(p, xq, x, scale=None, cap=0.0, mask=None):
+        q, k, v = lin(p + ".q_proj", xq), lin(p + ".k_proj", x), lin(p + ".v_proj", x)
+        q, k, v = (_heads(t, c.num_heads) for t in (q, k, v))
+        s = (q if scale is None else q * scale) @ k.transpose(-1, -2).contiguous() / math.sqrt(q.shape[-1])
+        s = cap * torch.tanh(s / cap) if cap else s
+        s = s if mask is None else s + mask
+        return lin(p + ".o_proj", (torch.softmax(s, -1) @ v).transpose(-2, -3).flatten(-2))
+
+    x = ws["token_embedding.weight"][torch.from_numpy(ids).to(DEV).long()].double() * math.sqrt(c.d_model)
+    mask = torch.from_numpy(padding).to(DEV).double() * -1e9
+    for i in range(c.num_layers):
+        p = f"text_layers.{i}"
+        h = ln(p + ".attn_ln", x)
+        x = x + attn(p + ".attn", h, h, cap=50.0, mask=mask)
+        x = x + lin(p + ".ffn_w2", torch.nn.functional.gelu(lin(p + ".ffn_w1", ln(p + ".ffn_ln", x))))
+    n = ln("text_pooler.ln", ln("text_exit_ln", x))
+    scale = torch.nn.functional.softplus(ws["text_pooler.attn._per_dim_scale"].double()) / math.log(2.0)
+    return attn("text_pooler.attn", ws["text_pooler.query"].double().view(1, -1), n, scale)[0]
+
+
+def exact(case, seed):
+    path, s = case["path"], _inputs(case, seed)
+    if path == "codec":
+        return _codec64(s["codes"])
+    if path == "style":
+        return {"embedding": _style64(s["ids"], s["padding"]), "tokens": None}
+    c, w = _depthformer64(case)
+    if "embs" in s:
+        embs = torch.from_numpy(s["embs"]).to(DEV).to(TORCH[case["dtype"]]).double()
+    if path == "depth_step":
+        x = _rms(_decoder64(c, w, "depth", embs.transpose(0, 1))[:, -1], w("decoder_norm"))
+        head = w("lm_head")
+        return x @ (head if case["level"] < 0 else head[OFFSET + CODES * case["level"]:][:CODES]).T
+    if path == "depth_full":
+        return _rms(_decoder64(c, w, "depth", embs), w("decoder_norm")) @ w("lm_head").T
+    enc = _encoder64(c, w, s["context"], case["dtype"])
+    if path == "batch_encode":
+        return enc
+    if path == "encode":
+        p, H = f"temporal_layers.{c.num_temporal_layers - 1}.cross_attn.", c.num_heads
+        return {"out": enc, "k": _heads(enc @ w(p + "k_proj").T, H), "v": _heads(enc @ w(p + "v_proj").T, H)}
+    if path == "temporal_step":
+        return _decoder64(c, w, "temporal", embs.transpose(0, 1), enc)[:, -1]
+    t, slices = _chunk64(c, w, enc, s["teacher"])
+    out = {"tokens": None, "slices": slices, "temporal": t}
+    return {**out, "drawn": None} if path == "chunk" else out
