@@ -470,14 +470,15 @@ def work(case):
 def tolerance(case):
     """Four times the distance from 64 bits that the paths show (16-bit types
     round every layer's outputs; fp32 paths differ by the order of sums).  A
-    drawn token follows its logits' rounding: 16-bit evaluations of a chunk
-    pick another of the 40 candidates in about a tenth of the draws."""
+    drawn token follows its logits' rounding: two evaluations of a chunk pick
+    another of the 40 candidates in 15 % (bf16), 2 % (fp16) and none (fp32) of
+    the draws; a one-frame chunk has 16 of them."""
     path = case["path"]
     if path in ("codec", "style"):
         return {"rel": 1e-5, "differ": 0.1}
     rel = {"bf16": 6e-2, "fp16": 8e-3, "fp32": 2e-5}[case["dtype"]]
     if path == "chunk":
-        return {"rel": rel, "differ": 0.25 if case["dtype"] != "fp32" else 0.02}
+        return {"rel": rel, "differ": {"bf16": 0.5, "fp16": 0.2, "fp32": 0.02}[case["dtype"]]}
     return {"rel": rel}
 
 
