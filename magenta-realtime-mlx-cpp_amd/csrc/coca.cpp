@@ -158,6 +158,7 @@ Coca::Coca(const TensorSource& w, const TensorSource& cbs, const CocaConfig& c, 
   patt_ = dalloc(PD);
   emb_ = dalloc(D);
   res_ = dalloc(D);
+  rvq_work_ = dalloc(2 * (D + c.codebook));
   for (int i = 0; i < c.num_layers; ++i) layer_out_.push_back(dalloc(static_cast<size_t>(L) * D));
 
   // the GEMM plan of one prompt (fixed: the prompt is always max_text_len rows)
@@ -324,7 +325,7 @@ void Coca::tokenize(const float* emb, int32_t* tokens) {
   MRT_REQUIRE(tokens, "musiccoca: null tokens");
   MRT_HIP_CHECK(hipSetDevice(device));
   if (emb) MRT_HIP_CHECK(hipMemcpyAsync(emb_, emb, c.d_model * 4, hipMemcpyHostToDevice, stream));
-  rvq_quantize(emb_, codebooks_, c.rvq_depth, c.codebook, c.d_model, res_, tok_, stream);
+  rvq_quantize(emb_, codebooks_, c.rvq_depth, c.codebook, c.d_model, rvq_work_, res_, tok_, stream);
   MRT_HIP_CHECK(hipMemcpyAsync(h_stage_, tok_, c.rvq_depth * 4, hipMemcpyDeviceToHost, stream));
   MRT_HIP_CHECK(hipStreamSynchronize(stream));
   std::copy(h_stage_, h_stage_ + c.rvq_depth, tokens);

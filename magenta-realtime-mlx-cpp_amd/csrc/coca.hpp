@@ -35,9 +35,10 @@ void layer_norm_rows(const float* x, int rows, int D, const float* w, const floa
 void coca_attention(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, int Sq, int Sk, int H,
                     int D, const float* qscale, float cap, const float* mask, float* out, hipStream_t s);
 // rvq_quantization (rvq.cpp:24-62) of one vector (D) against codebooks (K, C,
-// D), C <= 1024: tokens (K); residual (D) scratch.
-void rvq_quantize(const float* vec, const float* codebooks, int K, int C, int D, float* residual, int* tokens,
-                  hipStream_t s);
+// D), C <= 1024: tokens (K); work (2 (D + C)) scratch, residual (D) what the
+// last level leaves.
+void rvq_quantize(const float* vec, const float* codebooks, int K, int C, int D, float* work, float* residual,
+                  int* tokens, hipStream_t s);
 
 class Coca {
  public:
@@ -92,7 +93,7 @@ class Coca {
   int* ids_ = nullptr;
   float *mask_ = nullptr, *x_ = nullptr, *h_ = nullptr, *qkv_buf_ = nullptr, *att_ = nullptr, *y_ = nullptr,
         *f_ = nullptr, *n_ = nullptr, *pq_buf_ = nullptr, *pkv_buf_ = nullptr, *patt_ = nullptr, *emb_ = nullptr,
-        *res_ = nullptr;
+        *res_ = nullptr, *rvq_work_ = nullptr;
   std::vector<float*> layer_out_;
   int* tok_ = nullptr;
   int32_t* h_stage_ = nullptr;

@@ -121,3 +121,22 @@ def test_musiccoca_graph_replays_match_eager(gpu_available, size):
         np.testing.assert_array_equal(got, eager[i])
         sm.tokenize()
     sm.close()
+
+
+@pytest.mark.parametrize("codes,depth", [(1, 1), (3, 2), (61, 12), (257, 5)])
+def test_quantize_edges(codes, depth):
+    """Codebooks that fill no workgroup: equal distances take the lowest index
+    and each level quantises what the one before left.  Codes and vector hold
+    small integers, so every product and sum is exact in any order."""
+    import dataclasses
+
+    import mrt_df
+    cfg = dataclasses.replace(mrt_df.CocaConfig.tiny(), rvq_depth=depth, codebook_size=codes)
+    w = synth_bundle.make_coca_weights(cfg, seed=3)
+    rng = np.random.default_rng(codes)
+    cb = rng.integers(-3, 4, (depth, codes, cfg.d_model)).astype(np.float32)
+    cb[:, codes // 2:] = cb[:, :codes - codes // 2]  # every row twice (the middle of an odd count once)
+    w["codebooks"] = cb
+    sm = mrt_df.StyleModel(w, cfg)
+    vec = rng.integers(-9, 10, cfg.d_model).astype(np.float32)
+    np.testing.assert_array_equal(sm.tokenize(vec), M.rvq_quantization(vec[None], cb)[0][0])
