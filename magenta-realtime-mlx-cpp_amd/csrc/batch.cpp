@@ -48,11 +48,13 @@ Batch::Batch(Model& model, int streams, int max_frames, int enc_len)
   dkv_ = dalloc(static_cast<size_t>(c.num_depth_layers) * 2 * R * H * L * 64 * e);
   t_in_ = dalloc(R * D * e);
   d_in_ = dalloc(R * D * e);
-  xn_ = dalloc(R * std::max(D, FF) * e);
+  const size_t Rt = frag_rows(R);  // xn_, xf_, att_, ffh_ are GEMM inputs in fragment order
+  xn_ = dalloc(Rt * D * e);
+  xf_ = dalloc(Rt * D * e);
   ssq_ = static_cast<float*>(dalloc(static_cast<size_t>(R) * (D / 16) * 4));
   q_ = dalloc(R * HD * e);
-  att_ = dalloc(R * HD * e);
-  ffh_ = dalloc(R * FF * e);
+  att_ = dalloc(Rt * HD * e);
+  ffh_ = dalloc(Rt * FF * e);
   fsum_ = dalloc(R * D * e);
   logits_ = static_cast<float*>(dalloc(static_cast<size_t>(R) * 1024 * 4));
   noise_ = static_cast<float*>(dalloc(static_cast<size_t>(B) * F * L * 1024 * 4));
@@ -64,6 +66,7 @@ Batch::Batch(Model& model, int streams, int max_frames, int enc_len)
   MRT_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&h_pinned_), h_pinned_n_ * 4, hipHostMallocDefault));
   MRT_HIP_CHECK(hipEventCreate(&ev_[0]));
   MRT_HIP_CHECK(hipEventCreate(&ev_[1]));
+  fw_ = m.frag_weights(true, stream);
 }
 
 Batch::~Batch() {
@@ -104,50 +107,51 @@ void Batch::encode_device() {
 // ring slot f, or *fptr when non-null.
 void Batch::temporal_stack(int f, const int* fptr) {
   const Config& c = m.cfg;
+  const DType dt = m.dt;
   const int D = c.d_model, HD = c.hd(), FF = c.d_ff, H = c.num_heads;
   for (int i = 0; i < c.num_temporal_layers; ++i) {
-    const DecoderLayerW& W = m.tmp[i];
+    const FragLayer& W = fw_->tmp[i];
     char *tk = ring(tkv_, i, 0, F), *tv = ring(tkv_, i, 1, F);
     // layer 0's input is the frame mean (no row partials): a plain norm pass
     if (i == 0) {
-      rmsnorm_rows(DType::BF16, t_in_, W.norm_sa, 1e-6f, R, D, xn_, stream);
-      bgemm_qkv(xn_, R, D, W.wqkv, HD, q_, tk, tv, H, F, f, fptr, stream);
+      rmsnorm_rows_frag(dt, t_in_, m.tmp[i].norm_sa, 1e-6f, R, D, xn_, stream);
+      bgemm_qkv(dt, xn_, R, D, W.wqkv, HD, q_, tk, tv, H, F, f, fptr, stream);
     } else {
-      bgemm_qkv(t_in_, R, D, W.wqkv, HD, q_, tk, tv, H, F, f, fptr, stream, norm(W.norm_sa));
+      bgemm_qkv(dt, xf_, R, D, W.wqkv, HD, q_, tk, tv, H, F, f, fptr, stream, norm());
     }
-    self_attn_at(DType::BF16, R, q_, tk, tv, H, F, f + 1, f, fptr, m.tbias, m.tbuckets, att_, stream);
-    bgemm_resid(att_, R, HD, W.wo, D, t_in_, D, stream, ssq_);
-    bgemm_store(t_in_, R, D, W.wq_c, HD, q_, HD, stream, norm(W.norm_ca));
+    self_attn_at(dt, R, q_, tk, tv, H, F, f + 1, f, fptr, m.tbias, m.tbuckets, att_, stream, 0, nullptr, true);
+    bgemm_resid(dt, att_, R, HD, W.wo, D, t_in_, xf_, ssq_, stream);
+    bgemm_store(dt, xf_, R, D, W.wq_c, HD, q_, HD, stream, norm());
     cross_attn_rows(q_, ring(enc_.cross, i, 0, S), ring(enc_.cross, i, 1, S), R, H, S, att_, stream);
-    bgemm_resid(att_, R, HD, W.wo_c, D, t_in_, D, stream, ssq_);
-    bgemm_geglu(t_in_, R, D, W.w01, FF, ffh_, FF, stream, norm(W.norm_ff));
-    bgemm_resid(ffh_, R, FF, W.wo2, D, t_in_, D, stream, ssq_);
+    bgemm_resid(dt, att_, R, HD, W.wo_c, D, t_in_, xf_, ssq_, stream);
+    bgemm_geglu(dt, xf_, R, D, W.w01, FF, ffh_, stream, norm());
+    bgemm_resid(dt, ffh_, R, FF, W.wo2, D, t_in_, xf_, ssq_, stream);
   }
 }
 
 // Depth step l of every row in place on x (model.cpp:638-651 per row).
-// x_partials: the row partials of x are those the last bgemm_resid left
-// (the temporal step's output), else layer 0 normalises in its own pass.
 // qkv_fed: layer 0's q and ring slot l were written by the previous level's
-// draw from the q/k/v table (x = emb(token), a function of the token alone).
-void Batch::depth_stack(void* x, int l, bool x_partials, bool qkv_fed) {
+// draw from the q/k/v table (x = emb(token), a function of the token alone);
+// else layer 0 normalises in its own pass, whatever wrote x.
+void Batch::depth_stack(void* x, int l, bool qkv_fed) {
   const Config& c = m.cfg;
+  const DType dt = m.dt;
   const int D = c.d_model, HD = c.hd(), FF = c.d_ff, H = c.num_heads, L = c.rvq_depth;
   for (int i = 0; i < c.num_depth_layers; ++i) {
-    const DecoderLayerW& W = m.dep[i];
+    const FragLayer& W = fw_->dep[i];
     char *dk = ring(dkv_, i, 0, L), *dv = ring(dkv_, i, 1, L);
     if (i == 0 && qkv_fed) {
       // nothing to compute: q / k / v are in place
-    } else if (i == 0 && !x_partials) {
-      rmsnorm_rows(DType::BF16, x, W.norm_sa, 1e-6f, R, D, xn_, stream);
-      bgemm_qkv(xn_, R, D, W.wqkv, HD, q_, dk, dv, H, L, l, nullptr, stream);
+    } else if (i == 0) {
+      rmsnorm_rows_frag(dt, x, m.dep[i].norm_sa, 1e-6f, R, D, xn_, stream);
+      bgemm_qkv(dt, xn_, R, D, W.wqkv, HD, q_, dk, dv, H, L, l, nullptr, stream);
     } else {
-      bgemm_qkv(x, R, D, W.wqkv, HD, q_, dk, dv, H, L, l, nullptr, stream, norm(W.norm_sa));
+      bgemm_qkv(dt, xf_, R, D, W.wqkv, HD, q_, dk, dv, H, L, l, nullptr, stream, norm());
     }
-    self_attn_at(DType::BF16, R, q_, dk, dv, H, L, l + 1, l, nullptr, m.dbias, m.dbuckets, att_, stream);
-    bgemm_resid(att_, R, HD, W.wo, D, x, D, stream, ssq_);
-    bgemm_geglu(x, R, D, W.w01, FF, ffh_, FF, stream, norm(W.norm_ff));
-    bgemm_resid(ffh_, R, FF, W.wo2, D, x, D, stream, ssq_);
+    self_attn_at(dt, R, q_, dk, dv, H, L, l + 1, l, nullptr, m.dbias, m.dbuckets, att_, stream, 0, nullptr, true);
+    bgemm_resid(dt, att_, R, HD, W.wo, D, x, xf_, ssq_, stream);
+    bgemm_geglu(dt, xf_, R, D, W.w01, FF, ffh_, stream, norm());
+    bgemm_resid(dt, ffh_, R, FF, W.wo2, D, x, xf_, ssq_, stream);
   }
 }
 
@@ -178,13 +182,13 @@ void Batch::enqueue_frame(const GenOpts& o, int f, bool dynamic) {
   if (o.record_temporal) copy_dev(static_cast<char*>(o.record_temporal) + f * row_bytes, t_in_, row_bytes, stream);
   for (int l = 0; l < L; ++l) {
     void* x = l == 0 ? t_in_ : d_in_;
-    depth_stack(x, l, l == 0 && c.num_temporal_layers > 0, l > 0 && qkv_tab_ != nullptr);
-    const char* head = static_cast<const char*>(m.lm_head) + static_cast<size_t>(o.codec_offset + C * l) * D * 2;
+    depth_stack(x, l, l > 0 && qkv_tab_ != nullptr);
+    const int head0 = o.codec_offset + C * l;
     if (c.num_depth_layers > 0) {
-      bgemm_f32(x, R, D, head, C, logits_, C, stream, norm(m.dec_norm));
+      bgemm_f32(m.dt, xf_, R, D, fw_->head, head0, C, logits_, C, stream, norm());
     } else {
-      rmsnorm_rows(DType::BF16, x, m.dec_norm, 1e-6f, R, D, xn_, stream);
-      bgemm_f32(xn_, R, D, head, C, logits_, C, stream);
+      rmsnorm_rows_frag(m.dt, x, m.dec_norm, 1e-6f, R, D, xn_, stream);
+      bgemm_f32(m.dt, xn_, R, D, fw_->head, head0, C, logits_, C, stream);
     }
     if (o.record_slices)
       copy_dev(o.record_slices + (static_cast<size_t>(f) * L + l) * R * C, logits_, static_cast<size_t>(R) * C * 4,

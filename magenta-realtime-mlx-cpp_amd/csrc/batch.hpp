@@ -15,44 +15,63 @@ namespace mrt {
 
 constexpr int kBatchRows = 64;  // activation rows of one batched step (32 streams)
 
-// RMSNorm (eps, weights g) of a GEMM's input rows applied as they are loaded:
-// X then holds the raw residual rows, whose sums of squares are the K / 16
-// partials per row (row-major, K / 16 a row) that the bgemm_resid which last
-// wrote them left at ssq.  g == nullptr: X is used as it is.
+// Fragment order: the operands of the skinny GEMMs are stored as 16-row x
+// 32-column tiles, each tile the 64 lanes' 16-byte operands of one 16x16x32
+// matrix instruction (lane l: row l % 16, columns 8 (l / 16) .. + 7), tiles of a
+// row group back to back along K.  Element (m, k): frag_index (device_utils.hpp).
+// Activation buffers hold whole tiles: frag_rows(M) rows.
+inline int frag_rows(int M) { return (M + 15) / 16 * 16; }
+
+// Elements of an (N, K) weight matrix in fragment order (N padded to 16 rows,
+// and 16 rows more).
+size_t frag_weights_elems(int N, int K);
+// The matrix in fragment order; g non-null: column k times g[k], rounded to the
+// storage type (the RMSNorm weights of the input folded in, for BNorm inputs).
+// pairs: W is a packed wi_0 / wi_1 matrix (N = 2F rows, bgemm_geglu).
+void frag_weights(DType dt, const void* W, const void* g, int N, int K, bool pairs, void* out, hipStream_t s);
+// rmsnorm_rows (row-major in) with the result in fragment order, D <= 4096.
+void rmsnorm_rows_frag(DType dt, const void* x, const void* g, float eps, int M, int D, void* y, hipStream_t s);
+
+// RMSNorm of a GEMM's input rows: X then holds the raw residual rows, whose
+// sums of squares are the K / 16 partials per row that the bgemm_resid which
+// last wrote them left at ssq, and W the weights with the norm's weights folded
+// in (frag_weights).  ssq == nullptr: X is used as it is.
 struct BNorm {
-  const void* g = nullptr;
   const float* ssq = nullptr;
   float eps = 0.f;
 };
 
-// Skinny GEMMs Y (M x N) = X (M x K) . W^T, bf16 in, fp32 accumulation, M <= 64,
-// K % 32 == 0 (batch_kernels.hip).  Epilogues as the batch-1 GEMVs.
-void bgemm_store(const void* X, int M, int K, const void* W, int N, void* Y, int ldy, hipStream_t s,
+// Skinny GEMMs Y (M x N) = X (M x K) . W^T, 16-bit storage types, fp32
+// accumulation, M <= 64, K % 32 == 0, X and W in fragment order
+// (batch_kernels.hip).  Epilogues as the batch-1 GEMVs.
+void bgemm_store(DType dt, const void* X, int M, int K, const void* W, int N, void* Y, int ldy, hipStream_t s,
                  const BNorm& norm = {});
-void bgemm_f32(const void* X, int M, int K, const void* W, int N, float* Y, int ldy, hipStream_t s,
-               const BNorm& norm = {});
-// R += X . W^T (rounded as the batch-1 residual); ssq non-null: each updated
-// row's sums of squares over its 16-column tiles, (M, N / 16) floats.
-void bgemm_resid(const void* X, int M, int K, const void* W, int N, void* R, int ldr, hipStream_t s,
-                 float* ssq = nullptr);
+// Logits, rounded to the storage type: weight rows w_row0 .. + N.  groups > 1:
+// independent products, rows [g M, + M) of X against weight rows
+// w_row0 + g w_group_rows .. + N into Y rows g M + m.
+void bgemm_f32(DType dt, const void* X, int M, int K, const void* W, int w_row0, int N, float* Y, int ldy,
+               hipStream_t s, const BNorm& norm = {}, int groups = 1, int w_group_rows = 0);
+// R (M, N) += X . W^T (rounded as the batch-1 residual); the updated rows also
+// in fragment order to Rf, and each row's sums of squares over its 16-column
+// tiles to ssq (M, N / 16).
+void bgemm_resid(DType dt, const void* X, int M, int K, const void* W, int N, void* R, void* Rf, float* ssq,
+                 hipStream_t s);
 // W = [Wq; Wk; Wv] (3 HD rows): q -> Q (M, HD); k, v -> ring slot pos (or
 // *pos_ptr when non-null) of caches laid out (M, H, Lmax, 64).
-void bgemm_qkv(const void* X, int M, int K, const void* W, int HD, void* Q, void* Kc, void* Vc, int H, int Lmax, int pos,
-               const int* pos_ptr, hipStream_t s, const BNorm& norm = {});
+void bgemm_qkv(DType dt, const void* X, int M, int K, const void* W, int HD, void* Q, void* Kc, void* Vc, int H,
+               int Lmax, int pos, const int* pos_ptr, hipStream_t s, const BNorm& norm = {});
 // The same for rows m = P * pos + r (positions of one stream's frame, P CFG
 // rows each): k / v -> slot pos of ring row r (P, H, Lmax, 64).
-void bgemm_qkv_pos(const void* X, int M, int K, const void* W, int HD, void* Q, void* Kc, void* Vc, int H, int Lmax,
-                   int P, hipStream_t s);
-// groups independent products: rows [g rows, +rows) of X against
-// W + g * w_group_stride, logits rounded to bf16 into Y rows g rows + m.
-void bgemm_f32_grouped(const void* X, int rows, int K, const void* W, long w_group_stride, int N, float* Y, int ldy,
-                       int groups, hipStream_t s);
-// Gated GELU over the 32-row packed wi_0 / wi_1 matrix (2F rows) -> (M, F).
-void bgemm_geglu(const void* X, int M, int K, const void* W01, int F, void* Hout, int ldh, hipStream_t s,
+void bgemm_qkv_pos(DType dt, const void* X, int M, int K, const void* W, int HD, void* Q, void* Kc, void* Vc, int H,
+                   int Lmax, int P, hipStream_t s);
+// Gated GELU over the 32-row packed wi_0 / wi_1 matrix (2F rows) -> (M, F) in
+// fragment order.
+void bgemm_geglu(DType dt, const void* X, int M, int K, const void* W01, int F, void* Hout, hipStream_t s,
                  const BNorm& norm = {});
 
 // Cross attention (no bias, no mask, scale 1) of every (row, head) over S <=
-// 1024 encoder keys, caches laid out (rows, H, S, 64); out (rows, H * 64).
+// 1024 encoder keys, caches laid out (rows, H, S, 64); out (rows, H * 64) in
+// fragment order.
 void cross_attn_rows(const void* Q, const void* Kc, const void* Vc, int rows, int H, int S, void* out, hipStream_t s);
 
 // Gumbel noise of every draw for every stream: out (streams, frames, L, C).
@@ -89,9 +108,9 @@ class Batch {
  private:
   void enqueue_frame(const GenOpts& o, int f, bool dynamic);
   void temporal_stack(int f, const int* fptr);
-  void depth_stack(void* x, int l, bool x_partials, bool qkv_fed = false);
-  // the norm (weights g) of a GEMM input whose row partials are at ssq_
-  BNorm norm(const void* g) const { return BNorm{g, ssq_, 1e-6f}; }
+  void depth_stack(void* x, int l, bool qkv_fed);
+  // the norm of a GEMM input whose row partials are at ssq_
+  BNorm norm() const { return BNorm{ssq_, 1e-6f}; }
   void* dalloc(size_t bytes);
   char* ring(void* base, int layer, int kv, int len) const;
 
@@ -100,7 +119,10 @@ class Batch {
   bool encoded_ = false;
   void *tkv_ = nullptr, *dkv_ = nullptr;
   void *t_in_ = nullptr, *d_in_ = nullptr, *xn_ = nullptr, *q_ = nullptr, *att_ = nullptr, *ffh_ = nullptr;
-  float* ssq_ = nullptr;  // row partials of the last residual update: (R, d_model / 16)
+  // the last residual update: its rows in fragment order and their partials (R, d_model / 16)
+  void* xf_ = nullptr;
+  float* ssq_ = nullptr;
+  const FragWeights* fw_ = nullptr;  // the model's
   // the model's depth layer-0 q/k/v table of the current call's codec levels,
   // or nullptr (layer 0 computed at every level)
   const void* qkv_tab_ = nullptr;

@@ -2,11 +2,12 @@
 // together, R = 2B activation rows (both CFG rows of every stream), R <= 64.
 //
 // At R = 64 every weight row meets 64 activation rows, so the projections are
-// skinny GEMMs and run on the matrix cores: v_mfma_f32_16x16x32_bf16, one
+// skinny GEMMs and run on the matrix cores: v_mfma_f32_16x16x32_{bf16,f16}, one
 // block per 16 output columns, the 8 waves of a block splitting K and summing
 // their partial tiles through LDS in a fixed order (deterministic).  The
 // activations (R x K, at most 360 KB) are read by every block from L2; the
-// weights stream from HBM/MALL once per step.
+// weights stream from HBM/MALL once per step.  Both are kept in fragment order
+// (batch.hpp), so an operand load of a wave is 1 KB of consecutive addresses.
 #include <algorithm>
 #include <type_traits>
 
@@ -17,61 +18,84 @@
 namespace mrt {
 namespace {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kBgCols = 16;   // output columns per block
-constexpr int kBgChunk = 1;   // k-steps (of 32) per loop step of a wave: fewer live registers (per 32-stream chunk: 8: 243.6 ms, 4: 238.7, 2: 234.2, 1: 232.2)
-constexpr int kBgWaves = 8;   // waves per block, splitting K
+// The 16x16x32 matrix instruction of each 16-bit storage type.
+template <typename T>
+struct Mfma16;
+template <>
+struct Mfma16<bf16> {
+  typedef __bf16 v8 __attribute__((ext_vector_type(8)));
+  __device__ __forceinline__ static f32x4_t mma(uint4 a, uint4 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
+  }
+};
+template <>
+struct Mfma16<f16> {
+  typedef _Float16 v8 __attribute__((ext_vector_type(8)));
+  __device__ __forceinline__ static f32x4_t mma(uint4 a, uint4 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
+  }
+};
+
+constexpr int kBgCols = 16;  // output columns per block
+constexpr int kBgWaves = 8;  // waves per block, splitting K
 constexpr int kBgThreads = 64 * kBgWaves;
 
 // ---- epilogues: op(m, n, v[P]) with v the fp32 sums of output (m, n) ---------------
 
+template <typename T>
 struct BStore {
-  bf16* y;
+  T* y;
   int ldy;
-  __device__ void operator()(int m, int n, const float (&v)[1]) const { y[(size_t)m * ldy + n] = St<bf16>::st(v[0]); }
+  __device__ void operator()(int m, int n, const float (&v)[1]) const { y[(size_t)m * ldy + n] = St<T>::st(v[0]); }
 };
 
+template <typename T>
 struct BF32 {
   float* y;
   int ldy;
-  __device__ void operator()(int m, int n, const float (&v)[1]) const { y[(size_t)m * ldy + n] = St<bf16>::rnd(v[0]); }
+  __device__ void operator()(int m, int n, const float (&v)[1]) const { y[(size_t)m * ldy + n] = St<T>::rnd(v[0]); }
 };
 
 // Residual update; the residual values are read at the start of the kernel
-// (pre), so the epilogue does not wait for them.  `ssq` non-null: the sum of
-// squares of each updated row over the block's 16 columns goes to
-// ssq[m * ntiles + tile], the partials a normalised consumer reads (BNorm).
+// (pre), so the epilogue does not wait for them.  The updated rows are written
+// to r and, in fragment order, to rf; the sum of squares of each updated row
+// over the block's 16 columns goes to ssq[m * (N / 16) + tile], the partials a
+// normalised consumer reads (BNorm).
+template <typename T>
 struct BResid {
-  bf16* r;
+  T* r;
   int ldr;
+  T* rf;
   float* ssq;
   static constexpr bool kPre = true;
-  __device__ float pre(int m, int n) const { return St<bf16>::ld(r[(size_t)m * ldr + n]); }
+  __device__ float pre(int m, int n) const { return St<T>::ld(r[(size_t)m * ldr + n]); }
   __device__ float operator()(int m, int n, const float (&v)[1], float x) const {
-    const bf16 y = St<bf16>::st(x + St<bf16>::rnd(v[0]));
+    const T y = St<T>::st(x + St<T>::rnd(v[0]));
     r[(size_t)m * ldr + n] = y;
-    return St<bf16>::ld(y);
+    rf[frag_index(m, n, ldr >> 5)] = y;
+    return St<T>::ld(y);
   }
 };
 
 // n < HD: q; else k / v into ring slot pos (fixed, or *pos_ptr) of the caches
 // laid out (R, H, Lmax, 64).
+template <typename T>
 struct BQKV {
-  bf16* q;
-  bf16* kc;
-  bf16* vc;
+  T* q;
+  T* kc;
+  T* vc;
   int HD, H, Lmax, pos;
   const int* pos_ptr;
   __device__ void operator()(int m, int n, const float (&v)[1]) const {
-    const bf16 o = St<bf16>::st(v[0]);
+    const T o = St<T>::st(v[0]);
     const int which = n / HD, nn = n - which * HD;
     if (which == 0) {
       q[(size_t)m * HD + nn] = o;
     } else {
       const int p = pos_ptr ? *pos_ptr : pos;
-      bf16* c = which == 1 ? kc : vc;
+      T* c = which == 1 ? kc : vc;
       c[(((size_t)m * H + (nn >> 6)) * Lmax + p) * 64 + (nn & 63)] = o;
     }
   }
@@ -79,49 +103,41 @@ struct BQKV {
 
 // Rows m = P * pos + r (the positions of one frame, rows r = 0..P-1 each):
 // q -> Q row m; k / v -> ring slot pos of ring row r, caches (P, H, Lmax, 64).
+template <typename T>
 struct BQKVPos {
-  bf16* q;
-  bf16* kc;
-  bf16* vc;
+  T* q;
+  T* kc;
+  T* vc;
   int HD, H, Lmax, P;
   __device__ void operator()(int m, int n, const float (&v)[1]) const {
-    const bf16 o = St<bf16>::st(v[0]);
+    const T o = St<T>::st(v[0]);
     const int which = n / HD, nn = n - which * HD;
     if (which == 0) {
       q[(size_t)m * HD + nn] = o;
     } else {
       const int r = m % P, pos = m / P;
-      bf16* c = which == 1 ? kc : vc;
+      T* c = which == 1 ? kc : vc;
       c[(((size_t)r * H + (nn >> 6)) * Lmax + pos) * 64 + (nn & 63)] = o;
     }
   }
 };
 
+// Output (M, F) in fragment order: the input of the down projection.
+template <typename T>
 struct BGeglu {
-  bf16* h;
-  int ldh;
+  T* h;
+  int F;
   __device__ void operator()(int m, int j, const float (&v)[2]) const {
-    const float g = gelu_t<bf16>(St<bf16>::rnd(v[0]));
-    h[(size_t)m * ldh + j] = St<bf16>::st(g * St<bf16>::rnd(v[1]));
+    const float g = gelu_t<T>(St<T>::rnd(v[0]));
+    h[frag_index(m, j, F >> 5)] = St<T>::st(g * St<T>::rnd(v[1]));
   }
 };
 
 __device__ __forceinline__ int bg_geglu_row(int j, int p) { return (j >> 5) * 64 + (j & 31) + 32 * p; }
 
-// Y (M x nout) = X (M x K) . W^T with epilogue.  P = 1: output n reads weight
-// row n; P = 2: output j reads the gate / up rows of the 32-row packed wi_0 /
-// wi_1 matrix.  Operand fragments of the 16x16x32 MFMA: lane l holds row
-// (l % 16) of A and column (l % 16) of B over k = 8 (l / 16) .. + 7 of the
-// step; the 4 accumulators of lane l hold column l % 16, rows 4 (l / 16) + i.
-// Wave w of the 8 takes k-steps w, w + 8, ...; the 8 partial tiles are summed
-// in wave order.  Rows past M are zero, columns past nout re-read the last row
-// and are not stored.
-// RMSNorm of the activation rows applied as they are loaded (modules.cpp
-// RMSNorm, as rmsnorm_rows): row m of X is the raw residual, its sum of squares
-// the `parts` partials at ssq + m * parts (summed in order), element k scaled
-// to bf16(bf16(x * inv) * g[k]) with inv = 1 / sqrt(ss / K + eps).
+// The row sums of squares of an input that is normalised (BNorm): `parts`
+// partials per row at ssq + m * parts, summed in order.
 struct BNormDev {
-  const bf16* g;
   const float* ssq;
   int parts;
   float eps;
@@ -136,17 +152,6 @@ __device__ __forceinline__ float row16_sum(float v) {
   return v;
 }
 
-// Eight bf16 activations scaled by the row's inverse RMS and the norm weights.
-__device__ __forceinline__ uint4 norm8(uint4 x, uint4 g, float inv) {
-  const bf16* xe = reinterpret_cast<const bf16*>(&x);
-  const bf16* ge = reinterpret_cast<const bf16*>(&g);
-  uint4 out;
-  bf16* oe = reinterpret_cast<bf16*>(&out);
-#pragma unroll
-  for (int e = 0; e < 8; ++e) oe[e] = St<bf16>::st(St<bf16>::rnd(St<bf16>::ld(xe[e]) * inv) * St<bf16>::ld(ge[e]));
-  return out;
-}
-
 template <class Epi, class = void>
 struct HasPre {
   static constexpr bool value = false;
@@ -156,77 +161,108 @@ struct HasPre<Epi, decltype((void)Epi::kPre)> {
   static constexpr bool value = Epi::kPre;
 };
 
+template <class Epi>
+struct IsResid : std::false_type {};
+template <typename T>
+struct IsResid<BResid<T>> : std::true_type {};
+
+// Y (M x nout) = X (M x K) . W^T with epilogue, X and W in fragment order.
+// P = 1: output n is weight row w_row0 + n; P = 2: output j meets the gate / up
+// rows of the packed wi_0 / wi_1 matrix.  Operand fragments of the 16x16x32
+// MFMA: lane l holds row (l % 16) of A and column (l % 16) of B over
+// k = 8 (l / 16) .. + 7 of the step; the 4 accumulators of lane l hold column
+// l % 16, rows 4 (l / 16) + i.  Wave w of the 8 takes k-steps w, w + 8, ...; the
+// 8 partial tiles are summed in wave order.  Rows past M repeat the last row and
+// columns past nout meet other rows' weights; neither is stored.
+//
+// NORM: X holds raw residual rows and W the weights already multiplied by the
+// norm weights, so RMSNorm (modules.cpp:72-84) is the scaling of row m's sums
+// by inv(m) = 1 / sqrt(mean(x^2) + eps): it costs one multiplication an output
+// instead of two roundings of every activation in every block, and its chain
+// (partials, square root) runs beside the products.  Scaling the activations on
+// load took 3 us of the 9.7 us of the 3,072-wide output at 64 rows.
+//
 // Block (tile, ms) of the grid computes output columns [16 tile, +16) for the
 // MT row tiles [MT ms, +MT) of 16 rows: blocks sharing a column tile are
-// tile + ntiles * ms, on the same XCD when ntiles % 8 == 0 (blocks are dealt to
-// the 8 XCDs in turn), so the weight tile comes from HBM once and from that
-// XCD's L2 for the others.
-template <int P, int MT, bool NORM, class Epi>
-__global__ __launch_bounds__(kBgThreads) void k_bgemm(const bf16* __restrict__ X, int M, int K,
-                                                      const bf16* __restrict__ W, int nout, int ntiles, Epi epi,
-                                                      long w_group_stride, BNormDev nrm) {
+// tile + ntiles * ms, on the same XCD as ntiles is then padded to a multiple of
+// 8 (blocks are dealt to the 8 XCDs in turn), so the weight tile comes from HBM
+// once and from that XCD's L2 for the others.
+//
+// What bounds it is the launch and one or two memory round trips, so a wave
+// requests the operands of NST of its k-steps at once, without a branch between
+// the loads (a step past the end re-reads the last one and is not multiplied).
+// Fragment order is what makes that pay: rows 2 KB apart put the 16 rows of an
+// operand load into few L2 channels, and more of them in flight ran slower
+// (64 rows, alone, us: 3,072 outputs 6.6 row-major, 4.1 here; 2,816 gated pairs
+// 9.2, 5.8; 1,024 outputs 3.9, 2.9 at K = 1,024 and 6.8, 4.2 at K = 2,816; an
+// empty launch takes 1.9).
+template <typename T, int P, int MT, int NST, bool NORM, class Epi>
+__global__ __launch_bounds__(kBgThreads) void k_bgemm(const T* __restrict__ X, int M, int K, const T* __restrict__ W,
+                                                      int nout, int ntiles, Epi epi, int w_row0, int w_group_rows,
+                                                      BNormDev nrm) {
   // blockIdx.y = group g (grouped launch): rows [g M, g M + M) of X against
-  // W + g * w_group_stride, outputs at rows g M + m
+  // weight rows w_row0 + g * w_group_rows, outputs at rows g M + m
   const int grow = blockIdx.y * M;
-  X += (size_t)grow * K;
-  W += blockIdx.y * w_group_stride;
+  const int row0 = w_row0 + blockIdx.y * w_group_rows, skip = P == 1 ? row0 & 15 : 0;
   constexpr int kRows = 16 * MT;
   constexpr int kOut = kRows * kBgCols;                        // outputs of the block
   constexpr int kPer = (kOut + kBgThreads - 1) / kBgThreads;  // epilogue outputs per thread
   __shared__ float part[kBgWaves][kRows][kBgCols + 1];  // one part (gate / up) at a time
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  [[maybe_unused]] __shared__ float inv_s[kRows];
+  // the wave index as a scalar: matrix instructions ignore the lane mask, so the
+  // conditions around them must be branches
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tile = blockIdx.x % ntiles, m0 = (blockIdx.x / ntiles) * kRows;
-  const int j0 = tile * kBgCols;
+  const int j0 = tile * kBgCols - skip;  // output of the block's first column
+  if (j0 >= nout) return;                // a padding tile (launch_bgemm_t)
   const int c16 = lane & 15, kg = lane >> 4;
-  const bf16* wrow[P];
-#pragma unroll
-  for (int p = 0; p < P; ++p) {
-    const int j = min(j0 + c16, nout - 1);
-    wrow[p] = W + (size_t)(P == 1 ? j : bg_geglu_row(j, p)) * K + kg * 8;
-  }
-  const bf16* xrow[MT];
-  bool xin[MT];
+  const int nks = K / 32;
+
+  const T* wt = W + ((size_t)(P == 1 ? (row0 >> 4) + tile : tile) * nks * P) * 512 + lane * 8;
+  const T* xrow[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
-    const int m = m0 + 16 * t + c16;
-    xin[t] = m < M;
-    xrow[t] = X + (size_t)min(m, M - 1) * K + kg * 8;
+    const int r = grow + min(m0 + 16 * t + c16, M - 1);
+    xrow[t] = X + (size_t)(r >> 4) * nks * 512 + (kg * 16 + (r & 15)) * 8;
   }
-  float inv[MT];
-  const bf16* grow_g = nullptr;
-  if constexpr (NORM) {
-    // eight lanes per row: with 64 partials lane q sums [8 q, 8 q + 8) in
-    // order (other counts: lane 0 sums them all), and the eight sums meet by
-    // lane exchange (the same total in each lane)
-    __shared__ float inv_s[kRows];
-    const int r = tid >> 3, q = tid & 7;
-    float ss = 0.f;
-    if (r < kRows) {
-      const float* sp = nrm.ssq + (size_t)(grow + min(m0 + r, M - 1)) * nrm.parts;
-      if (nrm.parts == 64) {
-        const float4 u = *reinterpret_cast<const float4*>(sp + 8 * q);
-        const float4 w = *reinterpret_cast<const float4*>(sp + 8 * q + 4);
-        ss = ((((((u.x + u.y) + u.z) + u.w) + w.x) + w.y) + w.z) + w.w;
-      } else if (q == 0) {
-        for (int t = 0; t < nrm.parts; ++t) ss += sp[t];
-      }
-    }
-    ss += __shfl_xor(ss, 1);
-    ss += __shfl_xor(ss, 2);
-    ss += __shfl_xor(ss, 4);
-    if (r < kRows && q == 0) inv_s[r] = 1.0f / sqrtf(ss / (float)K + nrm.eps);
-    __syncthreads();
+  uint4 b[NST][P], a[NST][MT];
+  auto load = [&](int s0) {
 #pragma unroll
-    for (int t = 0; t < MT; ++t) inv[t] = inv_s[16 * t + c16];
-    grow_g = nrm.g + kg * 8;
-  }
+    for (int c = 0; c < NST; ++c) {
+      const int ks = min(s0 + kBgWaves * c, nks - 1);
+#pragma unroll
+      for (int p = 0; p < P; ++p) b[c][p] = ld_g16(wt + (size_t)(ks * P + p) * 512);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) a[c][t] = ld_g16(xrow[t] + (size_t)ks * 512);
+    }
+  };
+  load(wid);
   float pre[kPer];
   if constexpr (HasPre<Epi>::value) {
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
-      const int idx = tid + kBgThreads * i, m = m0 + idx / kBgCols, n = j0 + idx % kBgCols;
-      pre[i] = (idx < kOut && m < M && n < nout) ? epi.pre(grow + m, n) : 0.f;
+      const int idx = min(tid + kBgThreads * i, kOut - 1), m = m0 + idx / kBgCols, n = j0 + idx % kBgCols;
+      pre[i] = epi.pre(grow + min(m, M - 1), min(n, nout - 1));
     }
+  }
+  if constexpr (NORM) {
+    // eight lanes per row: with 64 partials lane q sums [8 q, 8 q + 8) in
+    // order (other counts: lane 0 sums them all), and the eight sums meet by
+    // lane exchange (the same total in each lane)
+    const int r = tid >> 3, q = tid & 7;
+    const float* sp = nrm.ssq + (size_t)(grow + min(m0 + min(r, kRows - 1), M - 1)) * nrm.parts;
+    float ss = 0.f;
+    if (nrm.parts == 64) {
+      const float4 u = *reinterpret_cast<const float4*>(sp + 8 * q);
+      const float4 w = *reinterpret_cast<const float4*>(sp + 8 * q + 4);
+      ss = ((((((u.x + u.y) + u.z) + u.w) + w.x) + w.y) + w.z) + w.w;
+    } else if (q == 0) {
+      for (int t = 0; t < nrm.parts; ++t) ss += sp[t];
+    }
+    ss += __shfl_xor(ss, 1);
+    ss += __shfl_xor(ss, 2);
+    ss += __shfl_xor(ss, 4);
+    if (r < kRows && q == 0) inv_s[r] = 1.0f / sqrtf(ss / (float)K + nrm.eps);  // read after the barrier below
   }
   f32x4_t acc[P][MT];
 #pragma unroll
@@ -234,35 +270,17 @@ __global__ __launch_bounds__(kBgThreads) void k_bgemm(const bf16* __restrict__ X
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[p][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  const int nks = K / 32;
-  for (int s0 = wid; s0 < nks; s0 += kBgWaves * kBgChunk) {
-    uint4 b[kBgChunk][P], a[kBgChunk][MT], gk[NORM ? kBgChunk : 1];
+  for (int s0 = wid; s0 < nks; s0 += kBgWaves * NST) {
 #pragma unroll
-    for (int c = 0; c < kBgChunk; ++c) {
-      const int ks = s0 + kBgWaves * c;
-      if (ks < nks) {
-#pragma unroll
-        for (int p = 0; p < P; ++p) b[c][p] = ld_g16(wrow[p] + ks * 32);
-#pragma unroll
-        for (int t = 0; t < MT; ++t) a[c][t] = xin[t] ? ld_g16(xrow[t] + ks * 32) : make_uint4(0u, 0u, 0u, 0u);
-        if constexpr (NORM) gk[c] = ld_g16(grow_g + ks * 32);
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < kBgChunk; ++c) {
+    for (int c = 0; c < NST; ++c) {
       if (s0 + kBgWaves * c < nks) {
-        if constexpr (NORM) {
-#pragma unroll
-          for (int t = 0; t < MT; ++t) a[c][t] = norm8(a[c][t], gk[c], inv[t]);
-        }
 #pragma unroll
         for (int p = 0; p < P; ++p)
 #pragma unroll
-          for (int t = 0; t < MT; ++t)
-            acc[p][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[c][t]),
-                                                                __builtin_bit_cast(bf16x8_t, b[c][p]), acc[p][t], 0, 0, 0);
+          for (int t = 0; t < MT; ++t) acc[p][t] = Mfma16<T>::mma(a[c][t], b[c][p], acc[p][t]);
       }
     }
+    if (s0 + kBgWaves * NST < nks) load(s0 + kBgWaves * NST);
   }
   float v[kPer][P];
 #pragma unroll
@@ -279,73 +297,146 @@ __global__ __launch_bounds__(kBgThreads) void k_bgemm(const bf16* __restrict__ X
       float a = part[0][m][n];
 #pragma unroll
       for (int w = 1; w < kBgWaves; ++w) a += part[w][m][n];
-      v[i][p] = a;
+      v[i][p] = NORM ? a * inv_s[m] : a;
     }
   }
-  if constexpr (std::is_same<Epi, BResid>::value) {
+  if constexpr (IsResid<Epi>::value) {
     // lanes 16 r .. 16 r + 15 of a wave hold the 16 columns of one output row
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
       const int idx = tid + kBgThreads * i, m = m0 + idx / kBgCols, n = idx % kBgCols;
       const bool ok = idx < kOut && m < M && j0 + n < nout;
       const float y = ok ? epi(grow + m, j0 + n, v[i], pre[i]) : 0.f;
-      if (epi.ssq != nullptr) {
-        const float ss = row16_sum(y * y);
-        if (ok && n == kBgCols - 1) epi.ssq[(size_t)(grow + m) * ntiles + tile] = ss;
-      }
+      const float ss = row16_sum(y * y);
+      if (ok && n == kBgCols - 1) epi.ssq[(size_t)(grow + m) * (epi.ldr / kBgCols) + tile] = ss;
     }
   } else {
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
-      const int idx = tid + kBgThreads * i, m = m0 + idx / kBgCols, n = idx % kBgCols;
-      if (idx >= kOut || m >= M || j0 + n >= nout) continue;
-      if constexpr (HasPre<Epi>::value)
-        epi(grow + m, j0 + n, v[i], pre[i]);
-      else
-        epi(grow + m, j0 + n, v[i]);
+      const int idx = tid + kBgThreads * i, m = m0 + idx / kBgCols, n = j0 + idx % kBgCols;
+      if (idx >= kOut || m >= M || n < 0 || n >= nout) continue;
+      epi(grow + m, n, v[i]);
     }
   }
 }
 
 // Row tiles per block: grids of fewer than 128 column tiles (the d_model-wide
 // outputs) split the rows until there are 256 blocks, one per CU; wider
-// outputs keep all rows in a block (measured faster: each block then reads the
-// activations once for twice the columns' work).
-template <int P, bool NORM, class Epi>
-void launch_bgemm_t(const bf16* X, int M, int K, const bf16* W, int nout, const Epi& epi, hipStream_t s, int groups,
-                    long w_group_stride, const BNormDev& nrm) {
-  const int ntiles = (nout + kBgCols - 1) / kBgCols, mtiles = (M + 15) / 16;
+// outputs keep all rows in a block (each block then reads the activations once
+// for twice the columns' work), the gated pairs at most two row tiles (64 rows:
+// 5.8 against 6.5 us with four).  A block holds 1, 2 or 4 row tiles, no more
+// than the rows need: the loads of unused ones cost as much (the 3,072-wide
+// output of 10 rows: 8.5 us with four).
+template <typename T, int P, bool NORM, class Epi>
+void launch_bgemm_t(const T* X, int M, int K, const T* W, int nout, const Epi& epi, hipStream_t s, int groups,
+                    int w_row0, int w_group_rows, const BNormDev& nrm) {
+  // a column tile more where the weight rows do not start on a tile
+  const bool shifted = P == 1 && (w_row0 % kBgCols != 0 || (groups > 1 && w_group_rows % kBgCols != 0));
+  const int ntiles = (nout + kBgCols - 1) / kBgCols + (shifted ? 1 : 0), mtiles = (M + 15) / 16;
   int ms = 1;
   while (ntiles < 128 && ms < 4 && ms < mtiles && ntiles * ms < 256) ms *= 2;
-  const dim3 grid(ntiles * ms, groups), block(kBgThreads);
-  if (ms == 1)
-    hipLaunchKernelGGL((k_bgemm<P, 4, NORM, Epi>), grid, block, 0, s, X, M, K, W, nout, ntiles, epi, w_group_stride,
-                       nrm);
-  else if (ms == 2)
-    hipLaunchKernelGGL((k_bgemm<P, 2, NORM, Epi>), grid, block, 0, s, X, M, K, W, nout, ntiles, epi, w_group_stride,
-                       nrm);
+  const int mt = (mtiles + ms - 1) / ms;
+  auto go = [&](auto k, int mt_block) {
+    const int mb = (mtiles + mt_block - 1) / mt_block, nt = mb > 1 ? (ntiles + 7) / 8 * 8 : ntiles;
+    hipLaunchKernelGGL(k, dim3(nt * mb, groups), dim3(kBgThreads), 0, s, X, M, K, W, nout, nt, epi, w_row0,
+                       w_group_rows, nrm);
+  };
+  // 12 steps in flight cover K <= 3072 with one row tile
+  if (mt == 1 && P == 1 && K > 32 * 4 * kBgWaves)
+    go(k_bgemm<T, P, 1, P == 1 ? 12 : 4, NORM, Epi>, 1);
+  else if (mt == 1)
+    go(k_bgemm<T, P, 1, 4, NORM, Epi>, 1);
+  else if (mt == 2 || P == 2)
+    go(k_bgemm<T, P, 2, 4, NORM, Epi>, 2);
   else
-    hipLaunchKernelGGL((k_bgemm<P, 1, NORM, Epi>), grid, block, 0, s, X, M, K, W, nout, ntiles, epi, w_group_stride,
-                       nrm);
+    go(k_bgemm<T, P, P == 2 ? 2 : 4, 4, NORM, Epi>, 4);
   MRT_HIP_CHECK(hipGetLastError());
 }
 
-// nrm.g non-null: X holds raw residual rows normalised on load (BNormDev),
-// their sums of squares the K / 16 partials per row a BResid GEMM of width K
-// wrote.
-template <int P, class Epi>
-void launch_bgemm(const bf16* X, int M, int K, const bf16* W, int nout, const Epi& epi, hipStream_t s, int groups = 1,
-                  long w_group_stride = 0, const BNorm& norm = {}) {
-  MRT_REQUIRE(M >= 1 && M <= kBatchRows, "batched GEMM: rows must be in [1, 64]");
+template <typename T, int P, class Epi>
+void launch_bgemm(const void* X, int M, int K, const void* W, int nout, const Epi& epi, hipStream_t s,
+                  const BNorm& norm = {}, int w_row0 = 0, int groups = 1, int w_group_rows = 0) {
+  MRT_REQUIRE(M >= 1 && M * groups <= kBatchRows, "batched GEMM: rows must be in [1, 64]");
   MRT_REQUIRE(K % 32 == 0 && K >= 32, "batched GEMM: K must be a multiple of 32");
-  MRT_REQUIRE(nout >= 1 && groups >= 1, "batched GEMM: no outputs");
-  if (norm.g != nullptr) {
-    MRT_REQUIRE(norm.ssq != nullptr && groups == 1, "batched GEMM: a normalised input needs its row partials");
-    const BNormDev d{static_cast<const bf16*>(norm.g), norm.ssq, K / kBgCols, norm.eps};
-    launch_bgemm_t<P, true>(X, M, K, W, nout, epi, s, groups, w_group_stride, d);
-  } else {
-    launch_bgemm_t<P, false>(X, M, K, W, nout, epi, s, groups, w_group_stride, BNormDev{nullptr, nullptr, 0, 0.f});
+  MRT_REQUIRE(nout >= 1 && groups >= 1 && w_row0 >= 0, "batched GEMM: no outputs");
+  const T* x = static_cast<const T*>(X);
+  const T* w = static_cast<const T*>(W);
+  if (norm.ssq != nullptr)
+    launch_bgemm_t<T, P, true>(x, M, K, w, nout, epi, s, groups, w_row0, w_group_rows,
+                               BNormDev{norm.ssq, K / kBgCols, norm.eps});
+  else
+    launch_bgemm_t<T, P, false>(x, M, K, w, nout, epi, s, groups, w_row0, w_group_rows, BNormDev{nullptr, 0, 0.f});
+}
+
+// Weights (N, K) -> fragment order, each element times g[k] where g is not
+// null (rounded to the storage type).  Block (tile, ks): 16 rows x 32 columns a
+// part; P = 2: the gate and up rows of 16 outputs of a packed matrix.  Rows past
+// N are zero.
+template <typename T, int P>
+__global__ __launch_bounds__(64) void k_frag_weights(const T* __restrict__ W, const T* __restrict__ g, int N, int K,
+                                                     T* __restrict__ out) {
+  using S = St<T>;
+  const int tile = blockIdx.x, ks = blockIdx.y, lane = threadIdx.x, nks = K / 32;
+  const int k0 = ks * 32 + (lane >> 4) * 8;
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int j = tile * 16 + (lane & 15), row = P == 1 ? j : bg_geglu_row(j, p);
+    uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    if (row < N) {
+      v = ld_g16(W + (size_t)row * K + k0);
+      if (g != nullptr) {
+        T* e = reinterpret_cast<T*>(&v);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) e[i] = S::st(S::ld(e[i]) * S::ld(g[k0 + i]));
+      }
+    }
+    *reinterpret_cast<uint4*>(out + (((size_t)tile * nks + ks) * P + p) * 512 + lane * 8) = v;
   }
+}
+
+// rmsnorm_rows with the result in fragment order (K = D): one wave per row, a
+// lane's 16-byte chunks lane, lane + 64, ... (the wave norm's order of sums).
+constexpr int kFragNormChunks = 8;  // D <= 4096
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_rmsnorm_frag(const T* __restrict__ x, const T* __restrict__ g, float eps,
+                                                      int M, int D, T* __restrict__ y) {
+  using S = St<T>;
+  const int lane = threadIdx.x & 63, r = blockIdx.x * 4 + (threadIdx.x >> 6);  // wave-uniform
+  if (r >= M) return;
+  const int nch = D / 8;
+  uint4 v[kFragNormChunks], gv[kFragNormChunks];
+#pragma unroll
+  for (int i = 0; i < kFragNormChunks; ++i)
+    if (64 * i < nch) {  // uniform
+      const int c = min(lane + 64 * i, nch - 1);
+      v[i] = ld_g16(x + (size_t)r * D + c * 8);
+      gv[i] = ld_g16(g + c * 8);
+    }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < kFragNormChunks; ++i)
+    if (lane + 64 * i < nch) {
+      const T* e = reinterpret_cast<const T*>(&v[i]);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const float f = S::ld(e[k]);
+        ss += f * f;
+      }
+    }
+  ss = wave_sum(ss);
+  const float inv = 1.0f / sqrtf(ss / (float)D + eps);
+#pragma unroll
+  for (int i = 0; i < kFragNormChunks; ++i)
+    if (lane + 64 * i < nch) {
+      const T* e = reinterpret_cast<const T*>(&v[i]);
+      const T* ge = reinterpret_cast<const T*>(&gv[i]);
+      uint4 o;
+      T* oe = reinterpret_cast<T*>(&o);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) oe[k] = S::st(S::rnd(S::ld(e[k]) * inv) * S::ld(ge[k]));
+      *reinterpret_cast<uint4*>(y + frag_index(r, (lane + 64 * i) * 8, D >> 5)) = o;
+    }
 }
 
 // Cross attention of one (row, head) over all S encoder keys (no bias, no
@@ -435,7 +526,7 @@ __global__ __launch_bounds__(256) void k_cross_attn_b(const bf16* __restrict__ Q
   if (tid < 64) {
     float o = 0.f;
     for (int g = 0; g < 32; ++g) o += red[g][tid];
-    out[(size_t)b * HD + h * 64 + tid] = St<bf16>::st(o / sum);
+    out[frag_index(b, h * 64 + tid, HD >> 5)] = St<bf16>::st(o / sum);
   }
 }
 
@@ -479,45 +570,78 @@ void cross_attn_rows(const void* Q, const void* Kc, const void* Vc, int rows, in
   MRT_HIP_CHECK(hipGetLastError());
 }
 
-void bgemm_store(const void* X, int M, int K, const void* W, int N, void* Y, int ldy, hipStream_t s, const BNorm& norm) {
-  launch_bgemm<1>(static_cast<const bf16*>(X), M, K, static_cast<const bf16*>(W), N, BStore{static_cast<bf16*>(Y), ldy},
-                  s, 1, 0, norm);
+#define MRT_DTYPE16(dt, ...)                                                         \
+  do {                                                                               \
+    MRT_REQUIRE((dt) != DType::F32, "batched GEMM: 16-bit storage types only");      \
+    if ((dt) == DType::BF16) {                                                       \
+      using T = bf16;                                                                \
+      __VA_ARGS__;                                                                   \
+    } else {                                                                         \
+      using T = f16;                                                                 \
+      __VA_ARGS__;                                                                   \
+    }                                                                                \
+  } while (0)
+
+// One tile more than the rows fill: a range of weight rows that does not start
+// on a tile may touch it (its outputs are not stored).
+size_t frag_weights_elems(int N, int K) { return (static_cast<size_t>((N + 15) / 16) + 1) * 16 * K; }
+
+void frag_weights(DType dt, const void* W, const void* g, int N, int K, bool pairs, void* out, hipStream_t s) {
+  MRT_REQUIRE(K % 32 == 0 && N >= 1, "fragment weights: K must be a multiple of 32");
+  MRT_REQUIRE(!pairs || N % 64 == 0, "fragment weights: gate / up pairs come in groups of 64 rows");
+  const int tiles = (pairs ? N / 2 : N + 15) / 16;
+  MRT_DTYPE16(dt, {
+    const auto k = pairs ? k_frag_weights<T, 2> : k_frag_weights<T, 1>;
+    hipLaunchKernelGGL(k, dim3(tiles, K / 32), dim3(64), 0, s, static_cast<const T*>(W), static_cast<const T*>(g), N,
+                       K, static_cast<T*>(out));
+  });
+  MRT_HIP_CHECK(hipGetLastError());
 }
 
-void bgemm_f32(const void* X, int M, int K, const void* W, int N, float* Y, int ldy, hipStream_t s, const BNorm& norm) {
-  launch_bgemm<1>(static_cast<const bf16*>(X), M, K, static_cast<const bf16*>(W), N, BF32{Y, ldy}, s, 1, 0, norm);
+void rmsnorm_rows_frag(DType dt, const void* x, const void* g, float eps, int M, int D, void* y, hipStream_t s) {
+  MRT_REQUIRE(D % 32 == 0 && D <= 512 * kFragNormChunks, "fragment norm: D must be a multiple of 32, at most 4096");
+  MRT_DTYPE16(dt, hipLaunchKernelGGL(k_rmsnorm_frag<T>, dim3((M + 3) / 4), dim3(256), 0, s, static_cast<const T*>(x),
+                                     static_cast<const T*>(g), eps, M, D, static_cast<T*>(y)));
+  MRT_HIP_CHECK(hipGetLastError());
 }
 
-void bgemm_resid(const void* X, int M, int K, const void* W, int N, void* R, int ldr, hipStream_t s, float* ssq) {
-  MRT_REQUIRE(ssq == nullptr || N % kBgCols == 0, "batched GEMM: row partials need whole 16-column tiles");
-  launch_bgemm<1>(static_cast<const bf16*>(X), M, K, static_cast<const bf16*>(W), N,
-                  BResid{static_cast<bf16*>(R), ldr, ssq}, s);
+void bgemm_store(DType dt, const void* X, int M, int K, const void* W, int N, void* Y, int ldy, hipStream_t s,
+                 const BNorm& norm) {
+  MRT_DTYPE16(dt, (launch_bgemm<T, 1>(X, M, K, W, N, BStore<T>{static_cast<T*>(Y), ldy}, s, norm)));
 }
 
-void bgemm_qkv(const void* X, int M, int K, const void* W, int HD, void* Q, void* Kc, void* Vc, int H, int Lmax, int pos,
-               const int* pos_ptr, hipStream_t s, const BNorm& norm) {
-  BQKV e{static_cast<bf16*>(Q), static_cast<bf16*>(Kc), static_cast<bf16*>(Vc), HD, H, Lmax, pos, pos_ptr};
-  launch_bgemm<1>(static_cast<const bf16*>(X), M, K, static_cast<const bf16*>(W), 3 * HD, e, s, 1, 0, norm);
+void bgemm_f32(DType dt, const void* X, int M, int K, const void* W, int w_row0, int N, float* Y, int ldy,
+               hipStream_t s, const BNorm& norm, int groups, int w_group_rows) {
+  MRT_DTYPE16(dt, (launch_bgemm<T, 1>(X, M, K, W, N, BF32<T>{Y, ldy}, s, norm, w_row0, groups, w_group_rows)));
 }
 
-void bgemm_qkv_pos(const void* X, int M, int K, const void* W, int HD, void* Q, void* Kc, void* Vc, int H, int Lmax,
-                   int P, hipStream_t s) {
+void bgemm_resid(DType dt, const void* X, int M, int K, const void* W, int N, void* R, void* Rf, float* ssq,
+                 hipStream_t s) {
+  MRT_REQUIRE(N % 32 == 0, "batched GEMM: residual rows must be whole fragments");
+  MRT_DTYPE16(dt, (launch_bgemm<T, 1>(X, M, K, W, N, BResid<T>{static_cast<T*>(R), N, static_cast<T*>(Rf), ssq}, s)));
+}
+
+void bgemm_qkv(DType dt, const void* X, int M, int K, const void* W, int HD, void* Q, void* Kc, void* Vc, int H,
+               int Lmax, int pos, const int* pos_ptr, hipStream_t s, const BNorm& norm) {
+  MRT_DTYPE16(dt, (launch_bgemm<T, 1>(X, M, K, W, 3 * HD,
+                                      BQKV<T>{static_cast<T*>(Q), static_cast<T*>(Kc), static_cast<T*>(Vc), HD, H,
+                                              Lmax, pos, pos_ptr},
+                                      s, norm)));
+}
+
+void bgemm_qkv_pos(DType dt, const void* X, int M, int K, const void* W, int HD, void* Q, void* Kc, void* Vc, int H,
+                   int Lmax, int P, hipStream_t s) {
   MRT_REQUIRE(P >= 1 && M % P == 0 && M / P <= Lmax, "batched GEMM: positions exceed the ring");
-  BQKVPos e{static_cast<bf16*>(Q), static_cast<bf16*>(Kc), static_cast<bf16*>(Vc), HD, H, Lmax, P};
-  launch_bgemm<1>(static_cast<const bf16*>(X), M, K, static_cast<const bf16*>(W), 3 * HD, e, s);
+  MRT_DTYPE16(dt, (launch_bgemm<T, 1>(X, M, K, W, 3 * HD,
+                                      BQKVPos<T>{static_cast<T*>(Q), static_cast<T*>(Kc), static_cast<T*>(Vc), HD, H,
+                                                 Lmax, P},
+                                      s)));
 }
 
-void bgemm_f32_grouped(const void* X, int rows, int K, const void* W, long w_group_stride, int N, float* Y, int ldy,
-                       int groups, hipStream_t s) {
-  launch_bgemm<1>(static_cast<const bf16*>(X), rows, K, static_cast<const bf16*>(W), N, BF32{Y, ldy}, s, groups,
-                  w_group_stride);
-}
-
-void bgemm_geglu(const void* X, int M, int K, const void* W01, int F, void* Hout, int ldh, hipStream_t s,
+void bgemm_geglu(DType dt, const void* X, int M, int K, const void* W01, int F, void* Hout, hipStream_t s,
                  const BNorm& norm) {
   MRT_REQUIRE(F % 32 == 0, "batched GEMM: d_ff must be a multiple of 32 (packed gate/up groups)");
-  launch_bgemm<2>(static_cast<const bf16*>(X), M, K, static_cast<const bf16*>(W01), F,
-                  BGeglu{static_cast<bf16*>(Hout), ldh}, s, 1, 0, norm);
+  MRT_DTYPE16(dt, (launch_bgemm<T, 2>(X, M, K, W01, F, BGeglu<T>{static_cast<T*>(Hout), F}, s, norm)));
 }
 
 }  // namespace mrt

@@ -276,7 +276,7 @@ __global__ __launch_bounds__(64) void k_self_attn(const T* __restrict__ Q, const
                                                   int qpos, const int* __restrict__ qpos_ptr, int pos_rows,
                                                   const T* __restrict__ bias_tab,
                                                   const int* __restrict__ buckets, const T* __restrict__ bias_row,
-                                                  T* __restrict__ out) {
+                                                  int out_nks, T* __restrict__ out) {
   using S = St<T>;
   constexpr int V = S::kVec;
   const int bh = blockIdx.x, b = bh / H, h = bh - b * H, lane = threadIdx.x;
@@ -291,6 +291,8 @@ __global__ __launch_bounds__(64) void k_self_attn(const T* __restrict__ Q, const
     len = qpos + 1;
   }
   const int HD = H * 64;
+  // out_nks > 0: in fragment order with that many k-steps
+  T* dst = out + (out_nks > 0 ? frag_index(b, h * 64 + lane, out_nks) : (size_t)b * HD + h * 64 + lane);
   __shared__ float qs[64];
   __shared__ float ps[kMaxSelfLen];
   const T* Kp = Kc + ((size_t)rb * H + h) * Lmax * 64;
@@ -336,7 +338,7 @@ __global__ __launch_bounds__(64) void k_self_attn(const T* __restrict__ Q, const
     __syncthreads();
     float o = 0.f;
     for (int t = 0; t < len; ++t) o = fmaf(ps[t], S::ld(vs[t * 64 + lane]), o);
-    out[(size_t)b * HD + h * 64 + lane] = S::st(o / sum);
+    *dst = S::st(o / sum);
     return;
   }
   qs[lane] = S::ld(Q[(size_t)b * HD + h * 64 + lane]);
@@ -367,7 +369,7 @@ __global__ __launch_bounds__(64) void k_self_attn(const T* __restrict__ Q, const
   __syncthreads();
   float o = 0.f;
   for (int j = 0; j < len; ++j) o = fmaf(ps[j], S::ld(Vp[(size_t)j * 64 + lane]), o);
-  out[(size_t)b * HD + h * 64 + lane] = S::st(o / sum);
+  *dst = S::st(o / sum);
 }
 
 // Full-sequence self attention (depth_forward_full, model.cpp:243-268): one
@@ -377,7 +379,7 @@ template <typename T>
 __global__ __launch_bounds__(64) void k_full_attn(const T* __restrict__ qkv, int K, int H,
                                                   const T* __restrict__ explicit_bias,
                                                   const T* __restrict__ bias_tab, const int* __restrict__ buckets,
-                                                  int causal, T* __restrict__ out) {
+                                                  int causal, int out_nks, T* __restrict__ out) {
   using S = St<T>;
   const int mh = blockIdx.x, m = mh / H, h = mh - m * H, lane = threadIdx.x;
   const int b = m / K, i = m - b * K;
@@ -403,7 +405,7 @@ __global__ __launch_bounds__(64) void k_full_attn(const T* __restrict__ qkv, int
   __syncthreads();
   float o = 0.f;
   for (int j = 0; j < len; ++j) o = fmaf(ps[j], S::ld(qkv[(size_t)(b * K + j) * ld + 2 * HD + h * 64 + lane]), o);
-  out[(size_t)m * HD + h * 64 + lane] = S::st(o / sum);
+  out[out_nks > 0 ? frag_index(m, h * 64 + lane, out_nks) : (size_t)m * HD + h * 64 + lane] = S::st(o / sum);
 }
 
 // Partial softmax-attention of one (row, head) over one block of keys.
@@ -512,7 +514,7 @@ void self_attn(DType dt, int nb, const void* Q, const void* Kc, const void* Vc, 
 
 void self_attn_at(DType dt, int nb, const void* Q, const void* Kc, const void* Vc, int H, int Lmax, int len,
                   int qpos, const int* qpos_ptr, const void* bias_tab, const int* buckets, void* out,
-                  hipStream_t s, int pos_rows, const void* bias_row) {
+                  hipStream_t s, int pos_rows, const void* bias_row, bool frag_out) {
   MRT_REQUIRE(qpos_ptr == nullptr || Lmax <= kMaxSelfLen, "self_attn: ring longer than the kernel's score buffer");
   MRT_REQUIRE(pos_rows == 0 || (nb % pos_rows == 0 && nb / pos_rows <= Lmax && Lmax <= kMaxSelfLen),
               "self_attn: positions exceed the ring");
@@ -520,7 +522,7 @@ void self_attn_at(DType dt, int nb, const void* Q, const void* Kc, const void* V
               "self_attn: an explicit bias needs a host-known query position");
   MRT_DTYPE_DISPATCH(dt, hipLaunchKernelGGL(k_self_attn<T>, dim3(nb * H), dim3(64), 0, s, (const T*)Q, (const T*)Kc,
                                             (const T*)Vc, H, Lmax, len, qpos, qpos_ptr, pos_rows,
-                                            (const T*)bias_tab, buckets, (const T*)bias_row, (T*)out));
+                                            (const T*)bias_tab, buckets, (const T*)bias_row, frag_out ? H * 2 : 0, (T*)out));
   MRT_HIP_CHECK(hipGetLastError());
 }
 
@@ -549,11 +551,11 @@ void bias_rows(DType dt, const void* table, const int* buckets, int H, int n, vo
 }
 
 void full_attn(DType dt, int nb, int K, int H, const void* qkv, const void* explicit_bias, const void* bias_tab,
-               const int* buckets, bool causal, void* out, hipStream_t s) {
+               const int* buckets, bool causal, void* out, hipStream_t s, bool frag_out) {
   MRT_REQUIRE(nb >= 1 && K >= 1 && K <= 64, "full_attn: K must be in [1, 64]");
   MRT_DTYPE_DISPATCH(dt, hipLaunchKernelGGL(k_full_attn<T>, dim3(nb * K * H), dim3(64), 0, s, (const T*)qkv, K, H,
                                             (const T*)explicit_bias, (const T*)bias_tab, buckets, causal ? 1 : 0,
-                                            (T*)out));
+                                            frag_out ? H * 2 : 0, (T*)out));
   MRT_HIP_CHECK(hipGetLastError());
 }
 

@@ -32,6 +32,13 @@ __device__ __forceinline__ T ld_g(const T* p) {
   return *(const __attribute__((address_space(1))) T*)(p);
 }
 
+// Element (m, k) of an activation matrix of K = 32 nks columns in fragment
+// order (batch.hpp): 16-row x 32-column tiles, each in the operand order of the
+// 16x16x32 matrix instructions.
+__device__ __forceinline__ size_t frag_index(int m, int k, int nks) {
+  return ((size_t)(m >> 4) * nks + (k >> 5)) * 512 + (((k >> 3) & 3) * 16 + (m & 15)) * 8 + (k & 7);
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

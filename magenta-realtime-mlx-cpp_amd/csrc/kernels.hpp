@@ -53,9 +53,10 @@ void self_attn(DType dt, int nb, const void* Q, const void* Kc, const void* Vc, 
 // is non-null (len = qpos + 1; the caller keeps it below Lmax).
 // pos_rows > 0 instead attends all positions of one frame at once: query row
 // b is position b / pos_rows of ring row b % pos_rows, causal (len = pos + 1).
+// frag_out: out in the skinny GEMMs' fragment order (batch.hpp).
 void self_attn_at(DType dt, int nb, const void* Q, const void* Kc, const void* Vc, int H, int Lmax, int len,
                   int qpos, const int* qpos_ptr, const void* bias_tab, const int* buckets, void* out,
-                  hipStream_t s, int pos_rows = 0, const void* bias_row = nullptr);
+                  hipStream_t s, int pos_rows = 0, const void* bias_row = nullptr, bool frag_out = false);
 // The rel-pos bias of steps 0..n-1 (precompute_{temporal,depth}_biases,
 // model.cpp:302-320) back to back: step f's (H, f + 1) block at element
 // H * f * (f + 1) / 2, entry [h][j] = table[bucket(f - j), h].
@@ -64,9 +65,9 @@ void bias_rows(DType dt, const void* table, const int* buckets, int H, int n, vo
 // depth pass): qkv (nb*K, 3*HD) rows m = b*K + i, [q | k | v]; query (b, i)
 // attends keys (b, j) for j <= i (causal) or all j < K, with the bias
 // explicit[(h*K + i)*K + j] when `explicit_bias` is set, else
-// bias_tab[buckets[max(i - j, 0)] * H + h]; scale 1.0; out (nb*K, HD).  K <= 64.
+// bias_tab[buckets[max(i - j, 0)] * H + h]; scale 1.0; out (nb*K, HD), frag_out: in fragment order.  K <= 64.
 void full_attn(DType dt, int nb, int K, int H, const void* qkv, const void* explicit_bias, const void* bias_tab,
-               const int* buckets, bool causal, void* out, hipStream_t s);
+               const int* buckets, bool causal, void* out, hipStream_t s, bool frag_out = false);
 // Cross-attention over S encoder keys (no bias/mask), split over key blocks.
 // ``part`` needs nb*H*nsplit*66 floats.
 void cross_attn(DType dt, int nb, const void* Q, const void* Kc, const void* Vc, int H,

@@ -400,11 +400,14 @@ State::State(Model& model, int rows_, int max_frames, int enc_len)
                               hipHostMallocDefault));
   {  // rows of the full-sequence depth pass and the speculative verification pass (2 L rows)
     const size_t R2 = 2 * L;
+    const size_t Rt = frag_rows(static_cast<int>(R2));  // GEMM inputs may be in fragment order
     sx_ = dalloc(R2 * D * e);
-    sxn_ = dalloc(R2 * std::max(D, FF) * e);
+    sxn_ = dalloc(Rt * std::max(D, FF) * e);
     sqkv_ = dalloc(R2 * 3 * HD * e);
-    satt_ = dalloc(R2 * HD * e);
-    sffh_ = dalloc(R2 * FF * e);
+    satt_ = dalloc(Rt * HD * e);
+    sffh_ = dalloc(Rt * FF * e);
+    sxf_ = dalloc(Rt * D * e);
+    sssq_ = static_cast<float*>(dalloc(R2 * (D / 16 + 1) * 4));
   }
   if (m.dt == DType::BF16) {  // speculative decoding
     const size_t R2 = 2 * L;
@@ -779,6 +782,7 @@ void State::enqueue_decode_spec(const GenOpts& o) {
   sp_rest.noise_frames = o.num_frames;  // one stream: noise row (frame * L + level)
   const char* head0 = static_cast<const char*>(m.lm_head) + static_cast<size_t>(o.codec_offset) * D * esz();
   const int ns = spec_count(o);
+  const FragWeights& fw = *fw_;
   for (int f = 0; f < o.num_frames; ++f) {
     if (f >= ns) {  // past the speculated frames: the plain decode
       enqueue_plain_frame(o, f, sp);
@@ -790,17 +794,19 @@ void State::enqueue_decode_spec(const GenOpts& o) {
     // verification pass: rows 2i + r
     spec_inputs(dt, t_out, m.emb, d_drafts_ + static_cast<size_t>(f) * L, L, D, sx_, stream);
     for (int i = 0; i < c.num_depth_layers; ++i) {
-      const DecoderLayerW& W = m.dep[i];
-      rmsnorm_rows(dt, sx_, W.norm_sa, 1e-6f, R2, D, sxn_, stream);
-      bgemm_qkv_pos(sxn_, R2, D, W.wqkv, HD, sq_, dk(i), dv(i), H, L, rows, stream);
-      self_attn_at(dt, R2, sq_, dk(i), dv(i), H, L, 0, 0, nullptr, m.dbias, m.dbuckets, satt_, stream, rows);
-      bgemm_resid(satt_, R2, HD, W.wo, D, sx_, D, stream);
-      rmsnorm_rows(dt, sx_, W.norm_ff, 1e-6f, R2, D, sxn_, stream);
-      bgemm_geglu(sxn_, R2, D, W.w01, FF, sffh_, FF, stream);
-      bgemm_resid(sffh_, R2, FF, W.wo2, D, sx_, D, stream);
+      const FragLayer& W = fw.dep[i];
+      rmsnorm_rows_frag(dt, sx_, m.dep[i].norm_sa, 1e-6f, R2, D, sxn_, stream);
+      bgemm_qkv_pos(dt, sxn_, R2, D, W.wqkv, HD, sq_, dk(i), dv(i), H, L, rows, stream);
+      self_attn_at(dt, R2, sq_, dk(i), dv(i), H, L, 0, 0, nullptr, m.dbias, m.dbuckets, satt_, stream, rows, nullptr,
+                   true);
+      bgemm_resid(dt, satt_, R2, HD, W.wo, D, sx_, sxf_, sssq_, stream);
+      rmsnorm_rows_frag(dt, sx_, m.dep[i].norm_ff, 1e-6f, R2, D, sxn_, stream);
+      bgemm_geglu(dt, sxn_, R2, D, W.w01, FF, sffh_, stream);
+      bgemm_resid(dt, sffh_, R2, FF, W.wo2, D, sx_, sxf_, sssq_, stream);
     }
-    rmsnorm_rows(dt, sx_, m.dec_norm, 1e-6f, R2, D, sxn_, stream);
-    bgemm_f32_grouped(sxn_, rows, D, head0, static_cast<long>(C) * D, C, slog_, C, L, stream);
+    // level i's 1024-row head slice for rows 2i, 2i + 1
+    rmsnorm_rows_frag(dt, sx_, m.dec_norm, 1e-6f, R2, D, sxn_, stream);
+    bgemm_f32(dt, sxn_, rows, D, fw.head, o.codec_offset, C, slog_, C, stream, {}, L, C);
     draw_levels(slog_, sp_all, f, L, sdrawn_, stream);
     int* decided = sdecided_ + f;
     sp_rest.decided = decided;
@@ -1015,6 +1021,25 @@ void State::depth_forward_full(const void* emb, int k, const void* bias, bool ca
   const int D = c.d_model, HD = c.hd(), FF = c.d_ff, H = c.num_heads, M = rows * k;
   MRT_HIP_CHECK(hipSetDevice(m.device));
   copy(sx_, emb, static_cast<size_t>(M) * D * esz());
+  // 16-bit rows that the skinny GEMMs hold: M <= 32 fills no tile of the
+  // encoder's GEMM (its 1,024-wide outputs ran 8 blocks, 16 us each; 292 us a
+  // call in all at k = 16, 125 us here)
+  if (m.frag_shapes() && M <= kBatchRows && c.num_depth_layers > 0) {
+    const FragWeights& fw = *m.frag_weights(true, stream);
+    const BNorm bn{sssq_, 1e-6f};
+    for (int i = 0; i < c.num_depth_layers; ++i) {
+      const FragLayer& W = fw.dep[i];
+      if (i == 0) rmsnorm_rows_frag(dt, sx_, m.dep[i].norm_sa, 1e-6f, M, D, sxn_, stream);
+      bgemm_store(dt, i == 0 ? sxn_ : sxf_, M, D, W.wqkv, 3 * HD, sqkv_, 3 * HD, stream, i == 0 ? BNorm{} : bn);
+      full_attn(dt, rows, k, H, sqkv_, bias, m.dbias, m.dbuckets, causal, satt_, stream, true);
+      bgemm_resid(dt, satt_, M, HD, W.wo, D, sx_, sxf_, sssq_, stream);
+      bgemm_geglu(dt, sxf_, M, D, W.w01, FF, sffh_, stream, bn);
+      bgemm_resid(dt, sffh_, M, FF, W.wo2, D, sx_, sxf_, sssq_, stream);
+    }
+    bgemm_f32(dt, sxf_, M, D, fw.head, 0, c.vocab_size, logits, c.vocab_size, stream, bn);
+    MRT_HIP_CHECK(hipStreamSynchronize(stream));
+    return;
+  }
   auto gemm_to = [&](const void* A, const void* W, int N, int K, GemmEpi kind, void* C) {
     GemmEpiArgs e;
     e.kind = kind;
@@ -1111,6 +1136,52 @@ void State::reset_cache(int kind) {
     temporal_len_ = 0;
   else
     depth_len_ = 0;
+}
+
+const FragWeights* Model::frag_weights(bool folded, hipStream_t s) {
+  MRT_REQUIRE(frag_shapes(), "fragment weights: 16-bit model with widths that are multiples of 32");
+  std::lock_guard<std::mutex> lock(frag_mu_);
+  if (frag_built_[folded]) return &frag_[folded];
+  MRT_HIP_CHECK(hipSetDevice(device));
+  const int D = cfg.d_model, HD = cfg.hd(), F = cfg.d_ff;
+  std::vector<void*> bufs;
+  FragWeights fw;
+  try {
+    auto place = [&](const void* W, const void* g, int N, int K, bool pairs = false) -> const void* {
+      void* out = nullptr;
+      MRT_HIP_CHECK(hipMalloc(&out, frag_weights_elems(N, K) * esz));
+      bufs.push_back(out);
+      mrt::frag_weights(dt, W, folded ? g : nullptr, N, K, pairs, out, s);
+      return out;
+    };
+    auto stack = [&](const std::vector<DecoderLayerW>& ws, bool temporal, std::vector<FragLayer>& out) {
+      for (size_t i = 0; i < ws.size(); ++i) {
+        const DecoderLayerW& w = ws[i];
+        FragLayer f;
+        f.wqkv = place(w.wqkv, i > 0 ? w.norm_sa : nullptr, 3 * HD, D);
+        f.wo = place(w.wo, nullptr, D, HD);
+        if (temporal) {
+          f.wq_c = place(w.wq_c, w.norm_ca, HD, D);
+          f.wo_c = place(w.wo_c, nullptr, D, HD);
+        }
+        f.w01 = place(w.w01, w.norm_ff, 2 * F, D, true);
+        f.wo2 = place(w.wo2, nullptr, D, F);
+        out.push_back(f);
+      }
+    };
+    if (folded) stack(tmp, true, fw.tmp);
+    stack(dep, false, fw.dep);
+    fw.head = place(lm_head, dep.empty() ? nullptr : dec_norm, cfg.vocab_size, D);
+    MRT_HIP_CHECK(hipStreamSynchronize(s));
+  } catch (...) {
+    (void)hipStreamSynchronize(s);
+    for (void* p : bufs) (void)hipFree(p);
+    throw;
+  }
+  allocs_.insert(allocs_.end(), bufs.begin(), bufs.end());
+  frag_[folded] = std::move(fw);
+  frag_built_[folded] = true;
+  return &frag_[folded];
 }
 
 const void* Model::depth_qkv_table(int codebook, int offset, hipStream_t s) {
@@ -1317,6 +1388,7 @@ void State::generate(const int32_t* enc_tokens_host, const GenOpts& o, int32_t* 
   dec_launches_ = persistent() ? decode_launches(o) : 0;
   // built once per (codebook, offset) before any capture; waits for the stream then
   qkv_table_ = frame_kernel_ && qkv_table_on_ ? m.depth_qkv_table(o.codebook, o.codec_offset, stream) : nullptr;
+  if (spec_drafts_) fw_ = m.frag_weights(false, stream);  // likewise
   hipGraphExec_t exec = o.use_graph ? decode_graph(o) : nullptr;
   {
     // persistent grids of other states on this device run before or after

@@ -63,6 +63,17 @@ struct DecoderLayerW {
   const void *norm_sa, *wqkv, *wo, *norm_ca, *wq_c, *wo_c, *norm_ff, *w01, *wo2;
 };
 
+// The decoder matrices of a layer in the skinny GEMMs' fragment order
+// (batch.hpp).  Folded: the norm weights of the input multiplied in where the
+// input comes from a residual GEMM: every wq_c and w01, and wqkv past layer 0.
+struct FragLayer {
+  const void *wqkv = nullptr, *wo = nullptr, *wq_c = nullptr, *wo_c = nullptr, *w01 = nullptr, *wo2 = nullptr;
+};
+struct FragWeights {
+  std::vector<FragLayer> tmp, dep;
+  const void* head = nullptr;  // lm_head (vocab rows); folded: times decoder_norm if there are depth layers
+};
+
 struct GenOpts;
 
 class Model {
@@ -131,6 +142,18 @@ class Model {
   // levels < 2 (the decode then computes layer 0).
   const void* depth_qkv_table(int codebook, int offset, hipStream_t s);
   static constexpr size_t kMaxQkvTables = 4;
+  // The decoder stacks and lm_head in fragment order (16-bit models with
+  // d_model, heads * 64 and d_ff multiples of 32): as many bytes again as the
+  // matrices themselves, built on first use on `s` (waits for it; never during
+  // a capture) and kept with the model.  folded: both stacks, for inputs that
+  // are normalised by scaling the sums (BNorm); else the depth stack and lm_head
+  // alone, for normalised inputs rounded as the persistent kernels round them
+  // (the speculative verification pass, whose draws are held against theirs).
+  const FragWeights* frag_weights(bool folded, hipStream_t s);
+  bool frag_shapes() const {
+    return dt != DType::F32 && cfg.d_model % 32 == 0 && cfg.d_model <= 4096 && cfg.hd() % 32 == 0 &&
+           cfg.d_ff % 32 == 0;
+  }
   static constexpr int kQkvChunkRows = 2048;
 
  private:
@@ -141,6 +164,9 @@ class Model {
   };
   std::mutex qkv_mu_;
   std::vector<QkvTable> qkv_tables_;
+  std::mutex frag_mu_;
+  FragWeights frag_[2];  // plain, folded
+  bool frag_built_[2] = {false, false};
   void* qkv_ws_ = nullptr;  // build workspace of the tables (kQkvChunkRows x d_model)
   std::vector<float> pe_host_;  // fp32 sinusoid table (max_encoder_length, d_model)
   static constexpr int kEmbedChunk = 4096;
@@ -308,6 +334,9 @@ class State {
   void *sx_ = nullptr, *sxn_ = nullptr, *sq_ = nullptr, *satt_ = nullptr, *sffh_ = nullptr, *sqkv_ = nullptr;
   float* slog_ = nullptr;
   int *sdrawn_ = nullptr, *sdecided_ = nullptr;  // sdecided_: (F) the accepted count n of each frame
+  const FragWeights* fw_ = nullptr;  // the model's, once a call speculates
+  void* sxf_ = nullptr;     // the rows of sx_ in fragment order, and their partials (skinny GEMMs)
+  float* sssq_ = nullptr;
   float spec_acc_ = -1.f;  // share of the last call's levels taken from the verification pass
   void* sfm_ = nullptr;  // scratch frame-mean rows of the sampler (the spec path writes its own)
   void print_trace();

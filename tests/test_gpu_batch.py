@@ -378,3 +378,28 @@ def test_batch_32_streams_full_chunk_teacher_forced(full):
         assert max(terrs) <= BF16_TOL, (s, max(terrs))
         agree = assert_argmax_flips_are_near_ties(sl, orec["slices"])
         print(f"stream {s}: max slice rel-err {errs.max():.3e}, argmax agreement {agree:.3f}")
+
+
+@pytest.mark.parametrize("B", [1, 8, 9, 16, 17, 32])
+def test_batch_row_tiles(tiny, B):
+    """Row counts at the edges of the GEMMs' 16-row tiles: stream b of a batch
+    of B decodes bit for bit as it does alone (the products of a row and their
+    order do not depend on the other rows), here on the level logits."""
+    import torch
+    mrt_df = tiny["mrt_df"]
+    F, L, C = 2, 16, C_TINY
+    teacher = _teacher(np.random.default_rng(21), B, F, C)
+    enc = np.concatenate([tiny["toks"][b % 3] for b in range(B)], axis=0)
+
+    def slices(streams):
+        b = mrt_df.Batch(tiny["model"], len(streams), max_frames=F)
+        rec = dict(slices=torch.zeros((F, L, 2 * len(streams), C), dtype=torch.float32, device="cuda"))
+        b.generate_tokens(np.concatenate([enc[2 * s:2 * s + 2] for s in streams], axis=0), _opts(tiny, F),
+                          seeds=list(streams), teacher=teacher[list(streams)], record=rec)
+        out = rec["slices"].cpu().numpy()
+        b.close()
+        return out
+
+    whole = slices(range(B))
+    for s in sorted({0, B // 2, B - 1}):
+        np.testing.assert_array_equal(whole[:, :, 2 * s:2 * s + 2], slices([s]))
