@@ -23,6 +23,7 @@ SOURCES = [
     "decode_kernels.hip",
     "sample_kernels.hip",
     "encoder_kernels.hip",
+    "split_kernels.hip",
     "persist_kernels.hip",
     "stream_kernels.hip",
     "batch_kernels.hip",

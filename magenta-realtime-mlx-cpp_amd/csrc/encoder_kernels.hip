@@ -4,16 +4,16 @@
 //
 // GEMM operands are both K-contiguous ("NT": activations (M, K) row-major,
 // weights (N, K) row-major as the bundle stores them).  bf16 and fp16 use
-// v_mfma_f32_32x32x16_{bf16,f16} with LDS-double-buffered tiles; fp32 uses a
-// VALU tile (parity mode).
-#include <atomic>
+// v_mfma_f32_32x32x16_{bf16,f16} with LDS-double-buffered tiles; fp32 splits its
+// operands into three bf16 parts for the same instruction (split_gemm.hpp), or
+// uses a VALU tile where the shapes do not fit.
 #include <cmath>
-#include <mutex>
-#include <set>
-#include <utility>
+#include <type_traits>
 
 #include "device_utils.hpp"
 #include "kernels.hpp"
+#include "mfma_ring.hpp"
+#include "split_gemm.hpp"
 
 namespace mrt {
 namespace {
@@ -152,9 +152,14 @@ struct GemmOut {
     const float gl = gelu_t<T>(S::rnd(g));
     C[(size_t)m * (N / 2) + j] = S::st(gl * S::rnd(u));
   }
+  // The same in fp32, stored as split rows (the next split GEMM's input).
+  __device__ __forceinline__ void put_geglu_split(int m, int n, float g, float u) const {
+    const int j = (n >> 6) * 32 + (n & 31);
+    store_split(static_cast<bf16*>(a.C), split_index(m, j, N / 2), gelu_t<float>(g) * u);
+  }
 };
 
-// ---- VALU tiled GEMM (fp32 parity path; also the 16-bit fallback) -----------------
+// ---- VALU tiled GEMM (shapes the matrix-core tiles do not take) ---------------------
 // 64x64 tile, BK 16, 256 threads, 4x4 outputs per thread at rows ty+16i and
 // columns tx+16j, so columns j and j+2 form a packed gate/up pair.
 template <typename T>
@@ -207,7 +212,6 @@ __global__ __launch_bounds__(256) void k_gemm_valu(const T* __restrict__ A, cons
 }
 
 // ---- 16-bit MFMA GEMM ----------------------------------------------------------------
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef float f32x8_t __attribute__((ext_vector_type(8)));
 
 // The 32x32x16 matrix instruction of each 16-bit storage type (fp32 accumulators).
@@ -235,18 +239,6 @@ constexpr int kBN = 128, kBK = 64, kStages = 2;
 // read (and 16 consecutive lanes of any ds_read_b128) fall in distinct banks.
 __device__ __forceinline__ int swz(int r) { return (r ^ (r >> 3)) & 7; }
 
-// s_waitcnt immediate waiting for vmcnt <= n (expcnt and lgkmcnt left alone).
-constexpr int vm_wait_imm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
-
-// Workgroup barrier of the global -> LDS rings: every LDS read this wave has
-// issued has returned (so another wave may refill that stage after the
-// barrier), then the waves meet.  Unlike __syncthreads() it does not wait for
-// this wave's loads still in flight to later stages (a release fence would
-// wait for every outstanding LDS write, direct-to-LDS loads included): the
-// stage about to be read is awaited with an explicit vmcnt before it.  The
-// asm is a compiler barrier for memory operations.
-__device__ __forceinline__ void ring_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // Epilogue of the MFMA GEMMs.  Accumulator r of tile (i, j) of a lane holds
 // row mb + 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4 and column
 // nb + 32 j + lane % 32 (j = 2p / 2p + 1: gate / up columns of gated-GELU pair p).
@@ -271,6 +263,18 @@ __device__ __forceinline__ void mfma_epilogue(const GemmOut<T>& out, const f32x1
 #pragma unroll
             for (int r = 0; r < 16; ++r)
               if (row(i, r) < M) out.put_geglu(row(i, r), nb + 64 * pj + col, acc[i][2 * pj][r], acc[i][2 * pj + 1][r]);
+      }
+      break;
+    case GemmEpi::GegluSplit:
+      if constexpr (NJ % 2 == 0 && std::is_same<T, float>::value) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int pj = 0; pj < NJ / 2; ++pj)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+              if (row(i, r) < M)
+                out.put_geglu_split(row(i, r), nb + 64 * pj + col, acc[i][2 * pj][r], acc[i][2 * pj + 1][r]);
       }
       break;
     case GemmEpi::Resid:
@@ -346,20 +350,6 @@ __device__ __forceinline__ void mfma_epilogue(const GemmOut<T>& out, const f32x1
 // Blocks per CU the register budget is sized for: two wherever the LDS ring
 // leaves room for two (at most 80 KB), else one.
 constexpr int gemm_min_blocks(int BM, int S, int BN) { return S * (BM + BN) * 128 <= 80 * 1024 ? 2 : 1; }
-
-// Tile of block L of a 1-D grid in the XCD-grouped order: blocks are dealt to
-// the 8 XCDs in turn (L % 8), each XCD takes a contiguous range of tile ids,
-// and tile ids run down GM row tiles before the next column tile, so the
-// blocks that one XCD runs together share GM A tiles and a few B tiles in its
-// L2.  A bijection of [0, tm * tn).
-__device__ __forceinline__ void grouped_tile(int L, int tm, int tn, int GM, int& mt, int& nt) {
-  const int tiles = tm * tn, x = L & 7, q = tiles >> 3, rem = tiles & 7;
-  const int pid = x * q + min(x, rem) + (L >> 3);
-  const int g = pid / (GM * tn), first = g * GM, gsz = min(tm - first, GM);
-  const int w = pid - g * GM * tn;
-  mt = first + w % gsz;
-  nt = w / gsz;
-}
 
 // GM = 0: block (x, y) of a 2-D grid computes tile (y, x); GM > 0: a 1-D grid
 // in the grouped_tile order.
@@ -448,32 +438,6 @@ __global__ __launch_bounds__(256, gemm_min_blocks(BM, S, BN)) void k_gemm_mfma(c
   __builtin_amdgcn_s_waitcnt(vm_wait_imm(0));  // no copy into LDS outlives the block
 
   mfma_epilogue<T, MI, NJ>(out, acc, M, m0 + wm * (BM / 2), n0 + wn * (BN / 2));
-}
-
-// Dynamic LDS above 64 KB needs an explicit allowance, once per kernel and device.
-void allow_dynamic_lds(const void* fn, size_t bytes) {
-  static std::mutex mu;
-  static std::set<std::pair<const void*, int>> done;
-  int dev = 0;
-  MRT_HIP_CHECK(hipGetDevice(&dev));
-  std::lock_guard<std::mutex> g(mu);
-  if (done.count({fn, dev})) return;
-  MRT_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
-  done.insert({fn, dev});
-}
-
-// Compute units of the current device (cached per device).
-int device_cus() {
-  constexpr int kMaxDev = 64;
-  static std::atomic<int> cache[kMaxDev] = {};
-  int dev = 0;
-  MRT_HIP_CHECK(hipGetDevice(&dev));
-  int v = (dev >= 0 && dev < kMaxDev) ? cache[dev].load(std::memory_order_relaxed) : 0;
-  if (v == 0) {
-    MRT_HIP_CHECK(hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev));
-    if (dev >= 0 && dev < kMaxDev) cache[dev].store(v, std::memory_order_relaxed);
-  }
-  return v;
 }
 
 template <typename T, int BM, int S = kStages, int BN = kBN, int GM = 0>
@@ -582,6 +546,54 @@ void launch_gemm_big(const T* A, const T* B, int M, int N, int K, const GemmOut<
   constexpr size_t lds = (size_t)kStages * kGBStage;
   allow_dynamic_lds(reinterpret_cast<const void*>(&k_gemm_big<T>), lds);
   hipLaunchKernelGGL(k_gemm_big<T>, dim3(N / kGB, (M + kGB - 1) / kGB), dim3(64 * kGBWaves), lds, s, A, B, M, N, K, out);
+}
+
+// C = A B^T in fp32 from split operands (split_gemm.hpp) with the GemmOut
+// epilogue, BM x BN x 32 tiles in the XCD-grouped order, 4 waves in a 2 x 2 grid,
+// one block per CU.  Rows past M read row M - 1 (not stored); N % BN == 0.
+template <int BM, int BN, int S>
+__global__ __launch_bounds__(256, 1) void k_gemm_split(const bf16* __restrict__ A, const bf16* __restrict__ B, int M,
+                                                       int N, int K, GemmOut<float> out) {
+  using Tile = SplitTile<BM, BN, 2, 2, S>;
+  extern __shared__ __align__(16) unsigned char lds[];
+  int mt, nt;
+  grouped_tile(blockIdx.x, (M + BM - 1) / BM, N / BN, 4, mt, nt);
+  const int m0 = mt * BM, n0 = nt * BN;
+  const size_t ldk = (size_t)(K >> 5) * kSplitGroup;
+  const bf16* a0[Tile::LA];
+  const bf16* b0[Tile::LB];
+#pragma unroll
+  for (int q = 0; q < Tile::LA; ++q) {
+    int row, chunk;
+    Tile::load_pos(q, row, chunk);
+    a0[q] = A + (size_t)min(m0 + row, M - 1) * ldk + chunk * 8;
+  }
+#pragma unroll
+  for (int q = 0; q < Tile::LB; ++q) {
+    int row, chunk;
+    Tile::load_pos(q, row, chunk);
+    b0[q] = B + (size_t)(n0 + row) * ldk + chunk * 8;
+  }
+  f32x16_t acc[Tile::MI][Tile::NJ];
+  Tile::run(lds, 0, K >> 5,
+            [&](int kt, const bf16* (&ap)[Tile::LA], const bf16* (&bp)[Tile::LB]) {
+#pragma unroll
+              for (int q = 0; q < Tile::LA; ++q) ap[q] = a0[q] + (size_t)kt * kSplitGroup;
+#pragma unroll
+              for (int q = 0; q < Tile::LB; ++q) bp[q] = b0[q] + (size_t)kt * kSplitGroup;
+            },
+            acc);
+  const int wid = threadIdx.x >> 6;
+  mfma_epilogue<float, Tile::MI, Tile::NJ>(out, acc, M, m0 + (wid >> 1) * (BM / 2), n0 + (wid & 1) * (BN / 2));
+}
+
+template <int BM, int BN, int S>
+void launch_gemm_split(const bf16* A, const bf16* B, int M, int N, int K, const GemmOut<float>& out, hipStream_t s) {
+  using Tile = SplitTile<BM, BN, 2, 2, S>;
+  allow_dynamic_lds(reinterpret_cast<const void*>(&k_gemm_split<BM, BN, S>), Tile::kLds);
+  const long tiles = (long)((M + BM - 1) / BM) * (N / BN);
+  MRT_REQUIRE(tiles <= 0x7fffffffL, "split gemm: too many tiles");
+  hipLaunchKernelGGL((k_gemm_split<BM, BN, S>), dim3((unsigned)tiles), dim3(256), Tile::kLds, s, A, B, M, N, K, out);
 }
 
 // ---- encoder self-attention (bidirectional, no mask, no bias, scale 1.0) -------------
@@ -961,6 +973,32 @@ void gemm(DType dt, const void* A, const void* B, int M, int N, int K, const Gem
   if (e.kind == GemmEpi::CrossKV)
     MRT_REQUIRE(e.HD == e.H * 64 && N % e.HD == 0 && M == e.nb * e.S, "gemm: bad cross-KV shape");
   MRT_DTYPE_DISPATCH(dt, gemm_t<T>(static_cast<const T*>(A), static_cast<const T*>(B), M, N, K, e, s, allow_mfma));
+  MRT_HIP_CHECK(hipGetLastError());
+}
+
+bool gemm_split_fits(int N, int K) { return N % kBN == 0 && K % 32 == 0 && K >= 32; }
+
+void gemm_split(const bf16* A, const bf16* B, int M, int N, int K, const GemmEpiArgs& e, hipStream_t s) {
+  MRT_REQUIRE(M >= 1 && gemm_split_fits(N, K), "split gemm: N must be a multiple of 128, K of 32");
+  if (e.kind == GemmEpi::CrossKV)
+    MRT_REQUIRE(e.HD == e.H * 64 && N % e.HD == 0 && M == e.nb * e.S, "gemm: bad cross-KV shape");
+  const GemmOut<float> out{e, N};
+  // The tile whose rounds over the CUs (one block each) take the fewest
+  // products; the 64-row tile reads more LDS a product (a factor of 1.15).
+  const long cus = device_cus();
+  auto cost = [&](int bm, int bn, double f) {
+    const long tiles = (long)((M + bm - 1) / bm) * (N / bn);
+    return (double)((tiles + cus - 1) / cus) * bm * bn * f;
+  };
+  const bool pairs = e.kind == GemmEpi::GegluSplit || e.kind == GemmEpi::Geglu;  // 64-column wave tiles
+  const double c64 = cost(64, 128, 1.15), c128 = cost(128, 128, 1.0);
+  const double cw = !pairs && N % 192 == 0 ? cost(128, 192, 1.0) : 1e30;
+  if (cw <= c128 && cw <= c64)
+    launch_gemm_split<128, 192, 2>(A, B, M, N, K, out, s);
+  else if (c128 <= c64)
+    launch_gemm_split<128, 128, 3>(A, B, M, N, K, out, s);
+  else
+    launch_gemm_split<64, 128, 4>(A, B, M, N, K, out, s);
   MRT_HIP_CHECK(hipGetLastError());
 }
 

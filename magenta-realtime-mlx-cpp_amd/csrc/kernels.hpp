@@ -159,6 +159,7 @@ enum class GemmEpi : int {
   CrossKV = 3,  // n = (layer*2 + kv)*HD + h*64 + d; m = b*S + s ->
                 //   C[(((layer*2+kv)*nb + b)*H + h)*S + s][d]
   StoreF32 = 4, // C (M, N) fp32, each value rounded to the model dtype first (logits)
+  GegluSplit = 5, // fp32: as Geglu, C split rows (split_gemm.hpp) of N/2 values
 };
 struct GemmEpiArgs {
   GemmEpi kind = GemmEpi::Store;
@@ -167,6 +168,14 @@ struct GemmEpiArgs {
 };
 void gemm(DType dt, const void* A, const void* B, int M, int N, int K, const GemmEpiArgs& e,
           hipStream_t s, bool allow_mfma = true);
+
+// The fp32 GEMM from split rows (split_gemm.hpp; six bytes a value): A (M, K),
+// B (N, K), N % 128 == 0, K % 32 == 0, and the row norm and encoder attention
+// that produce them (attention from fp32 q/k/v).
+bool gemm_split_fits(int N, int K);
+void gemm_split(const bf16* A, const bf16* B, int M, int N, int K, const GemmEpiArgs& e, hipStream_t s);
+void rmsnorm_rows_split(const float* x, const float* g, float eps, int M, int D, bf16* y, hipStream_t s);
+void encoder_attn_split(const float* qkv, int nb, int S, int H, bf16* out, hipStream_t s);
 
 // Bidirectional encoder self-attention, no mask, no bias, scale 1.0.
 // qkv (nb*S, 3*HD) row-major [q | k | v]; out (nb*S, HD).

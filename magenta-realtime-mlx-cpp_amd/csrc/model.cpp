@@ -9,6 +9,7 @@
 
 #include "batch.hpp"
 #include "kernels.hpp"
+#include "split_gemm.hpp"
 #include "persist.hpp"
 #include "spec.hpp"
 
@@ -367,10 +368,11 @@ State::State(Model& model, int rows_, int max_frames, int enc_len)
   const size_t M = static_cast<size_t>(rows) * S, e = esz();
   d_enc_tok = static_cast<int*>(dalloc(M * 4));
   ex = dalloc(M * D * e);
-  exn = dalloc(M * D * e);
+  const size_t ei = encoder_input_bytes(m.dt);
+  exn = dalloc(M * D * ei);
   eqkv = dalloc(M * 3 * HD * e);
-  eattn = dalloc(M * HD * e);
-  effh = dalloc(M * FF * e);
+  eattn = dalloc(M * HD * ei);
+  effh = dalloc(M * FF * ei);
   enc_out = dalloc(M * D * e);
   cross = dalloc(static_cast<size_t>(c.num_temporal_layers) * 2 * rows * H * S * 64 * e);
   tkv = dalloc(static_cast<size_t>(c.num_temporal_layers) * 2 * rows * H * F * 64 * e);
@@ -925,12 +927,32 @@ void State::encode(const int32_t* tokens_host) {
   encode_device();
 }
 
-void run_encoder(const Model& m, const EncoderBufs& b, hipStream_t s) {
+void run_encoder(Model& m, const EncoderBufs& b, hipStream_t s) {
   const Config& c = m.cfg;
   const int M = b.rows * b.S;
   const DType dt = m.dt;
   const int D = c.d_model, HD = c.hd(), FF = c.d_ff, H = c.num_heads;
   encoder_embed(dt, m.emb, m.pe, b.tok, M, b.S, D, b.ex, s);
+  if (const SplitWeights* sw = m.split_weights(s)) {
+    auto* xn = static_cast<bf16*>(b.exn);
+    auto* at = static_cast<bf16*>(b.eattn);
+    auto* fh = static_cast<bf16*>(b.effh);
+    auto* x = static_cast<float*>(b.ex);
+    for (size_t i = 0; i < m.enc.size(); ++i) {
+      const EncoderLayerW& L = m.enc[i];
+      const SplitLayer& W = sw->enc[i];
+      rmsnorm_rows_split(x, static_cast<const float*>(L.norm_attn), 1e-6f, M, D, xn, s);
+      gemm_split(xn, W.wqkv, M, 3 * HD, D, {GemmEpi::Store, b.eqkv}, s);
+      encoder_attn_split(static_cast<const float*>(b.eqkv), b.rows, b.S, H, at, s);
+      gemm_split(at, W.wo, M, D, HD, {GemmEpi::Resid, x}, s);
+      rmsnorm_rows_split(x, static_cast<const float*>(L.norm_ff), 1e-6f, M, D, xn, s);
+      gemm_split(xn, W.w01, M, 2 * FF, D, {GemmEpi::GegluSplit, fh}, s);
+      gemm_split(fh, W.wo2, M, D, FF, {GemmEpi::Resid, x}, s);
+    }
+    rmsnorm_rows(dt, b.ex, m.enc_norm, 1e-6f, M, D, b.enc_out, s);
+    project_cross_kv(m, b.enc_out, b.rows, b.S, b.cross, b.exn, s);
+    return;
+  }
   for (const auto& L : m.enc) {
     rmsnorm_rows(dt, b.ex, L.norm_attn, 1e-6f, M, D, b.exn, s);
     gemm(dt, b.exn, L.wqkv, M, 3 * HD, D, {GemmEpi::Store, b.eqkv}, s);
@@ -941,10 +963,10 @@ void run_encoder(const Model& m, const EncoderBufs& b, hipStream_t s) {
     gemm(dt, b.effh, L.wo2, M, D, FF, {GemmEpi::Resid, b.ex}, s);
   }
   rmsnorm_rows(dt, b.ex, m.enc_norm, 1e-6f, M, D, b.enc_out, s);
-  project_cross_kv(m, b.enc_out, b.rows, b.S, b.cross, s);
+  project_cross_kv(m, b.enc_out, b.rows, b.S, b.cross, b.exn, s);
 }
 
-void project_cross_kv(const Model& m, const void* enc_out, int rows, int S, void* cross, hipStream_t s) {
+void project_cross_kv(Model& m, const void* enc_out, int rows, int S, void* cross, void* work, hipStream_t s) {
   const Config& c = m.cfg;
   if (c.num_temporal_layers == 0) return;
   GemmEpiArgs e;
@@ -954,7 +976,14 @@ void project_cross_kv(const Model& m, const void* enc_out, int rows, int S, void
   e.H = c.num_heads;
   e.S = S;
   e.HD = c.hd();
-  gemm(m.dt, enc_out, m.wkv_cross, rows * S, c.num_temporal_layers * 2 * c.hd(), c.d_model, e, s);
+  const int N = c.num_temporal_layers * 2 * c.hd();
+  if (const SplitWeights* sw = m.split_weights(s)) {
+    auto* xs = static_cast<bf16*>(work);
+    split_rows(static_cast<const float*>(enc_out), static_cast<long>(rows) * S, c.d_model, xs, s);
+    gemm_split(xs, sw->wkv_cross, rows * S, N, c.d_model, e, s);
+  } else {
+    gemm(m.dt, enc_out, m.wkv_cross, rows * S, N, c.d_model, e, s);
+  }
 }
 
 // The encoder on the token ids already in d_enc_tok (range-checked by whoever
@@ -984,7 +1013,7 @@ void State::encode_device() {
 }
 
 void State::project_cross(const void* src) {
-  project_cross_kv(m, src, rows, S, cross, stream);
+  project_cross_kv(m, src, rows, S, cross, exn, stream);
   cross_ready_ = true;
 }
 
@@ -1136,6 +1165,44 @@ void State::reset_cache(int kind) {
     temporal_len_ = 0;
   else
     depth_len_ = 0;
+}
+
+bool Model::split_shapes() const {
+  const int D = cfg.d_model, HD = cfg.hd(), F = cfg.d_ff;
+  return dt == DType::F32 && D <= 4096 && gemm_split_fits(3 * HD, D) && gemm_split_fits(D, HD) &&
+         gemm_split_fits(2 * F, D) && gemm_split_fits(D, F);
+}
+
+const SplitWeights* Model::split_weights(hipStream_t s) {
+  if (!split_shapes()) return nullptr;
+  std::lock_guard<std::mutex> lock(split_mu_);
+  if (split_built_) return &split_;
+  MRT_HIP_CHECK(hipSetDevice(device));
+  const int D = cfg.d_model, HD = cfg.hd(), F = cfg.d_ff;
+  std::vector<void*> bufs;
+  SplitWeights sw;
+  try {
+    auto place = [&](const void* W, int N, int K) -> const bf16* {
+      void* out = nullptr;
+      MRT_HIP_CHECK(hipMalloc(&out, static_cast<size_t>(N) * K * 6));
+      bufs.push_back(out);
+      split_rows(static_cast<const float*>(W), N, K, static_cast<bf16*>(out), s);
+      return static_cast<bf16*>(out);
+    };
+    for (const EncoderLayerW& w : enc)
+      sw.enc.push_back(SplitLayer{place(w.wqkv, 3 * HD, D), place(w.wo, D, HD), place(w.w01, 2 * F, D),
+                                  place(w.wo2, D, F)});
+    if (cfg.num_temporal_layers > 0) sw.wkv_cross = place(wkv_cross, cfg.num_temporal_layers * 2 * HD, D);
+    MRT_HIP_CHECK(hipStreamSynchronize(s));
+  } catch (...) {
+    (void)hipStreamSynchronize(s);
+    for (void* p : bufs) (void)hipFree(p);
+    throw;
+  }
+  allocs_.insert(allocs_.end(), bufs.begin(), bufs.end());
+  split_ = std::move(sw);
+  split_built_ = true;
+  return &split_;
 }
 
 const FragWeights* Model::frag_weights(bool folded, hipStream_t s) {

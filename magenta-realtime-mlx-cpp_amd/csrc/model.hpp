@@ -74,6 +74,16 @@ struct FragWeights {
   const void* head = nullptr;  // lm_head (vocab rows); folded: times decoder_norm if there are depth layers
 };
 
+// An fp32 model's encoder matrices and cross K/V projection as split rows
+// (split_gemm.hpp).
+struct SplitLayer {
+  const bf16 *wqkv = nullptr, *wo = nullptr, *w01 = nullptr, *wo2 = nullptr;
+};
+struct SplitWeights {
+  std::vector<SplitLayer> enc;
+  const bf16* wkv_cross = nullptr;
+};
+
 struct GenOpts;
 
 class Model {
@@ -150,6 +160,11 @@ class Model {
   // alone, for normalised inputs rounded as the persistent kernels round them
   // (the speculative verification pass, whose draws are held against theirs).
   const FragWeights* frag_weights(bool folded, hipStream_t s);
+  // The split encoder of an fp32 model (1.5 times its matrices' bytes), kept in
+  // the same way; nullptr for 16-bit models and widths the split GEMM does not
+  // take.
+  const SplitWeights* split_weights(hipStream_t s);
+  bool split_shapes() const;
   bool frag_shapes() const {
     return dt != DType::F32 && cfg.d_model % 32 == 0 && cfg.d_model <= 4096 && cfg.hd() % 32 == 0 &&
            cfg.d_ff % 32 == 0;
@@ -164,6 +179,9 @@ class Model {
   };
   std::mutex qkv_mu_;
   std::vector<QkvTable> qkv_tables_;
+  std::mutex split_mu_;
+  SplitWeights split_;
+  bool split_built_ = false;
   std::mutex frag_mu_;
   FragWeights frag_[2];  // plain, folded
   bool frag_built_[2] = {false, false};
@@ -181,14 +199,17 @@ class Model {
 struct EncoderBufs {
   int rows = 0, S = 0;
   int* tok = nullptr;  // (rows, S) ids, range-checked by whoever wrote them
+  // exn, eattn and effh hold GEMM inputs: encoder_input_bytes a value
   void *ex = nullptr, *exn = nullptr, *eqkv = nullptr, *eattn = nullptr, *effh = nullptr;
   void* enc_out = nullptr;  // (rows, S, d_model)
   void* cross = nullptr;    // (Lt, k|v, rows, H, S, 64)
 };
 // Depthformer::encode (model.cpp:226-241) over every row, then the cross K/V
 // of every temporal layer (modules.cpp:448-455).
-void run_encoder(const Model& m, const EncoderBufs& b, hipStream_t s);
-void project_cross_kv(const Model& m, const void* enc_out, int rows, int S, void* cross, hipStream_t s);
+void run_encoder(Model& m, const EncoderBufs& b, hipStream_t s);
+// work: rows * S * d_model values of encoder_input_bytes.
+void project_cross_kv(Model& m, const void* enc_out, int rows, int S, void* cross, void* work, hipStream_t s);
+inline size_t encoder_input_bytes(DType dt) { return dt == DType::F32 ? 6 : 2; }
 
 struct GenOpts {
   int num_frames = 50;
