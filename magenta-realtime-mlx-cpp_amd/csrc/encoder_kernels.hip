@@ -4,9 +4,10 @@
 //
 // GEMM operands are both K-contiguous ("NT": activations (M, K) row-major,
 // weights (N, K) row-major as the bundle stores them).  bf16 and fp16 use
-// v_mfma_f32_32x32x16_{bf16,f16} with LDS-double-buffered tiles; fp32 splits its
+// v_mfma_f32_32x32x16_{bf16,f16} through the LDS ring of ring_gemm.hpp; fp32 splits its
 // operands into three bf16 parts for the same instruction (split_gemm.hpp), or
 // uses a VALU tile where the shapes do not fit.
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -152,11 +153,6 @@ struct GemmOut {
     const float gl = gelu_t<T>(S::rnd(g));
     C[(size_t)m * (N / 2) + j] = S::st(gl * S::rnd(u));
   }
-  // The same in fp32, stored as split rows (the next split GEMM's input).
-  __device__ __forceinline__ void put_geglu_split(int m, int n, float g, float u) const {
-    const int j = (n >> 6) * 32 + (n & 31);
-    store_split(static_cast<bf16*>(a.C), split_index(m, j, N / 2), gelu_t<float>(g) * u);
-  }
 };
 
 // ---- VALU tiled GEMM (shapes the matrix-core tiles do not take) ---------------------
@@ -211,389 +207,287 @@ __global__ __launch_bounds__(256) void k_gemm_valu(const T* __restrict__ A, cons
   }
 }
 
-// ---- 16-bit MFMA GEMM ----------------------------------------------------------------
-typedef float f32x8_t __attribute__((ext_vector_type(8)));
-
-// The 32x32x16 matrix instruction of each 16-bit storage type (fp32 accumulators).
+// ---- matrix-core GEMM ------------------------------------------------------------------
+// gelu_t of 16-bit types with tanh taken as (1 - t) / (1 + t), t = 2^(-2 |x| log2 e):
+// within 2e-7 of tanhf, far below the 16-bit rounding of 1 + tanh that is all the
+// formula keeps of it.  tanhf's two polynomial paths made the 181 M gated-GELUs of
+// 32 streams a 300 us epilogue.
 template <typename T>
-struct Mfma;
-template <>
-struct Mfma<bf16> {
-  typedef __bf16 v8 __attribute__((ext_vector_type(8)));
-  __device__ __forceinline__ static f32x16_t mma(v8 a, v8 b, f32x16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-  }
-};
-template <>
-struct Mfma<f16> {
-  typedef _Float16 v8 __attribute__((ext_vector_type(8)));
-  __device__ __forceinline__ static f32x16_t mma(v8 a, v8 b, f32x16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-  }
-};
+__device__ __forceinline__ float gelu16(float x) {
+  using S = St<T>;
+  const float x2 = S::rnd(x * x);
+  float t = S::rnd(S::rnd(0.044715f) * x2);
+  t = S::rnd(1.0f + t);
+  t = S::rnd(x * t);
+  const float inner = S::rnd(S::rnd(0.7978845608028654f) * t);
+  const float q = __builtin_amdgcn_exp2f(fabsf(inner) * -2.8853900817779268f);
+  const float th = S::rnd(copysignf((1.0f - q) * __builtin_amdgcn_rcpf(1.0f + q), inner));
+  t = S::rnd(1.0f + th);
+  t = S::rnd(x * t);
+  return S::rnd(0.5f * t);
+}
 
-constexpr int kBN = 128, kBK = 64, kStages = 2;
-
-// LDS rows of a tile are 64 elements = 8 chunks of 16 bytes; chunk c of row r is
-// stored at chunk c ^ swz(r), so the 32 rows x 2 chunks of an MFMA fragment
-// read (and 16 consecutive lanes of any ds_read_b128) fall in distinct banks.
-__device__ __forceinline__ int swz(int r) { return (r ^ (r >> 3)) & 7; }
-
-// Epilogue of the MFMA GEMMs.  Accumulator r of tile (i, j) of a lane holds
-// row mb + 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4 and column
-// nb + 32 j + lane % 32 (j = 2p / 2p + 1: gate / up columns of gated-GELU pair p).
-// The kind is resolved once per tile, and the residual epilogue loads every
-// residual before it stores anything: with the loads and stores of one
-// element interleaved, each load would wait for the previous element's store.
-template <typename T, int MI, int NJ = 2>
+// Epilogue of a wave's tile, first row mb, first column nb: a lane holds row
+// mb + 32 i + lane % 32 of tile (i, j) and four times four consecutive columns
+// (j = 2 p / 2 p + 1: gate / up columns of gated-GELU pair p).  16-bit results swap
+// halves between lanes l and l + 32, so that a lane stores 8 consecutive columns,
+// 16 bytes.  The kind is resolved once per tile, and the residual epilogue loads
+// every residual before it stores anything.
+template <typename T, int MI, int NJ>
 __device__ __forceinline__ void mfma_epilogue(const GemmOut<T>& out, const f32x16_t (&acc)[MI][NJ], int M, int mb,
                                               int nb) {
   using St_ = St<T>;
-  const int lane = threadIdx.x & 63, col = lane & 31, rl = 4 * (lane >> 5);
-  const int N = out.N;
+  constexpr bool k16 = sizeof(T) == 2;
+  constexpr int G = k16 ? 2 : 4, V = k16 ? 8 : 4;  // stores per 32 columns, columns per store
+  const int lane = threadIdx.x & 63, lh = lane >> 5;
+  const int N = out.N, m0 = mb + (lane & 31);
   T* C = static_cast<T*>(out.a.C);
-  auto row = [&](int i, int r) { return mb + 32 * i + 8 * (r >> 2) + rl + (r & 3); };
+  // the 16 bytes of group g of four (16 bit: groups 2 g and 2 g + 1 of the lane
+  // pair) from f(r), r = 0 .. 15, and their first column in the 32
+  auto pack = [&](int g, auto&& f) -> uint4 {
+    uint4 w;
+    if constexpr (k16) {
+      const uint32_t x0 = St_::bits(f(8 * g)) | (St_::bits(f(8 * g + 1)) << 16);
+      const uint32_t x1 = St_::bits(f(8 * g + 2)) | (St_::bits(f(8 * g + 3)) << 16);
+      const uint32_t y0 = St_::bits(f(8 * g + 4)) | (St_::bits(f(8 * g + 5)) << 16);
+      const uint32_t y1 = St_::bits(f(8 * g + 6)) | (St_::bits(f(8 * g + 7)) << 16);
+      const auto s0 = __builtin_amdgcn_permlane32_swap(x0, y0, false, false);
+      const auto s1 = __builtin_amdgcn_permlane32_swap(x1, y1, false, false);
+      w = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+    } else {
+      w = make_uint4(__float_as_uint(f(4 * g)), __float_as_uint(f(4 * g + 1)), __float_as_uint(f(4 * g + 2)),
+                     __float_as_uint(f(4 * g + 3)));
+    }
+    return w;
+  };
+  auto gelu = [](float x) {
+    if constexpr (k16)
+      return gelu16<T>(x);
+    else
+      return gelu_t<T>(x);
+  };
+  auto col = [&](int g) { return k16 ? 8 * (2 * g + lh) : 8 * g + 4 * lh; };
   switch (out.a.kind) {
     case GemmEpi::Geglu:
       if constexpr (NJ % 2 == 0) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
-          for (int pj = 0; pj < NJ / 2; ++pj)
+          for (int p = 0; p < NJ / 2; ++p)
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
-              if (row(i, r) < M) out.put_geglu(row(i, r), nb + 64 * pj + col, acc[i][2 * pj][r], acc[i][2 * pj + 1][r]);
+            for (int g = 0; g < G; ++g) {
+              const uint4 w = pack(g, [&](int r) {
+                return gelu(St_::rnd(acc[i][2 * p][r])) * St_::rnd(acc[i][2 * p + 1][r]);
+              });
+              const int m = m0 + 32 * i;
+              if (m < M) *reinterpret_cast<uint4*>(C + (size_t)m * (N / 2) + nb / 2 + 32 * p + col(g)) = w;
+            }
       }
       break;
     case GemmEpi::GegluSplit:
-      if constexpr (NJ % 2 == 0 && std::is_same<T, float>::value) {
+      if constexpr (NJ % 2 == 0 && !k16) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
-          for (int pj = 0; pj < NJ / 2; ++pj)
+          for (int p = 0; p < NJ / 2; ++p)
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
-              if (row(i, r) < M)
-                out.put_geglu_split(row(i, r), nb + 64 * pj + col, acc[i][2 * pj][r], acc[i][2 * pj + 1][r]);
+            for (int g = 0; g < 4; ++g) {
+              float v[4];
+#pragma unroll
+              for (int r = 0; r < 4; ++r) v[r] = gelu_t<float>(acc[i][2 * p][4 * g + r]) * acc[i][2 * p + 1][4 * g + r];
+              const int m = m0 + 32 * i;
+              if (m < M)
+                store_split4(static_cast<bf16*>(out.a.C), split_index(m, nb / 2 + 32 * p + col(g), N / 2), v);
+            }
       }
       break;
-    case GemmEpi::Resid:
+    case GemmEpi::Resid: {
+      uint4 old[MI][NJ][G];  // rows past M load row M - 1 (unconditional loads, issued together)
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          T old[16];  // rows past M load row M - 1 (unconditional loads, issued together)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) old[r] = C[(size_t)min(row(i, r), M - 1) * N + nb + 32 * j + col];
+          for (int g = 0; g < G; ++g)
+            old[i][j][g] =
+                *reinterpret_cast<const uint4*>(C + (size_t)min(m0 + 32 * i, M - 1) * N + nb + 32 * j + col(g));
 #pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if (row(i, r) < M)
-              C[(size_t)row(i, r) * N + nb + 32 * j + col] = St_::st(St_::ld(old[r]) + St_::rnd(acc[i][j][r]));
-        }
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int g = 0; g < G; ++g) {
+            const uint4 w = pack(g, [&](int r) { return acc[i][j][r]; });
+            const T* pw = reinterpret_cast<const T*>(&w);
+            const T* po = reinterpret_cast<const T*>(&old[i][j][g]);
+            uint4 res;
+            T* pr = reinterpret_cast<T*>(&res);
+#pragma unroll
+            for (int e = 0; e < V; ++e) pr[e] = St_::st(St_::ld(po[e]) + St_::ld(pw[e]));
+            const int m = m0 + 32 * i;
+            if (m < M) *reinterpret_cast<uint4*>(C + (size_t)m * N + nb + 32 * j + col(g)) = res;
+          }
       break;
+    }
     case GemmEpi::Store:
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if (row(i, r) < M) C[(size_t)row(i, r) * N + nb + 32 * j + col] = St_::st(acc[i][j][r]);
+          for (int g = 0; g < G; ++g) {
+            const uint4 w = pack(g, [&](int r) { return acc[i][j][r]; });
+            const int m = m0 + 32 * i;
+            if (m < M) *reinterpret_cast<uint4*>(C + (size_t)m * N + nb + 32 * j + col(g)) = w;
+          }
       break;
-    case GemmEpi::StoreF32:
+    case GemmEpi::StoreF32:  // a caller's buffer: aligned to its element only
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if (row(i, r) < M)
-              static_cast<float*>(out.a.C)[(size_t)row(i, r) * N + nb + 32 * j + col] = St_::rnd(acc[i][j][r]);
+          for (int r = 0; r < 16; ++r) {
+            const int m = m0 + 32 * i;
+            if (m < M)
+              static_cast<float*>(out.a.C)[(size_t)m * N + nb + 32 * j + 8 * (r >> 2) + 4 * lh + (r & 3)] =
+                  St_::rnd(acc[i][j][r]);
+          }
       break;
     default: {  // CrossKV: column n = (layer*2 + kv)*HD + h*64 + d, row m = b*S + s
-      size_t cbase[NJ];
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const int n = nb + 32 * j + col, lk = n / out.a.HD, nn = n - lk * out.a.HD;
-        cbase[j] = (((size_t)lk * out.a.nb) * out.a.H + (nn >> 6)) * out.a.S * 64 + (nn & 63);
-      }
-      const size_t bstride = (size_t)out.a.H * out.a.S * 64;
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = row(i, r);
-          if (m < M) {
-            const int b = m / out.a.S, sp = m - b * out.a.S;
-            const size_t ro = (size_t)b * bstride + (size_t)sp * 64;
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) C[cbase[j] + ro] = St_::st(acc[i][j][r]);
-          }
-        }
-    }
-  }
-}
-
-// C = A B^T (A (M, K), B (N, K) 16-bit, fp32 accumulation) with the GemmOut
-// epilogue.  Tile BM x BN x 64, 4 waves in a 2x2 grid (wave tile BM/2 x BN/2 =
-// (BM/64) x (BN/64) MFMA 32x32x16 tiles).  Tiles stream global -> LDS with direct
-// 16-byte loads (global_load_lds) through an S-deep ring: tile j + S - 1 is
-// requested while tile j is multiplied, and a wave waits only for its own
-// loads of tile j (vmcnt counts in order) before the barrier.  Where the grid
-// fills every CU twice, two stages (64 / 48 KB of LDS) leave room for 2-3
-// blocks per CU, which hides more latency than a deeper ring in one block
-// (measured); a grid of at most one tile per CU instead takes a deep ring in
-// its one block.  Rows past M read row M - 1 (their results are not stored).
-// Operand fragments of v_mfma_f32_32x32x16_{bf16,f16}: lane l holds row (l % 32)
-// and k = 8*(l / 32) .. +7 of both A (32x16) and B^T (32x16); the 16
-// accumulators of lane l hold column l % 32, rows 8*(r/4) + 4*(l/32) + r%4.
-// Blocks per CU the register budget is sized for: two wherever the LDS ring
-// leaves room for two (at most 80 KB), else one.
-constexpr int gemm_min_blocks(int BM, int S, int BN) { return S * (BM + BN) * 128 <= 80 * 1024 ? 2 : 1; }
-
-// GM = 0: block (x, y) of a 2-D grid computes tile (y, x); GM > 0: a 1-D grid
-// in the grouped_tile order.
-template <typename T, int BM, int S, int BN, int GM>
-__global__ __launch_bounds__(256, gemm_min_blocks(BM, S, BN)) void k_gemm_mfma(const T* __restrict__ A,
-                                                                               const T* __restrict__ B,
-                                                   int M, int N, int K, GemmOut<T> out) {
-  typedef typename Mfma<T>::v8 v8;
-  constexpr int MI = BM / 64;                        // MFMA tiles per wave in M
-  constexpr int NJ = BN / 64;                        // MFMA tiles per wave in N
-  constexpr int kStageBytes = (BM + BN) * 128;       // A rows then B rows, 128 bytes each
-  constexpr int LA = BM / 32 + BN / 32;              // load instructions per wave per tile
-  extern __shared__ __align__(16) unsigned char lds[];
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int wm = wid >> 1, wn = wid & 1;
-  int mt = blockIdx.y, nt = blockIdx.x;
-  if constexpr (GM > 0) grouped_tile(blockIdx.x, (M + BM - 1) / BM, N / BN, GM, mt, nt);
-  const int m0 = mt * BM, n0 = nt * BN;
-  const int nk = K / kBK;
-
-  // tile kt -> stage kt % S; wave w loads rows [w*BM/4, +BM/4) of A and
-  // [w*32, +32) of B, 8 rows (1 KB) per instruction
-  auto issue = [&](int kt) {
-    const int ktc = min(kt, nk - 1);  // past the end: reload the last tile into a free stage
-    unsigned char* st = lds + (kt % S) * kStageBytes;
-    const int r8 = lane >> 3, p = lane & 7;
-#pragma unroll
-    for (int q = 0; q < BM / 32; ++q) {
-      const int r = wid * (BM / 4) + q * 8 + r8;
-      const int gm = min(m0 + r, M - 1);
-      const T* src = A + (size_t)gm * K + ktc * kBK + ((p ^ swz(r)) << 3);
-      __builtin_amdgcn_global_load_lds((const MRT_GLOBAL void*)src,
-                                       (MRT_LDS void*)(st + (wid * (BM / 4) + q * 8) * 128), 16, 0, 0);
-    }
-#pragma unroll
-    for (int q = 0; q < BN / 32; ++q) {
-      const int r = wid * (BN / 4) + q * 8 + r8;
-      const T* src = B + (size_t)(n0 + r) * K + ktc * kBK + ((p ^ swz(r)) << 3);
-      __builtin_amdgcn_global_load_lds((const MRT_GLOBAL void*)src,
-                                       (MRT_LDS void*)(st + BM * 128 + (wid * (BN / 4) + q * 8) * 128), 16, 0, 0);
-    }
-  };
-
-  f32x16_t acc[MI][NJ];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-#pragma unroll
-  for (int kt = 0; kt < S - 1; ++kt) issue(kt);
-  const int lr = lane & 31, lh = lane >> 5;
-  for (int kt = 0; kt < nk; ++kt) {
-    __builtin_amdgcn_s_waitcnt(vm_wait_imm((S - 2) * LA));  // this wave's loads of tile kt have landed
-    ring_barrier();  // every wave's loads of tile kt; every wave is done with tile kt - 1
-    issue(kt + S - 1);
-    const unsigned char* st = lds + (kt % S) * kStageBytes;
-    // every fragment of the tile is read before the first product, so the
-    // LDS latency is paid once per tile, not once per 16-deep step
-    v8 a[kBK / 16][MI], b[kBK / 16][NJ];
-#pragma unroll
-    for (int ks = 0; ks < kBK / 16; ++ks) {
-      const int c = 2 * ks + lh;
+      size_t ro[MI];
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
-        const int r = wm * (BM / 2) + i * 32 + lr;
-        a[ks][i] = *reinterpret_cast<const v8*>(st + r * 128 + ((c ^ swz(r)) << 4));
+        const int m = m0 + 32 * i, b = m / out.a.S;
+        ro[i] = (size_t)b * out.a.H * out.a.S * 64 + (size_t)(m - b * out.a.S) * 64;
       }
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const int r = wn * (BN / 2) + j * 32 + lr;
-        b[ks][j] = *reinterpret_cast<const v8*>(st + BM * 128 + r * 128 + ((c ^ swz(r)) << 4));
+      for (int j = 0; j < NJ; ++j) {  // the 32 columns of a tile lie in one head
+        const int n = nb + 32 * j, lk = n / out.a.HD, nn = n - lk * out.a.HD;
+        T* base = C + ((size_t)lk * out.a.nb * out.a.H + (nn >> 6)) * out.a.S * 64 + (nn & 63);
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int g = 0; g < G; ++g) {
+            const uint4 w = pack(g, [&](int r) { return acc[i][j][r]; });
+            if (m0 + 32 * i < M) *reinterpret_cast<uint4*>(base + ro[i] + col(g)) = w;
+          }
       }
     }
-    __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of the products
-#pragma unroll
-    for (int ks = 0; ks < kBK / 16; ++ks)
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-          acc[i][j] = Mfma<T>::mma(a[ks][i], b[ks][j], acc[i][j]);
   }
-  __builtin_amdgcn_s_waitcnt(vm_wait_imm(0));  // no copy into LDS outlives the block
-
-  mfma_epilogue<T, MI, NJ>(out, acc, M, m0 + wm * (BM / 2), n0 + wn * (BN / 2));
 }
 
-template <typename T, int BM, int S = kStages, int BN = kBN, int GM = 0>
-void launch_gemm_mfma(const T* A, const T* B, int M, int N, int K, const GemmOut<T>& out, hipStream_t s) {
-  static_assert((S - 2) * (BM / 32 + BN / 32) < 64, "vmcnt holds at most 63 outstanding loads");
-  static_assert(BM % 64 == 0 && BN % 64 == 0, "wave tiles are whole 32x32 MFMA tiles");
-  constexpr size_t lds = (size_t)S * (BM + BN) * 128;
-  static_assert(lds <= 160 * 1024, "LDS of one CU");
-  MRT_REQUIRE(N % BN == 0, "gemm: N is not a multiple of the tile width");
-  allow_dynamic_lds(reinterpret_cast<const void*>(&k_gemm_mfma<T, BM, S, BN, GM>), lds);
-  const long tm = (M + BM - 1) / BM, tn = N / BN;
-  MRT_REQUIRE(GM == 0 || tm * tn <= 0x7fffffffL, "gemm: too many tiles");
-  const dim3 grid = GM > 0 ? dim3(static_cast<unsigned>(tm * tn)) : dim3(tn, tm);
-  hipLaunchKernelGGL((k_gemm_mfma<T, BM, S, BN, GM>), grid, dim3(256), lds, s, A, B, M, N, K, out);
-}
-
-// Large-M GEMM (the encoder of several streams): 256 x 256 x 64 tiles, 16
-// waves in a 4 x 4 grid (wave tile 64 x 64 = 2 x 2 MFMA 32x32x16 tiles, the
-// accumulators of k_gemm_mfma's waves), the same swizzled two-stage global ->
-// LDS ring.  Against 128 x 128 tiles it halves the operand bytes read from L2
-// per FLOP, which is what bounds the smaller tiles at these sizes.  Rows past
-// M read row M - 1 (not stored); N % 256 == 0.
-constexpr int kGB = 256;                 // block tile, M and N
-constexpr int kGBWaves = 16;
-constexpr int kGBStage = 2 * kGB * 128;  // A rows then B rows, 128 bytes (64 elements) each
-
-template <typename T>
-__global__ __launch_bounds__(64 * kGBWaves) void k_gemm_big(const T* __restrict__ A, const T* __restrict__ B,
-                                                            int M, int N, int K, GemmOut<T> out) {
-  typedef typename Mfma<T>::v8 v8;
-  constexpr int RW = kGB / kGBWaves;  // rows of A (and of B) each wave loads per stage
-  constexpr int LA = 2 * RW / 8;      // load instructions per wave per stage (8 rows each)
+// C = A B^T with the GemmOut epilogue (A (M, K), B (N, K): 16-bit rows, or split rows
+// of an fp32 matrix; fp32 accumulation).  One persistent block per CU: block L
+// takes tiles L, L + gridDim, .. (gridDim % 8 == 0) of the grouped_tile order.
+// The k-tiles of all its tiles are one stream through the ring: while a tile's
+// results are converted and stored, the next tile's first k-tiles land, and its
+// multiplies start while the stores drain (vmcnt counts in order: the first wait
+// of a tile leaves the previous tile's stores outstanding).  With one tile per block
+// the epilogue and the refill cost 7 of 33 us at 256 x 256 x 1,024: 731 us against
+// 666 us at 64,384 x 5,632 x 1,024 (1,115 TFLOP/s).  Rows past M read row M - 1 (not
+// stored); N % BN == 0.
+template <class Core, typename T, int BM, int BN, int WM, int WN, int S>
+__global__ __launch_bounds__(64 * WM * WN) void k_gemm_ring(const void* __restrict__ A, const void* __restrict__ B,
+                                                            int M, int N, int K, int GM, GemmOut<T> out) {
+  using Tile = RingTile<Core, BM, BN, WM, WN, S>;
   extern __shared__ __align__(16) unsigned char lds[];
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int wm = wid >> 2, wn = wid & 3;
-  const int m0 = blockIdx.y * kGB, n0 = blockIdx.x * kGB;
-  const int nk = K / kBK;
-
-  auto issue = [&](int kt) {
-    const int ktc = min(kt, nk - 1);
-    unsigned char* st = lds + (kt % kStages) * kGBStage;
-    const int r8 = lane >> 3, p = lane & 7;
-#pragma unroll
-    for (int q = 0; q < RW / 8; ++q) {
-      const int r = wid * RW + q * 8 + r8;
-      const int gm = min(m0 + r, M - 1);
-      const T* src = A + (size_t)gm * K + ktc * kBK + ((p ^ swz(r)) << 3);
-      __builtin_amdgcn_global_load_lds((const MRT_GLOBAL void*)src, (MRT_LDS void*)(st + (wid * RW + q * 8) * 128),
-                                       16, 0, 0);
-    }
-#pragma unroll
-    for (int q = 0; q < RW / 8; ++q) {
-      const int r = wid * RW + q * 8 + r8;
-      const T* src = B + (size_t)(n0 + r) * K + ktc * kBK + ((p ^ swz(r)) << 3);
-      __builtin_amdgcn_global_load_lds((const MRT_GLOBAL void*)src,
-                                       (MRT_LDS void*)(st + kGB * 128 + (wid * RW + q * 8) * 128), 16, 0, 0);
-    }
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tm = (M + BM - 1) / BM, tn = N / BN, tiles = tm * tn, nk = K / Core::kDepth;
+  const int x = blockIdx.x & 7, cnt = (tiles >> 3) + (x < (tiles & 7)), step = gridDim.x >> 3;
+  const size_t ld = (size_t)nk * Tile::kRow;  // bytes of an operand row
+  auto origin = [&](int i, int& m0, int& n0) {
+    int mt, nt;
+    grouped_tile(x + 8 * i, tm, tn, GM, mt, nt);
+    m0 = mt * BM;
+    n0 = nt * BN;
   };
+  int t = blockIdx.x >> 3;
+  if (t >= cnt) return;
 
-  f32x16_t acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-#pragma unroll
-  for (int kt = 0; kt < kStages - 1; ++kt) issue(kt);
-  const int lr = lane & 31, lh = lane >> 5;
-  for (int kt = 0; kt < nk; ++kt) {
-    __builtin_amdgcn_s_waitcnt(vm_wait_imm((kStages - 2) * LA));  // this wave's loads of tile kt have landed
-    ring_barrier();  // every wave's loads of tile kt; every wave is done with tile kt - 1
-    issue(kt + kStages - 1);
-    const unsigned char* st = lds + (kt % kStages) * kGBStage;
-    // one 16-deep step at a time: 16 waves leave 128 registers a lane, and
-    // reading further ahead spills
-#pragma unroll
-    for (int ks = 0; ks < kBK / 16; ++ks) {
-      const int c = 2 * ks + lh;
-      v8 a[2], b[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int r = wm * 64 + i * 32 + lr;
-        a[i] = *reinterpret_cast<const v8*>(st + r * 128 + ((c ^ swz(r)) << 4));
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int r = wn * 64 + j * 32 + lr;
-        b[j] = *reinterpret_cast<const v8*>(st + kGB * 128 + r * 128 + ((c ^ swz(r)) << 4));
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = Mfma<T>::mma(a[i], b[j], acc[i][j]);
-    }
-  }
-  __builtin_amdgcn_s_waitcnt(vm_wait_imm(0));  // no copy into LDS outlives the block
-
-  mfma_epilogue<T, 2>(out, acc, M, m0 + wm * 64, n0 + wn * 64);
-}
-
-template <typename T>
-void launch_gemm_big(const T* A, const T* B, int M, int N, int K, const GemmOut<T>& out, hipStream_t s) {
-  constexpr size_t lds = (size_t)kStages * kGBStage;
-  allow_dynamic_lds(reinterpret_cast<const void*>(&k_gemm_big<T>), lds);
-  hipLaunchKernelGGL(k_gemm_big<T>, dim3(N / kGB, (M + kGB - 1) / kGB), dim3(64 * kGBWaves), lds, s, A, B, M, N, K, out);
-}
-
-// C = A B^T in fp32 from split operands (split_gemm.hpp) with the GemmOut
-// epilogue, BM x BN x 32 tiles in the XCD-grouped order, 4 waves in a 2 x 2 grid,
-// one block per CU.  Rows past M read row M - 1 (not stored); N % BN == 0.
-template <int BM, int BN, int S>
-__global__ __launch_bounds__(256, 1) void k_gemm_split(const bf16* __restrict__ A, const bf16* __restrict__ B, int M,
-                                                       int N, int K, GemmOut<float> out) {
-  using Tile = SplitTile<BM, BN, 2, 2, S>;
-  extern __shared__ __align__(16) unsigned char lds[];
-  int mt, nt;
-  grouped_tile(blockIdx.x, (M + BM - 1) / BM, N / BN, 4, mt, nt);
-  const int m0 = mt * BM, n0 = nt * BN;
-  const size_t ldk = (size_t)(K >> 5) * kSplitGroup;
-  const bf16* a0[Tile::LA];
-  const bf16* b0[Tile::LB];
-#pragma unroll
-  for (int q = 0; q < Tile::LA; ++q) {
-    int row, chunk;
-    Tile::load_pos(q, row, chunk);
-    a0[q] = A + (size_t)min(m0 + row, M - 1) * ldk + chunk * 8;
-  }
+  // the next k-tile to request: tile lt, depth lk; byte offsets of this thread's
+  // chunks from the tile's first rows
+  int lt = t, lk = 0;
+  const char *ab, *bb;
+  unsigned ao[Tile::LA], bo[Tile::LB];
 #pragma unroll
   for (int q = 0; q < Tile::LB; ++q) {
     int row, chunk;
     Tile::load_pos(q, row, chunk);
-    b0[q] = B + (size_t)(n0 + row) * ldk + chunk * 8;
+    bo[q] = row * (unsigned)ld + chunk * 16;
   }
-  f32x16_t acc[Tile::MI][Tile::NJ];
-  Tile::run(lds, 0, K >> 5,
-            [&](int kt, const bf16* (&ap)[Tile::LA], const bf16* (&bp)[Tile::LB]) {
+  auto point = [&]() {
+    int m0, n0;
+    origin(lt, m0, n0);
+    ab = static_cast<const char*>(A) + m0 * ld;
+    bb = static_cast<const char*>(B) + n0 * ld;
 #pragma unroll
-              for (int q = 0; q < Tile::LA; ++q) ap[q] = a0[q] + (size_t)kt * kSplitGroup;
+    for (int q = 0; q < Tile::LA; ++q) {
+      int row, chunk;
+      Tile::load_pos(q, row, chunk);
+      ao[q] = min(row, M - 1 - m0) * (unsigned)ld + chunk * 16;
+    }
+  };
+  point();
+  auto issue = [&](unsigned char* stage) {
+    const char *a = ab + (size_t)lk * Tile::kRow, *b = bb + (size_t)lk * Tile::kRow;
 #pragma unroll
-              for (int q = 0; q < Tile::LB; ++q) bp[q] = b0[q] + (size_t)kt * kSplitGroup;
-            },
-            acc);
-  const int wid = threadIdx.x >> 6;
-  mfma_epilogue<float, Tile::MI, Tile::NJ>(out, acc, M, m0 + (wid >> 1) * (BM / 2), n0 + (wid & 1) * (BN / 2));
+    for (int q = 0; q < Tile::LA; ++q) Tile::load_a(stage, q, a + ao[q]);
+#pragma unroll
+    for (int q = 0; q < Tile::LB; ++q) Tile::load_b(stage, q, b + bo[q]);
+    if (++lk == nk) {
+      if (lt + step < cnt) {
+        lt += step;
+        lk = 0;
+        point();
+      } else {
+        lk = nk - 1;  // past the end: the last k-tile again, into a free stage
+      }
+    }
+  };
+
+  typename Tile::State s;
+  Tile::start(lds, s, issue);
+  // store instructions of a whole tile's epilogue (16 bytes each; the split
+  // gated-GELU pairs three times 8)
+  constexpr int kStores = Tile::MI * Tile::NJ * (sizeof(T) == 2 ? 2 : 4);
+  constexpr int kGegluStores = sizeof(T) == 2 ? kStores / 2 : kStores / 2 * 3;
+  const bool pairs = out.a.kind == GemmEpi::Geglu || out.a.kind == GemmEpi::GegluSplit;
+  const bool plain = out.a.kind == GemmEpi::Store || out.a.kind == GemmEpi::CrossKV;
+  bool stored = false;  // the previous tile's epilogue issued exactly those stores after the ring's loads
+  for (; t < cnt; t += step) {
+    int m0, n0;
+    origin(t, m0, n0);
+    s.clear();
+    Tile::reread(lds, s);  // the first fragments need no registers across the epilogue
+    for (int kt = 0; kt < nk; ++kt) {
+      const bool after = stored && kt == 0;
+      Tile::ktile(lds, s, issue, [&] {
+        if (after && plain)
+          Tile::template wait_loads<kStores>();
+        else if (after && pairs)
+          Tile::template wait_loads<kGegluStores>();
+        else
+          Tile::template wait_loads<>();
+      });
+    }
+    mfma_epilogue<T, Tile::MI, Tile::NJ>(out, s.acc, M, m0 + (wid / WN) * (BM / WM), n0 + (wid % WN) * (BN / WN));
+    asm volatile("" ::: "memory");  // the stores stay ahead of the next tile's waits
+    stored = m0 + BM <= M;
+  }
+  __builtin_amdgcn_s_waitcnt(vm_wait_imm(0));  // no copy into LDS outlives the block
 }
 
-template <int BM, int BN, int S>
-void launch_gemm_split(const bf16* A, const bf16* B, int M, int N, int K, const GemmOut<float>& out, hipStream_t s) {
-  using Tile = SplitTile<BM, BN, 2, 2, S>;
-  allow_dynamic_lds(reinterpret_cast<const void*>(&k_gemm_split<BM, BN, S>), Tile::kLds);
+template <class Core, typename T, int BM, int BN, int WM, int WN, int S>
+void launch_gemm_ring(const void* A, const void* B, int M, int N, int K, const GemmOut<T>& out, hipStream_t s) {
+  using Tile = RingTile<Core, BM, BN, WM, WN, S>;
+  const auto kernel = &k_gemm_ring<Core, T, BM, BN, WM, WN, S>;
+  allow_dynamic_lds(reinterpret_cast<const void*>(kernel), Tile::kLds);
   const long tiles = (long)((M + BM - 1) / BM) * (N / BN);
-  MRT_REQUIRE(tiles <= 0x7fffffffL, "split gemm: too many tiles");
-  hipLaunchKernelGGL((k_gemm_split<BM, BN, S>), dim3((unsigned)tiles), dim3(256), Tile::kLds, s, A, B, M, N, K, out);
+  MRT_REQUIRE(N % BN == 0 && K % Core::kDepth == 0 && tiles <= 0x7fffffffL, "gemm: tile does not fit the shape");
+  MRT_REQUIRE((long)K / Core::kDepth * Tile::kRow * (BM > BN ? BM : BN) <= 0xffffffffL, "gemm: rows too long");
+  const long grid = std::min((long)std::max(8, device_cus() & ~7), (tiles + 7) / 8 * 8);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(Tile::kThreads), Tile::kLds, s, A, B, M, N, K, 4, out);
 }
 
 // ---- encoder self-attention (bidirectional, no mask, no bias, scale 1.0) -------------
@@ -906,58 +800,53 @@ void rmsnorm_rows(DType dt, const void* x, const void* g, float eps, int M, int 
 
 namespace {
 
+// The tile whose rounds over the CUs (one block each) take the least time: rounds x
+// area x the tile's time per area relative to 256 x 256.  The factors are measured
+// times a round of the 16-bit kernel, K = 1,024: 256 x 256 30.7 us; 192 x 256 24.2
+// and 128 x 256 15.9 (1.05); 128 x 192 14.3 (1.25); 64 x 128 5.7 (1.5; its fragment
+// reads and its epilogue weigh more).  Gated-GELU pairs need wave tiles of whole
+// 64-column groups (not 128 x 192).
+template <class Core, typename T>
+void gemm_tiles(const void* A, const void* B, int M, int N, int K, const GemmEpiArgs& e, hipStream_t s) {
+  const GemmOut<T> out{e, N};
+  const long cus = std::max(8, device_cus() & ~7);
+  const bool pairs = e.kind == GemmEpi::Geglu || e.kind == GemmEpi::GegluSplit;
+  auto cost = [&](int bm, int bn, double f) {
+    if (N % bn) return 1e30;
+    const long tiles = (long)((M + bm - 1) / bm) * (N / bn);
+    return (double)((tiles + cus - 1) / cus) * bm * bn * f;
+  };
+  const double cw = pairs ? 1e30 : cost(128, 192, sizeof(T) == 2 ? 1.25 : 1.0);
+  if constexpr (sizeof(T) == 2) {
+    const double c64 = cost(64, 128, 1.5), c128 = cost(128, 256, 1.05), c192 = cost(192, 256, 1.05);
+    const double c256 = cost(256, 256, 1.0);
+    if (c256 <= std::min(std::min(c192, c128), std::min(cw, c64)))
+      launch_gemm_ring<Core, T, 256, 256, 4, 2, 2>(A, B, M, N, K, out, s);
+    else if (c192 <= std::min(c128, std::min(cw, c64)))
+      launch_gemm_ring<Core, T, 192, 256, 2, 4, 2>(A, B, M, N, K, out, s);
+    else if (c128 <= std::min(cw, c64))
+      launch_gemm_ring<Core, T, 128, 256, 2, 4, 3>(A, B, M, N, K, out, s);
+    else if (cw <= c64)
+      launch_gemm_ring<Core, T, 128, 192, 4, 2, 3>(A, B, M, N, K, out, s);
+    else
+      launch_gemm_ring<Core, T, 64, 128, 2, 2, 4>(A, B, M, N, K, out, s);
+  } else {
+    const double c64 = cost(64, 128, 1.15), c128 = cost(128, 128, 1.0);
+    if (cw <= std::min(c128, c64))
+      launch_gemm_ring<Core, T, 128, 192, 2, 2, 2>(A, B, M, N, K, out, s);
+    else if (c128 <= c64)
+      launch_gemm_ring<Core, T, 128, 128, 2, 2, 3>(A, B, M, N, K, out, s);
+    else
+      launch_gemm_ring<Core, T, 64, 128, 2, 2, 4>(A, B, M, N, K, out, s);
+  }
+}
+
 template <typename T>
 void gemm_t(const T* A, const T* B, int M, int N, int K, const GemmEpiArgs& e, hipStream_t s, bool allow_mfma) {
   GemmOut<T> out{e, N};
   if constexpr (sizeof(T) == 2) {
-    if (allow_mfma && N % kBN == 0 && K % kBK == 0) {
-      // Measured on MI355X (256 CUs) at 2 x 1006 x {1, 8, 32} rows: 256 x 256
-      // tiles of 16 waves for outputs up to 4096 wide once they give about
-      // one tile per CU (slower for the 5632- and 40960-wide outputs, where
-      // 2-3 smaller blocks per CU hide more latency); for the wider outputs
-      // other than the gated-GELU pairs (the 40960-wide cross K/V projection)
-      // 256 x 256 tiles of 4 waves with 128 x 128 wave tiles (half the LDS
-      // fragment reads per product) in the XCD-grouped order: 280 -> 234 us
-      // at one stream, 7.35 -> 6.41 ms at 32 (the gated-GELU output measured
-      // slower with them).  The XCD-grouped order also serves the 64-row
-      // tiles of one stream (O 12.6 -> 11.5 us, FFN down 25.3 -> 23.6 us),
-      // the 1024-wide output of K <= 1024 at 32 streams on 192-row tiles
-      // (the attention output projection: 249 -> 210 us against k_gemm_big;
-      // the FFN down projection, K = 2816, is as fast on k_gemm_big) and the
-      // gated-GELU output past two 192-row blocks per CU (1077 -> 998 us at
-      // 32 streams).  Below that every block streams
-      // its operands at the latency of the last-level cache, so the tile is
-      // chosen for the bytes it keeps in flight: a grid of at most one 64-row
-      // tile per CU takes a 4-deep ring (96 KB of LDS; 6 deep measured
-      // slower); a 128 x 192 tile with
-      // a 3-deep ring where that grid fits the CUs once (not for the
-      // gated-GELU pairs, which need wave tiles of whole 64-column groups);
-      // 192-row tiles where two blocks per CU (80 KB each) cover the grid
-      // once; else 128-row tiles when those give >= 1.5 tiles per CU, else
-      // 64-row tiles.
-      const long cus = device_cus();
-      const long t256 = (long)((M + kGB - 1) / kGB) * (N / kGB), t64 = (long)((M + 63) / 64) * (N / kBN);
-      const long t128x192 = N % 192 == 0 ? (long)((M + 127) / 128) * (N / 192) : 0;
-      const long t192 = (long)((M + 191) / 192) * (N / kBN);
-      if (N % kGB == 0 && N <= 4096 && t256 >= cus - cus / 8) {
-        if (N == 1024 && K <= 1024)
-          launch_gemm_mfma<T, 192, 2, 128, 2>(A, B, M, N, K, out, s);
-        else
-          launch_gemm_big<T>(A, B, M, N, K, out, s);
-      } else if (e.kind != GemmEpi::Geglu && N % 256 == 0 && N > 4096 && t256 >= cus)
-        launch_gemm_mfma<T, 256, 2, 256, 4>(A, B, M, N, K, out, s);
-      else if (t64 <= cus)
-        launch_gemm_mfma<T, 64, 4, 128, 4>(A, B, M, N, K, out, s);
-      else if (e.kind != GemmEpi::Geglu && t128x192 > 0 && t128x192 <= cus)
-        launch_gemm_mfma<T, 128, 3, 192>(A, B, M, N, K, out, s);
-      else if (t192 <= 2 * cus)
-        launch_gemm_mfma<T, 192, 2>(A, B, M, N, K, out, s);
-      else if (e.kind == GemmEpi::Geglu)
-        launch_gemm_mfma<T, 192, 2, 128, 4>(A, B, M, N, K, out, s);
-      else if ((long)((M + 127) / 128) * (N / kBN) >= 3 * cus / 2)
-        launch_gemm_mfma<T, 128>(A, B, M, N, K, out, s);
-      else
-        launch_gemm_mfma<T, 64>(A, B, M, N, K, out, s);
+    if (allow_mfma && N % 128 == 0 && K % 64 == 0) {
+      gemm_tiles<Core16<T>, T>(A, B, M, N, K, e, s);
       return;
     }
   }
@@ -976,29 +865,13 @@ void gemm(DType dt, const void* A, const void* B, int M, int N, int K, const Gem
   MRT_HIP_CHECK(hipGetLastError());
 }
 
-bool gemm_split_fits(int N, int K) { return N % kBN == 0 && K % 32 == 0 && K >= 32; }
+bool gemm_split_fits(int N, int K) { return N % 128 == 0 && K % 32 == 0 && K >= 32; }
 
 void gemm_split(const bf16* A, const bf16* B, int M, int N, int K, const GemmEpiArgs& e, hipStream_t s) {
   MRT_REQUIRE(M >= 1 && gemm_split_fits(N, K), "split gemm: N must be a multiple of 128, K of 32");
   if (e.kind == GemmEpi::CrossKV)
     MRT_REQUIRE(e.HD == e.H * 64 && N % e.HD == 0 && M == e.nb * e.S, "gemm: bad cross-KV shape");
-  const GemmOut<float> out{e, N};
-  // The tile whose rounds over the CUs (one block each) take the fewest
-  // products; the 64-row tile reads more LDS a product (a factor of 1.15).
-  const long cus = device_cus();
-  auto cost = [&](int bm, int bn, double f) {
-    const long tiles = (long)((M + bm - 1) / bm) * (N / bn);
-    return (double)((tiles + cus - 1) / cus) * bm * bn * f;
-  };
-  const bool pairs = e.kind == GemmEpi::GegluSplit || e.kind == GemmEpi::Geglu;  // 64-column wave tiles
-  const double c64 = cost(64, 128, 1.15), c128 = cost(128, 128, 1.0);
-  const double cw = !pairs && N % 192 == 0 ? cost(128, 192, 1.0) : 1e30;
-  if (cw <= c128 && cw <= c64)
-    launch_gemm_split<128, 192, 2>(A, B, M, N, K, out, s);
-  else if (c128 <= c64)
-    launch_gemm_split<128, 128, 3>(A, B, M, N, K, out, s);
-  else
-    launch_gemm_split<64, 128, 4>(A, B, M, N, K, out, s);
+  gemm_tiles<CoreSplit, float>(A, B, M, N, K, e, s);
   MRT_HIP_CHECK(hipGetLastError());
 }
 
