@@ -29,6 +29,7 @@ SOURCES = [
     "batch_kernels.hip",
     "spec_kernels.hip",
     "codec_kernels.hip",
+    "conv_split.hip",
     "coca_kernels.hip",
     "probe_kernels.hip",
     "safetensors.cpp",

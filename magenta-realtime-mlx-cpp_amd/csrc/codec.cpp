@@ -2,6 +2,7 @@
 // the decode sequence (system.cpp:373-390: rvq_dequantization, the decoder,
 // istft_postprocess).
 #include "codec.hpp"
+#include "kernels.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -31,6 +32,24 @@ float* Codec::dalloc(size_t floats) {
   return static_cast<float*>(d);
 }
 
+bf16* Codec::salloc(size_t values) { return reinterpret_cast<bf16*>(dalloc((values * 6 + 3) / 4)); }
+
+template <class F>
+void* Codec::pack(int K, int N, F&& value) {
+  std::vector<float> h(static_cast<size_t>(K) * N);
+  for (int k = 0; k < K; ++k)
+    for (int n = 0; n < N; ++n)
+      h[split_ ? static_cast<size_t>(n) * K + k : static_cast<size_t>(k) * N + n] = value(k, n);
+  if (!split_) {
+    float* d = dalloc(h.size());
+    MRT_HIP_CHECK(hipMemcpy(d, h.data(), h.size() * 4, hipMemcpyHostToDevice));
+    return d;
+  }
+  bf16* d = salloc(h.size());
+  split_upload(h.data(), N, K, d, stream);
+  return d;
+}
+
 // WNConv2d (spectrostream.cpp:125-139): stored (O, I, kH, kW) -> one sub-problem
 // with rows (t * I + c), t = kh * kW + kw, columns O padded to the tile width.
 Codec::Conv Codec::pack_conv(const TensorSource& w, const std::string& name, int o, int i, int kh, int kw) {
@@ -42,16 +61,10 @@ Codec::Conv Codec::pack_conv(const TensorSource& w, const std::string& name, int
   c.cin = i;
   c.cout = o;
   c.cout_pad = round_up(o, 64);
-  std::vector<float> h(static_cast<size_t>(kh) * kw * i * c.cout_pad, 0.f);
-  for (int oo = 0; oo < o; ++oo)
-    for (int ii = 0; ii < i; ++ii)
-      for (int y = 0; y < kh; ++y)
-        for (int x = 0; x < kw; ++x)
-          h[(static_cast<size_t>(y * kw + x) * i + ii) * c.cout_pad + oo] =
-              t.data[((static_cast<size_t>(oo) * i + ii) * kh + y) * kw + x];
-  float* d = dalloc(h.size());
-  MRT_HIP_CHECK(hipMemcpy(d, h.data(), h.size() * 4, hipMemcpyHostToDevice));
-  c.w.push_back(d);
+  c.w.push_back(pack(kh * kw * i, c.cout_pad, [&](int k, int oo) {
+    const int tap = k / i, ii = k - tap * i;
+    return oo < o ? t.data[(static_cast<size_t>(oo) * i + ii) * kh * kw + tap] : 0.f;
+  }));
   c.bias = dalloc(o);
   MRT_HIP_CHECK(hipMemcpy(c.bias, b.data, o * 4, hipMemcpyHostToDevice));
   return c;
@@ -73,18 +86,10 @@ Codec::Conv Codec::pack_transposed(const TensorSource& w, const std::string& nam
   for (int ph = 0; ph < sh; ++ph)
     for (int pw = 0; pw < sw; ++pw) {
       const int nj = (kh - ph + sh - 1) / sh, ni = (kw - pw + sw - 1) / sw;
-      std::vector<float> h(static_cast<size_t>(nj) * ni * i * c.cout_pad, 0.f);
-      for (int j = 0; j < nj; ++j)
-        for (int q = 0; q < ni; ++q) {
-          const int y = ph + sh * j, x = pw + sw * q, tap = j * ni + q;
-          for (int ii = 0; ii < i; ++ii)
-            for (int oo = 0; oo < o; ++oo)
-              h[(static_cast<size_t>(tap) * i + ii) * c.cout_pad + oo] =
-                  t.data[((static_cast<size_t>(ii) * o + oo) * kh + y) * kw + x];
-        }
-      float* d = dalloc(h.size());
-      MRT_HIP_CHECK(hipMemcpy(d, h.data(), h.size() * 4, hipMemcpyHostToDevice));
-      c.w.push_back(d);
+      c.w.push_back(pack(nj * ni * i, c.cout_pad, [&](int k, int oo) {
+        const int tap = k / i, ii = k - tap * i, y = ph + sh * (tap / ni), x = pw + sw * (tap % ni);
+        return oo < o ? t.data[((static_cast<size_t>(ii) * o + oo) * kh + y) * kw + x] : 0.f;
+      }));
     }
   c.bias = dalloc(o);
   MRT_HIP_CHECK(hipMemcpy(c.bias, b.data, o * 4, hipMemcpyHostToDevice));
@@ -146,6 +151,9 @@ Codec::Codec(const TensorSource& w, const TensorSource& cbs, const CodecConfig& 
   MRT_HIP_CHECK(hipEventCreate(&ev_[0]));
   MRT_HIP_CHECK(hipEventCreate(&ev_[1]));
 
+  split_ = E % 32 == 0 && P % 32 == 0 && C0 % 32 == 0 && (2 * cfg.hop) % 32 == 0 && cfg.blocks[0].out_ch % 64 == 0;
+  for (const CodecBlockCfg& b : cfg.blocks) split_ = split_ && b.in_ch % 32 == 0 && b.out_ch % 32 == 0;
+
   const HostTensor& cb = cbs.tensor("codebooks");
   const size_t cbn = static_cast<size_t>(cfg.levels) * cfg.codebook * E;
   codebooks_ = dalloc(cbn);
@@ -163,7 +171,7 @@ Codec::Codec(const TensorSource& w, const TensorSource& cbs, const CodecConfig& 
     blk_c_.push_back(pack_conv(w, p + ".conv", b.out_ch, b.out_ch, b.kph, b.kpw));
     blk_sc_.push_back(b.in_ch != b.out_ch ? pack_conv(w, p + ".shortcut", b.out_ch, b.in_ch, 1, 1) : Conv{});
   }
-  {  // output conv: compact (kh, kw, cin, 2) for the vector-ALU kernel
+  {  // output conv: compact (cin, kh, kw, 2) for the vector-ALU kernel
     const int ci = cfg.blocks.back().out_ch, k = cfg.out_k;
     MRT_REQUIRE(k == 7 && ci % 8 == 0, "codec: output conv shape");
     const HostTensor& t = w.tensor("output_conv.weight");
@@ -172,7 +180,8 @@ Codec::Codec(const TensorSource& w, const TensorSource& cbs, const CodecConfig& 
       for (int c = 0; c < ci; ++c)
         for (int y = 0; y < k; ++y)
           for (int x = 0; x < k; ++x)
-            h[((static_cast<size_t>(y) * k + x) * ci + c) * 2 + o] = t.data[((static_cast<size_t>(o) * ci + c) * k + y) * k + x];
+            h[((static_cast<size_t>(c) * k + y) * k + x) * 2 + o] =
+                t.data[((static_cast<size_t>(o) * ci + c) * k + y) * k + x];
     out_w_ = dalloc(h.size());
     MRT_HIP_CHECK(hipMemcpy(out_w_, h.data(), h.size() * 4, hipMemcpyHostToDevice));
     out_b_ = dalloc(2);
@@ -194,19 +203,14 @@ Codec::Codec(const TensorSource& w, const TensorSource& cbs, const CodecConfig& 
     istft_.cin = 2 * F;
     istft_.cout = N;
     istft_.cout_pad = round_up(N, 64);
-    std::vector<float> h(static_cast<size_t>(2 * F) * istft_.cout_pad, 0.f);
-    for (int k = 0; k < F; ++k)
-      for (int t = 0; t < N; ++t) {
-        const long kt = (static_cast<long>(k) * t) % N;
-        const double ang = 2.0 * M_PI * static_cast<double>(kt) / N;
-        const double c = k == 0 ? 1.0 : 2.0;
-        h[static_cast<size_t>(2 * k) * istft_.cout_pad + t] = static_cast<float>(c * std::cos(ang) / N * syn[t]);
-        h[static_cast<size_t>(2 * k + 1) * istft_.cout_pad + t] =
-            static_cast<float>(-c * std::sin(ang) / N * syn[t]);
-      }
-    float* d = dalloc(h.size());
-    MRT_HIP_CHECK(hipMemcpy(d, h.data(), h.size() * 4, hipMemcpyHostToDevice));
-    istft_.w.push_back(d);
+    istft_.w.push_back(pack(2 * F, istft_.cout_pad, [&](int r, int t) {
+      if (t >= N) return 0.f;
+      const int k = r / 2;
+      const long kt = (static_cast<long>(k) * t) % N;
+      const double ang = 2.0 * M_PI * static_cast<double>(kt) / N;
+      const double c = k == 0 ? 1.0 : 2.0;
+      return static_cast<float>(r % 2 == 0 ? c * std::cos(ang) / N * syn[t] : -c * std::sin(ang) / N * syn[t]);
+    }));
   }
 
   // activations at max_frames
@@ -214,12 +218,26 @@ Codec::Codec(const TensorSource& w, const TensorSource& cbs, const CodecConfig& 
   tok_ = static_cast<int*>(static_cast<void*>(dalloc(static_cast<size_t>(max_frames) * cfg.levels)));
   emb_ = dalloc(static_cast<size_t>(Hn) * E);
   skip_ = dalloc(static_cast<size_t>(Hn) * P);
-  p1_ = dalloc(static_cast<size_t>(Hn) * P);
   x0_ = dalloc(static_cast<size_t>(Hn) * P);
-  x0e_ = dalloc(static_cast<size_t>(Hn) * P);
-  t0_ = dalloc(static_cast<size_t>(Hn) * P);
   x1_ = dalloc(static_cast<size_t>(Hn) * P);
-  x1e_ = dalloc(static_cast<size_t>(Hn) * P);
+  auto both = [&](float*& f, bf16*& s, size_t values) {  // read by convolutions only
+    if (split_)
+      s = salloc(values);
+    else
+      f = dalloc(values);
+  };
+  both(p1_, p1s_, static_cast<size_t>(Hn) * P);
+  both(x0e_, x0es_, static_cast<size_t>(Hn) * P);
+  both(t0_, t0s_, static_cast<size_t>(Hn) * P);
+  both(x1e_, x1es_, static_cast<size_t>(Hn) * P);
+  if (split_) {
+    embs_ = salloc(static_cast<size_t>(Hn) * E);
+    if (cfg.blocks[0].in_ch != cfg.blocks[0].out_ch) x1s_ = salloc(static_cast<size_t>(Hn) * P);
+    int zmax = std::max(std::max(E, P), 2 * cfg.hop);
+    for (const CodecBlockCfg& b : cfg.blocks) zmax = std::max(zmax, std::max(b.in_ch, b.out_ch));
+    zeros_ = salloc(zmax);
+    MRT_HIP_CHECK(hipMemsetAsync(zeros_, 0, static_cast<size_t>(zmax) * 6, stream));
+  }
   size_t tmax = 0, rmax = 0;
   int n = 1, H = Hn, W = cfg.unfold;
   for (size_t i = 0; i < cfg.blocks.size(); ++i) {
@@ -230,15 +248,20 @@ Codec::Codec(const TensorSource& w, const TensorSource& cbs, const CodecConfig& 
     const size_t outn = static_cast<size_t>(n) * H * W * b.out_ch;
     tmax = std::max(tmax, outn);
     blk_out_.push_back(dalloc(outn));
-    blk_oute_.push_back(dalloc(outn));
+    const bool last = i + 1 == cfg.blocks.size();  // read by the output conv
+    blk_oute_.push_back(!split_ || last ? dalloc(outn) : nullptr);
+    blk_outes_.push_back(split_ && !last ? salloc(outn) : nullptr);
+    blk_outs_.push_back(split_ && !last && cfg.blocks[i + 1].in_ch != cfg.blocks[i + 1].out_ch ? salloc(outn)
+                                                                                              : nullptr);
     blk_out_n_.push_back(outn);
     if (i == 0) n = 2;
   }
   MRT_REQUIRE(W == cfg.hop, "codec: the decoder's width must reach hop frequency bins");
-  tbuf_ = dalloc(tmax);
+  both(tbuf_, tbufs_, tmax);
   rbuf_ = dalloc(std::max<size_t>(rmax, 1));
   const int Hs = H - cfg.temporal_crop;
   spec_ = dalloc(static_cast<size_t>(2) * Hs * cfg.hop * 2);
+  if (split_) specs_ = salloc(static_cast<size_t>(2) * Hs * cfg.hop * 2);
   wf_ = dalloc(static_cast<size_t>(2) * Hs * cfg.n_fft);
   audio_ = dalloc(static_cast<size_t>(max_frames) * cfg.samples_per_frame * 2);
 }
@@ -264,15 +287,23 @@ const Codec::Plan& Codec::plan(int frames) {
   auto pl = std::make_unique<Plan>();
   pl->frames = frames;
   std::vector<std::vector<ConvSub>> subs;
-  size_t need_partial = 0;
+  size_t need_partial = 0, need_counters = 0;
 
   auto add = [&](ConvLaunch L, std::vector<ConvSub> s) {
+    MRT_REQUIRE(L.cin % 16 == 0 && L.cout % L.split == 0, "codec plan: channel layout");
+    int rows = 64;
+    if (split_) {
+      MRT_REQUIRE(L.xs && L.cin % 32 == 0 && (!(L.ys || L.ys_elu) || L.split % 32 == 0), "codec plan: split layout");
+      conv_split_plan(L, s.data(), static_cast<int>(s.size()));
+      rows = conv_split_tile_rows(L);
+    }
     int tiles = 0;
     for (auto& q : s) {
       q.tile0 = tiles;
       const long M = static_cast<long>(L.n) * q.gy * q.gx;
-      MRT_REQUIRE(M >= 1 && q.ntaps >= 1 && q.ntaps <= kConvMaxTaps, "codec plan: empty sub-problem");
-      tiles += static_cast<int>((M + 63) / 64);
+      MRT_REQUIRE(M >= 1 && M <= 0x7fffffffL - 256 && q.ntaps >= 1 && q.ntaps <= kConvMaxTaps,
+                  "codec plan: empty sub-problem");
+      tiles += static_cast<int>((M + rows - 1) / rows);
       // output / residual coordinates at the grid's corners (affine, monotone)
       for (int y : {0, q.gy - 1})
         for (int x : {0, q.gx - 1}) {
@@ -282,26 +313,34 @@ const Codec::Plan& Codec::plan(int frames) {
             MRT_REQUIRE(oy / L.rh < L.res_h && ox / L.rw < L.res_w, "codec plan: residual out of range");
         }
     }
-    MRT_REQUIRE(L.cin % 16 == 0 && L.cout % L.split == 0, "codec plan: channel layout");
-    // split-K when the tiles alone give fewer than 2 workgroups per CU:
-    // ~512 workgroups, >= 2 K chunks per slice
-    L.ksplit = 1;
-    L.rows = tiles * 64;
-    const int blocks = tiles * (L.cout_pad / 64);
-    if (blocks < 512) {
-      int min_nk = 1 << 30;
-      for (auto& q : s) min_nk = std::min(min_nk, q.ntaps * (L.cin / (L.cin % 32 == 0 ? 32 : 16)));
-      L.ksplit = std::max(1, std::min({(512 + blocks - 1) / blocks, min_nk / 2, 16}));
+    if (split_) {
+      need_partial = std::max(need_partial, conv_split_partial(L, tiles));
+      need_counters = std::max(need_counters, conv_split_counters(L, tiles));
+    } else {
+      // split-K when the tiles alone give fewer than 2 workgroups per CU:
+      // ~512 workgroups, >= 2 K chunks per slice
+      L.ksplit = 1;
+      L.rows = tiles * 64;
+      const int blocks = tiles * (L.cout_pad / 64);
+      if (blocks < 512) {
+        int min_nk = 1 << 30;
+        for (auto& q : s) min_nk = std::min(min_nk, q.ntaps * (L.cin / (L.cin % 32 == 0 ? 32 : 16)));
+        L.ksplit = std::max(1, std::min({(512 + blocks - 1) / blocks, min_nk / 2, 16}));
+      }
+      if (L.ksplit > 1) need_partial = std::max(need_partial, static_cast<size_t>(L.ksplit) * L.rows * L.cout_pad);
     }
-    if (L.ksplit > 1) need_partial = std::max(need_partial, static_cast<size_t>(L.ksplit) * L.rows * L.cout_pad);
     pl->launches.push_back(L);
     pl->tiles_m.push_back(tiles);
     pl->tiles_n.push_back(L.cout_pad / 64);
     subs.push_back(std::move(s));
   };
-  auto base = [&](const Conv& c, const float* x, int n, int hin, int win, float* y, int hout, int wout) {
+  // input x (fp32) or xs (split), output y
+  auto base = [&](const Conv& c, const float* x, const bf16* xs, int n, int hin, int win, float* y, int hout,
+                  int wout) {
     ConvLaunch L{};
     L.x = x;
+    L.xs = xs;
+    L.zeros = zeros_;
     L.n = n;
     L.hin = hin;
     L.win = win;
@@ -334,12 +373,14 @@ const Codec::Plan& Codec::plan(int frames) {
 
   const int Hn = frames + cfg.temporal_pad;
   // Res1x1Block input_proj (spectrostream.cpp:174-181) on (1, Hn, 1, E)
-  add(base(proj_sc_, emb_, 1, Hn, 1, skip_, Hn, 1), regular(proj_sc_, Hn, 1, 1, 1, 0, 0, 0));
+  add(base(proj_sc_, emb_, embs_, 1, Hn, 1, skip_, Hn, 1), regular(proj_sc_, Hn, 1, 1, 1, 0, 0, 0));
   {
-    ConvLaunch L = base(proj_c1_, emb_, 1, Hn, 1, p1_, Hn, 1);
+    ConvLaunch L = base(proj_c1_, emb_, embs_, 1, Hn, 1, p1_, Hn, 1);
+    L.ys = p1s_;
     L.act_out = kActElu;
     add(L, regular(proj_c1_, Hn, 1, 1, 1, 0, 0, 0));
-    ConvLaunch L2 = base(proj_c2_, p1_, 1, Hn, 1, x0_, Hn, 1);
+    ConvLaunch L2 = base(proj_c2_, p1_, p1s_, 1, Hn, 1, x0_, Hn, 1);
+    L2.ys_elu = x0es_;
     L2.y_elu = x0e_;  // elu(x0): input_conv's first conv reads it as is
     L2.res = skip_;
     L2.res_h = Hn;
@@ -350,11 +391,14 @@ const Codec::Plan& Codec::plan(int frames) {
   const int W0 = cfg.unfold;
   // Res3x3Block input_conv, causal (spectrostream.cpp:191-200): pads top 2, left 1
   {
-    ConvLaunch L = base(in_c1_, x0e_, 1, Hn, W0, t0_, Hn, W0);
+    ConvLaunch L = base(in_c1_, x0e_, x0es_, 1, Hn, W0, t0_, Hn, W0);
+    L.ys = t0s_;
     L.act_out = kActElu;
     add(L, regular(in_c1_, Hn, W0, 3, 3, 2, 1, 0));
-    ConvLaunch L2 = base(in_c2_, t0_, 1, Hn, W0, x1_, Hn, W0);
+    ConvLaunch L2 = base(in_c2_, t0_, t0s_, 1, Hn, W0, x1_, Hn, W0);
     L2.y_elu = x1e_;
+    L2.ys = x1s_;
+    L2.ys_elu = x1es_;
     L2.res = x0_;
     L2.res_h = Hn;
     L2.res_w = W0;
@@ -363,6 +407,7 @@ const Codec::Plan& Codec::plan(int frames) {
   // DecoderResBlocks (spectrostream.cpp:224-262)
   const float* x = x1_;   // raw: the residual / shortcut input
   const float* xe = x1e_;  // elu(x): the transposed conv's input
+  const bf16 *xs = x1s_, *xes = x1es_;  // the same, split
   int n = 1, H = Hn, W = W0;
   for (size_t i = 0; i < cfg.blocks.size(); ++i) {
     const CodecBlockCfg& b = cfg.blocks[i];
@@ -370,12 +415,13 @@ const Codec::Plan& Codec::plan(int frames) {
     const int cs = (b.ktw - b.sw) / 2;       // crop_w_start
     const float* res = x;
     if (b.in_ch != b.out_ch) {  // shortcut on the input grid, repeated by the epilogue below
-      add(base(blk_sc_[i], x, n, H, W, rbuf_, H, W), regular(blk_sc_[i], H, W, 1, 1, 0, 0, 0));
+      add(base(blk_sc_[i], x, xs, n, H, W, rbuf_, H, W), regular(blk_sc_[i], H, W, 1, 1, 0, 0, 0));
       res = rbuf_;
     }
     // conv_transpose(elu(x)) + bias, cropped, then elu: one sub-problem per phase
     {
-      ConvLaunch L = base(blk_t_[i], xe, n, H, W, tbuf_, Ho, Wo);
+      ConvLaunch L = base(blk_t_[i], xe, xes, n, H, W, tbuf_, Ho, Wo);
+      L.ys = tbufs_;
       L.act_out = kActElu;
       std::vector<ConvSub> ph_subs;
       int wi = 0;
@@ -404,8 +450,10 @@ const Codec::Plan& Codec::plan(int frames) {
     // conv(causal pad(elu'd T)) + bias + residual (repeated by the stride)
     {
       const int top = b.kph - 1, left = (b.kpw - 1) / 2;
-      ConvLaunch L = base(blk_c_[i], tbuf_, n, Ho, Wo, blk_out_[i], Ho, Wo);
+      ConvLaunch L = base(blk_c_[i], tbuf_, tbufs_, n, Ho, Wo, blk_out_[i], Ho, Wo);
       L.y_elu = blk_oute_[i];
+      L.ys = blk_outs_[i];
+      L.ys_elu = blk_outes_[i];
       L.res = res;
       L.res_h = H;
       L.res_w = W;
@@ -416,6 +464,8 @@ const Codec::Plan& Codec::plan(int frames) {
     }
     x = blk_out_[i];
     xe = blk_oute_[i];
+    xs = blk_outs_[i];
+    xes = blk_outes_[i];
     if (i == 0) n = 2;
     H = Ho;
     W = Wo;
@@ -428,14 +478,23 @@ const Codec::Plan& Codec::plan(int frames) {
   pl->out_w = W;
   pl->out_hs = Hs;
   // iSTFT frames: spec (2 Hs rows of 2 hop) x basis (2 hop, n_fft)
-  add(base(istft_, spec_, 1, 2 * Hs, 1, wf_, 2 * Hs, 1), regular(istft_, 2 * Hs, 1, 1, 1, 0, 0, 0));
+  add(base(istft_, spec_, specs_, 1, 2 * Hs, 1, wf_, 2 * Hs, 1), regular(istft_, 2 * Hs, 1, 1, 1, 0, 0, 0));
 
   if (need_partial > partial_n_) {
     MRT_HIP_CHECK(hipStreamSynchronize(stream));  // an older, smaller buffer may still be in use
     partial_ = dalloc(need_partial);
     partial_n_ = need_partial;
   }
-  for (auto& L : pl->launches) L.partial = partial_;
+  if (need_counters > counters_n_) {
+    MRT_HIP_CHECK(hipStreamSynchronize(stream));
+    counters_ = reinterpret_cast<unsigned*>(dalloc(need_counters));
+    MRT_HIP_CHECK(hipMemsetAsync(counters_, 0, need_counters * 4, stream));
+    counters_n_ = need_counters;
+  }
+  for (auto& L : pl->launches) {
+    L.partial = partial_;
+    L.counters = counters_;
+  }
   // upload every launch's sub-problems into one device array
   size_t total = 0;
   for (auto& s : subs) total += s.size();
@@ -457,13 +516,15 @@ void Codec::enqueue(const int* tokens_dev, int frames, float* audio_dev) {
   const Plan& pl = plan(frames);
   MRT_HIP_CHECK(hipEventRecord(ev_[0], stream));
   rvq_dequant(tokens_dev, frames, cfg.levels, codebooks_, cfg.codebook, cfg.embedding_dim, cfg.temporal_pad, emb_,
-              stream);
+              embs_, stream);
   for (size_t l = 0; l < pl.launches.size(); ++l) {
     if (static_cast<int>(l) == pl.out_at)
       out_conv(blk_oute_.back(), 2, pl.out_h, pl.out_w, cfg.blocks.back().out_ch, cfg.temporal_crop, false, out_w_,
-               out_b_,
-               spec_, pl.out_hs, stream);
-    conv_launch(pl.launches[l], pl.tiles_m[l], pl.tiles_n[l], stream);
+               out_b_, spec_, specs_, pl.out_hs, stream);
+    if (split_)
+      conv_split_launch(pl.launches[l], pl.tiles_m[l], stream);
+    else
+      conv_launch(pl.launches[l], pl.tiles_m[l], pl.tiles_n[l], stream);
   }
   const int Hs = spec_frames(frames);
   overlap_add(wf_, Hs, cfg.n_fft, frames * cfg.samples_per_frame, audio_dev, stream);

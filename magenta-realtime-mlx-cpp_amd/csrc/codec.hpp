@@ -3,8 +3,9 @@
 // post-processor (spectrostream.cpp:593-681), in fp32 as the reference runs
 // it (system.cpp:118-119, 373-390).
 //
-// Every convolution is an implicit GEMM on the fp32 matrix cores
-// (codec_kernels.hip): M = output pixels, N = output channels, K = taps x
+// Every convolution is an implicit GEMM on the bf16 matrix cores with fp32 operands
+// split into three parts (conv_split.hip), or on the fp32 matrix cores where a
+// channel count is no multiple of 32 (codec_kernels.hip): M = output pixels, N = output channels, K = taps x
 // input channels, activations NHWC.  A transposed convolution is launched as
 // one sub-problem per output stride phase, each a stride-1 convolution over
 // the input (no multiplies by inserted zeros); crops are output offsets; the
@@ -37,7 +38,7 @@ struct ConvSub {
   int oys, oyo, oxs, oxo;
   int ntaps;
   int tile0;  // first M tile of this sub-problem in the launch
-  const float* w;
+  const void* w;  // fp32 [tap][c][o], or split rows (o, taps x cin) for a split launch
   int16_t dy[kConvMaxTaps];
   int16_t dx[kConvMaxTaps];
 };
@@ -62,21 +63,40 @@ struct ConvLaunch {
   int ksplit, rows;
   float* partial;
   float* y_elu;  // when non-null, also elu(result) here (same layout): the next ELU'd input
+  // Split launches (conv_split.hip; cin % 32 == 0, input already ELU'd): input and
+  // outputs as split rows (split_gemm.hpp), one row a pixel; y may be null then.
+  // partial holds one tile of sums per (tile, slice), counters (zero between
+  // launches) one word per tile.
+  const bf16* xs;
+  const bf16* zeros;  // cin split zeros
+  bf16 *ys, *ys_elu;  // result and elu(result), when non-null
+  int tile;           // tile shape (conv_split_plan)
+  unsigned* counters;
 };
+
+// Tile shape and K split of a split launch whose other fields are set; pixels a tile
+// row covers, and the fp32 values / words of partial and counters it needs.
+void conv_split_plan(ConvLaunch& a, const ConvSub* subs, int nsub);
+int conv_split_tile_rows(const ConvLaunch& a);
+size_t conv_split_partial(const ConvLaunch& a, int tiles_m);
+size_t conv_split_counters(const ConvLaunch& a, int tiles_m);
+void conv_split_launch(const ConvLaunch& a, int tiles_m, hipStream_t s);
 
 // One convolution launch (plus its split-K finish when a.ksplit > 1).
 void conv_launch(const ConvLaunch& a, int tiles_m, int tiles_n, hipStream_t s);
 // emb (frames + pad, dim): rows < frames = sum over levels k < levels of
 // codebooks[k][tokens[f * levels + k]] (fp32, level order); the pad rows 0.
-// Ids outside [0, codebook) are read as 0.
+// Ids outside [0, codebook) are read as 0.  emb_split (may be null): the same as
+// split rows.
 void rvq_dequant(const int* tokens, int frames, int levels, const float* codebooks, int codebook, int dim, int pad,
-                 float* emb, hipStream_t s);
+                 float* emb, bf16* emb_split, hipStream_t s);
 // The output conv: x (n, H, W, cin) -> out (n, Hs, W, 2) = conv7x7(elu(x))
 // (x already ELU'd when !elu_in) with causal padding (top 6, left 3, right 3)
-// over input rows from `crop` on, plus bias; w packed (kh, kw, cin, 2); cin a
-// multiple of 8.
+// over input rows from `crop` on, plus bias; w packed (cin, kh, kw, 2); cin a
+// multiple of 8.  out_split (may be null): the rows (n, Hs) of W x 2 values as
+// split rows too (W % 16 == 0).
 void out_conv(const float* x, int n, int H, int W, int cin, int crop, bool elu_in, const float* w, const float* bias,
-              float* out, int Hs, hipStream_t s);
+              float* out, bf16* out_split, int Hs, hipStream_t s);
 // audio (T, 2) from windowed frames wf (2 * H, n_fft): overlap-add at hop
 // n_fft / 2 (spectrostream.cpp:649-667), trimmed to T, channels interleaved.
 void overlap_add(const float* wf, int H, int n_fft, int T, float* audio, hipStream_t s);
@@ -136,7 +156,7 @@ class Codec {
 
  private:
   struct Conv {  // packed GEMM weights of one convolution (one entry per sub-problem)
-    std::vector<float*> w;
+    std::vector<void*> w;
     float* bias = nullptr;
     int cin = 0, cout = 0, cout_pad = 0;
   };
@@ -151,13 +171,18 @@ class Codec {
   const Plan& plan(int frames);
   void enqueue(const int* tokens_dev, int frames, float* audio_dev);
   float* dalloc(size_t floats);
+  bf16* salloc(size_t values);  // split values
+  // Uploads packed weights (K, N) given as value(k, n): fp32 rows of N, or split rows
+  // of K in split mode.
+  template <class F>
+  void* pack(int K, int N, F&& value);
   Conv pack_conv(const TensorSource& w, const std::string& name, int o, int i, int kh, int kw);
   Conv pack_transposed(const TensorSource& w, const std::string& name, int i, int o, int kh, int kw, int sh, int sw);
 
   std::vector<void*> allocs_;
   float* codebooks_ = nullptr;
   Conv proj_sc_, proj_c1_, proj_c2_, in_c1_, in_c2_, istft_;
-  float *out_w_ = nullptr, *out_b_ = nullptr;  // output conv (kh, kw, cin, 2), bias (2)
+  float *out_w_ = nullptr, *out_b_ = nullptr;  // output conv (cin, kh, kw, 2), bias (2)
   std::vector<Conv> blk_t_, blk_c_, blk_sc_;
   float *emb_ = nullptr, *skip_ = nullptr, *p1_ = nullptr, *x0_ = nullptr, *t0_ = nullptr, *x1_ = nullptr;
   float *x0e_ = nullptr, *x1e_ = nullptr;  // elu(x0), elu(x1)
@@ -167,6 +192,14 @@ class Codec {
   int* tok_ = nullptr;
   int last_frames_ = 0;
   std::map<int, std::unique_ptr<Plan>> plans_;
+  // Split mode (every channel count a multiple of 32): the convolutions run on split
+  // operands, and these take the place of the fp32 buffers that only feed them.
+  bool split_ = false;
+  bf16 *embs_ = nullptr, *p1s_ = nullptr, *x0es_ = nullptr, *t0s_ = nullptr, *x1s_ = nullptr, *x1es_ = nullptr;
+  bf16 *tbufs_ = nullptr, *specs_ = nullptr, *zeros_ = nullptr;
+  std::vector<bf16*> blk_outs_, blk_outes_;
+  unsigned* counters_ = nullptr;
+  size_t counters_n_ = 0;
   float* partial_ = nullptr;  // split-K partial sums (grown by plan())
   size_t partial_n_ = 0;
   hipEvent_t ev_[2] = {nullptr, nullptr};

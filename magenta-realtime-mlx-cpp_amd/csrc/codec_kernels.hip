@@ -1,5 +1,5 @@
-// Codec decode kernels (fp32): the implicit-GEMM convolution on the matrix
-// cores, RVQ dequantisation and the iSTFT overlap-add.
+// Codec decode kernels (fp32): the implicit-GEMM convolution on the fp32 matrix
+// cores (channel counts that conv_split.hip does not take), RVQ dequantisation and the iSTFT overlap-add.
 //
 // k_conv<BM, BN, KC>: a BM x BN output tile (pixels x channels) per
 // 256-thread workgroup (64 x 64: larger tiles measured slower, fewer
@@ -12,6 +12,7 @@
 // register sets).  LDS strides: A rows KC + 4 floats (the 16 rows x 4 k lanes of
 // an A fragment hit 64 distinct banks), B rows 80 floats (the same for B).
 #include "codec.hpp"
+#include "split_gemm.hpp"
 
 #include <type_traits>
 
@@ -60,7 +61,7 @@ __global__ __launch_bounds__(kThreads) void k_conv(ConvLaunch a) {
   const int M = a.n * gy * gx;
   const int m0 = ((int)blockIdx.x - sub->tile0) * BM;
   const int n0 = (int)blockIdx.y * BN;
-  const float* __restrict__ W = sub->w;
+  const float* __restrict__ W = static_cast<const float*>(sub->w);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
 
@@ -231,26 +232,28 @@ __global__ __launch_bounds__(256) void k_conv_finish(ConvLaunch a) {
 // The output convolution (Cout = 2, a 7 x 7 kernel, causal padding, the
 // first `crop` rows dropped; spectrostream.cpp:420-427) on the vector ALUs:
 // a matrix-core tile would be 2 of 16 columns.  Workgroup: 4 output rows x
-// 128 columns of one image and 256 threads, two halves over the input
-// channels (waves 0-1 and 2-3, so the weights a wave needs are uniform and
-// come through scalar loads); a thread owns a 4-pixel strip x 2 outputs.
-// The input halo (4 + 6 rows x 128 + 6 columns) is staged through LDS 8
-// channels at a time (4 per half) with the ELU applied; the halves' sums
-// meet in LDS at the end.
-constexpr int kOcRows = 4, kOcCols = 128, kOcStrip = 4, kOcThreads = 256;
+// 128 columns of one image and 512 threads, four parts over the input
+// channels (two waves each, so the weights a wave needs are uniform and come
+// through scalar loads, the 98 of a channel in one run: a load per tap stalled
+// the wave 49 times a channel); a thread owns a 4-pixel strip x 2 outputs and
+// reads its inputs 16 bytes at a time.  The input halo (4 + 6 rows x 128 + 6
+// columns) is staged through LDS 8 channels at a time (2 per part) with the ELU
+// applied; the parts' sums meet in LDS at the end.
+constexpr int kOcRows = 4, kOcCols = 128, kOcStrip = 4, kOcThreads = 512, kOcParts = 4;
 constexpr int kOcCh = 8, kOcK = 7;
-constexpr int kOcHaloR = kOcRows + kOcK - 1, kOcHaloC = kOcCols + kOcK - 1;
-constexpr int kOcPlane = kOcHaloR * kOcHaloC;
+constexpr int kOcHaloR = kOcRows + kOcK - 1, kOcHaloC = kOcCols + kOcK - 1, kOcPitch = kOcHaloC + 2;
+constexpr int kOcPlane = kOcHaloR * kOcPitch;
+static_assert(kOcPitch % 4 == 0, "16-byte reads of a strip: 12 floats from column 4 t, at most 136");
 
 __global__ __launch_bounds__(kOcThreads) void k_out_conv(const float* __restrict__ x, int H, int W, int cin, int crop,
                                                          int elu_in, const float* __restrict__ w,
                                                          const float* __restrict__ bias, float* __restrict__ out,
-                                                         int Hs) {
-  __shared__ float hl[kOcCh * kOcPlane];  // (channel, halo row, halo column)
+                                                         bf16* __restrict__ out_split, int Hs) {
+  __shared__ __attribute__((aligned(16))) float hl[kOcCh * kOcPlane];  // (channel, halo row, halo column)
   const int tid = threadIdx.x;
   const int img = blockIdx.z;
   const int y0 = blockIdx.y * kOcRows, x0 = blockIdx.x * kOcCols;
-  const int half = __builtin_amdgcn_readfirstlane(tid >> 7);  // wave-uniform
+  const int part = __builtin_amdgcn_readfirstlane(tid >> 7);  // wave-uniform
   const int st = tid & 127;
   const int ty = st / (kOcCols / kOcStrip), tx = (st % (kOcCols / kOcStrip)) * kOcStrip;
   float acc[kOcStrip][2];
@@ -260,7 +263,7 @@ __global__ __launch_bounds__(kOcThreads) void k_out_conv(const float* __restrict
   const int iy0 = y0 + crop - (kOcK - 1), ix0 = x0 - (kOcK - 1) / 2;
   for (int c0 = 0; c0 < cin; c0 += kOcCh) {
     __syncthreads();  // the previous chunk's reads are done
-    for (int i = tid; i < kOcPlane * 2; i += kOcThreads) {
+    for (int i = tid; i < kOcHaloR * kOcHaloC * 2; i += kOcThreads) {
       const int hh = i & 1, pix = i >> 1;
       const int r = pix / kOcHaloC, q = pix - r * kOcHaloC;
       const int iy = iy0 + r, ix = ix0 + q;
@@ -274,7 +277,7 @@ __global__ __launch_bounds__(kOcThreads) void k_out_conv(const float* __restrict
           v.w = elu1(v.w);
         }
       }
-      float* d = hl + (hh * 4) * kOcPlane + pix;
+      float* d = hl + (hh * 4) * kOcPlane + r * kOcPitch + q;
       d[0] = v.x;
       d[kOcPlane] = v.y;
       d[2 * kOcPlane] = v.z;
@@ -282,18 +285,24 @@ __global__ __launch_bounds__(kOcThreads) void k_out_conv(const float* __restrict
     }
     __syncthreads();
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int ch = c0 + half * 4 + c;
-      const float* hc = hl + (half * 4 + c) * kOcPlane;
+    for (int c = 0; c < kOcCh / kOcParts; ++c) {
+      const int lc = part * (kOcCh / kOcParts) + c;
+      const float* hc = hl + lc * kOcPlane;
+      const float* wc = w + (size_t)(c0 + lc) * (kOcK * kOcK * 2);
 #pragma unroll
       for (int kh = 0; kh < kOcK; ++kh) {
-        float in[kOcStrip + kOcK - 1];
+        float in[12];
 #pragma unroll
-        for (int q = 0; q < kOcStrip + kOcK - 1; ++q) in[q] = hc[(ty + kh) * kOcHaloC + tx + q];
+        for (int q = 0; q < 12; q += 4) {
+          const float4 v = *reinterpret_cast<const float4*>(hc + (ty + kh) * kOcPitch + tx + q);
+          in[q] = v.x;
+          in[q + 1] = v.y;
+          in[q + 2] = v.z;
+          in[q + 3] = v.w;
+        }
 #pragma unroll
         for (int kw = 0; kw < kOcK; ++kw) {
-          const float* wk = w + ((size_t)(kh * kOcK + kw) * cin + ch) * 2;
-          const float w0 = wk[0], w1 = wk[1];
+          const float w0 = wc[(kh * kOcK + kw) * 2], w1 = wc[(kh * kOcK + kw) * 2 + 1];
 #pragma unroll
           for (int p = 0; p < kOcStrip; ++p) {
             acc[p][0] = fmaf(in[p + kw], w0, acc[p][0]);
@@ -303,18 +312,19 @@ __global__ __launch_bounds__(kOcThreads) void k_out_conv(const float* __restrict
       }
     }
   }
-  // the upper half's sums join the lower half's through LDS
+  // the other parts' sums join part 0's through LDS, in order
   __syncthreads();
   float* red = hl;
-  if (half == 1) {
+  if (part > 0) {
 #pragma unroll
-    for (int p = 0; p < kOcStrip; ++p) {
-      red[(p * 2) * 128 + st] = acc[p][0];
-      red[(p * 2 + 1) * 128 + st] = acc[p][1];
-    }
+    for (int p = 0; p < kOcStrip * 2; ++p) red[((part - 1) * kOcStrip * 2 + p) * 128 + st] = acc[p >> 1][p & 1];
   }
   __syncthreads();
-  if (half == 1) return;
+  if (part > 0) return;
+#pragma unroll
+  for (int q = 0; q < kOcParts - 1; ++q)
+#pragma unroll
+    for (int p = 0; p < kOcStrip * 2; ++p) acc[p >> 1][p & 1] += red[(q * kOcStrip * 2 + p) * 128 + st];
   const int oy = y0 + ty;
   if (oy >= Hs) return;
 #pragma unroll
@@ -322,13 +332,18 @@ __global__ __launch_bounds__(kOcThreads) void k_out_conv(const float* __restrict
     const int ox = x0 + tx + p;
     if (ox >= W) continue;
     float* o = out + ((size_t)(img * Hs + oy) * W + ox) * 2;
-    o[0] = acc[p][0] + red[(p * 2) * 128 + st] + bias[0];
-    o[1] = acc[p][1] + red[(p * 2 + 1) * 128 + st] + bias[1];
+    o[0] = acc[p][0] + bias[0];
+    o[1] = acc[p][1] + bias[1];
+    if (out_split) {
+      store_split(out_split, split_index((size_t)img * Hs + oy, 2 * ox, 2 * W), o[0]);
+      store_split(out_split, split_index((size_t)img * Hs + oy, 2 * ox + 1, 2 * W), o[1]);
+    }
   }
 }
 
 __global__ void k_rvq_dequant(const int* __restrict__ tokens, int frames, int levels,
-                              const float* __restrict__ cb, int codebook, int dim, float* __restrict__ emb) {
+                              const float* __restrict__ cb, int codebook, int dim, float* __restrict__ emb,
+                              bf16* __restrict__ emb_split) {
   const int f = blockIdx.x;
   for (int d = threadIdx.x; d < dim; d += blockDim.x) {
     float s = 0.f;
@@ -340,6 +355,7 @@ __global__ void k_rvq_dequant(const int* __restrict__ tokens, int frames, int le
       }
     }
     emb[(size_t)f * dim + d] = s;
+    if (emb_split) store_split(emb_split, split_index(f, d, dim), s);
   }
 }
 
@@ -372,17 +388,18 @@ void conv_launch(const ConvLaunch& a, int tiles_m, int tiles_n, hipStream_t s) {
 }
 
 void out_conv(const float* x, int n, int H, int W, int cin, int crop, bool elu_in, const float* w, const float* bias,
-              float* out, int Hs, hipStream_t s) {
+              float* out, bf16* out_split, int Hs, hipStream_t s) {
   MRT_REQUIRE(cin % kOcCh == 0, "codec: output conv input channels must be a multiple of 8");
   const dim3 grid((W + kOcCols - 1) / kOcCols, (Hs + kOcRows - 1) / kOcRows, n);
-  hipLaunchKernelGGL(k_out_conv, grid, dim3(kOcThreads), 0, s, x, H, W, cin, crop, elu_in ? 1 : 0, w, bias, out, Hs);
+  hipLaunchKernelGGL(k_out_conv, grid, dim3(kOcThreads), 0, s, x, H, W, cin, crop, elu_in ? 1 : 0, w, bias, out,
+                     out_split, Hs);
   MRT_HIP_CHECK(hipGetLastError());
 }
 
 void rvq_dequant(const int* tokens, int frames, int levels, const float* codebooks, int codebook, int dim, int pad,
-                 float* emb, hipStream_t s) {
+                 float* emb, bf16* emb_split, hipStream_t s) {
   hipLaunchKernelGGL(k_rvq_dequant, dim3(frames + pad), dim3(256), 0, s, tokens, frames, levels, codebooks, codebook,
-                     dim, emb);
+                     dim, emb, emb_split);
   MRT_HIP_CHECK(hipGetLastError());
 }
 

@@ -174,6 +174,8 @@ void gemm(DType dt, const void* A, const void* B, int M, int N, int K, const Gem
 // that produce them (attention from fp32 q/k/v).
 bool gemm_split_fits(int N, int K);
 void gemm_split(const bf16* A, const bf16* B, int M, int N, int K, const GemmEpiArgs& e, hipStream_t s);
+// W (N, K) fp32 in host memory -> split rows on the device (waits for s).
+void split_upload(const float* W, long N, int K, bf16* out, hipStream_t s);
 void rmsnorm_rows_split(const float* x, const float* g, float eps, int M, int D, bf16* y, hipStream_t s);
 void encoder_attn_split(const float* qkv, int nb, int S, int H, bf16* out, hipStream_t s);
 

@@ -248,6 +248,19 @@ void split_rows(const float* W, long N, int K, bf16* out, hipStream_t s) {
   MRT_HIP_CHECK(hipGetLastError());
 }
 
+void split_upload(const float* W, long N, int K, bf16* out, hipStream_t s) {
+  void* d = nullptr;
+  const size_t bytes = (size_t)N * K * 4;
+  MRT_HIP_CHECK(hipMalloc(&d, bytes));
+  hipError_t e = hipMemcpy(d, W, bytes, hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    split_rows(static_cast<const float*>(d), N, K, out, s);
+    e = hipStreamSynchronize(s);
+  }
+  (void)hipFree(d);
+  MRT_HIP_CHECK(e);
+}
+
 void rmsnorm_rows_split(const float* x, const float* g, float eps, int M, int D, bf16* y, hipStream_t s) {
   MRT_REQUIRE(M >= 1 && D % 32 == 0 && D <= 4096, "split norm: D must be a multiple of 32, at most 4096");
   const dim3 grid((M + 3) / 4), block(256);
