@@ -3,6 +3,7 @@
 // launch sequence of MusicCoCaEncoder::embed_text (musiccoca.cpp:272-294) and
 // StyleModel::tokenize (style_model.cpp:88-104).
 #include "coca.hpp"
+#include "kernels.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -29,7 +30,7 @@ float* Coca::dalloc(size_t floats) {
 
 // Linear (musiccoca.cpp:85-98), stored (out, in): several stored matrices
 // with the same input width stacked along the output axis, packed (in,
-// out_pad) for the GEMM, biases concatenated.
+// out_pad) for the GEMM (split mode: out_pad split rows), biases concatenated.
 Coca::Lin Coca::pack(const TensorSource& w, const std::vector<std::string>& names, int in) {
   Lin l;
   l.in = in;
@@ -42,13 +43,18 @@ Coca::Lin Coca::pack(const TensorSource& w, const std::vector<std::string>& name
     const HostTensor& b = w.tensor(n + ".bias");
     const int o = static_cast<int>(t.shape[0]);
     for (int r = 0; r < o; ++r) {
-      for (int c = 0; c < in; ++c) h[static_cast<size_t>(c) * l.out_pad + o0 + r] = t.data[static_cast<size_t>(r) * in + c];
+      for (int c = 0; c < in; ++c)
+        h[split_ ? static_cast<size_t>(o0 + r) * in + c : static_cast<size_t>(c) * l.out_pad + o0 + r] =
+            t.data[static_cast<size_t>(r) * in + c];
       hb[o0 + r] = b.data[r];
     }
     o0 += o;
   }
-  l.w = dalloc(h.size());
-  MRT_HIP_CHECK(hipMemcpy(l.w, h.data(), h.size() * 4, hipMemcpyHostToDevice));
+  l.w = dalloc(split_ ? h.size() / 2 * 3 : h.size());
+  if (split_)
+    split_upload(h.data(), l.out_pad, in, static_cast<bf16*>(l.w), stream);
+  else
+    MRT_HIP_CHECK(hipMemcpy(l.w, h.data(), h.size() * 4, hipMemcpyHostToDevice));
   l.b = dalloc(l.out);
   MRT_HIP_CHECK(hipMemcpy(l.b, hb.data(), hb.size() * 4, hipMemcpyHostToDevice));
   return l;
@@ -100,6 +106,7 @@ Coca::Coca(const TensorSource& w, const TensorSource& cbs, const CocaConfig& c, 
   MRT_HIP_CHECK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
   MRT_HIP_CHECK(hipEventCreate(&ev_[0]));
   MRT_HIP_CHECK(hipEventCreate(&ev_[1]));
+  split_ = D % 32 == 0 && F % 32 == 0 && HD % 32 == 0 && PD % 32 == 0;
   MRT_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&h_stage_), 64 * 1024, hipHostMallocDefault));
   auto up = [&](const std::string& n) {
     const HostTensor& t = w.tensor(n);
@@ -147,15 +154,28 @@ Coca::Coca(const TensorSource& w, const TensorSource& cbs, const CocaConfig& c, 
   tok_ = static_cast<int*>(static_cast<void*>(dalloc(c.rvq_depth)));
   mask_ = dalloc(L);
   x_ = dalloc(static_cast<size_t>(L) * D);
-  h_ = dalloc(static_cast<size_t>(L) * D);
   y_ = dalloc(static_cast<size_t>(L) * D);
-  n_ = dalloc(static_cast<size_t>(L) * D);
+  auto both = [&](float*& f, bf16*& sp, size_t values) {  // read by GEMMs only
+    if (split_)
+      sp = reinterpret_cast<bf16*>(dalloc((values * 6 + 3) / 4));
+    else
+      f = dalloc(values);
+  };
+  both(h_, hs_, static_cast<size_t>(L) * D);
+  both(n_, ns_, static_cast<size_t>(L) * D);
+  both(att_, atts_, static_cast<size_t>(L) * HD);
+  both(f_, fs_, static_cast<size_t>(L) * F);
+  both(patt_, patts_, PD);
+  if (split_) {
+    const size_t zb = static_cast<size_t>(std::max(std::max(D, F), std::max(HD, PD))) * 6;
+    zeros_ = reinterpret_cast<bf16*>(dalloc((zb + 3) / 4));
+    MRT_HIP_CHECK(hipMemsetAsync(zeros_, 0, zb, stream));
+    pquerys_ = reinterpret_cast<bf16*>(dalloc((static_cast<size_t>(D) * 6 + 3) / 4));
+    split_upload(w.tensor("text_pooler.query").data, 1, D, pquerys_, stream);
+  }
   qkv_buf_ = dalloc(static_cast<size_t>(L) * qkv_[0].out);
-  att_ = dalloc(static_cast<size_t>(L) * HD);
-  f_ = dalloc(static_cast<size_t>(L) * F);
   pq_buf_ = dalloc(PD);
   pkv_buf_ = dalloc(static_cast<size_t>(L) * 2 * PD);
-  patt_ = dalloc(PD);
   emb_ = dalloc(D);
   res_ = dalloc(D);
   rvq_work_ = dalloc(2 * (D + c.codebook));
@@ -164,17 +184,17 @@ Coca::Coca(const TensorSource& w, const TensorSource& cbs, const CocaConfig& c, 
   // the GEMM plan of one prompt (fixed: the prompt is always max_text_len rows)
   for (int i = 0; i < c.num_layers; ++i) {
     const float* xin = i == 0 ? x_ : layer_out_[i - 1];
-    plan_gemm(h_, L, qkv_[i], qkv_buf_, nullptr, kActNone);
-    plan_gemm(att_, L, o_[i], y_, xin, kActNone);
-    plan_gemm(h_, L, w1_[i], f_, nullptr, kActGelu);
-    plan_gemm(f_, L, w2_[i], layer_out_[i], y_, kActNone);
+    plan_gemm(h_, hs_, L, qkv_[i], qkv_buf_, nullptr, nullptr, kActNone);
+    plan_gemm(att_, atts_, L, o_[i], y_, nullptr, xin, kActNone);
+    plan_gemm(h_, hs_, L, w1_[i], f_, fs_, nullptr, kActGelu);
+    plan_gemm(f_, fs_, L, w2_[i], layer_out_[i], nullptr, y_, kActNone);
   }
-  plan_gemm(pquery_, 1, pq_, pq_buf_, nullptr, kActNone);
-  plan_gemm(n_, L, pkv_, pkv_buf_, nullptr, kActNone);
-  plan_gemm(patt_, 1, po_, emb_, nullptr, kActNone);
+  plan_gemm(pquery_, pquerys_, 1, pq_, pq_buf_, nullptr, nullptr, kActNone);
+  plan_gemm(n_, ns_, L, pkv_, pkv_buf_, nullptr, nullptr, kActNone);
+  plan_gemm(patt_, patts_, 1, po_, emb_, nullptr, nullptr, kActNone);
   // one sub-problem per GEMM in device memory; split-K workspace
   std::vector<ConvSub> subs(steps_.size());
-  size_t need = 0;
+  size_t need = 0, words = 0;
   for (size_t s = 0; s < steps_.size(); ++s) {
     ConvSub& q = subs[s];
     q = ConvSub{};  // rows (0, y, 0) -> output (y, 0), one tap at offset 0
@@ -183,22 +203,36 @@ Coca::Coca(const TensorSource& w, const TensorSource& cbs, const CocaConfig& c, 
     q.oys = q.oxs = 1;
     q.ntaps = 1;
     q.w = steps_[s].w;
-    need = std::max(need, static_cast<size_t>(steps_[s].L.ksplit) * steps_[s].L.rows * steps_[s].L.cout_pad);
+    if (split_) {
+      need = std::max(need, conv_split_partial(steps_[s].L, steps_[s].tiles_m));
+      words = std::max(words, conv_split_counters(steps_[s].L, steps_[s].tiles_m));
+    } else {
+      need = std::max(need, static_cast<size_t>(steps_[s].L.ksplit) * steps_[s].L.rows * steps_[s].L.cout_pad);
+    }
   }
   MRT_HIP_CHECK(hipMalloc(&subs_dev_, subs.size() * sizeof(ConvSub)));
   MRT_HIP_CHECK(hipMemcpy(subs_dev_, subs.data(), subs.size() * sizeof(ConvSub), hipMemcpyHostToDevice));
   partial_ = dalloc(std::max<size_t>(need, 1));
+  if (split_) {
+    counters_ = reinterpret_cast<unsigned*>(dalloc(words));
+    MRT_HIP_CHECK(hipMemsetAsync(counters_, 0, words * 4, stream));
+  }
   for (size_t s = 0; s < steps_.size(); ++s) {
     steps_[s].L.subs = subs_dev_ + s;
     steps_[s].L.partial = partial_;
+    steps_[s].L.counters = counters_;
   }
 }
 
 // One GEMM y (M, out) = x (M, in) W^T + b (+ res) (act), as a one-tap
 // implicit-GEMM launch (its sub-problem is uploaded with the others).
-void Coca::plan_gemm(const float* x, int M, const Lin& l, float* y, const float* res, int act) {
+void Coca::plan_gemm(const float* x, const bf16* xs, int M, const Lin& l, float* y, bf16* ys, const float* res,
+                     int act) {
   ConvLaunch L{};
   L.x = x;
+  L.xs = xs;
+  L.zeros = zeros_;
+  L.ys = ys;
   L.n = 1;
   L.hin = M;
   L.win = 1;
@@ -216,6 +250,16 @@ void Coca::plan_gemm(const float* x, int M, const Lin& l, float* y, const float*
   L.rh = L.rw = 1;
   L.act_out = act;
   L.nsub = 1;
+  if (split_) {
+    ConvSub q{};
+    q.gy = M;
+    q.gx = 1;
+    q.ntaps = 1;
+    conv_split_plan(L, &q, 1);
+    const int rows = conv_split_tile_rows(L);
+    steps_.push_back(Step{L, (M + rows - 1) / rows, l.out_pad / 64, l.w});
+    return;
+  }
   const int tiles = (M + 63) / 64;
   L.rows = tiles * 64;
   const int blocks = tiles * (l.out_pad / 64);
@@ -223,6 +267,14 @@ void Coca::plan_gemm(const float* x, int M, const Lin& l, float* y, const float*
   L.ksplit = blocks < 512 ? std::max(1, std::min({(512 + blocks - 1) / blocks, nk / 2, 16})) : 1;
   MRT_REQUIRE(l.in % 16 == 0, "musiccoca: GEMM inputs must be multiples of 16 wide");
   steps_.push_back(Step{L, tiles, l.out_pad / 64, l.w});
+}
+
+void Coca::gemm_step(size_t i) {
+  const Step& s = steps_[i];
+  if (split_)
+    conv_split_launch(s.L, s.tiles_m, stream);
+  else
+    conv_launch(s.L, s.tiles_m, s.tiles_n, stream);
 }
 
 Coca::~Coca() {
@@ -247,30 +299,30 @@ void Coca::enqueue_text() {
   size_t s = 0;
   for (int i = 0; i < c.num_layers; ++i) {
     const float* xin = i == 0 ? x_ : layer_out_[i - 1];
-    layer_norm_rows(xin, L, D, ln1w_[i], ln1b_[i], 1e-5f, h_, stream);
-    conv_launch(steps_[s].L, steps_[s].tiles_m, steps_[s].tiles_n, stream);  // q | k | v
+    layer_norm_rows(xin, L, D, ln1w_[i], ln1b_[i], 1e-5f, h_, hs_, stream);
+    gemm_step(s);  // q | k | v
     ++s;
     coca_attention(qkv_buf_, 3 * HD, qkv_buf_ + HD, 3 * HD, qkv_buf_ + 2 * HD, 3 * HD, L, L, c.num_heads, c.d_head,
-                   nullptr, 50.0f, mask_, att_, stream);
-    conv_launch(steps_[s].L, steps_[s].tiles_m, steps_[s].tiles_n, stream);  // o + residual
+                   nullptr, 50.0f, mask_, att_, atts_, stream);
+    gemm_step(s);  // o + residual
     ++s;
-    layer_norm_rows(y_, L, D, ln2w_[i], ln2b_[i], 1e-5f, h_, stream);
-    conv_launch(steps_[s].L, steps_[s].tiles_m, steps_[s].tiles_n, stream);  // w1 + GELU
+    layer_norm_rows(y_, L, D, ln2w_[i], ln2b_[i], 1e-5f, h_, hs_, stream);
+    gemm_step(s);  // w1 + GELU
     ++s;
-    conv_launch(steps_[s].L, steps_[s].tiles_m, steps_[s].tiles_n, stream);  // w2 + residual
+    gemm_step(s);  // w2 + residual
     ++s;
   }
   // exit LayerNorm, then the pooler's own LayerNorm (musiccoca.cpp:225-231, 291-293)
-  layer_norm_rows(layer_out_.back(), L, D, exit_w_, exit_b_, 1e-5f, y_, stream);
-  layer_norm_rows(y_, L, D, pln_w_, pln_b_, 1e-5f, n_, stream);
+  layer_norm_rows(layer_out_.back(), L, D, exit_w_, exit_b_, 1e-5f, y_, nullptr, stream);
+  layer_norm_rows(y_, L, D, pln_w_, pln_b_, 1e-5f, n_, ns_, stream);
   const int PD = c.num_heads * c.pooler_d_head;
-  conv_launch(steps_[s].L, steps_[s].tiles_m, steps_[s].tiles_n, stream);  // pooler q (1 row)
+  gemm_step(s);  // pooler q (1 row)
   ++s;
-  conv_launch(steps_[s].L, steps_[s].tiles_m, steps_[s].tiles_n, stream);  // pooler k | v
+  gemm_step(s);  // pooler k | v
   ++s;
   coca_attention(pq_buf_, PD, pkv_buf_, 2 * PD, pkv_buf_ + PD, 2 * PD, 1, L, c.num_heads, c.pooler_d_head, pscale_,
-                 0.0f, nullptr, patt_, stream);
-  conv_launch(steps_[s].L, steps_[s].tiles_m, steps_[s].tiles_n, stream);  // pooler o
+                 0.0f, nullptr, patt_, patts_, stream);
+  gemm_step(s);  // pooler o
 }
 
 void Coca::embed_text(const int32_t* ids, const float* padding, float* emb) {

@@ -25,15 +25,17 @@ struct CocaConfig {
 // x (rows, D) = table[ids] * scale.
 void coca_embed(const int* ids, int rows, const float* table, int vocab, int D, float scale, float* x,
                 hipStream_t s);
-// LayerNorm over the last axis (musiccoca.cpp:71-79): rows of D <= 4096.
-void layer_norm_rows(const float* x, int rows, int D, const float* w, const float* b, float eps, float* y,
+// LayerNorm over the last axis (musiccoca.cpp:71-79): rows of D <= 4096.  Rows go to
+// y, or where ys is given to ys as split rows (split_gemm.hpp).
+void layer_norm_rows(const float* x, int rows, int D, const float* w, const float* b, float eps, float* y, bf16* ys,
                      hipStream_t s);
 // Multi-head attention core (musiccoca.cpp:155-176): q (Sq, ldq), k / v (Sk,
 // ldk / ldv), head h at columns h * D; logits (q * qscale) . k / sqrt(D),
 // capped cap * tanh(x / cap) when cap > 0, plus mask (Sk) when non-null,
-// softmax over the keys; out (Sq, H * D).  Sk <= 256, D <= 256.
+// softmax over the keys; out (Sq, H * D), or outs as split rows where given.
+// Sk <= 256, D <= 256.
 void coca_attention(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, int Sq, int Sk, int H,
-                    int D, const float* qscale, float cap, const float* mask, float* out, hipStream_t s);
+                    int D, const float* qscale, float cap, const float* mask, float* out, bf16* outs, hipStream_t s);
 // rvq_quantization (rvq.cpp:24-62) of one vector (D) against codebooks (K, C,
 // D), C <= 1024: tokens (K); work (2 (D + C)) scratch, residual (D) what the
 // last level leaves.
@@ -68,18 +70,19 @@ class Coca {
 
  private:
   struct Lin {
-    float* w = nullptr;  // (in, out_pad), packed
+    void* w = nullptr;   // (in, out_pad) fp32, or out_pad split rows of in values
     float* b = nullptr;  // (out)
     int in = 0, out = 0, out_pad = 0;
   };
   struct Step {  // one GEMM launch
     ConvLaunch L;
     int tiles_m, tiles_n;
-    const float* w;  // packed weights of its single sub-problem
+    const void* w;  // packed weights of its single sub-problem
   };
   Lin pack(const TensorSource& w, const std::vector<std::string>& names, int in);
   void enqueue_text();
-  void plan_gemm(const float* x, int M, const Lin& l, float* y, const float* res, int act);
+  void plan_gemm(const float* x, const bf16* xs, int M, const Lin& l, float* y, bf16* ys, const float* res, int act);
+  void gemm_step(size_t i);
   float* dalloc(size_t floats);
 
   std::vector<void*> allocs_;
@@ -95,6 +98,12 @@ class Coca {
         *f_ = nullptr, *n_ = nullptr, *pq_buf_ = nullptr, *pkv_buf_ = nullptr, *patt_ = nullptr, *emb_ = nullptr,
         *res_ = nullptr, *rvq_work_ = nullptr;
   std::vector<float*> layer_out_;
+  // Split mode (every width a multiple of 32): the GEMMs run on split operands
+  // (conv_split.hip), which take the place of the fp32 buffers that only feed them.
+  bool split_ = false;
+  bf16 *hs_ = nullptr, *atts_ = nullptr, *fs_ = nullptr, *ns_ = nullptr, *patts_ = nullptr, *pquerys_ = nullptr,
+       *zeros_ = nullptr;
+  unsigned* counters_ = nullptr;
   int* tok_ = nullptr;
   int32_t* h_stage_ = nullptr;
   std::vector<Step> steps_;  // every GEMM of embed_text, in order

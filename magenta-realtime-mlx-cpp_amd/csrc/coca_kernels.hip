@@ -1,8 +1,9 @@
 // MusicCoCa text-path kernels (fp32): embedding, LayerNorm, the attention
 // core and RVQ quantisation.  The projections run on the codec's matrix-core
-// GEMM (codec_kernels.hip).
+// GEMM (conv_split.hip; codec_kernels.hip for widths it does not take).
 #include "coca.hpp"
 #include "device_utils.hpp"
+#include "split_gemm.hpp"
 
 namespace mrt {
 namespace {
@@ -42,7 +43,8 @@ __global__ void k_coca_embed(const int* __restrict__ ids, const float* __restric
 // musiccoca.cpp:71-79: mean, centred, variance of the centred values, then
 // centred * rsqrt(var + eps) * w + b.  One workgroup per row.
 __global__ __launch_bounds__(kT) void k_layer_norm(const float* __restrict__ x, int D, const float* __restrict__ w,
-                                                   const float* __restrict__ b, float eps, float* __restrict__ y) {
+                                                   const float* __restrict__ b, float eps, float* __restrict__ y,
+                                                   bf16* __restrict__ ys) {
   __shared__ float red[kT / 64];
   const float* xr = x + (size_t)blockIdx.x * D;
   float s = 0.f;
@@ -55,7 +57,13 @@ __global__ __launch_bounds__(kT) void k_layer_norm(const float* __restrict__ x, 
   }
   const float var = block_sum(v, red) / (float)D;
   const float inv = rsqrtf(var + eps);
-  for (int d = threadIdx.x; d < D; d += kT) y[(size_t)blockIdx.x * D + d] = (xr[d] - mean) * inv * w[d] + b[d];
+  for (int d = threadIdx.x; d < D; d += kT) {
+    const float o = (xr[d] - mean) * inv * w[d] + b[d];
+    if (ys)
+      store_split(ys, split_index(blockIdx.x, d, D), o);
+    else
+      y[(size_t)blockIdx.x * D + d] = o;
+  }
 }
 
 // One workgroup per (query, head): thread j < Sk scores key j, the softmax
@@ -65,7 +73,7 @@ __global__ __launch_bounds__(kT) void k_coca_attention(const float* __restrict__
                                                        const float* __restrict__ v, int ldv, int Sk, int D,
                                                        const float* __restrict__ qscale, float cap,
                                                        const float* __restrict__ mask, float* __restrict__ out,
-                                                       int ldo) {
+                                                       bf16* __restrict__ outs, int ldo) {
   __shared__ float qs[256];
   __shared__ float p[256];
   __shared__ float red[kT / 64];
@@ -93,7 +101,10 @@ __global__ __launch_bounds__(kT) void k_coca_attention(const float* __restrict__
   for (int d = threadIdx.x; d < D; d += kT) {
     float acc = 0.f;
     for (int t = 0; t < Sk; ++t) acc += p[t] * v[(size_t)t * ldv + h * D + d];
-    out[(size_t)i * ldo + h * D + d] = acc;
+    if (outs)
+      store_split(outs, split_index(i, h * D + d, ldo), acc);
+    else
+      out[(size_t)i * ldo + h * D + d] = acc;
   }
 }
 
@@ -109,7 +120,8 @@ __global__ __launch_bounds__(kT) void k_coca_attention_tile(const float* __restr
                                                             const float* __restrict__ k, int ldk,
                                                             const float* __restrict__ v, int ldv, int Sq, int Sk,
                                                             int D, float cap, const float* __restrict__ mask,
-                                                            float* __restrict__ out, int ldo) {
+                                                            float* __restrict__ out, bf16* __restrict__ outs,
+                                                            int ldo) {
   __shared__ float ks[kAttSk][kAttD + 1];
   __shared__ float vs[kAttSk][kAttD + 1];
   __shared__ float qs[kAttQ][kAttD];
@@ -170,7 +182,10 @@ __global__ __launch_bounds__(kT) void k_coca_attention_tile(const float* __restr
   if (l < D) {
     float acc = 0.f;
     for (int j = 0; j < Sk; ++j) acc += ps[r][j] * vs[j][l];
-    out[(size_t)(q0 + r) * ldo + h * D + l] = acc;
+    if (outs)
+      store_split(outs, split_index(q0 + r, h * D + l, ldo), acc);
+    else
+      out[(size_t)(q0 + r) * ldo + h * D + l] = acc;
   }
 }
 
@@ -266,23 +281,23 @@ void coca_embed(const int* ids, int rows, const float* table, int vocab, int D, 
   MRT_HIP_CHECK(hipGetLastError());
 }
 
-void layer_norm_rows(const float* x, int rows, int D, const float* w, const float* b, float eps, float* y,
+void layer_norm_rows(const float* x, int rows, int D, const float* w, const float* b, float eps, float* y, bf16* ys,
                      hipStream_t s) {
-  hipLaunchKernelGGL(k_layer_norm, dim3(rows), dim3(kT), 0, s, x, D, w, b, eps, y);
+  hipLaunchKernelGGL(k_layer_norm, dim3(rows), dim3(kT), 0, s, x, D, w, b, eps, y, ys);
   MRT_HIP_CHECK(hipGetLastError());
 }
 
 void coca_attention(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, int Sq, int Sk, int H,
-                    int D, const float* qscale, float cap, const float* mask, float* out, hipStream_t s) {
+                    int D, const float* qscale, float cap, const float* mask, float* out, bf16* outs, hipStream_t s) {
   MRT_REQUIRE(Sk >= 1 && Sk <= kT && D >= 1 && D <= 256, "coca attention: Sk <= 256 and d_head <= 256");
   if (!qscale && Sk <= kAttSk && D <= kAttD && D % 4 == 0 && ldk % 4 == 0 && ldv % 4 == 0 &&
       reinterpret_cast<uintptr_t>(k) % 16 == 0 && reinterpret_cast<uintptr_t>(v) % 16 == 0) {
     // query blocks with the head's K / V in LDS
     hipLaunchKernelGGL(k_coca_attention_tile, dim3((Sq + kAttQ - 1) / kAttQ, H), dim3(kT), 0, s, q, ldq, k, ldk, v,
-                       ldv, Sq, Sk, D, cap, mask, out, H * D);
+                       ldv, Sq, Sk, D, cap, mask, out, outs, H * D);
   } else {
     hipLaunchKernelGGL(k_coca_attention, dim3(Sq, H), dim3(kT), 0, s, q, ldq, k, ldk, v, ldv, Sk, D, qscale, cap,
-                       mask, out, H * D);
+                       mask, out, outs, H * D);
   }
   MRT_HIP_CHECK(hipGetLastError());
 }

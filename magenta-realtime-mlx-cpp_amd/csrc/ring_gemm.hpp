@@ -51,6 +51,7 @@ struct Core16 {
     c = Mfma<T>::mma(b[0], a[0], c);
   }
   static constexpr int kProducts = 1;
+  static constexpr bool kFine = false;
 };
 
 template <class Core, int BM, int BN, int WM, int WN, int S>
@@ -77,6 +78,7 @@ struct RingTile {
 
   struct State {
     f32x16_t acc[MI][NJ];  // (i, j), r: row 32 i + lane % 32, column 32 j + 8 (r / 4) + 4 (lane / 32) + r % 4
+    f32x16_t low[Core::kFine ? MI : 1][Core::kFine ? NJ : 1];  // sums of all products but the last
     v8 a[2][MI][Core::kParts], b[2][NJ][Core::kParts];
     int slot = 0;  // ring stage of the next k-tile
     __device__ void clear() {
@@ -85,7 +87,19 @@ struct RingTile {
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+          for (int r = 0; r < 16; ++r) {
+            acc[i][j][r] = 0.f;
+            if constexpr (Core::kFine) low[i][j][r] = 0.f;
+          }
+    }
+    // acc the whole sums
+    __device__ void settle() {
+      if constexpr (Core::kFine) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) acc[i][j] += low[i][j];
+      }
     }
   };
 
@@ -162,7 +176,12 @@ struct RingTile {
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) Core::mma(s.a[d][i], s.b[d][j], u, s.acc[i][j]);
+        for (int j = 0; j < NJ; ++j) {
+          if constexpr (Core::kFine)
+            Core::mma(s.a[d][i], s.b[d][j], u, u + 1 < Core::kProducts ? s.low[i][j] : s.acc[i][j]);
+          else
+            Core::mma(s.a[d][i], s.b[d][j], u, s.acc[i][j]);
+        }
   }
   // One product, then its share of the next step's LDS reads.
   __device__ static void interleave() {

@@ -66,6 +66,7 @@ struct CoreSplit {
   typedef __bf16 v8 __attribute__((ext_vector_type(8)));
   static constexpr int kChunks = 12, kSteps = 2, kParts = 3, kDepth = 32;
   static constexpr int kProducts = 6;
+  static constexpr bool kFine = false;
   __device__ static int place(int r, int chunk) {
     const int c = chunk + ((r >> 2) & 3);
     return c >= 12 ? c - 12 : c;
@@ -80,6 +81,13 @@ struct CoreSplit {
     constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
     c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[pb[u]], a[pa[u]], c, 0, 0, 0);
   }
+};
+
+// The same with the five small products summed apart from the largest, so that the
+// whole sum is rounded once per 16 terms instead of six times: for tiles with the
+// registers to spare.
+struct CoreSplitFine : CoreSplit {
+  static constexpr bool kFine = true;
 };
 
 // W (N, K) fp32 -> split rows (split_kernels.hip).
