@@ -66,7 +66,7 @@ Batch::Batch(Model& model, int streams, int max_frames, int enc_len)
   MRT_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&h_pinned_), h_pinned_n_ * 4, hipHostMallocDefault));
   MRT_HIP_CHECK(hipEventCreate(&ev_[0]));
   MRT_HIP_CHECK(hipEventCreate(&ev_[1]));
-  fw_ = m.frag_weights(true, stream);
+  fw_ = m.frag_weights(stream);
 }
 
 Batch::~Batch() {
@@ -111,46 +111,50 @@ void Batch::temporal_stack(int f, const int* fptr) {
   const int D = c.d_model, HD = c.hd(), FF = c.d_ff, H = c.num_heads;
   for (int i = 0; i < c.num_temporal_layers; ++i) {
     const FragLayer& W = fw_->tmp[i];
+    const DecoderLayerW& G = m.tmp[i];  // its norms
     char *tk = ring(tkv_, i, 0, F), *tv = ring(tkv_, i, 1, F);
     // layer 0's input is the frame mean (no row partials): a plain norm pass
     if (i == 0) {
-      rmsnorm_rows_frag(dt, t_in_, m.tmp[i].norm_sa, 1e-6f, R, D, xn_, stream);
+      rmsnorm_rows_frag(dt, t_in_, G.norm_sa, 1e-6f, R, D, xn_, stream);
       bgemm_qkv(dt, xn_, R, D, W.wqkv, HD, q_, tk, tv, H, F, f, fptr, stream);
     } else {
-      bgemm_qkv(dt, xf_, R, D, W.wqkv, HD, q_, tk, tv, H, F, f, fptr, stream, norm());
+      bgemm_qkv(dt, xf_, R, D, W.wqkv, HD, q_, tk, tv, H, F, f, fptr, stream, norm(G.norm_sa));
     }
     self_attn_at(dt, R, q_, tk, tv, H, F, f + 1, f, fptr, m.tbias, m.tbuckets, att_, stream, 0, nullptr, true);
     bgemm_resid(dt, att_, R, HD, W.wo, D, t_in_, xf_, ssq_, stream);
-    bgemm_store(dt, xf_, R, D, W.wq_c, HD, q_, HD, stream, norm());
+    bgemm_store(dt, xf_, R, D, W.wq_c, HD, q_, HD, stream, norm(G.norm_ca));
     cross_attn_rows(q_, ring(enc_.cross, i, 0, S), ring(enc_.cross, i, 1, S), R, H, S, att_, stream);
     bgemm_resid(dt, att_, R, HD, W.wo_c, D, t_in_, xf_, ssq_, stream);
-    bgemm_geglu(dt, xf_, R, D, W.w01, FF, ffh_, stream, norm());
+    bgemm_geglu(dt, xf_, R, D, W.w01, FF, ffh_, stream, norm(G.norm_ff));
     bgemm_resid(dt, ffh_, R, FF, W.wo2, D, t_in_, xf_, ssq_, stream);
   }
 }
 
 // Depth step l of every row in place on x (model.cpp:638-651 per row).
-// qkv_fed: layer 0's q and ring slot l were written by the previous level's
-// draw from the q/k/v table (x = emb(token), a function of the token alone);
-// else layer 0 normalises in its own pass, whatever wrote x.
-void Batch::depth_stack(void* x, int l, bool qkv_fed) {
+// x_partials: the row partials of x are those the last bgemm_resid left, its
+// fragments those at xf_ (the temporal step's output), else layer 0 normalises
+// in its own pass.  qkv_fed: layer 0's q and ring slot l were written by the
+// previous level's draw from the q/k/v table (x = emb(token), a function of the
+// token alone).
+void Batch::depth_stack(void* x, int l, bool x_partials, bool qkv_fed) {
   const Config& c = m.cfg;
   const DType dt = m.dt;
   const int D = c.d_model, HD = c.hd(), FF = c.d_ff, H = c.num_heads, L = c.rvq_depth;
   for (int i = 0; i < c.num_depth_layers; ++i) {
     const FragLayer& W = fw_->dep[i];
+    const DecoderLayerW& G = m.dep[i];
     char *dk = ring(dkv_, i, 0, L), *dv = ring(dkv_, i, 1, L);
     if (i == 0 && qkv_fed) {
       // nothing to compute: q / k / v are in place
-    } else if (i == 0) {
-      rmsnorm_rows_frag(dt, x, m.dep[i].norm_sa, 1e-6f, R, D, xn_, stream);
+    } else if (i == 0 && !x_partials) {
+      rmsnorm_rows_frag(dt, x, G.norm_sa, 1e-6f, R, D, xn_, stream);
       bgemm_qkv(dt, xn_, R, D, W.wqkv, HD, q_, dk, dv, H, L, l, nullptr, stream);
     } else {
-      bgemm_qkv(dt, xf_, R, D, W.wqkv, HD, q_, dk, dv, H, L, l, nullptr, stream, norm());
+      bgemm_qkv(dt, xf_, R, D, W.wqkv, HD, q_, dk, dv, H, L, l, nullptr, stream, norm(G.norm_sa));
     }
     self_attn_at(dt, R, q_, dk, dv, H, L, l + 1, l, nullptr, m.dbias, m.dbuckets, att_, stream, 0, nullptr, true);
     bgemm_resid(dt, att_, R, HD, W.wo, D, x, xf_, ssq_, stream);
-    bgemm_geglu(dt, xf_, R, D, W.w01, FF, ffh_, stream, norm());
+    bgemm_geglu(dt, xf_, R, D, W.w01, FF, ffh_, stream, norm(G.norm_ff));
     bgemm_resid(dt, ffh_, R, FF, W.wo2, D, x, xf_, ssq_, stream);
   }
 }
@@ -182,10 +186,10 @@ void Batch::enqueue_frame(const GenOpts& o, int f, bool dynamic) {
   if (o.record_temporal) copy_dev(static_cast<char*>(o.record_temporal) + f * row_bytes, t_in_, row_bytes, stream);
   for (int l = 0; l < L; ++l) {
     void* x = l == 0 ? t_in_ : d_in_;
-    depth_stack(x, l, l > 0 && qkv_tab_ != nullptr);
+    depth_stack(x, l, l == 0 && c.num_temporal_layers > 0, l > 0 && qkv_tab_ != nullptr);
     const int head0 = o.codec_offset + C * l;
     if (c.num_depth_layers > 0) {
-      bgemm_f32(m.dt, xf_, R, D, fw_->head, head0, C, logits_, C, stream, norm());
+      bgemm_f32(m.dt, xf_, R, D, fw_->head, head0, C, logits_, C, stream, norm(m.dec_norm));
     } else {
       rmsnorm_rows_frag(m.dt, x, m.dec_norm, 1e-6f, R, D, xn_, stream);
       bgemm_f32(m.dt, xn_, R, D, fw_->head, head0, C, logits_, C, stream);

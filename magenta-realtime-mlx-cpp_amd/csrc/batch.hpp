@@ -25,18 +25,18 @@ inline int frag_rows(int M) { return (M + 15) / 16 * 16; }
 // Elements of an (N, K) weight matrix in fragment order (N padded to 16 rows,
 // and 16 rows more).
 size_t frag_weights_elems(int N, int K);
-// The matrix in fragment order; g non-null: column k times g[k], rounded to the
-// storage type (the RMSNorm weights of the input folded in, for BNorm inputs).
-// pairs: W is a packed wi_0 / wi_1 matrix (N = 2F rows, bgemm_geglu).
-void frag_weights(DType dt, const void* W, const void* g, int N, int K, bool pairs, void* out, hipStream_t s);
+// The matrix in fragment order.  pairs: W is a packed wi_0 / wi_1 matrix (N = 2F
+// rows, bgemm_geglu).
+void frag_weights(DType dt, const void* W, int N, int K, bool pairs, void* out, hipStream_t s);
 // rmsnorm_rows (row-major in) with the result in fragment order, D <= 4096.
 void rmsnorm_rows_frag(DType dt, const void* x, const void* g, float eps, int M, int D, void* y, hipStream_t s);
 
-// RMSNorm of a GEMM's input rows: X then holds the raw residual rows, whose
-// sums of squares are the K / 16 partials per row that the bgemm_resid which
-// last wrote them left at ssq, and W the weights with the norm's weights folded
-// in (frag_weights).  ssq == nullptr: X is used as it is.
+// RMSNorm (eps, weights g) of a GEMM's input rows applied between their load and
+// the products: X then holds the raw residual rows, whose sums of squares are
+// the K / 16 partials per row that the bgemm_resid which last wrote them left at
+// ssq.  g == nullptr: X is used as it is.
 struct BNorm {
+  const void* g = nullptr;
   const float* ssq = nullptr;
   float eps = 0.f;
 };
@@ -108,9 +108,9 @@ class Batch {
  private:
   void enqueue_frame(const GenOpts& o, int f, bool dynamic);
   void temporal_stack(int f, const int* fptr);
-  void depth_stack(void* x, int l, bool qkv_fed);
-  // the norm of a GEMM input whose row partials are at ssq_
-  BNorm norm() const { return BNorm{ssq_, 1e-6f}; }
+  void depth_stack(void* x, int l, bool x_partials, bool qkv_fed);
+  // the norm (weights g) of a GEMM input whose row partials are at ssq_
+  BNorm norm(const void* g) const { return BNorm{g, ssq_, 1e-6f}; }
   void* dalloc(size_t bytes);
   char* ring(void* base, int layer, int kv, int len) const;
 

@@ -14,6 +14,7 @@
 #include "batch.hpp"
 #include "device_utils.hpp"
 #include "kernels.hpp"
+#include "mfma_ring.hpp"
 
 namespace mrt {
 namespace {
@@ -135,9 +136,11 @@ struct BGeglu {
 
 __device__ __forceinline__ int bg_geglu_row(int j, int p) { return (j >> 5) * 64 + (j & 31) + 32 * p; }
 
-// The row sums of squares of an input that is normalised (BNorm): `parts`
-// partials per row at ssq + m * parts, summed in order.
+// An input that is normalised (BNorm): the norm weights, and the row sums of
+// squares as `parts` partials per row at ssq + m * parts, summed in order.
+template <typename T>
 struct BNormDev {
+  const T* g;
   const float* ssq;
   int parts;
   float eps;
@@ -150,6 +153,28 @@ __device__ __forceinline__ float row16_sum(float v) {
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x114, 0xf, 0xf, true));  // row_shr:4
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x118, 0xf, 0xf, true));  // row_shr:8
   return v;
+}
+
+// Sum over each 8 lanes, in every lane: pairs, quads, then the other quad.
+__device__ __forceinline__ float group8_sum(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));   // quad [1,0,3,2]
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));   // quad [2,3,0,1]
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true));  // row_half_mirror
+  return v;
+}
+
+// Eight activations x normalised as rmsnorm_rows rounds them: x times the row's
+// inverse RMS, rounded, times the norm weights, rounded.
+template <typename T>
+__device__ __forceinline__ uint4 norm8(uint4 x, uint4 g, float inv) {
+  using S = St<T>;
+  const T* xe = reinterpret_cast<const T*>(&x);
+  const T* ge = reinterpret_cast<const T*>(&g);
+  uint4 out;
+  T* oe = reinterpret_cast<T*>(&out);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) oe[e] = S::st(S::rnd(S::ld(xe[e]) * inv) * S::ld(ge[e]));
+  return out;
 }
 
 template <class Epi, class = void>
@@ -175,14 +200,15 @@ struct IsResid<BResid<T>> : std::true_type {};
 // 8 partial tiles are summed in wave order.  Rows past M repeat the last row and
 // columns past nout meet other rows' weights; neither is stored.
 //
-// NORM: X holds raw residual rows and W the weights already multiplied by the
-// norm weights, so RMSNorm (modules.cpp:72-84) is the scaling of row m's sums
-// by inv(m) = 1 / sqrt(mean(x^2) + eps): it costs one multiplication an output
-// instead of two roundings of every activation in every block, and its chain
-// (partials, square root) runs beside the products.  Scaling the activations on
-// load took 3 us of the 9.7 us of the 3,072-wide output at 64 rows.
+// NORM: X holds raw residual rows, and a wave normalises its operands between
+// their load and the products, rounded as the separate norm rounds them
+// (modules.cpp:72-84): a norm folded into the weights would round those once more,
+// and below the smallest normal fp16 value lose their bits.  The row's inverse RMS
+// (partials, square root, a barrier) and the normalised operands are computed while
+// the weights are in flight: those are requested last, as loads return in order
+// (32 streams x 50 frames 183.5 ms; weights first 190.2).
 //
-// Block (tile, ms) of the grid computes output columns [16 tile, +16) for the
+// Block (tile, ms) of the grid computes output columns [16 C tile, +16 C) for the
 // MT row tiles [MT ms, +MT) of 16 rows: blocks sharing a column tile are
 // tile + ntiles * ms, on the same XCD as ntiles is then padded to a multiple of
 // 8 (blocks are dealt to the 8 XCDs in turn), so the weight tile comes from HBM
@@ -195,29 +221,34 @@ struct IsResid<BResid<T>> : std::true_type {};
 // operand load into few L2 channels, and more of them in flight ran slower
 // (64 rows, alone, us: 3,072 outputs 6.6 row-major, 4.1 here; 2,816 gated pairs
 // 9.2, 5.8; 1,024 outputs 3.9, 2.9 at K = 1,024 and 6.8, 4.2 at K = 2,816; an
-// empty launch takes 1.9).
-template <typename T, int P, int MT, int NST, bool NORM, class Epi>
+// empty launch takes 1.9; inputs that are not normalised).
+template <typename T, int P, int C, int MT, int NST, bool NORM, class Epi>
 __global__ __launch_bounds__(kBgThreads) void k_bgemm(const T* __restrict__ X, int M, int K, const T* __restrict__ W,
                                                       int nout, int ntiles, Epi epi, int w_row0, int w_group_rows,
-                                                      BNormDev nrm) {
+                                                      BNormDev<T> nrm) {
+  static_assert(P == 1 || C == 1, "gate / up pairs: one column tile a block");
+  static_assert(C == 1 || !HasPre<Epi>::value, "the residual epilogue: one column tile a block");
   // blockIdx.y = group g (grouped launch): rows [g M, g M + M) of X against
   // weight rows w_row0 + g * w_group_rows, outputs at rows g M + m
   const int grow = blockIdx.y * M;
   const int row0 = w_row0 + blockIdx.y * w_group_rows, skip = P == 1 ? row0 & 15 : 0;
+  constexpr int kW = P * C;                                    // weight tiles of the block
   constexpr int kRows = 16 * MT;
-  constexpr int kOut = kRows * kBgCols;                        // outputs of the block
-  constexpr int kPer = (kOut + kBgThreads - 1) / kBgThreads;  // epilogue outputs per thread
-  __shared__ float part[kBgWaves][kRows][kBgCols + 1];  // one part (gate / up) at a time
+  constexpr int kOut = kRows * kBgCols;                        // outputs of a column tile
+  constexpr int kPer = (kOut + kBgThreads - 1) / kBgThreads;  // of them per thread
+  __shared__ float part[kBgWaves][kRows][kBgCols + 1];  // one weight tile at a time
   [[maybe_unused]] __shared__ float inv_s[kRows];
   // the wave index as a scalar: matrix instructions ignore the lane mask, so the
   // conditions around them must be branches
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int tile = blockIdx.x % ntiles, m0 = (blockIdx.x / ntiles) * kRows;
+  const int tile = (blockIdx.x % ntiles) * C, m0 = (blockIdx.x / ntiles) * kRows;
   const int j0 = tile * kBgCols - skip;  // output of the block's first column
   if (j0 >= nout) return;                // a padding tile (launch_bgemm_t)
   const int c16 = lane & 15, kg = lane >> 4;
   const int nks = K / 32;
 
+  // weight tile w of k-step ks: the P parts of an output tile alternate, column
+  // tiles lie a whole K apart
   const T* wt = W + ((size_t)(P == 1 ? (row0 >> 4) + tile : tile) * nks * P) * 512 + lane * 8;
   const T* xrow[MT];
 #pragma unroll
@@ -225,17 +256,41 @@ __global__ __launch_bounds__(kBgThreads) void k_bgemm(const T* __restrict__ X, i
     const int r = grow + min(m0 + 16 * t + c16, M - 1);
     xrow[t] = X + (size_t)(r >> 4) * nks * 512 + (kg * 16 + (r & 15)) * 8;
   }
-  uint4 b[NST][P], a[NST][MT];
+  uint4 b[NST][kW], a[NST][MT];
+  [[maybe_unused]] uint4 gk[NORM ? NST : 1];
+  auto weights = [&](int c, int ks) {
+#pragma unroll
+    for (int w = 0; w < kW; ++w) b[c][w] = ld_g16(wt + (size_t)(C == 1 ? ks * P + w : w * nks + ks) * 512);
+  };
   auto load = [&](int s0) {
 #pragma unroll
     for (int c = 0; c < NST; ++c) {
       const int ks = min(s0 + kBgWaves * c, nks - 1);
 #pragma unroll
-      for (int p = 0; p < P; ++p) b[c][p] = ld_g16(wt + (size_t)(ks * P + p) * 512);
-#pragma unroll
       for (int t = 0; t < MT; ++t) a[c][t] = ld_g16(xrow[t] + (size_t)ks * 512);
+      if constexpr (NORM) gk[c] = ld_g16(nrm.g + ks * 32 + kg * 8);
+      if constexpr (!NORM) weights(c, ks);
+    }
+    if constexpr (NORM) {  // the weights last: the rest is at work before they are there
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int c = 0; c < NST; ++c) weights(c, min(s0 + kBgWaves * c, nks - 1));
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
+  // eight lanes per row r: with 64 partials lane q sums [8 q, 8 q + 8) in order
+  // (other counts: lane 0 sums them all)
+  [[maybe_unused]] const int r = tid >> 3, q = tid & 7;
+  [[maybe_unused]] float4 su, sw;
+  [[maybe_unused]] const float* sp = nullptr;
+  if constexpr (NORM) {
+    sp = nrm.ssq + (size_t)(grow + min(m0 + min(r, kRows - 1), M - 1)) * nrm.parts;
+    if (nrm.parts == 64) {
+      su = *reinterpret_cast<const float4*>(sp + 8 * q);
+      sw = *reinterpret_cast<const float4*>(sp + 8 * q + 4);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
   load(wid);
   float pre[kPer];
   if constexpr (HasPre<Epi>::value) {
@@ -245,77 +300,81 @@ __global__ __launch_bounds__(kBgThreads) void k_bgemm(const T* __restrict__ X, i
       pre[i] = epi.pre(grow + min(m, M - 1), min(n, nout - 1));
     }
   }
+  [[maybe_unused]] float inv[MT];
   if constexpr (NORM) {
-    // eight lanes per row: with 64 partials lane q sums [8 q, 8 q + 8) in
-    // order (other counts: lane 0 sums them all), and the eight sums meet by
-    // lane exchange (the same total in each lane)
-    const int r = tid >> 3, q = tid & 7;
-    const float* sp = nrm.ssq + (size_t)(grow + min(m0 + min(r, kRows - 1), M - 1)) * nrm.parts;
     float ss = 0.f;
     if (nrm.parts == 64) {
-      const float4 u = *reinterpret_cast<const float4*>(sp + 8 * q);
-      const float4 w = *reinterpret_cast<const float4*>(sp + 8 * q + 4);
-      ss = ((((((u.x + u.y) + u.z) + u.w) + w.x) + w.y) + w.z) + w.w;
+      ss = ((((((su.x + su.y) + su.z) + su.w) + sw.x) + sw.y) + sw.z) + sw.w;
     } else if (q == 0) {
       for (int t = 0; t < nrm.parts; ++t) ss += sp[t];
     }
-    ss += __shfl_xor(ss, 1);
-    ss += __shfl_xor(ss, 2);
-    ss += __shfl_xor(ss, 4);
-    if (r < kRows && q == 0) inv_s[r] = 1.0f / sqrtf(ss / (float)K + nrm.eps);  // read after the barrier below
+    ss = group8_sum(ss);
+    if (r < kRows && q == 0) inv_s[r] = 1.0f / sqrtf(ss / (float)K + nrm.eps);
+    ring_barrier();  // not __syncthreads(): the operands stay in flight
+#pragma unroll
+    for (int t = 0; t < MT; ++t) inv[t] = inv_s[16 * t + c16];
   }
-  f32x4_t acc[P][MT];
+  f32x4_t acc[kW][MT];
 #pragma unroll
-  for (int p = 0; p < P; ++p)
+  for (int w = 0; w < kW; ++w)
 #pragma unroll
-    for (int t = 0; t < MT; ++t) acc[p][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < MT; ++t) acc[w][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   for (int s0 = wid; s0 < nks; s0 += kBgWaves * NST) {
+    if constexpr (NORM) {
+#pragma unroll
+      for (int c = 0; c < NST; ++c)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) a[c][t] = norm8<T>(a[c][t], gk[c], inv[t]);
+    }
 #pragma unroll
     for (int c = 0; c < NST; ++c) {
       if (s0 + kBgWaves * c < nks) {
 #pragma unroll
-        for (int p = 0; p < P; ++p)
+        for (int w = 0; w < kW; ++w)
 #pragma unroll
-          for (int t = 0; t < MT; ++t) acc[p][t] = Mfma16<T>::mma(a[c][t], b[c][p], acc[p][t]);
+          for (int t = 0; t < MT; ++t) acc[w][t] = Mfma16<T>::mma(a[c][t], b[c][w], acc[w][t]);
       }
     }
     if (s0 + kBgWaves * NST < nks) load(s0 + kBgWaves * NST);
   }
-  float v[kPer][P];
 #pragma unroll
-  for (int p = 0; p < P; ++p) {
-    if (p > 0) __syncthreads();  // the previous part has been read
+  for (int ct = 0; ct < C; ++ct) {
+    float v[kPer][P];
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
+    for (int p = 0; p < P; ++p) {
+      if (ct + p > 0) __syncthreads();  // the previous weight tile's sums have been read
 #pragma unroll
-      for (int i = 0; i < 4; ++i) part[wid][16 * t + 4 * kg + i][c16] = acc[p][t][i];
-    __syncthreads();
+      for (int t = 0; t < MT; ++t)
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int idx = min(tid + kBgThreads * i, kOut - 1), m = idx / kBgCols, n = idx % kBgCols;
-      float a = part[0][m][n];
+        for (int i = 0; i < 4; ++i) part[wid][16 * t + 4 * kg + i][c16] = acc[ct + p][t][i];
+      __syncthreads();
 #pragma unroll
-      for (int w = 1; w < kBgWaves; ++w) a += part[w][m][n];
-      v[i][p] = NORM ? a * inv_s[m] : a;
+      for (int i = 0; i < kPer; ++i) {
+        const int idx = min(tid + kBgThreads * i, kOut - 1), m = idx / kBgCols, n = idx % kBgCols;
+        float sum = part[0][m][n];
+#pragma unroll
+        for (int w = 1; w < kBgWaves; ++w) sum += part[w][m][n];
+        v[i][p] = sum;
+      }
     }
-  }
-  if constexpr (IsResid<Epi>::value) {
-    // lanes 16 r .. 16 r + 15 of a wave hold the 16 columns of one output row
+    if constexpr (IsResid<Epi>::value) {
+      // lanes 16 r .. 16 r + 15 of a wave hold the 16 columns of one output row
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int idx = tid + kBgThreads * i, m = m0 + idx / kBgCols, n = idx % kBgCols;
-      const bool ok = idx < kOut && m < M && j0 + n < nout;
-      const float y = ok ? epi(grow + m, j0 + n, v[i], pre[i]) : 0.f;
-      const float ss = row16_sum(y * y);
-      if (ok && n == kBgCols - 1) epi.ssq[(size_t)(grow + m) * (epi.ldr / kBgCols) + tile] = ss;
-    }
-  } else {
+      for (int i = 0; i < kPer; ++i) {
+        const int idx = tid + kBgThreads * i, m = m0 + idx / kBgCols, n = idx % kBgCols;
+        const bool ok = idx < kOut && m < M && j0 + n < nout;
+        const float y = ok ? epi(grow + m, j0 + n, v[i], pre[i]) : 0.f;
+        const float ss = row16_sum(y * y);
+        if (ok && n == kBgCols - 1) epi.ssq[(size_t)(grow + m) * (epi.ldr / kBgCols) + tile] = ss;
+      }
+    } else {
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int idx = tid + kBgThreads * i, m = m0 + idx / kBgCols, n = j0 + idx % kBgCols;
-      if (idx >= kOut || m >= M || n < 0 || n >= nout) continue;
-      epi(grow + m, n, v[i]);
+      for (int i = 0; i < kPer; ++i) {
+        const int idx = tid + kBgThreads * i, m = m0 + idx / kBgCols, n = j0 + ct * kBgCols + idx % kBgCols;
+        if (idx >= kOut || m >= M || n < 0 || n >= nout) continue;
+        epi(grow + m, n, v[i]);
+      }
     }
   }
 }
@@ -324,32 +383,37 @@ __global__ __launch_bounds__(kBgThreads) void k_bgemm(const T* __restrict__ X, i
 // outputs) split the rows until there are 256 blocks, one per CU; wider
 // outputs keep all rows in a block (each block then reads the activations once
 // for twice the columns' work), the gated pairs at most two row tiles (64 rows:
-// 5.8 against 6.5 us with four).  A block holds 1, 2 or 4 row tiles, no more
+// 5.8 against 6.5 us with four).  Where the input is normalised, a block of the
+// wide outputs takes two column tiles and two row tiles instead of one and four:
+// as many products, half the rows to normalise.  A block holds 1, 2 or 4 row tiles, no more
 // than the rows need: the loads of unused ones cost as much (the 3,072-wide
 // output of 10 rows: 8.5 us with four).
 template <typename T, int P, bool NORM, class Epi>
 void launch_bgemm_t(const T* X, int M, int K, const T* W, int nout, const Epi& epi, hipStream_t s, int groups,
-                    int w_row0, int w_group_rows, const BNormDev& nrm) {
+                    int w_row0, int w_group_rows, const BNormDev<T>& nrm) {
   // a column tile more where the weight rows do not start on a tile
   const bool shifted = P == 1 && (w_row0 % kBgCols != 0 || (groups > 1 && w_group_rows % kBgCols != 0));
   const int ntiles = (nout + kBgCols - 1) / kBgCols + (shifted ? 1 : 0), mtiles = (M + 15) / 16;
   int ms = 1;
   while (ntiles < 128 && ms < 4 && ms < mtiles && ntiles * ms < 256) ms *= 2;
   const int mt = (mtiles + ms - 1) / ms;
-  auto go = [&](auto k, int mt_block) {
-    const int mb = (mtiles + mt_block - 1) / mt_block, nt = mb > 1 ? (ntiles + 7) / 8 * 8 : ntiles;
+  auto go = [&](auto k, int mt_block, int c_block = 1) {
+    const int mb = (mtiles + mt_block - 1) / mt_block, nb = (ntiles + c_block - 1) / c_block;
+    const int nt = mb > 1 ? (nb + 7) / 8 * 8 : nb;
     hipLaunchKernelGGL(k, dim3(nt * mb, groups), dim3(kBgThreads), 0, s, X, M, K, W, nout, nt, epi, w_row0,
                        w_group_rows, nrm);
   };
   // 12 steps in flight cover K <= 3072 with one row tile
   if (mt == 1 && P == 1 && K > 32 * 4 * kBgWaves)
-    go(k_bgemm<T, P, 1, P == 1 ? 12 : 4, NORM, Epi>, 1);
+    go(k_bgemm<T, P, 1, 1, P == 1 ? 12 : 4, NORM, Epi>, 1);
   else if (mt == 1)
-    go(k_bgemm<T, P, 1, 4, NORM, Epi>, 1);
+    go(k_bgemm<T, P, 1, 1, 4, NORM, Epi>, 1);
   else if (mt == 2 || P == 2)
-    go(k_bgemm<T, P, 2, 4, NORM, Epi>, 2);
+    go(k_bgemm<T, P, 1, 2, 4, NORM, Epi>, 2);
+  else if (NORM && !shifted && nout % (2 * kBgCols) == 0)
+    go(k_bgemm<T, P, NORM && P == 1 && !HasPre<Epi>::value ? 2 : 1, 2, 4, NORM, Epi>, 2, 2);
   else
-    go(k_bgemm<T, P, P == 2 ? 2 : 4, 4, NORM, Epi>, 4);
+    go(k_bgemm<T, P, 1, P == 2 ? 2 : 4, 4, NORM, Epi>, 4);
   MRT_HIP_CHECK(hipGetLastError());
 }
 
@@ -361,35 +425,29 @@ void launch_bgemm(const void* X, int M, int K, const void* W, int nout, const Ep
   MRT_REQUIRE(nout >= 1 && groups >= 1 && w_row0 >= 0, "batched GEMM: no outputs");
   const T* x = static_cast<const T*>(X);
   const T* w = static_cast<const T*>(W);
-  if (norm.ssq != nullptr)
-    launch_bgemm_t<T, P, true>(x, M, K, w, nout, epi, s, groups, w_row0, w_group_rows,
-                               BNormDev{norm.ssq, K / kBgCols, norm.eps});
-  else
-    launch_bgemm_t<T, P, false>(x, M, K, w, nout, epi, s, groups, w_row0, w_group_rows, BNormDev{nullptr, 0, 0.f});
+  if constexpr (!HasPre<Epi>::value) {  // the residual update's input is never normalised
+    if (norm.g != nullptr) {
+      MRT_REQUIRE(norm.ssq != nullptr, "batched GEMM: a normalised input needs its row partials");
+      launch_bgemm_t<T, P, true>(x, M, K, w, nout, epi, s, groups, w_row0, w_group_rows,
+                                 BNormDev<T>{static_cast<const T*>(norm.g), norm.ssq, K / kBgCols, norm.eps});
+      return;
+    }
+  }
+  launch_bgemm_t<T, P, false>(x, M, K, w, nout, epi, s, groups, w_row0, w_group_rows,
+                              BNormDev<T>{nullptr, nullptr, 0, 0.f});
 }
 
-// Weights (N, K) -> fragment order, each element times g[k] where g is not
-// null (rounded to the storage type).  Block (tile, ks): 16 rows x 32 columns a
+// Weights (N, K) -> fragment order.  Block (tile, ks): 16 rows x 32 columns a
 // part; P = 2: the gate and up rows of 16 outputs of a packed matrix.  Rows past
 // N are zero.
 template <typename T, int P>
-__global__ __launch_bounds__(64) void k_frag_weights(const T* __restrict__ W, const T* __restrict__ g, int N, int K,
-                                                     T* __restrict__ out) {
-  using S = St<T>;
+__global__ __launch_bounds__(64) void k_frag_weights(const T* __restrict__ W, int N, int K, T* __restrict__ out) {
   const int tile = blockIdx.x, ks = blockIdx.y, lane = threadIdx.x, nks = K / 32;
   const int k0 = ks * 32 + (lane >> 4) * 8;
 #pragma unroll
   for (int p = 0; p < P; ++p) {
     const int j = tile * 16 + (lane & 15), row = P == 1 ? j : bg_geglu_row(j, p);
-    uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (row < N) {
-      v = ld_g16(W + (size_t)row * K + k0);
-      if (g != nullptr) {
-        T* e = reinterpret_cast<T*>(&v);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) e[i] = S::st(S::ld(e[i]) * S::ld(g[k0 + i]));
-      }
-    }
+    const uint4 v = row < N ? ld_g16(W + (size_t)row * K + k0) : make_uint4(0u, 0u, 0u, 0u);
     *reinterpret_cast<uint4*>(out + (((size_t)tile * nks + ks) * P + p) * 512 + lane * 8) = v;
   }
 }
@@ -586,14 +644,14 @@ void cross_attn_rows(const void* Q, const void* Kc, const void* Vc, int rows, in
 // on a tile may touch it (its outputs are not stored).
 size_t frag_weights_elems(int N, int K) { return (static_cast<size_t>((N + 15) / 16) + 1) * 16 * K; }
 
-void frag_weights(DType dt, const void* W, const void* g, int N, int K, bool pairs, void* out, hipStream_t s) {
+void frag_weights(DType dt, const void* W, int N, int K, bool pairs, void* out, hipStream_t s) {
   MRT_REQUIRE(K % 32 == 0 && N >= 1, "fragment weights: K must be a multiple of 32");
   MRT_REQUIRE(!pairs || N % 64 == 0, "fragment weights: gate / up pairs come in groups of 64 rows");
   const int tiles = (pairs ? N / 2 : N + 15) / 16;
   MRT_DTYPE16(dt, {
     const auto k = pairs ? k_frag_weights<T, 2> : k_frag_weights<T, 1>;
-    hipLaunchKernelGGL(k, dim3(tiles, K / 32), dim3(64), 0, s, static_cast<const T*>(W), static_cast<const T*>(g), N,
-                       K, static_cast<T*>(out));
+    hipLaunchKernelGGL(k, dim3(tiles, K / 32), dim3(64), 0, s, static_cast<const T*>(W), N, K,
+                       static_cast<T*>(out));
   });
   MRT_HIP_CHECK(hipGetLastError());
 }

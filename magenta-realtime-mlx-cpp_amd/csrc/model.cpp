@@ -1052,20 +1052,22 @@ void State::depth_forward_full(const void* emb, int k, const void* bias, bool ca
   copy(sx_, emb, static_cast<size_t>(M) * D * esz());
   // 16-bit rows that the skinny GEMMs hold: M <= 32 fills no tile of the
   // encoder's GEMM (its 1,024-wide outputs ran 8 blocks, 16 us each; 292 us a
-  // call in all at k = 16, 125 us here)
+  // call in all at k = 16, 135 us here)
   if (m.frag_shapes() && M <= kBatchRows && c.num_depth_layers > 0) {
-    const FragWeights& fw = *m.frag_weights(true, stream);
-    const BNorm bn{sssq_, 1e-6f};
+    const FragWeights& fw = *m.frag_weights(stream);
+    auto norm = [&](const void* g) { return BNorm{g, sssq_, 1e-6f}; };
     for (int i = 0; i < c.num_depth_layers; ++i) {
       const FragLayer& W = fw.dep[i];
       if (i == 0) rmsnorm_rows_frag(dt, sx_, m.dep[i].norm_sa, 1e-6f, M, D, sxn_, stream);
-      bgemm_store(dt, i == 0 ? sxn_ : sxf_, M, D, W.wqkv, 3 * HD, sqkv_, 3 * HD, stream, i == 0 ? BNorm{} : bn);
+      bgemm_store(dt, i == 0 ? sxn_ : sxf_, M, D, W.wqkv, 3 * HD, sqkv_, 3 * HD, stream, i == 0 ? BNorm{} : norm(m.dep[i].norm_sa));
       full_attn(dt, rows, k, H, sqkv_, bias, m.dbias, m.dbuckets, causal, satt_, stream, true);
       bgemm_resid(dt, satt_, M, HD, W.wo, D, sx_, sxf_, sssq_, stream);
-      bgemm_geglu(dt, sxf_, M, D, W.w01, FF, sffh_, stream, bn);
+      bgemm_geglu(dt, sxf_, M, D, W.w01, FF, sffh_, stream, norm(m.dep[i].norm_ff));
       bgemm_resid(dt, sffh_, M, FF, W.wo2, D, sx_, sxf_, sssq_, stream);
     }
-    bgemm_f32(dt, sxf_, M, D, fw.head, 0, c.vocab_size, logits, c.vocab_size, stream, bn);
+    // the head's many blocks would each normalise all rows: one pass instead
+    rmsnorm_rows_frag(dt, sx_, m.dec_norm, 1e-6f, M, D, sxn_, stream);
+    bgemm_f32(dt, sxn_, M, D, fw.head, 0, c.vocab_size, logits, c.vocab_size, stream);
     MRT_HIP_CHECK(hipStreamSynchronize(stream));
     return;
   }
@@ -1205,40 +1207,39 @@ const SplitWeights* Model::split_weights(hipStream_t s) {
   return &split_;
 }
 
-const FragWeights* Model::frag_weights(bool folded, hipStream_t s) {
+const FragWeights* Model::frag_weights(hipStream_t s) {
   MRT_REQUIRE(frag_shapes(), "fragment weights: 16-bit model with widths that are multiples of 32");
   std::lock_guard<std::mutex> lock(frag_mu_);
-  if (frag_built_[folded]) return &frag_[folded];
+  if (frag_built_) return &frag_;
   MRT_HIP_CHECK(hipSetDevice(device));
   const int D = cfg.d_model, HD = cfg.hd(), F = cfg.d_ff;
   std::vector<void*> bufs;
   FragWeights fw;
   try {
-    auto place = [&](const void* W, const void* g, int N, int K, bool pairs = false) -> const void* {
+    auto place = [&](const void* W, int N, int K, bool pairs = false) -> const void* {
       void* out = nullptr;
       MRT_HIP_CHECK(hipMalloc(&out, frag_weights_elems(N, K) * esz));
       bufs.push_back(out);
-      mrt::frag_weights(dt, W, folded ? g : nullptr, N, K, pairs, out, s);
+      mrt::frag_weights(dt, W, N, K, pairs, out, s);
       return out;
     };
     auto stack = [&](const std::vector<DecoderLayerW>& ws, bool temporal, std::vector<FragLayer>& out) {
-      for (size_t i = 0; i < ws.size(); ++i) {
-        const DecoderLayerW& w = ws[i];
+      for (const DecoderLayerW& w : ws) {
         FragLayer f;
-        f.wqkv = place(w.wqkv, i > 0 ? w.norm_sa : nullptr, 3 * HD, D);
-        f.wo = place(w.wo, nullptr, D, HD);
+        f.wqkv = place(w.wqkv, 3 * HD, D);
+        f.wo = place(w.wo, D, HD);
         if (temporal) {
-          f.wq_c = place(w.wq_c, w.norm_ca, HD, D);
-          f.wo_c = place(w.wo_c, nullptr, D, HD);
+          f.wq_c = place(w.wq_c, HD, D);
+          f.wo_c = place(w.wo_c, D, HD);
         }
-        f.w01 = place(w.w01, w.norm_ff, 2 * F, D, true);
-        f.wo2 = place(w.wo2, nullptr, D, F);
+        f.w01 = place(w.w01, 2 * F, D, true);
+        f.wo2 = place(w.wo2, D, F);
         out.push_back(f);
       }
     };
-    if (folded) stack(tmp, true, fw.tmp);
+    stack(tmp, true, fw.tmp);
     stack(dep, false, fw.dep);
-    fw.head = place(lm_head, dep.empty() ? nullptr : dec_norm, cfg.vocab_size, D);
+    fw.head = place(lm_head, cfg.vocab_size, D);
     MRT_HIP_CHECK(hipStreamSynchronize(s));
   } catch (...) {
     (void)hipStreamSynchronize(s);
@@ -1246,9 +1247,9 @@ const FragWeights* Model::frag_weights(bool folded, hipStream_t s) {
     throw;
   }
   allocs_.insert(allocs_.end(), bufs.begin(), bufs.end());
-  frag_[folded] = std::move(fw);
-  frag_built_[folded] = true;
-  return &frag_[folded];
+  frag_ = std::move(fw);
+  frag_built_ = true;
+  return &frag_;
 }
 
 const void* Model::depth_qkv_table(int codebook, int offset, hipStream_t s) {
@@ -1455,7 +1456,7 @@ void State::generate(const int32_t* enc_tokens_host, const GenOpts& o, int32_t* 
   dec_launches_ = persistent() ? decode_launches(o) : 0;
   // built once per (codebook, offset) before any capture; waits for the stream then
   qkv_table_ = frame_kernel_ && qkv_table_on_ ? m.depth_qkv_table(o.codebook, o.codec_offset, stream) : nullptr;
-  if (spec_drafts_) fw_ = m.frag_weights(false, stream);  // likewise
+  if (spec_drafts_) fw_ = m.frag_weights(stream);  // likewise
   hipGraphExec_t exec = o.use_graph ? decode_graph(o) : nullptr;
   {
     // persistent grids of other states on this device run before or after

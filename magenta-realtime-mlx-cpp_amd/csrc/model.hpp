@@ -64,14 +64,13 @@ struct DecoderLayerW {
 };
 
 // The decoder matrices of a layer in the skinny GEMMs' fragment order
-// (batch.hpp).  Folded: the norm weights of the input multiplied in where the
-// input comes from a residual GEMM: every wq_c and w01, and wqkv past layer 0.
+// (batch.hpp).
 struct FragLayer {
   const void *wqkv = nullptr, *wo = nullptr, *wq_c = nullptr, *wo_c = nullptr, *w01 = nullptr, *wo2 = nullptr;
 };
 struct FragWeights {
   std::vector<FragLayer> tmp, dep;
-  const void* head = nullptr;  // lm_head (vocab rows); folded: times decoder_norm if there are depth layers
+  const void* head = nullptr;  // lm_head (vocab rows)
 };
 
 // An fp32 model's encoder matrices and cross K/V projection as split rows
@@ -155,11 +154,8 @@ class Model {
   // The decoder stacks and lm_head in fragment order (16-bit models with
   // d_model, heads * 64 and d_ff multiples of 32): as many bytes again as the
   // matrices themselves, built on first use on `s` (waits for it; never during
-  // a capture) and kept with the model.  folded: both stacks, for inputs that
-  // are normalised by scaling the sums (BNorm); else the depth stack and lm_head
-  // alone, for normalised inputs rounded as the persistent kernels round them
-  // (the speculative verification pass, whose draws are held against theirs).
-  const FragWeights* frag_weights(bool folded, hipStream_t s);
+  // a capture) and kept with the model.
+  const FragWeights* frag_weights(hipStream_t s);
   // The split encoder of an fp32 model (1.5 times its matrices' bytes), kept in
   // the same way; nullptr for 16-bit models and widths the split GEMM does not
   // take.
@@ -183,8 +179,8 @@ class Model {
   SplitWeights split_;
   bool split_built_ = false;
   std::mutex frag_mu_;
-  FragWeights frag_[2];  // plain, folded
-  bool frag_built_[2] = {false, false};
+  FragWeights frag_;
+  bool frag_built_ = false;
   void* qkv_ws_ = nullptr;  // build workspace of the tables (kQkvChunkRows x d_model)
   std::vector<float> pe_host_;  // fp32 sinusoid table (max_encoder_length, d_model)
   static constexpr int kEmbedChunk = 4096;

@@ -403,3 +403,28 @@ def test_batch_row_tiles(tiny, B):
     whole = slices(range(B))
     for s in sorted({0, B // 2, B - 1}):
         np.testing.assert_array_equal(whole[:, :, 2 * s:2 * s + 2], slices([s]))
+
+
+@pytest.mark.parametrize("B", [17, 24, 32])
+def test_batch_row_tiles_full_size(full, B):
+    """More than 32 rows at the benchmark dims, where the wide normalised outputs
+    take two column tiles a block: a stream's logits are bit for bit those it has
+    alone."""
+    import torch
+    mrt_df = full["mrt_df"]
+    F, L, C = 1, 16, 1024
+    teacher = _teacher(np.random.default_rng(B), B, F, C)
+    opts = mrt_df.GenOptions(num_frames=F, rvq_depth=L, temperature=1.1, top_k=40, guidance_weight=5.0, seed=0,
+                             codebook_size=C, codec_offset=2)
+
+    def slices(streams):
+        b = mrt_df.Batch(full["model"], len(streams), max_frames=F)
+        sl = torch.zeros((F, L, 2 * len(streams), C), dtype=torch.float32, device="cuda")
+        b.generate_tokens(np.concatenate([full["toks"][s % 4] for s in streams], axis=0), opts, seeds=list(streams),
+                          teacher=teacher[list(streams)], record=dict(slices=sl))
+        b.close()
+        return sl.cpu().numpy()
+
+    whole = slices(range(B))
+    for s in (0, B // 2, B - 1):
+        np.testing.assert_array_equal(whole[:, :, 2 * s:2 * s + 2], slices([s]))
