@@ -471,6 +471,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_ring(const void* __restri
           Tile::template wait_loads<>();
       });
     }
+    s.settle();
     mfma_epilogue<T, Tile::MI, Tile::NJ>(out, s.acc, M, m0 + (wid / WN) * (BM / WM), n0 + (wid % WN) * (BN / WN));
     asm volatile("" ::: "memory");  // the stores stay ahead of the next tile's waits
     stored = m0 + BM <= M;
@@ -871,7 +872,7 @@ void gemm_split(const bf16* A, const bf16* B, int M, int N, int K, const GemmEpi
   MRT_REQUIRE(M >= 1 && gemm_split_fits(N, K), "split gemm: N must be a multiple of 128, K of 32");
   if (e.kind == GemmEpi::CrossKV)
     MRT_REQUIRE(e.HD == e.H * 64 && N % e.HD == 0 && M == e.nb * e.S, "gemm: bad cross-KV shape");
-  gemm_tiles<CoreSplit, float>(A, B, M, N, K, e, s);
+  gemm_tiles<CoreSplitFine, float>(A, B, M, N, K, e, s);
   MRT_HIP_CHECK(hipGetLastError());
 }
 
