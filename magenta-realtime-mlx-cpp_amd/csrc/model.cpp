@@ -145,7 +145,7 @@ const void* Model::upload(const std::vector<float>& host) {
   const size_t bytes = host.size() * esz;
   void* d = nullptr;
   MRT_HIP_CHECK(hipMalloc(&d, std::max<size_t>(bytes, 256)));
-  allocs_.push_back(d);
+  allocs_.add(d);
   std::vector<uint8_t> tmp(bytes);
   convert(dt, host.data(), host.size(), tmp.data());
   MRT_HIP_CHECK(hipMemcpy(d, tmp.data(), bytes, hipMemcpyHostToDevice));
@@ -156,7 +156,7 @@ const void* Model::upload(const std::vector<float>& host) {
 const void* Model::upload_i32(const std::vector<int>& host) {
   void* d = nullptr;
   MRT_HIP_CHECK(hipMalloc(&d, host.size() * 4));
-  allocs_.push_back(d);
+  allocs_.add(d);
   MRT_HIP_CHECK(hipMemcpy(d, host.data(), host.size() * 4, hipMemcpyHostToDevice));
   return d;
 }
@@ -231,9 +231,9 @@ Model::Model(const TensorSource& src, const Config& c, DType dtype, int dev)
     void* t = nullptr;
     void* d = nullptr;
     MRT_HIP_CHECK(hipMalloc(&t, n_rows * esz));
-    allocs_.push_back(t);
+    allocs_.add(t);
     MRT_HIP_CHECK(hipMalloc(&d, n_rows * esz));
-    allocs_.push_back(d);
+    allocs_.add(d);
     precompute_biases(0, kBiasRows, t);
     precompute_biases(1, kBiasRows, d);
     tbias_rows = t;
@@ -306,7 +306,7 @@ Model::Model(const TensorSource& src, const Config& c, DType dtype, int dev)
 
 Model::~Model() {
   (void)hipSetDevice(device);
-  for (void* p : allocs_) (void)hipFree(p);
+  allocs_.drain([](void* p) { (void)hipFree(p); });
   if (embed_ids_host_) (void)hipHostFree(embed_ids_host_);
 }
 
@@ -320,7 +320,7 @@ void Model::embed_tokens(const int32_t* ids, int n, void* out, hipStream_t s) {
   if (embed_ids_dev_ == nullptr) {
     void* d = nullptr;
     MRT_HIP_CHECK(hipMalloc(&d, kEmbedChunk * sizeof(int)));
-    allocs_.push_back(d);
+    allocs_.add(d);
     embed_ids_dev_ = static_cast<int*>(d);
     MRT_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&embed_ids_host_), kEmbedChunk * sizeof(int),
                                 hipHostMallocDefault));
@@ -1201,7 +1201,7 @@ const SplitWeights* Model::split_weights(hipStream_t s) {
     for (void* p : bufs) (void)hipFree(p);
     throw;
   }
-  allocs_.insert(allocs_.end(), bufs.begin(), bufs.end());
+  allocs_.add(bufs);
   split_ = std::move(sw);
   split_built_ = true;
   return &split_;
@@ -1246,7 +1246,7 @@ const FragWeights* Model::frag_weights(hipStream_t s) {
     for (void* p : bufs) (void)hipFree(p);
     throw;
   }
-  allocs_.insert(allocs_.end(), bufs.begin(), bufs.end());
+  allocs_.add(bufs);
   frag_ = std::move(fw);
   frag_built_ = true;
   return &frag_;
@@ -1270,11 +1270,11 @@ const void* Model::depth_qkv_table(int codebook, int offset, hipStream_t s) {
   const int rows = (L - 1) * codebook;
   if (qkv_ws_ == nullptr) {
     MRT_HIP_CHECK(hipMalloc(&qkv_ws_, static_cast<size_t>(kQkvChunkRows) * D * esz));
-    allocs_.push_back(qkv_ws_);
+    allocs_.add(qkv_ws_);
   }
   void* out = nullptr;
   MRT_HIP_CHECK(hipMalloc(&out, static_cast<size_t>(rows) * 3 * HD * esz));
-  allocs_.push_back(out);
+  allocs_.add(out);
   for (int r0 = 0; r0 < rows; r0 += kQkvChunkRows) {
     const int n = std::min(kQkvChunkRows, rows - r0);
     const char* x = static_cast<const char*>(emb) + (static_cast<size_t>(offset) + r0) * D * esz;

@@ -11,6 +11,7 @@
 #include <mutex>
 #include <vector>
 
+#include "alloc_list.hpp"
 #include "common.hpp"
 #include "persist.hpp"
 #include "safetensors.hpp"
@@ -168,7 +169,7 @@ class Model {
   static constexpr int kQkvChunkRows = 2048;
 
  private:
-  std::vector<void*> allocs_;
+  AllocList allocs_;
   struct QkvTable {
     int codebook, offset;
     void* rows;
