@@ -30,6 +30,16 @@ Batch::Batch(Model& model, int streams, int max_frames, int enc_len)
   MRT_REQUIRE(S >= 1 && S <= c.max_encoder_length, "enc_len must be in [1, max_encoder_length]");
   MRT_REQUIRE(c.d_model % 32 == 0 && c.hd() % 32 == 0 && c.d_ff % 32 == 0,
               "batched streams need d_model, heads * 64 and d_ff multiples of 32");
+  try {
+    setup();
+  } catch (...) {
+    release();
+    throw;
+  }
+}
+
+void Batch::setup() {
+  const Config& c = m.cfg;
   MRT_HIP_CHECK(hipSetDevice(m.device));
   MRT_HIP_CHECK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
   const size_t D = c.d_model, HD = c.hd(), FF = c.d_ff, H = c.num_heads, L = c.rvq_depth, e = 2;
@@ -66,10 +76,14 @@ Batch::Batch(Model& model, int streams, int max_frames, int enc_len)
   MRT_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&h_pinned_), h_pinned_n_ * 4, hipHostMallocDefault));
   MRT_HIP_CHECK(hipEventCreate(&ev_[0]));
   MRT_HIP_CHECK(hipEventCreate(&ev_[1]));
-  fw_ = m.frag_weights(stream);
+  tmp_ = m.frag_temporal(stream);
+  dep_ = m.frag_depth(stream);
+  if (tmp_ == nullptr || dep_ == nullptr) throw Error(3, "batched streams: no device memory for the laid-out weights");
 }
 
-Batch::~Batch() {
+Batch::~Batch() { release(); }
+
+void Batch::release() {
   (void)hipSetDevice(m.device);
   if (stream) (void)hipStreamSynchronize(stream);
   if (graph_exec_) (void)hipGraphExecDestroy(graph_exec_);
@@ -110,7 +124,7 @@ void Batch::temporal_stack(int f, const int* fptr) {
   const DType dt = m.dt;
   const int D = c.d_model, HD = c.hd(), FF = c.d_ff, H = c.num_heads;
   for (int i = 0; i < c.num_temporal_layers; ++i) {
-    const FragLayer& W = fw_->tmp[i];
+    const FragLayer& W = (*tmp_)[i];
     const DecoderLayerW& G = m.tmp[i];  // its norms
     char *tk = ring(tkv_, i, 0, F), *tv = ring(tkv_, i, 1, F);
     // layer 0's input is the frame mean (no row partials): a plain norm pass
@@ -141,7 +155,7 @@ void Batch::depth_stack(void* x, int l, bool x_partials, bool qkv_fed) {
   const DType dt = m.dt;
   const int D = c.d_model, HD = c.hd(), FF = c.d_ff, H = c.num_heads, L = c.rvq_depth;
   for (int i = 0; i < c.num_depth_layers; ++i) {
-    const FragLayer& W = fw_->dep[i];
+    const FragLayer& W = dep_->layers[i];
     const DecoderLayerW& G = m.dep[i];
     char *dk = ring(dkv_, i, 0, L), *dv = ring(dkv_, i, 1, L);
     if (i == 0 && qkv_fed) {
@@ -189,10 +203,10 @@ void Batch::enqueue_frame(const GenOpts& o, int f, bool dynamic) {
     depth_stack(x, l, l == 0 && c.num_temporal_layers > 0, l > 0 && qkv_tab_ != nullptr);
     const int head0 = o.codec_offset + C * l;
     if (c.num_depth_layers > 0) {
-      bgemm_f32(m.dt, xf_, R, D, fw_->head, head0, C, logits_, C, stream, norm(m.dec_norm));
+      bgemm_f32(m.dt, xf_, R, D, dep_->head, head0, C, logits_, C, stream, norm(m.dec_norm));
     } else {
       rmsnorm_rows_frag(m.dt, x, m.dec_norm, 1e-6f, R, D, xn_, stream);
-      bgemm_f32(m.dt, xn_, R, D, fw_->head, head0, C, logits_, C, stream);
+      bgemm_f32(m.dt, xn_, R, D, dep_->head, head0, C, logits_, C, stream);
     }
     if (o.record_slices)
       copy_dev(o.record_slices + (static_cast<size_t>(f) * L + l) * R * C, logits_, static_cast<size_t>(R) * C * 4,

@@ -112,6 +112,8 @@ class Batch {
   // the norm (weights g) of a GEMM input whose row partials are at ssq_
   BNorm norm(const void* g) const { return BNorm{g, ssq_, 1e-6f}; }
   void* dalloc(size_t bytes);
+  void setup();
+  void release();
   char* ring(void* base, int layer, int kv, int len) const;
 
   std::vector<void*> allocs_;
@@ -122,7 +124,8 @@ class Batch {
   // the last residual update: its rows in fragment order and their partials (R, d_model / 16)
   void* xf_ = nullptr;
   float* ssq_ = nullptr;
-  const FragWeights* fw_ = nullptr;  // the model's
+  const std::vector<FragLayer>* tmp_ = nullptr;  // the model's
+  const FragDepth* dep_ = nullptr;
   // the model's depth layer-0 q/k/v table of the current call's codec levels,
   // or nullptr (layer 0 computed at every level)
   const void* qkv_tab_ = nullptr;

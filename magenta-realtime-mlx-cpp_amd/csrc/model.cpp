@@ -408,8 +408,10 @@ State::State(Model& model, int rows_, int max_frames, int enc_len)
     sqkv_ = dalloc(R2 * 3 * HD * e);
     satt_ = dalloc(Rt * HD * e);
     sffh_ = dalloc(Rt * FF * e);
-    sxf_ = dalloc(Rt * D * e);
-    sssq_ = static_cast<float*>(dalloc(R2 * (D / 16 + 1) * 4));
+    if (m.frag_shapes()) {
+      sxf_ = dalloc(Rt * D * e);
+      sssq_ = static_cast<float*>(dalloc(R2 * (D / 16) * 4));
+    }
   }
   if (m.dt == DType::BF16) {  // speculative decoding
     const size_t R2 = 2 * L;
@@ -784,7 +786,7 @@ void State::enqueue_decode_spec(const GenOpts& o) {
   sp_rest.noise_frames = o.num_frames;  // one stream: noise row (frame * L + level)
   const char* head0 = static_cast<const char*>(m.lm_head) + static_cast<size_t>(o.codec_offset) * D * esz();
   const int ns = spec_count(o);
-  const FragWeights& fw = *fw_;
+  const FragDepth& fw = *fw_;
   for (int f = 0; f < o.num_frames; ++f) {
     if (f >= ns) {  // past the speculated frames: the plain decode
       enqueue_plain_frame(o, f, sp);
@@ -796,7 +798,7 @@ void State::enqueue_decode_spec(const GenOpts& o) {
     // verification pass: rows 2i + r
     spec_inputs(dt, t_out, m.emb, d_drafts_ + static_cast<size_t>(f) * L, L, D, sx_, stream);
     for (int i = 0; i < c.num_depth_layers; ++i) {
-      const FragLayer& W = fw.dep[i];
+      const FragLayer& W = fw.layers[i];
       rmsnorm_rows_frag(dt, sx_, m.dep[i].norm_sa, 1e-6f, R2, D, sxn_, stream);
       bgemm_qkv_pos(dt, sxn_, R2, D, W.wqkv, HD, sq_, dk(i), dv(i), H, L, rows, stream);
       self_attn_at(dt, R2, sq_, dk(i), dv(i), H, L, 0, 0, nullptr, m.dbias, m.dbuckets, satt_, stream, rows, nullptr,
@@ -1053,11 +1055,12 @@ void State::depth_forward_full(const void* emb, int k, const void* bias, bool ca
   // 16-bit rows that the skinny GEMMs hold: M <= 32 fills no tile of the
   // encoder's GEMM (its 1,024-wide outputs ran 8 blocks, 16 us each; 292 us a
   // call in all at k = 16, 135 us here)
-  if (m.frag_shapes() && M <= kBatchRows && c.num_depth_layers > 0) {
-    const FragWeights& fw = *m.frag_weights(stream);
+  const FragDepth* fd = m.frag_shapes() && M <= kBatchRows && c.num_depth_layers > 0 ? m.frag_depth(stream) : nullptr;
+  if (fd != nullptr) {
+    const FragDepth& fw = *fd;
     auto norm = [&](const void* g) { return BNorm{g, sssq_, 1e-6f}; };
     for (int i = 0; i < c.num_depth_layers; ++i) {
-      const FragLayer& W = fw.dep[i];
+      const FragLayer& W = fw.layers[i];
       if (i == 0) rmsnorm_rows_frag(dt, sx_, m.dep[i].norm_sa, 1e-6f, M, D, sxn_, stream);
       bgemm_store(dt, i == 0 ? sxn_ : sxf_, M, D, W.wqkv, 3 * HD, sqkv_, 3 * HD, stream, i == 0 ? BNorm{} : norm(m.dep[i].norm_sa));
       full_attn(dt, rows, k, H, sqkv_, bias, m.dbias, m.dbuckets, causal, satt_, stream, true);
@@ -1175,81 +1178,104 @@ bool Model::split_shapes() const {
          gemm_split_fits(2 * F, D) && gemm_split_fits(D, F);
 }
 
+namespace {
+
+struct HipDev {
+  hipStream_t s;
+  bool alloc(void** p, size_t bytes) const {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      return false;
+    }
+    MRT_HIP_CHECK(e);
+    return true;
+  }
+  void free(void* p) const { (void)hipFree(p); }
+  void sync() const { MRT_HIP_CHECK(hipStreamSynchronize(s)); }
+};
+
+}  // namespace
+
 const SplitWeights* Model::split_weights(hipStream_t s) {
   if (!split_shapes()) return nullptr;
   std::lock_guard<std::mutex> lock(split_mu_);
   if (split_built_) return &split_;
   MRT_HIP_CHECK(hipSetDevice(device));
   const int D = cfg.d_model, HD = cfg.hd(), F = cfg.d_ff;
-  std::vector<void*> bufs;
+  AllocGroup<HipDev> group(HipDev{s});
   SplitWeights sw;
-  try {
-    auto place = [&](const void* W, int N, int K) -> const bf16* {
-      void* out = nullptr;
-      MRT_HIP_CHECK(hipMalloc(&out, static_cast<size_t>(N) * K * 6));
-      bufs.push_back(out);
-      split_rows(static_cast<const float*>(W), N, K, static_cast<bf16*>(out), s);
-      return static_cast<bf16*>(out);
-    };
-    for (const EncoderLayerW& w : enc)
-      sw.enc.push_back(SplitLayer{place(w.wqkv, 3 * HD, D), place(w.wo, D, HD), place(w.w01, 2 * F, D),
-                                  place(w.wo2, D, F)});
-    if (cfg.num_temporal_layers > 0) sw.wkv_cross = place(wkv_cross, cfg.num_temporal_layers * 2 * HD, D);
-    MRT_HIP_CHECK(hipStreamSynchronize(s));
-  } catch (...) {
-    (void)hipStreamSynchronize(s);
-    for (void* p : bufs) (void)hipFree(p);
-    throw;
-  }
-  allocs_.add(bufs);
+  auto place = [&](const void* W, int N, int K) {
+    auto* out = static_cast<bf16*>(group.alloc(static_cast<size_t>(N) * K * 6));
+    if (out) split_rows(static_cast<const float*>(W), N, K, out, s);
+    return static_cast<const bf16*>(out);
+  };
+  for (const EncoderLayerW& w : enc)
+    sw.enc.push_back(SplitLayer{place(w.wqkv, 3 * HD, D), place(w.wo, D, HD), place(w.w01, 2 * F, D),
+                                place(w.wo2, D, F)});
+  if (cfg.num_temporal_layers > 0) sw.wkv_cross = place(wkv_cross, cfg.num_temporal_layers * 2 * HD, D);
+  if (!group.keep(allocs_)) return nullptr;
   split_ = std::move(sw);
   split_built_ = true;
   return &split_;
 }
 
-const FragWeights* Model::frag_weights(hipStream_t s) {
+namespace {
+
+// W (N, K) in fragment order, or nullptr (AllocGroup::alloc).
+const void* place_frags(AllocGroup<HipDev>& group, DType dt, const void* W, int N, int K, bool pairs, hipStream_t s) {
+  void* out = group.alloc(frag_weights_elems(N, K) * dtype_size(dt));
+  if (out) frag_weights(dt, W, N, K, pairs, out, s);
+  return out;
+}
+
+std::vector<FragLayer> place_stack(AllocGroup<HipDev>& group, DType dt, const Config& c,
+                                   const std::vector<DecoderLayerW>& ws, bool temporal, hipStream_t s) {
+  const int D = c.d_model, HD = c.hd(), F = c.d_ff;
+  std::vector<FragLayer> out;
+  for (const DecoderLayerW& w : ws) {
+    FragLayer f;
+    f.wqkv = place_frags(group, dt, w.wqkv, 3 * HD, D, false, s);
+    f.wo = place_frags(group, dt, w.wo, D, HD, false, s);
+    if (temporal) {
+      f.wq_c = place_frags(group, dt, w.wq_c, HD, D, false, s);
+      f.wo_c = place_frags(group, dt, w.wo_c, D, HD, false, s);
+    }
+    f.w01 = place_frags(group, dt, w.w01, 2 * F, D, true, s);
+    f.wo2 = place_frags(group, dt, w.wo2, D, F, false, s);
+    out.push_back(f);
+  }
+  return out;
+}
+
+}  // namespace
+
+const FragDepth* Model::frag_depth(hipStream_t s) {
   MRT_REQUIRE(frag_shapes(), "fragment weights: 16-bit model with widths that are multiples of 32");
   std::lock_guard<std::mutex> lock(frag_mu_);
-  if (frag_built_) return &frag_;
+  if (frag_depth_built_) return &frag_depth_;
   MRT_HIP_CHECK(hipSetDevice(device));
-  const int D = cfg.d_model, HD = cfg.hd(), F = cfg.d_ff;
-  std::vector<void*> bufs;
-  FragWeights fw;
-  try {
-    auto place = [&](const void* W, int N, int K, bool pairs = false) -> const void* {
-      void* out = nullptr;
-      MRT_HIP_CHECK(hipMalloc(&out, frag_weights_elems(N, K) * esz));
-      bufs.push_back(out);
-      mrt::frag_weights(dt, W, N, K, pairs, out, s);
-      return out;
-    };
-    auto stack = [&](const std::vector<DecoderLayerW>& ws, bool temporal, std::vector<FragLayer>& out) {
-      for (const DecoderLayerW& w : ws) {
-        FragLayer f;
-        f.wqkv = place(w.wqkv, 3 * HD, D);
-        f.wo = place(w.wo, D, HD);
-        if (temporal) {
-          f.wq_c = place(w.wq_c, HD, D);
-          f.wo_c = place(w.wo_c, D, HD);
-        }
-        f.w01 = place(w.w01, 2 * F, D, true);
-        f.wo2 = place(w.wo2, D, F);
-        out.push_back(f);
-      }
-    };
-    stack(tmp, true, fw.tmp);
-    stack(dep, false, fw.dep);
-    fw.head = place(lm_head, cfg.vocab_size, D);
-    MRT_HIP_CHECK(hipStreamSynchronize(s));
-  } catch (...) {
-    (void)hipStreamSynchronize(s);
-    for (void* p : bufs) (void)hipFree(p);
-    throw;
-  }
-  allocs_.add(bufs);
-  frag_ = std::move(fw);
-  frag_built_ = true;
-  return &frag_;
+  AllocGroup<HipDev> group(HipDev{s});
+  FragDepth fd;
+  fd.layers = place_stack(group, dt, cfg, dep, false, s);
+  fd.head = place_frags(group, dt, lm_head, cfg.vocab_size, cfg.d_model, false, s);
+  if (!group.keep(allocs_)) return nullptr;
+  frag_depth_ = std::move(fd);
+  frag_depth_built_ = true;
+  return &frag_depth_;
+}
+
+const std::vector<FragLayer>* Model::frag_temporal(hipStream_t s) {
+  MRT_REQUIRE(frag_shapes(), "fragment weights: 16-bit model with widths that are multiples of 32");
+  std::lock_guard<std::mutex> lock(frag_mu_);
+  if (frag_temporal_built_) return &frag_temporal_;
+  MRT_HIP_CHECK(hipSetDevice(device));
+  AllocGroup<HipDev> group(HipDev{s});
+  std::vector<FragLayer> layers = place_stack(group, dt, cfg, tmp, true, s);
+  if (!group.keep(allocs_)) return nullptr;
+  frag_temporal_ = std::move(layers);
+  frag_temporal_built_ = true;
+  return &frag_temporal_;
 }
 
 const void* Model::depth_qkv_table(int codebook, int offset, hipStream_t s) {
@@ -1446,6 +1472,8 @@ void State::generate(const int32_t* enc_tokens_host, const GenOpts& o, int32_t* 
   // overwrites them.  Without a previous call of the same length it does not
   // speculate (as the reference's first chunk).
   spec_drafts_ = speculating(o) && prev_frames_ == o.num_frames;
+  // built once before any capture; without the memory for it the call decodes plainly
+  if (spec_drafts_) spec_drafts_ = (fw_ = m.frag_depth(stream)) != nullptr;
   if (spec_drafts_) copy(d_drafts_, d_tokens, nt * 4);
 
   if (persistent()) reserve_epochs(decode_launches(o));
@@ -1456,7 +1484,6 @@ void State::generate(const int32_t* enc_tokens_host, const GenOpts& o, int32_t* 
   dec_launches_ = persistent() ? decode_launches(o) : 0;
   // built once per (codebook, offset) before any capture; waits for the stream then
   qkv_table_ = frame_kernel_ && qkv_table_on_ ? m.depth_qkv_table(o.codebook, o.codec_offset, stream) : nullptr;
-  if (spec_drafts_) fw_ = m.frag_weights(stream);  // likewise
   hipGraphExec_t exec = o.use_graph ? decode_graph(o) : nullptr;
   {
     // persistent grids of other states on this device run before or after

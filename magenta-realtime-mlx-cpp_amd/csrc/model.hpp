@@ -69,8 +69,8 @@ struct DecoderLayerW {
 struct FragLayer {
   const void *wqkv = nullptr, *wo = nullptr, *wq_c = nullptr, *wo_c = nullptr, *w01 = nullptr, *wo2 = nullptr;
 };
-struct FragWeights {
-  std::vector<FragLayer> tmp, dep;
+struct FragDepth {
+  std::vector<FragLayer> layers;
   const void* head = nullptr;  // lm_head (vocab rows)
 };
 
@@ -152,14 +152,16 @@ class Model {
   // levels < 2 (the decode then computes layer 0).
   const void* depth_qkv_table(int codebook, int offset, hipStream_t s);
   static constexpr size_t kMaxQkvTables = 4;
-  // The decoder stacks and lm_head in fragment order (16-bit models with
-  // d_model, heads * 64 and d_ff multiples of 32): as many bytes again as the
-  // matrices themselves, built on first use on `s` (waits for it; never during
-  // a capture) and kept with the model.
-  const FragWeights* frag_weights(hipStream_t s);
+  // The depth stack with lm_head, and the temporal stack, in fragment order
+  // (16-bit models with d_model, heads * 64 and d_ff multiples of 32): as many
+  // bytes again as those matrices themselves, each built on first use on `s`
+  // (waits for it; never during a capture) and kept with the model; nullptr where
+  // there is no memory for it.
+  const FragDepth* frag_depth(hipStream_t s);
+  const std::vector<FragLayer>* frag_temporal(hipStream_t s);
   // The split encoder of an fp32 model (1.5 times its matrices' bytes), kept in
-  // the same way; nullptr for 16-bit models and widths the split GEMM does not
-  // take.
+  // the same way; nullptr also for 16-bit models and widths the split GEMM does
+  // not take.
   const SplitWeights* split_weights(hipStream_t s);
   bool split_shapes() const;
   bool frag_shapes() const {
@@ -180,8 +182,9 @@ class Model {
   SplitWeights split_;
   bool split_built_ = false;
   std::mutex frag_mu_;
-  FragWeights frag_;
-  bool frag_built_ = false;
+  FragDepth frag_depth_;
+  std::vector<FragLayer> frag_temporal_;
+  bool frag_depth_built_ = false, frag_temporal_built_ = false;
   void* qkv_ws_ = nullptr;  // build workspace of the tables (kQkvChunkRows x d_model)
   std::vector<float> pe_host_;  // fp32 sinusoid table (max_encoder_length, d_model)
   static constexpr int kEmbedChunk = 4096;
@@ -352,7 +355,7 @@ class State {
   void *sx_ = nullptr, *sxn_ = nullptr, *sq_ = nullptr, *satt_ = nullptr, *sffh_ = nullptr, *sqkv_ = nullptr;
   float* slog_ = nullptr;
   int *sdrawn_ = nullptr, *sdecided_ = nullptr;  // sdecided_: (F) the accepted count n of each frame
-  const FragWeights* fw_ = nullptr;  // the model's, once a call speculates
+  const FragDepth* fw_ = nullptr;  // the model's, once a call speculates
   void* sxf_ = nullptr;     // the rows of sx_ in fragment order, and their partials (skinny GEMMs)
   float* sssq_ = nullptr;
   float spec_acc_ = -1.f;  // share of the last call's levels taken from the verification pass

@@ -1,7 +1,12 @@
-"""The list of a model's allocations takes additions from several threads: the
-parts built on first use are built on whichever thread comes first, and distinct
-states of one model may be driven from distinct threads.  The list is compiled
-for the CPU under the thread sanitizer."""
+"""A model's allocations, compiled for the CPU.
+
+  * The list takes additions from several threads (under the thread sanitizer): the
+    parts built on first use are built on whichever thread comes first, and distinct
+    states of one model may be driven from distinct threads.
+  * A group of allocations is kept as a whole, or given back as a whole where there
+    is no memory for one of them (the caller then goes without that part) or where
+    building throws.
+"""
 
 from __future__ import annotations
 
@@ -10,7 +15,7 @@ import subprocess
 
 CSRC = pathlib.Path(__file__).resolve().parents[1] / "magenta-realtime-mlx-cpp_amd" / "csrc"
 
-PROGRAM = r"""
+THREADS = r"""
 #include <cstdint>
 #include <set>
 #include <thread>
@@ -37,13 +42,74 @@ int main() {
 """
 
 
-def test_allocations_added_from_several_threads(tmp_path):
-    src, exe = tmp_path / "alloc_list.cpp", tmp_path / "alloc_list"
-    src.write_text(PROGRAM)
-    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-fsanitize=thread", f"-I{CSRC}", str(src), "-o", str(exe),
-                    "-lpthread"], check=True)
+GROUPS = r"""
+#include <set>
+#include <stdexcept>
+#include "alloc_list.hpp"
+struct Dev {
+  std::set<void*>* live;
+  int* left;  // allocations that there is memory for
+  int* syncs;
+  bool alloc(void** p, size_t bytes) const {
+    if (bytes == 0) throw std::runtime_error("other error");
+    if (*left == 0) return false;
+    --*left;
+    *p = new char[bytes];
+    live->insert(*p);
+    return true;
+  }
+  void free(void* p) const {
+    if (live->erase(p) != 1) throw std::runtime_error("freed twice");
+    delete[] static_cast<char*>(p);
+  }
+  void sync() const { ++*syncs; }
+};
+int main() {
+  std::set<void*> live;
+  int left = 0, syncs = 0;
+  const Dev dev{&live, &left, &syncs};
+  mrt::AllocList list;
+  for (int room = 0; room <= 3; ++room) {  // three allocations, memory for `room` of them
+    left = room;
+    mrt::AllocGroup<Dev> g(dev);
+    int got = 0;
+    for (int i = 0; i < 3; ++i) got += g.alloc(8) != nullptr;
+    if (got != room) return 1;
+    left = 9;  // memory again does not mend the group
+    if (room < 3 && g.alloc(8) != nullptr) return 2;
+    if (g.keep(list) != (room == 3)) return 3;
+    if (live.size() != (room == 3 ? 3u : 0u) || syncs != room + 1) return 4;
+  }
+  left = 2;
+  try {  // a build that throws gives its allocations back, after the work that writes them
+    mrt::AllocGroup<Dev> g(dev);
+    g.alloc(8);
+    g.alloc(0);
+    return 5;
+  } catch (const std::runtime_error&) {
+  }
+  if (live.size() != 3 || syncs != 5) return 6;
+  list.drain([&](void* p) { dev.free(p); });
+  return live.empty() ? 0 : 7;
+}
+"""
+
+
+def run(tmp_path, program, *flags):
+    src, exe = tmp_path / "allocs.cpp", tmp_path / "allocs"
+    src.write_text(program)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-g", *flags, f"-I{CSRC}", str(src), "-o", str(exe), "-lpthread"],
+                   check=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
-    assert r.returncode == 0, r.stdout + r.stderr
+    assert r.returncode == 0, (r.returncode, r.stdout + r.stderr)
+
+
+def test_allocations_added_from_several_threads(tmp_path):
+    run(tmp_path, THREADS, "-fsanitize=thread")
+
+
+def test_groups_are_kept_or_given_back(tmp_path):
+    run(tmp_path, GROUPS, "-fsanitize=address")
 
 
 def test_model_keeps_its_allocations_in_the_list():

@@ -181,3 +181,33 @@ def test_reset_cache(tiny):
         st.reset_cache("cross")
     st.close()
     m.close()
+
+
+def test_depth_forward_full_lays_out_the_depth_stack_only(gpu_available):
+    """The first call of a 16-bit model lays out the matrices that the pass reads: the
+    device memory that it takes is that of the depth stack and lm_head, within 32 MB of
+    allocation granularity and scratch, and a second call takes none."""
+    import torch
+    import mrt_df
+    import synth_bundle
+    cfg = mrt_df.Config.bench()
+    w = synth_bundle.make_weights(cfg, seed=1234, threads=16)
+    reads = 2 * sum(v.size for k, v in w.items() if k.startswith("depth_layers") or k == "lm_head.weight")
+    m = mrt_df.Depthformer(w, cfg, dtype="bf16")
+    st = m.new_state(max_frames=1)
+    embs = torch.zeros((2, 16, cfg.d_model), dtype=torch.bfloat16, device="cuda")
+    out = st.depth_forward_full(embs[:, :1].contiguous())  # torch's own pool, the module's code
+    del out
+    st.close()
+    m.close()
+    m = mrt_df.Depthformer(w, cfg, dtype="bf16")
+    st = m.new_state(max_frames=1)
+    free = [torch.cuda.mem_get_info()[0]]
+    for _ in range(2):
+        st.depth_forward_full(embs[:, :1].contiguous())
+        torch.cuda.synchronize()
+        free.append(torch.cuda.mem_get_info()[0])
+    assert free[0] - free[1] <= reads + (32 << 20), (free, reads)
+    assert free[1] - free[2] <= 1 << 20, free
+    st.close()
+    m.close()
