@@ -9,7 +9,9 @@
 #include "batch.hpp"
 #include "coca.hpp"
 #include "codec.hpp"
+#include "kernels.hpp"
 #include "model.hpp"
+#include "split_gemm.hpp"
 #include "stream.hpp"
 
 struct mrt_df {
@@ -453,6 +455,50 @@ int mrt_probe_pingpong(int device, int peer, int rounds, float* us_one_way) {
   return guarded([&] {
     if (!us_one_way) throw mrt::Error(MRT_ERR_INVALID, "null argument");
     *us_one_way = mrt::probe_pingpong(device, peer, rounds);
+  });
+}
+
+// Not part of the interface (mrt_df.h): one GEMM of the encoder on device buffers, for
+// tests of single kernels.  path 0: as gemm() picks, 1: vector ALUs, 2: fp32 operands
+// split first (gemm_split).  tile: -1 the rule's; *taken: the tile of a matrix-core
+// GEMM of this shape by the rule.
+int mrt_test_gemm(int dtype, int path, const void* A, const void* B, int M, int N, int K, int kind, int tile, int nb,
+                  int H, int S, int HD, void* C, int* taken) {
+  return guarded([&] {
+    if (!A || !B || !C || !taken) throw mrt::Error(MRT_ERR_INVALID, "null argument");
+    mrt::GemmEpiArgs e;
+    e.kind = static_cast<mrt::GemmEpi>(kind);
+    e.C = C;
+    e.nb = nb;
+    e.H = H;
+    e.S = S;
+    e.HD = HD;
+    e.tile = tile;
+    const auto dt = static_cast<mrt::DType>(dtype);
+    *taken = N % 128 == 0 ? mrt::gemm_tile(dt, M, N, e.kind) : -1;
+    if (path == 2) {
+      mrt::bf16* sp[2] = {nullptr, nullptr};
+      auto free_all = [&] {
+        (void)hipDeviceSynchronize();
+        for (mrt::bf16* p : sp) (void)hipFree(p);
+      };
+      try {
+        const void* src[2] = {A, B};
+        const int rows[2] = {M, N};
+        for (int i = 0; i < 2; ++i) {
+          MRT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&sp[i]), static_cast<size_t>(rows[i]) * K * 6));
+          mrt::split_rows(static_cast<const float*>(src[i]), rows[i], K, sp[i], nullptr);
+        }
+        mrt::gemm_split(sp[0], sp[1], M, N, K, e, nullptr);
+      } catch (...) {
+        free_all();
+        throw;
+      }
+      free_all();
+    } else {
+      mrt::gemm(dt, A, B, M, N, K, e, nullptr, path == 0);
+    }
+    MRT_HIP_CHECK(hipDeviceSynchronize());
   });
 }
 

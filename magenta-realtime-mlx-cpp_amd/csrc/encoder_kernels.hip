@@ -210,7 +210,7 @@ __global__ __launch_bounds__(256) void k_gemm_valu(const T* __restrict__ A, cons
 // ---- matrix-core GEMM ------------------------------------------------------------------
 // gelu_t of 16-bit types with tanh taken as (1 - t) / (1 + t), t = 2^(-2 |x| log2 e):
 // within 2e-7 of tanhf, far below the 16-bit rounding of 1 + tanh that is all the
-// formula keeps of it.  tanhf's two polynomial paths made the 181 M gated-GELUs of
+// formula keeps of it (every finite bf16 and fp16 value has gelu_t's result).  tanhf's two polynomial paths made the 181 M gated-GELUs of
 // 32 streams a 300 us epilogue.
 template <typename T>
 __device__ __forceinline__ float gelu16(float x) {
@@ -260,16 +260,10 @@ __device__ __forceinline__ void mfma_epilogue(const GemmOut<T>& out, const f32x1
     }
     return w;
   };
-  auto gelu = [](float x) {
-    if constexpr (k16)
-      return gelu16<T>(x);
-    else
-      return gelu_t<T>(x);
-  };
   auto col = [&](int g) { return k16 ? 8 * (2 * g + lh) : 8 * g + 4 * lh; };
   switch (out.a.kind) {
-    case GemmEpi::Geglu:
-      if constexpr (NJ % 2 == 0) {
+    case GemmEpi::Geglu:  // 16 bit only (gemm_tiles)
+      if constexpr (NJ % 2 == 0 && k16) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -277,14 +271,14 @@ __device__ __forceinline__ void mfma_epilogue(const GemmOut<T>& out, const f32x1
 #pragma unroll
             for (int g = 0; g < G; ++g) {
               const uint4 w = pack(g, [&](int r) {
-                return gelu(St_::rnd(acc[i][2 * p][r])) * St_::rnd(acc[i][2 * p + 1][r]);
+                return gelu16<T>(St_::rnd(acc[i][2 * p][r])) * St_::rnd(acc[i][2 * p + 1][r]);
               });
               const int m = m0 + 32 * i;
               if (m < M) *reinterpret_cast<uint4*>(C + (size_t)m * (N / 2) + nb / 2 + 32 * p + col(g)) = w;
             }
       }
       break;
-    case GemmEpi::GegluSplit:
+    case GemmEpi::GegluSplit:  // fp32 only
       if constexpr (NJ % 2 == 0 && !k16) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
@@ -448,11 +442,11 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_ring(const void* __restri
 
   typename Tile::State s;
   Tile::start(lds, s, issue);
-  // store instructions of a whole tile's epilogue (16 bytes each; the split
-  // gated-GELU pairs three times 8)
+  // store instructions of a whole tile's epilogue: 16 bytes each, half as many for
+  // the 16-bit gated-GELU pairs; three times 8 bytes for 16 of the fp32 pairs' (split)
   constexpr int kStores = Tile::MI * Tile::NJ * (sizeof(T) == 2 ? 2 : 4);
   constexpr int kGegluStores = sizeof(T) == 2 ? kStores / 2 : kStores / 2 * 3;
-  const bool pairs = out.a.kind == GemmEpi::Geglu || out.a.kind == GemmEpi::GegluSplit;
+  const bool pairs = out.a.kind == (sizeof(T) == 2 ? GemmEpi::Geglu : GemmEpi::GegluSplit);
   const bool plain = out.a.kind == GemmEpi::Store || out.a.kind == GemmEpi::CrossKV;
   bool stored = false;  // the previous tile's epilogue issued exactly those stores after the ring's loads
   for (; t < cnt; t += step) {
@@ -801,44 +795,69 @@ void rmsnorm_rows(DType dt, const void* x, const void* g, float eps, int M, int 
 
 namespace {
 
+// The tiles, in the order in which they are preferred, with their time per area
+// relative to the first.
+struct GemmTile {
+  int bm, bn;
+  double f;
+};
+constexpr GemmTile kTiles16[] = {{256, 256, 1.0}, {192, 256, 1.05}, {128, 256, 1.05}, {128, 192, 1.25}, {64, 128, 1.5}};
+constexpr GemmTile kTiles32[] = {{128, 192, 1.0}, {128, 128, 1.0}, {64, 128, 1.15}};
+
+bool gemm_pairs(GemmEpi kind) { return kind == GemmEpi::Geglu || kind == GemmEpi::GegluSplit; }
+
+// Gated-GELU pairs need wave tiles of whole 64-column groups (not 192 columns).
+bool tile_takes(const GemmTile& t, int N, GemmEpi kind) { return N % t.bn == 0 && !(gemm_pairs(kind) && t.bn == 192); }
+
 // The tile whose rounds over the CUs (one block each) take the least time: rounds x
 // area x the tile's time per area relative to 256 x 256.  The factors are measured
 // times a round of the 16-bit kernel, K = 1,024: 256 x 256 30.7 us; 192 x 256 24.2
 // and 128 x 256 15.9 (1.05); 128 x 192 14.3 (1.25); 64 x 128 5.7 (1.5; its fragment
-// reads and its epilogue weigh more).  Gated-GELU pairs need wave tiles of whole
-// 64-column groups (not 128 x 192).
+// reads and its epilogue weigh more).
+template <int n>
+int best_tile(const GemmTile (&tiles)[n], int M, int N, GemmEpi kind) {
+  const long cus = std::max(8, device_cus() & ~7);
+  int best = -1;
+  double least = 0.;
+  for (int i = 0; i < n; ++i) {
+    const GemmTile& t = tiles[i];
+    if (!tile_takes(t, N, kind)) continue;
+    const long count = (long)((M + t.bm - 1) / t.bm) * (N / t.bn);
+    const double cost = (double)((count + cus - 1) / cus) * t.bm * t.bn * t.f;
+    if (best < 0 || cost < least) best = i, least = cost;
+  }
+  return best;
+}
+
+}  // namespace
+
+int gemm_tile(DType dt, int M, int N, GemmEpi kind) {
+  return dt == DType::F32 ? best_tile(kTiles32, M, N, kind) : best_tile(kTiles16, M, N, kind);
+}
+
+namespace {
+
 template <class Core, typename T>
 void gemm_tiles(const void* A, const void* B, int M, int N, int K, const GemmEpiArgs& e, hipStream_t s) {
   const GemmOut<T> out{e, N};
-  const long cus = std::max(8, device_cus() & ~7);
-  const bool pairs = e.kind == GemmEpi::Geglu || e.kind == GemmEpi::GegluSplit;
-  auto cost = [&](int bm, int bn, double f) {
-    if (N % bn) return 1e30;
-    const long tiles = (long)((M + bm - 1) / bm) * (N / bn);
-    return (double)((tiles + cus - 1) / cus) * bm * bn * f;
-  };
-  const double cw = pairs ? 1e30 : cost(128, 192, sizeof(T) == 2 ? 1.25 : 1.0);
+  const int tile = e.tile >= 0 ? e.tile : gemm_tile(sizeof(T) == 2 ? DType::BF16 : DType::F32, M, N, e.kind);
   if constexpr (sizeof(T) == 2) {
-    const double c64 = cost(64, 128, 1.5), c128 = cost(128, 256, 1.05), c192 = cost(192, 256, 1.05);
-    const double c256 = cost(256, 256, 1.0);
-    if (c256 <= std::min(std::min(c192, c128), std::min(cw, c64)))
-      launch_gemm_ring<Core, T, 256, 256, 4, 2, 2>(A, B, M, N, K, out, s);
-    else if (c192 <= std::min(c128, std::min(cw, c64)))
-      launch_gemm_ring<Core, T, 192, 256, 2, 4, 2>(A, B, M, N, K, out, s);
-    else if (c128 <= std::min(cw, c64))
-      launch_gemm_ring<Core, T, 128, 256, 2, 4, 3>(A, B, M, N, K, out, s);
-    else if (cw <= c64)
-      launch_gemm_ring<Core, T, 128, 192, 4, 2, 3>(A, B, M, N, K, out, s);
-    else
-      launch_gemm_ring<Core, T, 64, 128, 2, 2, 4>(A, B, M, N, K, out, s);
+    MRT_REQUIRE(tile >= 0 && tile < 5 && tile_takes(kTiles16[tile], N, e.kind), "gemm: tile does not fit the shape");
+    switch (tile) {
+      case 0: launch_gemm_ring<Core, T, 256, 256, 4, 2, 2>(A, B, M, N, K, out, s); break;
+      case 1: launch_gemm_ring<Core, T, 192, 256, 2, 4, 2>(A, B, M, N, K, out, s); break;
+      case 2: launch_gemm_ring<Core, T, 128, 256, 2, 4, 3>(A, B, M, N, K, out, s); break;
+      case 3: launch_gemm_ring<Core, T, 128, 192, 4, 2, 3>(A, B, M, N, K, out, s); break;
+      default: launch_gemm_ring<Core, T, 64, 128, 2, 2, 4>(A, B, M, N, K, out, s); break;
+    }
   } else {
-    const double c64 = cost(64, 128, 1.15), c128 = cost(128, 128, 1.0);
-    if (cw <= std::min(c128, c64))
-      launch_gemm_ring<Core, T, 128, 192, 2, 2, 2>(A, B, M, N, K, out, s);
-    else if (c128 <= c64)
-      launch_gemm_ring<Core, T, 128, 128, 2, 2, 3>(A, B, M, N, K, out, s);
-    else
-      launch_gemm_ring<Core, T, 64, 128, 2, 2, 4>(A, B, M, N, K, out, s);
+    MRT_REQUIRE(e.kind != GemmEpi::Geglu, "gemm: fp32 pairs are written split");
+    MRT_REQUIRE(tile >= 0 && tile < 3 && tile_takes(kTiles32[tile], N, e.kind), "gemm: tile does not fit the shape");
+    switch (tile) {
+      case 0: launch_gemm_ring<Core, T, 128, 192, 2, 2, 2>(A, B, M, N, K, out, s); break;
+      case 1: launch_gemm_ring<Core, T, 128, 128, 2, 2, 3>(A, B, M, N, K, out, s); break;
+      default: launch_gemm_ring<Core, T, 64, 128, 2, 2, 4>(A, B, M, N, K, out, s); break;
+    }
   }
 }
 
@@ -859,6 +878,7 @@ void gemm_t(const T* A, const T* B, int M, int N, int K, const GemmEpiArgs& e, h
 void gemm(DType dt, const void* A, const void* B, int M, int N, int K, const GemmEpiArgs& e,
           hipStream_t s, bool allow_mfma) {
   MRT_REQUIRE(M >= 1 && N >= 1 && K >= 1, "gemm: empty problem");
+  MRT_REQUIRE(e.kind != GemmEpi::GegluSplit, "gemm: split pairs come from split operands");
   if (e.kind == GemmEpi::Geglu) MRT_REQUIRE(N % 64 == 0, "gemm: gated-GELU needs N % 64 == 0");
   if (e.kind == GemmEpi::CrossKV)
     MRT_REQUIRE(e.HD == e.H * 64 && N % e.HD == 0 && M == e.nb * e.S, "gemm: bad cross-KV shape");

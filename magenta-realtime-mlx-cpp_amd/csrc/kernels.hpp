@@ -159,13 +159,16 @@ enum class GemmEpi : int {
   CrossKV = 3,  // n = (layer*2 + kv)*HD + h*64 + d; m = b*S + s ->
                 //   C[(((layer*2+kv)*nb + b)*H + h)*S + s][d]
   StoreF32 = 4, // C (M, N) fp32, each value rounded to the model dtype first (logits)
-  GegluSplit = 5, // fp32: as Geglu, C split rows (split_gemm.hpp) of N/2 values
+  GegluSplit = 5, // gemm_split: as Geglu (which it refuses), C split rows (split_gemm.hpp) of N/2 values
 };
 struct GemmEpiArgs {
   GemmEpi kind = GemmEpi::Store;
   void* C = nullptr;
   int nb = 2, H = 16, S = 1, HD = 1024;
+  int tile = -1;  // matrix-core tile (index, gemm_tile), -1: the rule's
 };
+// The tile that the matrix-core GEMM takes: its index among those of the type.
+int gemm_tile(DType dt, int M, int N, GemmEpi kind);
 void gemm(DType dt, const void* A, const void* B, int M, int N, int K, const GemmEpiArgs& e,
           hipStream_t s, bool allow_mfma = true);
 
