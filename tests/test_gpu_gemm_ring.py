@@ -1,4 +1,5 @@
-"""The encoder prefill's persistent GEMM at the edges of its tiles."""
+"""The encoder prefill through the persistent GEMM, whole: small widths, which take its
+64 x 128 tile (test_gpu_gemm_tiles.py has every tile by itself)."""
 
 from __future__ import annotations
 
@@ -18,8 +19,8 @@ TOL = {"bf16": 1.2e-2, "fp16": 1.5e-3}
 @pytest.mark.parametrize("dtype", ["bf16", "fp16"])
 @pytest.mark.parametrize("S", [1, 31, 33, 64, 65, 96, 97, 129, 200])
 def test_encode_edges(gpu_available, S, dtype):
-    """Row counts 2 S at the edges of the 64- to 256-row tiles and of the 32-row
-    matrix instruction; the output rows past the last are not written."""
+    """Row counts 2 S at the edges of the 64-row tile and of the 32-row matrix
+    instruction, against the oracle; a second encode finds the buffers of the first."""
     import mrt_df
     import synth_bundle
     from oracle import depthformer_oracle as O
@@ -39,8 +40,8 @@ def test_encode_edges(gpu_available, S, dtype):
 
 
 def test_many_rows_equal_few(gpu_available):
-    """Rows do not depend on the tile that computes them: 32 streams (several tiles a
-    block) against one stream, bit for bit."""
+    """Rows do not depend on the rows beside them: 32 streams (several tiles a block)
+    against one stream, bit for bit."""
     import mrt_df
     import synth_bundle
     cfg = dataclasses.replace(mrt_df.Config.tiny(8), max_encoder_length=300)

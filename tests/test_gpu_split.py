@@ -23,8 +23,9 @@ def rel(a, b):
 @pytest.mark.parametrize("ffn_scale", [1.0, 2.0 ** 40])
 @pytest.mark.parametrize("S", [1, 33, 63, 64, 65, 127, 129, 200])
 def test_encode_edges(gpu_available, S, ffn_scale):
-    """Context lengths at the edges of the 64- and 128-row tiles and of the key
-    tile pairs, and hidden FFN values far outside the range of 16-bit floats."""
+    """Context lengths at the edges of the 64-row tile (the one that these widths take)
+    and of the key tile pairs, and hidden FFN values far outside the range of 16-bit
+    floats."""
     import mrt_df
     import synth_bundle
     from oracle import depthformer_oracle as O
