@@ -466,6 +466,11 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_ring(const void* __restri
       });
     }
     s.settle();
+    if constexpr (sizeof(T) == 4)
+      resum_not_finite<Tile>(s, [&](int row, int col) {
+        return split_dot(reinterpret_cast<const bf16*>(static_cast<const char*>(A) + min(m0 + row, M - 1) * ld),
+                         reinterpret_cast<const bf16*>(static_cast<const char*>(B) + (n0 + col) * ld), nk, 0.f);
+      });
     mfma_epilogue<T, Tile::MI, Tile::NJ>(out, s.acc, M, m0 + (wid / WN) * (BM / WM), n0 + (wid % WN) * (BN / WN));
     asm volatile("" ::: "memory");  // the stores stay ahead of the next tile's waits
     stored = m0 + BM <= M;

@@ -138,6 +138,14 @@ struct RingTile {
   // The first fragments of the next k-tile again.
   __device__ static void reread(unsigned char* lds, State& s) { read(lds + s.slot * kStage, 0, 0, s); }
 
+  // Row and column of sum e (acc[e / 16 / NJ][e / 16 % NJ], r = e % 16) in the tile.
+  __device__ static void sum_pos(int e, int& row, int& col) {
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = e / 16 / NJ, j = e / 16 % NJ, r = e % 16;
+    row = (wid / WN) * (BM / WM) + 32 * i + (lane & 31);
+    col = (wid % WN) * (BN / WN) + 32 * j + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+  }
+
   // Extra: vector memory instructions issued after the loads waited for.
   template <int Extra = 0>
   __device__ static void wait_loads() {

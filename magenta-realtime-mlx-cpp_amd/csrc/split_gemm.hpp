@@ -31,8 +31,10 @@ __host__ __device__ inline size_t split_index(size_t r, int k, int K) {
   return (r * (size_t)(K >> 5) + (k >> 5)) * kSplitGroup + (k & 31);
 }
 
-// The parts of a float.  A value that rounds up to infinity keeps a truncated
-// first part; infinities and NaN are their first part alone.
+// The parts of a float: exact for values of at least 2^-110 (below, bits under
+// bf16's smallest subnormal, 2^-133, are lost).  A value that rounds up to infinity
+// keeps a truncated first part; infinities and NaN are their first part alone
+// (resum_not_finite has their products).
 __device__ __forceinline__ void split3(float a, bf16 (&p)[3]) {
   p[0] = f2bf(a);
   if ((p[0] & 0x7fff) == 0x7f80) p[0] = (bf16)(__float_as_uint(a) >> 16);
@@ -96,6 +98,58 @@ struct CoreSplit {
 struct CoreSplitFine : CoreSplit {
   static constexpr bool kFine = true;
 };
+
+// sum + the products of `groups` groups of two split rows, as fused multiply-adds of
+// the whole floats.
+__device__ inline float split_dot(const bf16* a, const bf16* b, int groups, float sum) {
+  for (int g = 0; g < groups; ++g, a += kSplitGroup, b += kSplitGroup)
+    for (int e = 0; e < 32; e += 8) {
+      uint4 u[3], v[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        u[p] = ld_g16(a + 32 * p + e);
+        v[p] = ld_g16(b + 32 * p + e);
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        auto whole = [&](const uint4 (&q)[3]) {
+          return (bf2f(reinterpret_cast<const bf16*>(&q[0])[k]) + bf2f(reinterpret_cast<const bf16*>(&q[1])[k])) +
+                 bf2f(reinterpret_cast<const bf16*>(&q[2])[k]);
+        };
+        sum = fmaf(whole(u), whole(v), sum);
+      }
+    }
+  return sum;
+}
+
+// An infinity times the other operand's small parts, zeros or of the other sign, is
+// NaN where the float product is infinite.  So sums that are not finite are taken
+// again as plain fp32 sums: sum_of(row, column of the tile).  A product and an add per
+// sum look for them; a tile that holds one costs as much as the vector ALUs take.
+template <class Tile, class F>
+__device__ __forceinline__ void resum_not_finite(typename Tile::State& s, F&& sum_of) {
+  constexpr int kSums = Tile::MI * Tile::NJ * 16;
+  float t[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int e = 0; e < kSums; ++e) t[e & 3] = fmaf(s.acc[e / 16 / Tile::NJ][e / 16 % Tile::NJ][e % 16], 0.f, t[e & 3]);
+  t[0] = (t[0] + t[1]) + (t[2] + t[3]);
+  if (__builtin_expect(__ballot(t[0] != t[0]) == 0, true)) return;
+#pragma unroll 1
+  for (int e = 0; e < kSums; ++e) {
+    float v = 0.f;
+#pragma unroll
+    for (int q = 0; q < kSums; ++q) v = q == e ? s.acc[q / 16 / Tile::NJ][q / 16 % Tile::NJ][q % 16] : v;
+    if (fabsf(v) < INFINITY) continue;
+    int row, col;
+    Tile::sum_pos(e, row, col);
+    v = sum_of(row, col);
+#pragma unroll
+    for (int q = 0; q < kSums; ++q) {
+      float& c = reinterpret_cast<float*>(&s.acc[q / 16 / Tile::NJ][q / 16 % Tile::NJ])[q % 16];
+      c = q == e ? v : c;
+    }
+  }
+}
 
 // W (N, K) fp32 -> split rows (split_kernels.hip).
 void split_rows(const float* W, long N, int K, bf16* out, hipStream_t s);

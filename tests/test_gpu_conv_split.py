@@ -44,3 +44,32 @@ def test_frame_counts(gpu_available, full, frames):
     for i in range(7):
         assert rel(codec.read(mrt_df.CODEC_BUF_BLOCK0 + i, rec[f"block{i}"].shape), rec[f"block{i}"]) <= TOL
     np.testing.assert_array_equal(codec.decode(tok), first)
+
+
+def test_infinite_activations(gpu_available):
+    """One frame whose first projection overflows: every residual of it is -inf from
+    there on and every ELU of one is -1, so the audio is finite, as the oracle has it.
+    (An infinite activation meets weights of three parts with both signs.)"""
+    import mrt_df
+    w = synth_bundle.make_codec_weights(synth_bundle.CodecShape.reference())
+    w = {k: np.array(v) for k, v in w.items()}
+    w["codebooks"][:, :, 0] = 0
+    w["codebooks"][0, 5, 0] = 4.0
+    w["input_proj.conv1.weight"][0] = 0
+    w["input_proj.conv1.weight"][0, 0] = 3e38
+    w["input_proj.conv2.weight"][:, 0] = -np.abs(w["input_proj.conv2.weight"][:, 0]) - 1e-3
+    for k in w:
+        if k.startswith("decoder_blocks") and k.endswith("shortcut.weight"):
+            w[k] = np.abs(w[k]) + 1e-4
+    tok = np.random.default_rng(3).integers(6, 1024, (4, 16)).astype(np.int32)
+    tok[2, 0] = 5
+    rec = {}
+    with np.errstate(all="ignore"):
+        ref = C.OracleCodec(w, C.CodecConfig.reference(), "fp32").decode(tok, rec)
+    assert np.isfinite(ref).all() and np.isneginf(rec["block6"]).any()
+    codec = mrt_df.Codec(w, max_frames=4)
+    got = codec.decode(tok)
+    last = codec.read(mrt_df.CODEC_BUF_BLOCK0 + 6, rec["block6"].shape)
+    codec.close()
+    assert np.isfinite(got).all() and rel(got, ref) <= TOL
+    np.testing.assert_array_equal(np.isneginf(last), np.isneginf(rec["block6"]))

@@ -142,6 +142,34 @@ def test_gated_gelu_of_every_value(gemm, dtype):
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("tile", range(3))
+@pytest.mark.parametrize("M,K", [(5, 32), (200, 160)])
+def test_split_gemm_not_finite(gemm, M, K, tile):
+    """Infinities, NaN and overflow of fp32 operands give what fp32 products give: an
+    infinite element meets weights with one, two and three parts of both signs."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M)
+    A = torch.randn((M, K), generator=g, device="cuda")
+    B = torch.randn((N, K), generator=g, device="cuda")
+    B[1::3] = B[1::3].bfloat16().float()  # their second and third parts are zero
+    B[2::3, 3] = 0
+    inf, big = float("inf"), 3.0e38
+    A[0, 3], A[1, 7], A[2, 0], A[3, K - 1] = inf, -inf, float("nan"), big
+    A[4, 3], A[4, 9] = inf, -inf
+    B[5, 7], B[6, 1] = inf, float("nan")
+    C = torch.zeros((M, N), device="cuda")
+    gemm("fp32", 2, A, B, STORE, C, tile)
+    want = (A.double().cpu() @ B.double().cpu().T)
+    want = torch.where(want.abs() > 3.4028235e38, torch.sign(want) * inf, want)
+    got = C.double().cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(torch.isinf(got), torch.isinf(want))
+    assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)])
+    ok = torch.isfinite(want)
+    scale = A.double().abs().nan_to_num(0, 0, 0).cpu() @ B.double().abs().nan_to_num(0, 0, 0).cpu().T
+    assert bool(((got - want)[ok].abs() <= 2.0 ** -22 * scale[ok]).all())
+
+
 @pytest.mark.parametrize("dtype,M,n,kind,tile", [
     ("bf16", 64384, 5632, GEGLU, 0), ("bf16", 2012, 5632, GEGLU, 1), ("bf16", 8048, 1024, RESID, 2),
     ("bf16", 2012, 3072, STORE, 3), ("bf16", 2012, 1024, RESID, 4), ("fp32", 2012, 3072, STORE, 0),
