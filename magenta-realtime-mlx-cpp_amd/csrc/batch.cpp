@@ -129,7 +129,7 @@ void Batch::temporal_stack(int f, const int* fptr) {
     char *tk = ring(tkv_, i, 0, F), *tv = ring(tkv_, i, 1, F);
     // layer 0's input is the frame mean (no row partials): a plain norm pass
     if (i == 0) {
-      rmsnorm_rows_frag(dt, t_in_, G.norm_sa, 1e-6f, R, D, xn_, stream);
+      rmsnorm_rows(dt, t_in_, G.norm_sa, 1e-6f, R, D, xn_, stream, true);
       bgemm_qkv(dt, xn_, R, D, W.wqkv, HD, q_, tk, tv, H, F, f, fptr, stream);
     } else {
       bgemm_qkv(dt, xf_, R, D, W.wqkv, HD, q_, tk, tv, H, F, f, fptr, stream, norm(G.norm_sa));
@@ -161,7 +161,7 @@ void Batch::depth_stack(void* x, int l, bool x_partials, bool qkv_fed) {
     if (i == 0 && qkv_fed) {
       // nothing to compute: q / k / v are in place
     } else if (i == 0 && !x_partials) {
-      rmsnorm_rows_frag(dt, x, G.norm_sa, 1e-6f, R, D, xn_, stream);
+      rmsnorm_rows(dt, x, G.norm_sa, 1e-6f, R, D, xn_, stream, true);
       bgemm_qkv(dt, xn_, R, D, W.wqkv, HD, q_, dk, dv, H, L, l, nullptr, stream);
     } else {
       bgemm_qkv(dt, xf_, R, D, W.wqkv, HD, q_, dk, dv, H, L, l, nullptr, stream, norm(G.norm_sa));
@@ -205,7 +205,7 @@ void Batch::enqueue_frame(const GenOpts& o, int f, bool dynamic) {
     if (c.num_depth_layers > 0) {
       bgemm_f32(m.dt, xf_, R, D, dep_->head, head0, C, logits_, C, stream, norm(m.dec_norm));
     } else {
-      rmsnorm_rows_frag(m.dt, x, m.dec_norm, 1e-6f, R, D, xn_, stream);
+      rmsnorm_rows(m.dt, x, m.dec_norm, 1e-6f, R, D, xn_, stream, true);
       bgemm_f32(m.dt, xn_, R, D, dep_->head, head0, C, logits_, C, stream);
     }
     if (o.record_slices)

@@ -28,8 +28,6 @@ size_t frag_weights_elems(int N, int K);
 // The matrix in fragment order.  pairs: W is a packed wi_0 / wi_1 matrix (N = 2F
 // rows, bgemm_geglu).
 void frag_weights(DType dt, const void* W, int N, int K, bool pairs, void* out, hipStream_t s);
-// rmsnorm_rows (row-major in) with the result in fragment order, D <= 4096.
-void rmsnorm_rows_frag(DType dt, const void* x, const void* g, float eps, int M, int D, void* y, hipStream_t s);
 
 // RMSNorm (eps, weights g) of a GEMM's input rows applied between their load and
 // the products: X then holds the raw residual rows, whose sums of squares are

@@ -452,51 +452,6 @@ __global__ __launch_bounds__(64) void k_frag_weights(const T* __restrict__ W, in
   }
 }
 
-// rmsnorm_rows with the result in fragment order (K = D): one wave per row, a
-// lane's 16-byte chunks lane, lane + 64, ... (the wave norm's order of sums).
-constexpr int kFragNormChunks = 8;  // D <= 4096
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_rmsnorm_frag(const T* __restrict__ x, const T* __restrict__ g, float eps,
-                                                      int M, int D, T* __restrict__ y) {
-  using S = St<T>;
-  const int lane = threadIdx.x & 63, r = blockIdx.x * 4 + (threadIdx.x >> 6);  // wave-uniform
-  if (r >= M) return;
-  const int nch = D / 8;
-  uint4 v[kFragNormChunks], gv[kFragNormChunks];
-#pragma unroll
-  for (int i = 0; i < kFragNormChunks; ++i)
-    if (64 * i < nch) {  // uniform
-      const int c = min(lane + 64 * i, nch - 1);
-      v[i] = ld_g16(x + (size_t)r * D + c * 8);
-      gv[i] = ld_g16(g + c * 8);
-    }
-  float ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < kFragNormChunks; ++i)
-    if (lane + 64 * i < nch) {
-      const T* e = reinterpret_cast<const T*>(&v[i]);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const float f = S::ld(e[k]);
-        ss += f * f;
-      }
-    }
-  ss = wave_sum(ss);
-  const float inv = 1.0f / sqrtf(ss / (float)D + eps);
-#pragma unroll
-  for (int i = 0; i < kFragNormChunks; ++i)
-    if (lane + 64 * i < nch) {
-      const T* e = reinterpret_cast<const T*>(&v[i]);
-      const T* ge = reinterpret_cast<const T*>(&gv[i]);
-      uint4 o;
-      T* oe = reinterpret_cast<T*>(&o);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) oe[k] = S::st(S::rnd(S::ld(e[k]) * inv) * S::ld(ge[k]));
-      *reinterpret_cast<uint4*>(y + frag_index(r, (lane + 64 * i) * 8, D >> 5)) = o;
-    }
-}
-
 // Cross attention of one (row, head) over all S encoder keys (no bias, no
 // mask, scale 1.0: modules.cpp:243-295), one 256-thread block per pair.  A
 // wave reads 8 whole K (then V) rows per 16-byte load instruction: thread t
@@ -653,13 +608,6 @@ void frag_weights(DType dt, const void* W, int N, int K, bool pairs, void* out, 
     hipLaunchKernelGGL(k, dim3(tiles, K / 32), dim3(64), 0, s, static_cast<const T*>(W), N, K,
                        static_cast<T*>(out));
   });
-  MRT_HIP_CHECK(hipGetLastError());
-}
-
-void rmsnorm_rows_frag(DType dt, const void* x, const void* g, float eps, int M, int D, void* y, hipStream_t s) {
-  MRT_REQUIRE(D % 32 == 0 && D <= 512 * kFragNormChunks, "fragment norm: D must be a multiple of 32, at most 4096");
-  MRT_DTYPE16(dt, hipLaunchKernelGGL(k_rmsnorm_frag<T>, dim3((M + 3) / 4), dim3(256), 0, s, static_cast<const T*>(x),
-                                     static_cast<const T*>(g), eps, M, D, static_cast<T*>(y)));
   MRT_HIP_CHECK(hipGetLastError());
 }
 

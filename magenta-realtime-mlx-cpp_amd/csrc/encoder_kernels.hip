@@ -30,11 +30,18 @@ __global__ void k_encoder_embed(const T* __restrict__ emb, const T* __restrict__
     x[(size_t)r * D + d] = St<T>::st(St<T>::ld(e[d]) + St<T>::ld(p[d]));
 }
 
+// Where a norm leaves element d of row r: row-major, or in the fragment order of the
+// skinny GEMMs (batch.hpp; D % 32 == 0).
+template <bool FRAG>
+__device__ __forceinline__ size_t norm_index(int r, int d, int D) {
+  return FRAG ? frag_index(r, d, D >> 5) : (size_t)r * D + d;
+}
+
 // Rows of up to 256 * kNormPer elements: each thread keeps its elements in
 // registers between the sum of squares and the scaling (one read of x).
 constexpr int kNormPer = 8;
 
-template <typename T>
+template <typename T, bool FRAG>
 __global__ __launch_bounds__(256) void k_rmsnorm_rows_reg(const T* __restrict__ x, const T* __restrict__ g,
                                                           float eps, int D, T* __restrict__ y) {
   using S = St<T>;
@@ -56,14 +63,14 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows_reg(const T* __restrict__ 
 #pragma unroll
   for (int i = 0; i < kNormPer; ++i) {
     const int d = tid + 256 * i;
-    if (d < D) y[(size_t)r * D + d] = S::st(S::rnd(v[i] * inv) * S::ld(g[d]));
+    if (d < D) y[norm_index<FRAG>(r, d, D)] = S::st(S::rnd(v[i] * inv) * S::ld(g[d]));
   }
 }
 
 // One wave per row of D = 64 V NV elements (V per 16-byte chunk): a lane keeps
 // its NV chunks in registers between the sum of squares and the scaling, and
 // the row's sum is one wave reduction (no LDS, no barrier); four rows per block.
-template <typename T, int NV>
+template <typename T, int NV, bool FRAG>
 __global__ __launch_bounds__(256) void k_rmsnorm_rows_wave(const T* __restrict__ x, const T* __restrict__ g,
                                                            float eps, int M, int D, T* __restrict__ y) {
   using S = St<T>;
@@ -90,7 +97,6 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows_wave(const T* __restrict__
   }
   ss = wave_sum(ss);
   const float inv = 1.0f / sqrtf(ss / (float)D + eps);
-  uint4* yr = reinterpret_cast<uint4*>(y + (size_t)r * D);
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const T* e = reinterpret_cast<const T*>(&v[i]);
@@ -99,11 +105,11 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows_wave(const T* __restrict__
     T* oe = reinterpret_cast<T*>(&o);
 #pragma unroll
     for (int k = 0; k < V; ++k) oe[k] = S::st(S::rnd(S::ld(e[k]) * inv) * S::ld(ge[k]));
-    yr[lane + 64 * i] = o;
+    *reinterpret_cast<uint4*>(y + norm_index<FRAG>(r, (lane + 64 * i) * V, D)) = o;
   }
 }
 
-template <typename T>
+template <typename T, bool FRAG>
 __global__ __launch_bounds__(256) void k_rmsnorm_rows(const T* __restrict__ x, const T* __restrict__ g,
                                                       float eps, int D, T* __restrict__ y) {
   using S = St<T>;
@@ -120,7 +126,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows(const T* __restrict__ x, c
   __syncthreads();
   const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)D + eps);
   for (int d = tid; d < D; d += 256)
-    y[(size_t)r * D + d] = S::st(S::rnd(S::ld(xr[d]) * inv) * S::ld(g[d]));
+    y[norm_index<FRAG>(r, d, D)] = S::st(S::rnd(S::ld(xr[d]) * inv) * S::ld(g[d]));
 }
 
 // ---- GEMM epilogue ----------------------------------------------------------------
@@ -765,7 +771,7 @@ namespace {
 
 // The wave-per-row norm for rows of 64 V NV elements (NV <= 4) on 16-byte
 // aligned pointers; false when the shape or alignment does not fit.
-template <typename T>
+template <typename T, bool FRAG>
 bool rmsnorm_rows_wave(const T* x, const T* g, float eps, int M, int D, T* y, hipStream_t s) {
   constexpr int W = 64 * St<T>::kVec;
   const bool aligned = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(g) |
@@ -773,28 +779,36 @@ bool rmsnorm_rows_wave(const T* x, const T* g, float eps, int M, int D, T* y, hi
   if (!aligned || D % W != 0 || D / W < 1 || D / W > 4) return false;
   const dim3 grid((M + 3) / 4), block(256);
   switch (D / W) {
-    case 1: hipLaunchKernelGGL((k_rmsnorm_rows_wave<T, 1>), grid, block, 0, s, x, g, eps, M, D, y); break;
-    case 2: hipLaunchKernelGGL((k_rmsnorm_rows_wave<T, 2>), grid, block, 0, s, x, g, eps, M, D, y); break;
-    case 3: hipLaunchKernelGGL((k_rmsnorm_rows_wave<T, 3>), grid, block, 0, s, x, g, eps, M, D, y); break;
-    default: hipLaunchKernelGGL((k_rmsnorm_rows_wave<T, 4>), grid, block, 0, s, x, g, eps, M, D, y); break;
+    case 1: hipLaunchKernelGGL((k_rmsnorm_rows_wave<T, 1, FRAG>), grid, block, 0, s, x, g, eps, M, D, y); break;
+    case 2: hipLaunchKernelGGL((k_rmsnorm_rows_wave<T, 2, FRAG>), grid, block, 0, s, x, g, eps, M, D, y); break;
+    case 3: hipLaunchKernelGGL((k_rmsnorm_rows_wave<T, 3, FRAG>), grid, block, 0, s, x, g, eps, M, D, y); break;
+    default: hipLaunchKernelGGL((k_rmsnorm_rows_wave<T, 4, FRAG>), grid, block, 0, s, x, g, eps, M, D, y); break;
   }
   return true;
 }
 
+template <typename T, bool FRAG>
+void rmsnorm_rows_t(const void* xv, const void* gv, float eps, int M, int D, void* yv, hipStream_t s) {
+  const T *x = static_cast<const T*>(xv), *g = static_cast<const T*>(gv);
+  T* y = static_cast<T*>(yv);
+  if (rmsnorm_rows_wave<T, FRAG>(x, g, eps, M, D, y, s)) return;
+  hipLaunchKernelGGL((D <= 256 * kNormPer ? k_rmsnorm_rows_reg<T, FRAG> : k_rmsnorm_rows<T, FRAG>), dim3(M), dim3(256),
+                     0, s, x, g, eps, D, y);
+}
+
 }  // namespace
 
-void rmsnorm_rows(DType dt, const void* x, const void* g, float eps, int M, int D, void* y,
-                  hipStream_t s) {
-  bool done = false;
-  MRT_DTYPE_DISPATCH(dt, done = rmsnorm_rows_wave<T>(static_cast<const T*>(x), static_cast<const T*>(g), eps, M, D,
-                                                      static_cast<T*>(y), s));
-  if (done) {
-    MRT_HIP_CHECK(hipGetLastError());
-    return;
+void rmsnorm_rows(DType dt, const void* x, const void* g, float eps, int M, int D, void* y, hipStream_t s,
+                  bool frag_out) {
+  if (frag_out) {
+    MRT_REQUIRE(dt != DType::F32 && D % 32 == 0, "norm: fragments hold 16-bit rows of whole 32 columns");
+    if (dt == DType::BF16)
+      rmsnorm_rows_t<bf16, true>(x, g, eps, M, D, y, s);
+    else
+      rmsnorm_rows_t<f16, true>(x, g, eps, M, D, y, s);
+  } else {
+    MRT_DTYPE_DISPATCH(dt, (rmsnorm_rows_t<T, false>(x, g, eps, M, D, y, s)));
   }
-  const bool reg = D <= 256 * kNormPer;
-  MRT_DTYPE_DISPATCH(dt, hipLaunchKernelGGL(reg ? k_rmsnorm_rows_reg<T> : k_rmsnorm_rows<T>, dim3(M), dim3(256), 0,
-                                            s, (const T*)x, (const T*)g, eps, D, (T*)y));
   MRT_HIP_CHECK(hipGetLastError());
 }
 

@@ -147,9 +147,10 @@ void draw_levels(const float* logits, const SampleParams& p, int frame, int leve
 // x[r, :] = round(emb[tok[r]] + pe_T[r % S])    (model.cpp:231-236)
 void encoder_embed(DType dt, const void* emb, const void* pe, const int* tok, int M, int S,
                    int D, void* x, hipStream_t s);
-// y[r, :] = rmsnorm(x[r, :]) * g   (model dtype in and out)
+// y[r, :] = rmsnorm(x[r, :]) * g   (model dtype in and out); frag_out: y in the skinny
+// GEMMs' fragment order (batch.hpp)
 void rmsnorm_rows(DType dt, const void* x, const void* g, float eps, int M, int D, void* y,
-                  hipStream_t s);
+                  hipStream_t s, bool frag_out = false);
 
 // GEMM C[m, n] = sum_k A[m, k] * B[n, k]; A (M, K) and B (N, K) row-major.
 enum class GemmEpi : int {

@@ -799,17 +799,17 @@ void State::enqueue_decode_spec(const GenOpts& o) {
     spec_inputs(dt, t_out, m.emb, d_drafts_ + static_cast<size_t>(f) * L, L, D, sx_, stream);
     for (int i = 0; i < c.num_depth_layers; ++i) {
       const FragLayer& W = fw.layers[i];
-      rmsnorm_rows_frag(dt, sx_, m.dep[i].norm_sa, 1e-6f, R2, D, sxn_, stream);
+      rmsnorm_rows(dt, sx_, m.dep[i].norm_sa, 1e-6f, R2, D, sxn_, stream, true);
       bgemm_qkv_pos(dt, sxn_, R2, D, W.wqkv, HD, sq_, dk(i), dv(i), H, L, rows, stream);
       self_attn_at(dt, R2, sq_, dk(i), dv(i), H, L, 0, 0, nullptr, m.dbias, m.dbuckets, satt_, stream, rows, nullptr,
                    true);
       bgemm_resid(dt, satt_, R2, HD, W.wo, D, sx_, sxf_, sssq_, stream);
-      rmsnorm_rows_frag(dt, sx_, m.dep[i].norm_ff, 1e-6f, R2, D, sxn_, stream);
+      rmsnorm_rows(dt, sx_, m.dep[i].norm_ff, 1e-6f, R2, D, sxn_, stream, true);
       bgemm_geglu(dt, sxn_, R2, D, W.w01, FF, sffh_, stream);
       bgemm_resid(dt, sffh_, R2, FF, W.wo2, D, sx_, sxf_, sssq_, stream);
     }
     // level i's 1024-row head slice for rows 2i, 2i + 1
-    rmsnorm_rows_frag(dt, sx_, m.dec_norm, 1e-6f, R2, D, sxn_, stream);
+    rmsnorm_rows(dt, sx_, m.dec_norm, 1e-6f, R2, D, sxn_, stream, true);
     bgemm_f32(dt, sxn_, rows, D, fw.head, o.codec_offset, C, slog_, C, stream, {}, L, C);
     draw_levels(slog_, sp_all, f, L, sdrawn_, stream);
     int* decided = sdecided_ + f;
@@ -1061,7 +1061,7 @@ void State::depth_forward_full(const void* emb, int k, const void* bias, bool ca
     auto norm = [&](const void* g) { return BNorm{g, sssq_, 1e-6f}; };
     for (int i = 0; i < c.num_depth_layers; ++i) {
       const FragLayer& W = fw.layers[i];
-      if (i == 0) rmsnorm_rows_frag(dt, sx_, m.dep[i].norm_sa, 1e-6f, M, D, sxn_, stream);
+      if (i == 0) rmsnorm_rows(dt, sx_, m.dep[i].norm_sa, 1e-6f, M, D, sxn_, stream, true);
       bgemm_store(dt, i == 0 ? sxn_ : sxf_, M, D, W.wqkv, 3 * HD, sqkv_, 3 * HD, stream, i == 0 ? BNorm{} : norm(m.dep[i].norm_sa));
       full_attn(dt, rows, k, H, sqkv_, bias, m.dbias, m.dbuckets, causal, satt_, stream, true);
       bgemm_resid(dt, satt_, M, HD, W.wo, D, sx_, sxf_, sssq_, stream);
@@ -1069,7 +1069,7 @@ void State::depth_forward_full(const void* emb, int k, const void* bias, bool ca
       bgemm_resid(dt, sffh_, M, FF, W.wo2, D, sx_, sxf_, sssq_, stream);
     }
     // the head's many blocks would each normalise all rows: one pass instead
-    rmsnorm_rows_frag(dt, sx_, m.dec_norm, 1e-6f, M, D, sxn_, stream);
+    rmsnorm_rows(dt, sx_, m.dec_norm, 1e-6f, M, D, sxn_, stream, true);
     bgemm_f32(dt, sxn_, M, D, fw.head, 0, c.vocab_size, logits, c.vocab_size, stream);
     MRT_HIP_CHECK(hipStreamSynchronize(stream));
     return;

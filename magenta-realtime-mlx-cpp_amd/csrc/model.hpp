@@ -165,8 +165,7 @@ class Model {
   const SplitWeights* split_weights(hipStream_t s);
   bool split_shapes() const;
   bool frag_shapes() const {
-    return dt != DType::F32 && cfg.d_model % 32 == 0 && cfg.d_model <= 4096 && cfg.hd() % 32 == 0 &&
-           cfg.d_ff % 32 == 0;
+    return dt != DType::F32 && cfg.d_model % 32 == 0 && cfg.hd() % 32 == 0 && cfg.d_ff % 32 == 0;
   }
   static constexpr int kQkvChunkRows = 2048;
 
