@@ -523,6 +523,7 @@ __global__ __launch_bounds__(64) void k_enc_attn(const T* __restrict__ qkv, int 
       Ks[r][lane] = St_::ld(row[HD + lane]);
       Vs[r][lane] = St_::ld(row[2 * HD + lane]);
     }
+    for (int r = nk; r < 64; ++r) Vs[r][lane] = 0.f;  // met by zero weights: LDS may hold NaN
     __syncthreads();
     float sc[64];
     float mt = -INFINITY;
