@@ -7,9 +7,12 @@
 namespace mrt {
 namespace {
 
+// W may be a caller's tensor, aligned to its element only (global loads of 16 bytes
+// need no more).
 __global__ __launch_bounds__(256) void k_split_rows(const float* __restrict__ W, size_t n4, bf16* __restrict__ out) {
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) {
-    const float4 v = reinterpret_cast<const float4*>(W)[i];
+    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+    const f4 v = reinterpret_cast<const f4*>(W)[i];
     const size_t e = 4 * i;  // rows are whole groups, so groups run through the matrix
     store_split4(out, (e >> 5) * kSplitGroup + (e & 31), {v.x, v.y, v.z, v.w});
   }

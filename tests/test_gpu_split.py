@@ -20,6 +20,28 @@ def rel(a, b):
     return float(np.linalg.norm(np.asarray(a, np.float64) - b) / np.linalg.norm(np.asarray(b, np.float64)))
 
 
+def test_encoder_output_of_any_alignment(gpu_available):
+    """An fp32 encoder output that the caller passes may start at any float."""
+    import mrt_df
+    import synth_bundle
+    import torch
+    cfg = mrt_df.Config.tiny(8)
+    m = mrt_df.Depthformer(synth_bundle.make_weights(cfg, seed=3, norm_jitter=0.1), cfg, dtype="fp32")
+    st = m.new_state(max_frames=1, enc_len=33)
+    n = 2 * 33 * cfg.d_model
+    flat = torch.randn(n + 4, device="cuda")
+    x = torch.randn((2, cfg.d_model), device="cuda")
+    outs = []
+    for off in range(4):
+        enc = flat[off:off + n]
+        enc.copy_(torch.arange(n, device="cuda") % 97 / 97.0 - 0.5)
+        st.reset_cache("temporal")
+        outs.append(st.temporal_step(x, 0, enc_out=enc.view(2, 33, cfg.d_model)).cpu())
+        assert torch.equal(outs[-1], outs[0]), off
+    st.close()
+    m.close()
+
+
 @pytest.mark.parametrize("ffn_scale", [1.0, 2.0 ** 40])
 @pytest.mark.parametrize("S", [1, 33, 63, 64, 65, 127, 129, 200])
 def test_encode_edges(gpu_available, S, ffn_scale):
