@@ -821,8 +821,8 @@ struct GemmTile {
   int bm, bn;
   double f;
 };
-constexpr GemmTile kTiles16[] = {{256, 256, 1.0}, {192, 256, 1.05}, {128, 256, 1.05}, {128, 192, 1.25}, {64, 128, 1.5}};
-constexpr GemmTile kTiles32[] = {{128, 192, 1.0}, {128, 128, 1.0}, {64, 128, 1.15}};
+constexpr GemmTile kTiles16[] = {{256, 256, 1.0}, {192, 256, 1.03}, {128, 256, 1.14}, {128, 192, 1.24}, {64, 128, 2.0}};
+constexpr GemmTile kTiles32[] = {{128, 192, 1.0}, {128, 128, 1.06}, {64, 128, 1.22}};
 
 bool gemm_pairs(GemmEpi kind) { return kind == GemmEpi::Geglu || kind == GemmEpi::GegluSplit; }
 
@@ -830,10 +830,12 @@ bool gemm_pairs(GemmEpi kind) { return kind == GemmEpi::Geglu || kind == GemmEpi
 bool tile_takes(const GemmTile& t, int N, GemmEpi kind) { return N % t.bn == 0 && !(gemm_pairs(kind) && t.bn == 192); }
 
 // The tile whose rounds over the CUs (one block each) take the least time: rounds x
-// area x the tile's time per area relative to 256 x 256.  The factors are measured
-// times a round of the 16-bit kernel, K = 1,024: 256 x 256 30.7 us; 192 x 256 24.2
-// and 128 x 256 15.9 (1.05); 128 x 192 14.3 (1.25); 64 x 128 5.7 (1.5; its fragment
-// reads and its epilogue weigh more).
+// area x the tile's time per area.  The factors are measured: three rounds on 256
+// CUs, operands from memory, us, 16 bit at K = 1,024 and 2,816: 256 x 256 106 and 248;
+// 192 x 256 84.3 and 193; 128 x 256 61.9 and 142; 128 x 192 49.4 and 115; 64 x 128
+// 27.2 and 60.8 (its fragment reads and its epilogue weigh more); fp32: 128 x 192 190
+// and 507; 128 x 128 137 and 353; 64 x 128 80.7 and 196.  The residual and gated
+// epilogues leave the ratios as they are within 6 %.
 template <int n>
 int best_tile(const GemmTile (&tiles)[n], int M, int N, GemmEpi kind) {
   const long cus = std::max(8, device_cus() & ~7);
