@@ -385,7 +385,7 @@ __device__ __forceinline__ void mfma_epilogue(const GemmOut<T>& out, const f32x1
 // multiplies start while the stores drain (vmcnt counts in order: the first wait
 // of a tile leaves the previous tile's stores outstanding).  With one tile per block
 // the epilogue and the refill cost 7 of 33 us at 256 x 256 x 1,024: 731 us against
-// 666 us at 64,384 x 5,632 x 1,024 (1,115 TFLOP/s).  Rows past M read row M - 1 (not
+// 666 us at 64,384 x 5,632 x 1,024 (1,115 TFLOP/s; operands in cache).  Rows past M read row M - 1 (not
 // stored); N % BN == 0.
 template <class Core, typename T, int BM, int BN, int WM, int WN, int S>
 __global__ __launch_bounds__(64 * WM * WN) void k_gemm_ring(const void* __restrict__ A, const void* __restrict__ B,

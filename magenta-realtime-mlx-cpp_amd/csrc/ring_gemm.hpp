@@ -4,8 +4,8 @@
 // A wave keeps two fragment sets: the fragments of a 16-deep step are read from
 // LDS between the products of the step before it, also across the barrier to the
 // next k-tile, so LDS reads and matrix instructions of one wave overlap (all
-// reads of a k-tile ahead of its products: 830 TFLOP/s at 64,384 x 5,632 x 1,024,
-// two 192 x 128 blocks a CU).  The products are taken as B A^T, so a lane's
+// reads of a k-tile ahead of its products: 818 us, 908 TFLOP/s, at 64,384 x 5,632 x
+// 1,024 in cache, two 192 x 128 blocks a CU; this loop 666 us).  The products are taken as B A^T, so a lane's
 // accumulators lie along one output row and the epilogue stores 16 bytes a lane.
 #pragma once
 
