@@ -460,7 +460,8 @@ int mrt_probe_pingpong(int device, int peer, int rounds, float* us_one_way) {
 
 // Not part of the interface (mrt_df.h): one GEMM of the encoder on device buffers, for
 // tests of single kernels.  path 0: as gemm() picks, 1: vector ALUs, 2: fp32 operands
-// split first (gemm_split).  tile: -1 the rule's; *taken: the tile of a matrix-core
+// split first (gemm_split), 3: 16-bit rows laid out first (bgemm_seq_*; gated GELU leaves
+// C in fragment order).  tile: -1 the rule's; *taken: the tile of a matrix-core
 // GEMM of this shape by the rule.
 int mrt_test_gemm(int dtype, int path, const void* A, const void* B, int M, int N, int K, int kind, int tile, int nb,
                   int H, int S, int HD, void* C, int* taken) {
@@ -476,7 +477,7 @@ int mrt_test_gemm(int dtype, int path, const void* A, const void* B, int M, int 
     e.tile = tile;
     const auto dt = static_cast<mrt::DType>(dtype);
     *taken = N % 128 == 0 ? mrt::gemm_tile(dt, M, N, e.kind) : -1;
-    if (path == 2) {
+    if (path == 2 || path == 3) {
       mrt::bf16* sp[2] = {nullptr, nullptr};
       auto free_all = [&] {
         (void)hipDeviceSynchronize();
@@ -485,11 +486,25 @@ int mrt_test_gemm(int dtype, int path, const void* A, const void* B, int M, int 
       try {
         const void* src[2] = {A, B};
         const int rows[2] = {M, N};
+        const bool pairs = e.kind == mrt::GemmEpi::Geglu;
         for (int i = 0; i < 2; ++i) {
-          MRT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&sp[i]), static_cast<size_t>(rows[i]) * K * 6));
-          mrt::split_rows(static_cast<const float*>(src[i]), rows[i], K, sp[i], nullptr);
+          const size_t bytes = path == 2 ? static_cast<size_t>(rows[i]) * K * 6 : mrt::frag_weights_elems(rows[i], K) * 2;
+          MRT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&sp[i]), bytes));
+          if (path == 2)
+            mrt::split_rows(static_cast<const float*>(src[i]), rows[i], K, sp[i], nullptr);
+          else
+            mrt::frag_weights(dt, src[i], rows[i], K, i == 1 && pairs, sp[i], nullptr);
         }
-        mrt::gemm_split(sp[0], sp[1], M, N, K, e, nullptr);
+        if (path == 2)
+          mrt::gemm_split(sp[0], sp[1], M, N, K, e, nullptr);
+        else if (pairs)
+          mrt::bgemm_seq_geglu(dt, sp[0], M, K, sp[1], N / 2, C, nullptr);
+        else if (e.kind == mrt::GemmEpi::Resid)
+          mrt::bgemm_seq_resid(dt, sp[0], M, K, sp[1], N, C, nullptr);
+        else if (e.kind == mrt::GemmEpi::StoreF32)
+          mrt::bgemm_seq_f32(dt, sp[0], M, K, sp[1], N, static_cast<float*>(C), nullptr);
+        else
+          mrt::bgemm_seq_store(dt, sp[0], M, K, sp[1], N, C, nullptr);
       } catch (...) {
         free_all();
         throw;

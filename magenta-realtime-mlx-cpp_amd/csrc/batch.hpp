@@ -67,6 +67,14 @@ void bgemm_qkv_pos(DType dt, const void* X, int M, int K, const void* W, int HD,
 void bgemm_geglu(DType dt, const void* X, int M, int K, const void* W01, int F, void* Hout, hipStream_t s,
                  const BNorm& norm = {});
 
+// The same products with every output summed over k in order, bit for bit as gemm()
+// sums them (any M): row-major Y (M, N), fp32 logits, R += X . W^T, and gated GELU
+// in fragment order.
+void bgemm_seq_store(DType dt, const void* X, int M, int K, const void* W, int N, void* Y, hipStream_t s);
+void bgemm_seq_f32(DType dt, const void* X, int M, int K, const void* W, int N, float* Y, hipStream_t s);
+void bgemm_seq_resid(DType dt, const void* X, int M, int K, const void* W, int N, void* R, hipStream_t s);
+void bgemm_seq_geglu(DType dt, const void* X, int M, int K, const void* W01, int F, void* Hout, hipStream_t s);
+
 // Cross attention (no bias, no mask, scale 1) of every (row, head) over S <=
 // 1024 encoder keys, caches laid out (rows, H, S, 64); out (rows, H * 64) in
 // fragment order.

@@ -438,6 +438,106 @@ void launch_bgemm(const void* X, int M, int K, const void* W, int nout, const Ep
                               BNormDev<T>{nullptr, nullptr, 0, 0.f});
 }
 
+// The same product with every output's sum taken over k in order in one accumulator,
+// as the encoder's GEMM takes it (a chain of 16x16x32 instructions gives bit for bit
+// what its 32x32x16 chain gives), for the full-sequence depth pass: its logits do not
+// depend on which GEMM ran.  A block is one wave: NW weight tiles (the P parts of an
+// output tile, or column tiles) against one row tile.  The chain is short (0.5 us at
+// K = 1,024); what bounds it is the operands' round trip, so a wave keeps two runs of
+// kSeqRun k-steps requested, all of K = 1,024.
+constexpr int kSeqRun = 16;
+
+template <typename T>
+struct SResid {
+  T* r;
+  int ldr;
+  static constexpr bool kPre = true;
+  __device__ float pre(int m, int n) const { return St<T>::ld(r[(size_t)m * ldr + n]); }
+  __device__ void operator()(int m, int n, const float (&v)[1], float x) const {
+    r[(size_t)m * ldr + n] = St<T>::st(x + St<T>::rnd(v[0]));
+  }
+};
+
+template <typename T, int P, int NW, class Epi>
+__global__ __launch_bounds__(64) void k_bgemm_seq(const T* __restrict__ X, int M, int K, const T* __restrict__ W,
+                                                  int nout, Epi epi) {
+  static_assert(P == 1 || NW == P, "gate / up pairs: one column tile a block");
+  constexpr int C = NW / P;
+  const int lane = threadIdx.x, c16 = lane & 15, kg = lane >> 4, nks = K / 32;
+  // eight columns of blocks, then the same eight for the next row tile: blocks of one
+  // column run together on one XCD (blocks are dealt to the 8 XCDs in turn)
+  const int mt = (M + 15) / 16, id = blockIdx.x / 8;
+  const int tile = (id / mt * 8 + blockIdx.x % 8) * C, m0 = id % mt * 16;
+  if (tile * kBgCols >= nout) return;
+  const T* wt = W + (size_t)tile * nks * P * 512 + lane * 8;
+  const int r = min(m0 + c16, M - 1);
+  const T* xr = X + (size_t)(r >> 4) * nks * 512 + (kg * 16 + (r & 15)) * 8;
+  float pre[C][4];
+  if constexpr (HasPre<Epi>::value) {
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        pre[c][i] = epi.pre(min(m0 + 4 * kg + i, M - 1), min((tile + c) * kBgCols + c16, nout - 1));
+  }
+  uint4 a[2][kSeqRun], b[2][kSeqRun][NW];
+  auto load = [&](int d, int s0) {  // a step past the end re-reads the last one and is not multiplied
+#pragma unroll
+    for (int s = 0; s < kSeqRun; ++s) {
+      const int ks = min(s0 + s, nks - 1);
+#pragma unroll
+      for (int w = 0; w < NW; ++w) b[d][s][w] = ld_g16(wt + (size_t)(P == 1 ? w * nks + ks : ks * P + w) * 512);
+      a[d][s] = ld_g16(xr + (size_t)ks * 512);
+    }
+  };
+  f32x4_t acc[NW];
+#pragma unroll
+  for (int w = 0; w < NW; ++w) acc[w] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto run = [&](int d, int s0) {
+#pragma unroll
+    for (int s = 0; s < kSeqRun; ++s)
+      if (s0 + s < nks) {  // uniform: a branch, matrix instructions ignore the lane mask
+#pragma unroll
+        for (int w = 0; w < NW; ++w) acc[w] = Mfma16<T>::mma(a[d][s], b[d][s][w], acc[w]);
+      }
+    if (s0 + 2 * kSeqRun < nks) load(d, s0 + 2 * kSeqRun);
+  };
+  load(0, 0);
+  if (kSeqRun < nks) load(1, kSeqRun);
+  for (int s0 = 0; s0 < nks; s0 += 2 * kSeqRun) {
+    run(0, s0);
+    if (s0 + kSeqRun < nks) run(1, s0 + kSeqRun);
+  }
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = m0 + 4 * kg + i, n = (tile + c) * kBgCols + c16;
+      if (m >= M || n >= nout) continue;
+      float v[P];
+#pragma unroll
+      for (int p = 0; p < P; ++p) v[p] = acc[c * P + p][i];
+      if constexpr (HasPre<Epi>::value)
+        epi(m, n, v, pre[c][i]);
+      else
+        epi(m, n, v);
+    }
+}
+
+// Two column tiles a wave where that still leaves several waves a CU (the head): half
+// the reads of X.
+template <typename T, int P, class Epi>
+void launch_bgemm_seq(const void* X, int M, int K, const void* W, int nout, const Epi& epi, hipStream_t s) {
+  MRT_REQUIRE(M >= 1 && K % 32 == 0 && K >= 32 && nout >= 1, "sequential GEMM: K must be a multiple of 32");
+  const int tiles = (nout + kBgCols - 1) / kBgCols, mt = (M + 15) / 16;
+  const T *x = static_cast<const T*>(X), *w = static_cast<const T*>(W);
+  if (P == 1 && tiles * mt >= 1024)
+    hipLaunchKernelGGL((k_bgemm_seq<T, P, 2, Epi>), dim3((tiles + 15) / 16 * 8 * mt), dim3(64), 0, s, x, M, K, w, nout, epi);
+  else
+    hipLaunchKernelGGL((k_bgemm_seq<T, P, P, Epi>), dim3((tiles + 7) / 8 * 8 * mt), dim3(64), 0, s, x, M, K, w, nout, epi);
+  MRT_HIP_CHECK(hipGetLastError());
+}
+
 // Weights (N, K) -> fragment order.  Block (tile, ks): 16 rows x 32 columns a
 // part; P = 2: the gate and up rows of 16 outputs of a packed matrix.  Rows past
 // N are zero.
@@ -649,6 +749,23 @@ void bgemm_geglu(DType dt, const void* X, int M, int K, const void* W01, int F, 
                  const BNorm& norm) {
   MRT_REQUIRE(F % 32 == 0, "batched GEMM: d_ff must be a multiple of 32 (packed gate/up groups)");
   MRT_DTYPE16(dt, (launch_bgemm<T, 2>(X, M, K, W01, F, BGeglu<T>{static_cast<T*>(Hout), F}, s, norm)));
+}
+
+void bgemm_seq_store(DType dt, const void* X, int M, int K, const void* W, int N, void* Y, hipStream_t s) {
+  MRT_DTYPE16(dt, (launch_bgemm_seq<T, 1>(X, M, K, W, N, BStore<T>{static_cast<T*>(Y), N}, s)));
+}
+
+void bgemm_seq_f32(DType dt, const void* X, int M, int K, const void* W, int N, float* Y, hipStream_t s) {
+  MRT_DTYPE16(dt, (launch_bgemm_seq<T, 1>(X, M, K, W, N, BF32<T>{Y, N}, s)));
+}
+
+void bgemm_seq_resid(DType dt, const void* X, int M, int K, const void* W, int N, void* R, hipStream_t s) {
+  MRT_DTYPE16(dt, (launch_bgemm_seq<T, 1>(X, M, K, W, N, SResid<T>{static_cast<T*>(R), N}, s)));
+}
+
+void bgemm_seq_geglu(DType dt, const void* X, int M, int K, const void* W01, int F, void* Hout, hipStream_t s) {
+  MRT_REQUIRE(F % 32 == 0, "sequential GEMM: d_ff must be a multiple of 32 (packed gate/up groups)");
+  MRT_DTYPE16(dt, (launch_bgemm_seq<T, 2>(X, M, K, W01, F, BGeglu<T>{static_cast<T*>(Hout), F}, s)));
 }
 
 }  // namespace mrt

@@ -1052,25 +1052,23 @@ void State::depth_forward_full(const void* emb, int k, const void* bias, bool ca
   const int D = c.d_model, HD = c.hd(), FF = c.d_ff, H = c.num_heads, M = rows * k;
   MRT_HIP_CHECK(hipSetDevice(m.device));
   copy(sx_, emb, static_cast<size_t>(M) * D * esz());
-  // 16-bit rows that the skinny GEMMs hold: M <= 32 fills no tile of the
-  // encoder's GEMM (its 1,024-wide outputs ran 8 blocks, 16 us each; 292 us a
-  // call in all at k = 16, 135 us here)
-  const FragDepth* fd = m.frag_shapes() && M <= kBatchRows && c.num_depth_layers > 0 ? m.frag_depth(stream) : nullptr;
+  // 16-bit rows: the path below on the skinny GEMMs, with the same sums (M <= 64 fills
+  // no tile of the encoder's GEMM: its 1,024-wide outputs ran 8 blocks, 16 us each;
+  // 292 us a call in all at k = 16, 152 us here)
+  const FragDepth* fd = m.frag_shapes() && M <= kBatchRows ? m.frag_depth(stream) : nullptr;
   if (fd != nullptr) {
-    const FragDepth& fw = *fd;
-    auto norm = [&](const void* g) { return BNorm{g, sssq_, 1e-6f}; };
     for (int i = 0; i < c.num_depth_layers; ++i) {
-      const FragLayer& W = fw.layers[i];
-      if (i == 0) rmsnorm_rows(dt, sx_, m.dep[i].norm_sa, 1e-6f, M, D, sxn_, stream, true);
-      bgemm_store(dt, i == 0 ? sxn_ : sxf_, M, D, W.wqkv, 3 * HD, sqkv_, 3 * HD, stream, i == 0 ? BNorm{} : norm(m.dep[i].norm_sa));
+      const FragLayer& W = fd->layers[i];
+      rmsnorm_rows(dt, sx_, m.dep[i].norm_sa, 1e-6f, M, D, sxn_, stream, true);
+      bgemm_seq_store(dt, sxn_, M, D, W.wqkv, 3 * HD, sqkv_, stream);
       full_attn(dt, rows, k, H, sqkv_, bias, m.dbias, m.dbuckets, causal, satt_, stream, true);
-      bgemm_resid(dt, satt_, M, HD, W.wo, D, sx_, sxf_, sssq_, stream);
-      bgemm_geglu(dt, sxf_, M, D, W.w01, FF, sffh_, stream, norm(m.dep[i].norm_ff));
-      bgemm_resid(dt, sffh_, M, FF, W.wo2, D, sx_, sxf_, sssq_, stream);
+      bgemm_seq_resid(dt, satt_, M, HD, W.wo, D, sx_, stream);
+      rmsnorm_rows(dt, sx_, m.dep[i].norm_ff, 1e-6f, M, D, sxn_, stream, true);
+      bgemm_seq_geglu(dt, sxn_, M, D, W.w01, FF, sffh_, stream);
+      bgemm_seq_resid(dt, sffh_, M, FF, W.wo2, D, sx_, stream);
     }
-    // the head's many blocks would each normalise all rows: one pass instead
     rmsnorm_rows(dt, sx_, m.dec_norm, 1e-6f, M, D, sxn_, stream, true);
-    bgemm_f32(dt, sxn_, M, D, fw.head, 0, c.vocab_size, logits, c.vocab_size, stream);
+    bgemm_seq_f32(dt, sxn_, M, D, fd->head, c.vocab_size, logits, stream);
     MRT_HIP_CHECK(hipStreamSynchronize(stream));
     return;
   }

@@ -170,6 +170,46 @@ def test_split_gemm_not_finite(gemm, M, K, tile):
     assert bool(((got - want)[ok].abs() <= 2.0 ** -22 * scale[ok]).all())
 
 
+@pytest.mark.parametrize("kind", [STORE, RESID, STORE_F32, GEGLU])
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+def test_sequential_skinny_gemm(gemm, dtype, kind):
+    """The skinny GEMM of the full-sequence depth pass sums every output as the encoder's
+    GEMM does: bit for bit, on random operands, at the edges of its 16-row tiles and of
+    its runs of 16 k-steps, and with two column tiles a wave (16,384 columns)."""
+    import torch
+    dt = gemm.dt[dtype]
+    g = torch.Generator(device="cuda").manual_seed(7)
+    for M, K, n in [(1, 64, 128), (15, 512, 384), (16, 576, 128), (17, 1024, 384), (32, 1088, 128), (33, 2816, 128),
+                    (64, 2112, 256), (17, 1088, 16384), (1, 64, 16384)]:
+        A = torch.randn((M, K), generator=g, device="cuda").to(dt)
+        B = (torch.randn((n, K), generator=g, device="cuda") / K ** 0.5).to(dt)
+        out = torch.float32 if kind == STORE_F32 else dt
+        cols = n // 2 if kind == GEGLU else n
+        want = torch.randn((M, cols), generator=g, device="cuda").to(out)
+        mp = -(-M // 16) * 16
+        C = torch.full((mp + 1, cols), 7, device="cuda", dtype=out)
+        if kind == RESID:
+            C[:M] = want
+        gemm(dtype, 0, A, B, kind, want)
+        gemm(dtype, 3, A, B, kind, C)
+        if kind == GEGLU:  # 16-row x 32-column tiles: (column group of 8, row, 8)
+            assert bool((C[mp:] == 7).all())
+            C = C[:mp].reshape(mp // 16, cols // 32, 4, 16, 8).permute(0, 3, 1, 2, 4).reshape(mp, cols)
+        assert torch.equal(C[:M], want), (M, K, n)
+        assert bool((C[M:] == 7).all())
+
+
+def test_sequential_skinny_gemm_odd_columns(gemm):
+    """A last column tile by itself, and one partly filled; exact sums."""
+    import torch
+    for n in (16400, 16390, 24):
+        A, B = operands("bf16", 33, 1088, n=n)
+        C = torch.full((35, n), 7, device="cuda", dtype=torch.float32)
+        gemm("bf16", 3, A.bfloat16(), B.bfloat16(), STORE_F32, C)
+        want = (A.double() @ B.double().T).float().bfloat16().float()
+        assert torch.equal(C[:33], want) and bool((C[33:] == 7).all()), n
+
+
 @pytest.mark.parametrize("dtype,M,n,kind,tile", [
     ("bf16", 64384, 5632, GEGLU, 0), ("bf16", 2012, 5632, GEGLU, 1), ("bf16", 8048, 1024, RESID, 2),
     ("bf16", 2012, 3072, STORE, 3), ("bf16", 2012, 1024, RESID, 4), ("fp32", 2012, 3072, STORE, 0),
