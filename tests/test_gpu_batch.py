@@ -304,7 +304,7 @@ def test_batch_full_size_32_streams(full):
 def test_batch_encoder_full_size(full, B):
     """Encoder prefill of B streams at the benchmark dims (2B x 1006 rows, each
     stream its own random context and style).  These are the shapes that take
-    the 256 x 256-tile GEMM (k_gemm_big: outputs <= 4096 wide with >= 512 tiles):
+    the GEMM's 256 x 256 tiles (test_gpu_gemm_tiles.py has the rule):
     the QKV projection (3072 wide) at 8 and 32 streams, and the O and FFN-down
     projections (1024 wide) at 32.  Every stream's rows must be bit-exact with a
     single-stream encode of the same tokens (smaller tiles, the same k order per
