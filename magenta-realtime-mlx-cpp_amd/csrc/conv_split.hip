@@ -190,7 +190,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void k_conv_split(ConvLaunch a)
     const int m = min(m0 + row, M - 1), img = m / gyx, r = m - img * gyx, y = r / gx, x = r - y * gx;
     const bf16* w = static_cast<const bf16*>(sub->w) + (size_t)(n0 + col) * nk_all * kSplitGroup;
     float sum = 0.f;
-    for (int t = 0; t < sub->ntaps; ++t, w += cpt * kSplitGroup) {
+    for (int t = 0; t < sub->ntaps && sum == sum; ++t, w += cpt * kSplitGroup) {
       const int iy = y + sub->dy[t], ix = x + sub->dx[t];
       const bool in = (unsigned)iy < (unsigned)a.hin && (unsigned)ix < (unsigned)a.win;
       sum = split_dot(in ? a.xs + ((size_t)(img * a.hin + iy) * a.win + ix) * (cpt * kSplitGroup) : a.zeros, w, cpt,

@@ -100,9 +100,9 @@ struct CoreSplitFine : CoreSplit {
 };
 
 // sum + the products of `groups` groups of two split rows, as fused multiply-adds of
-// the whole floats.
+// the whole floats; NaN as soon as the sum is.
 __device__ inline float split_dot(const bf16* a, const bf16* b, int groups, float sum) {
-  for (int g = 0; g < groups; ++g, a += kSplitGroup, b += kSplitGroup)
+  for (int g = 0; g < groups && sum == sum; ++g, a += kSplitGroup, b += kSplitGroup)
     for (int e = 0; e < 32; e += 8) {
       uint4 u[3], v[3];
 #pragma unroll
@@ -125,7 +125,8 @@ __device__ inline float split_dot(const bf16* a, const bf16* b, int groups, floa
 // An infinity times the other operand's small parts, zeros or of the other sign, is
 // NaN where the float product is infinite.  So sums that are not finite are taken
 // again as plain fp32 sums: sum_of(row, column of the tile).  A product and an add per
-// sum look for them; a tile that holds one costs as much as the vector ALUs take.
+// sum look for them; where there are some, those take the vector ALUs' time (51 codec
+// frames of nothing but NaN, whose sums end early: 43 ms against 2.7).
 template <class Tile, class F>
 __device__ __forceinline__ void resum_not_finite(typename Tile::State& s, F&& sum_of) {
   constexpr int kSums = Tile::MI * Tile::NJ * 16;
